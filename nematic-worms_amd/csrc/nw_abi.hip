@@ -535,7 +535,7 @@ void collideFilaments(float *force, float *sortedPos, float *sortedVel, float *s
     NW_HIP(launch_collide_filaments(reinterpret_cast<float4 *>(force), reinterpret_cast<const float4 *>(sortedPos),
                                     reinterpret_cast<const float4 *>(sortedVel),
                                     reinterpret_cast<const float4 *>(sortedTangent), gridParticleIndex, cellStart,
-                                    cellEnd, numParticles, numCells, kp, s.stream));
+                                    cellEnd, numParticles, kp, s.stream));
 }
 
 void collide(float *force, float *sortedPos, float *sortedVel, float *sortedTangent, uint *gridParticleIndex,

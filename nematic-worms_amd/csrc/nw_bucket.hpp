@@ -141,7 +141,7 @@ hipError_t launch_srd_cells(const BucketPlan &bp, BucketScratch &s, uint32_t *id
 hipError_t launch_srd_rotate(const uint32_t *hash, const float4 *com, const float *lam, float4 *pos, float4 *vel,
                              uint32_t NT, uint32_t N, float dt, float cosA, float sinA, int iso, const KP &kp,
                              hipStream_t st);
-// pair pass over CSR offsets; sortedCell may be NULL (cells recomputed from positions)
+// pair pass over CSR offsets and the cell of every sorted slot
 hipError_t launch_collide_off(float4 *force, const float4 *sPos, const float4 *sVel, const float4 *sTan,
                               const uint32_t *sIdx, const uint32_t *off, const uint32_t *sortedCell, uint32_t n,
                               const KP &kp, hipStream_t st);

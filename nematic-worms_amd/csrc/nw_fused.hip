@@ -8,28 +8,14 @@
 //                   cross-lane shuffles)
 //   cell sort       nw_bucket.hip (stable, atomic-free, gathers the records)
 //   k_collide_rows  pair forces, neighbour rows staged in LDS, one flattened
-//                   candidate list per bead (k_collide_csr without LDS for
-//                   stencils over several z layers)
+//                   candidate list per bead (stencils over several z layers:
+//                   nw_pairs.hip)
 // computing the per-call path's expressions in the same order, except that
 // pair terms are accumulated one by one rather than per cell.
 #include "nw_bucket.hpp"
-#include "nw_physics.hpp"
+#include "nw_pair.hpp"
 
 namespace nw {
-
-// cell coordinates of sorted bead i: from the sort's cell ids when given
-// (already wrapped into the grid), else from the position
-__device__ __forceinline__ void bead_cell(const KP &kp, const uint32_t *__restrict__ sCell, uint32_t i, f3 r, int &gx,
-                                          int &gy, int &gz) {
-    const SimParams &p = kp.p;
-    if (sCell) {
-        cell_xyz(kp, sCell[i], gx, gy, gz);
-    } else {
-        gx = wrap_mod(cell_coord(r.x, p.origin.x, p.cellSize.x), p.gridSize.x);
-        gy = wrap_mod(cell_coord(r.y, p.origin.y, p.cellSize.y), p.gridSize.y);
-        gz = wrap_mod(cell_coord(r.z, p.origin.z, p.cellSize.z), p.gridSize.z);
-    }
-}
 
 // ===========================================================================
 // MD front
@@ -173,53 +159,6 @@ __global__ __launch_bounds__(kBlock) void k_filament_tangents(const float4 *__re
 // leaves the term unchanged).  The global and the LDS kernel below follow this
 // order exactly and agree bit for bit.
 // ===========================================================================
-template <int MODE, bool TAN>
-struct Owner {
-    f3 r, v, t;
-    uint32_t fil, ch;
-};
-
-// one candidate's terms (collideParticles / bond / WCA, then the extensile
-// term), skipped for the bead itself and, in WCA mode, for its own worm
-template <int MODE, bool TAN, bool UNIT = false>
-__device__ __forceinline__ void add_pair(const KP &kp, const Owner<MODE, TAN> &o, float rc2, float w, f3 &acc,
-                                         f3 r2, uint32_t fil2, uint32_t ch2, f3 v2, f3 t2) {
-    const SimParams &p = kp.p;
-    const bool same = o.fil == fil2;
-    if (MODE == 0) {
-        if (same && ch2 == o.ch) return;
-        f3 t;
-        if (same && ((o.ch + 1u == ch2) || (o.ch - 1u == ch2)))
-            t = bond_hookean(p, o.r, r2, p.bondSpringK, p.bondSpringL);
-        else
-            t = dem_force(p, o.r, r2, o.v, v2);
-        acc += UNIT ? t : w * t;
-    } else {
-        if (same) return;
-        const f3 t = wca_force(p, kp.e, o.r, r2, rc2);
-        acc += UNIT ? t : w * t;
-    }
-    if (TAN && !same) {
-        const f3 t = extensile_force(p, o.r, r2, o.t, t2, p.activity);
-        acc += UNIT ? t : w * t;
-    }
-}
-
-// beadBase: the first bead id of the system (a replica's offset in the
-// batched step; worm and chain indices are the system's own)
-template <int MODE, bool TAN>
-__device__ __forceinline__ void add_run_global(const KP &kp, const Owner<MODE, TAN> &o, float rc2, float w, f3 &acc,
-                                               uint32_t a, uint32_t b, const float4 *__restrict__ sPos,
-                                               const float4 *__restrict__ sVel, const float4 *__restrict__ sTan,
-                                               const uint32_t *__restrict__ sIdx, uint32_t beadBase) {
-    for (uint32_t j = a; j < b; ++j) {
-        uint32_t fil2, ch2;
-        worm_of(kp, sIdx[j] - beadBase, fil2, ch2);
-        add_pair<MODE, TAN>(kp, o, rc2, w, acc, mk(sPos[j]), fil2, ch2, MODE == 0 ? mk(sVel[j]) : mk(0.f, 0.f, 0.f),
-                            TAN ? mk(sTan[j]) : mk(0.f, 0.f, 0.f));
-    }
-}
-
 // sorted-slot runs of the three x cells around cx in the row starting at
 // cell `base`: one run, or two across the x wrap (Gx >= 3)
 __device__ __forceinline__ void row_runs(const uint32_t *__restrict__ off, uint32_t base, int cx, uint32_t Gx,
@@ -309,60 +248,17 @@ __device__ __forceinline__ void add_layer_global(const KP &kp, const Owner<MODE,
 }
 
 // every candidate of the owner from global memory, in stencil order (off:
-// the CSR offsets of the system's cells, indexed by its own cell ids)
+// the CSR offsets of the system's cells, indexed by its own cell ids; a
+// stencil of one layer, gridSize.x >= 3)
 template <int MODE, bool TAN>
 __device__ __forceinline__ void add_all_global(const KP &kp, const Owner<MODE, TAN> &o, float rc2, f3 &acc, int gx,
                                                int gy, int gz, const uint32_t *__restrict__ off,
                                                const float4 *__restrict__ sPos, const float4 *__restrict__ sVel,
                                                const float4 *__restrict__ sTan, const uint32_t *__restrict__ sIdx,
                                                uint32_t beadBase = 0) {
-    const SimParams &p = kp.p;
-    const uint32_t Gx = p.gridSize.x;
-    const AxisCells ay = axis_cells_in(gy, p.gridSize.y, false);
-    const AxisCells az = axis_cells_in(gz, p.gridSize.z, kp.e.stencil == NW_STENCIL_2D);
-    if (az.n == 1 && Gx >= 3) {
-        add_layer_global<MODE, TAN>(kp, o, rc2, acc, gx, ay, uint32_t(az.c[0]), az.w[0], off, sPos, sVel, sTan, sIdx,
-                                    beadBase);
-        return;
-    }
-#pragma unroll
-    for (int zi = 0; zi < 3; ++zi) {
-        if (zi >= az.n) break;
-#pragma unroll
-        for (int yi = 0; yi < 3; ++yi) {
-            if (yi >= ay.n) break;
-            const float wzy = az.w[zi] * ay.w[yi];
-            const uint32_t base = (uint32_t(az.c[zi]) * p.gridSize.y + uint32_t(ay.c[yi])) * Gx;
-            if (Gx >= 3) {
-                uint32_t a0, a1, b0, b1;
-                row_runs(off, base, gx, Gx, a0, a1, b0, b1);
-                add_run_global<MODE, TAN>(kp, o, rc2, wzy, acc, a0, a1, sPos, sVel, sTan, sIdx, beadBase);
-                add_run_global<MODE, TAN>(kp, o, rc2, wzy, acc, b0, b1, sPos, sVel, sTan, sIdx, beadBase);
-            } else {
-                const AxisCells ax = axis_cells_in(gx, Gx, false);
-#pragma unroll
-                for (int xi = 0; xi < 3; ++xi) {
-                    if (xi >= ax.n) break;
-                    const uint32_t h = base + uint32_t(ax.c[xi]);
-                    add_run_global<MODE, TAN>(kp, o, rc2, wzy * ax.w[xi], acc, off[h], off[h + 1], sPos, sVel,
-                                              sTan, sIdx, beadBase);
-                }
-            }
-        }
-    }
-}
-
-template <int MODE, bool TAN>
-__device__ __forceinline__ Owner<MODE, TAN> load_owner(const KP &kp, uint32_t i, uint32_t me,
-                                                       const float4 *__restrict__ sPos,
-                                                       const float4 *__restrict__ sVel,
-                                                       const float4 *__restrict__ sTan) {
-    Owner<MODE, TAN> o;
-    o.r = mk(sPos[i]);
-    o.v = MODE == 0 ? mk(sVel[i]) : mk(0.f, 0.f, 0.f);
-    o.t = TAN ? mk(sTan[i]) : mk(0.f, 0.f, 0.f);
-    worm_of(kp, me, o.fil, o.ch);
-    return o;
+    const AxisCells ay = axis_cells_in(gy, kp.p.gridSize.y, false);
+    const float wz = kp.e.stencil == NW_STENCIL_2D ? 1.0f : axis_cells_in(gz, kp.p.gridSize.z, false).w[0];
+    add_layer_global<MODE, TAN>(kp, o, rc2, acc, gx, ay, uint32_t(gz), wz, off, sPos, sVel, sTan, sIdx, beadBase);
 }
 
 __device__ __forceinline__ void add_force(float4 *__restrict__ force, uint32_t me, f3 acc) {
@@ -382,7 +278,7 @@ __global__ __launch_bounds__(kBlock) void k_collide_csr(float4 *__restrict__ for
     const uint32_t me = sIdx[i];
     const Owner<MODE, TAN> o = load_owner<MODE, TAN>(kp, i, me, sPos, sVel, sTan);
     int gx, gy, gz;
-    bead_cell(kp, sCell, i, o.r, gx, gy, gz);
+    cell_xyz(kp, sCell[i], gx, gy, gz);
     f3 acc = mk(0.f, 0.f, 0.f);
     add_all_global<MODE, TAN>(kp, o, kp.e.wcaCutoff * kp.e.wcaCutoff, acc, gx, gy, gz, off, sPos, sVel, sTan, sIdx);
     add_force(force, me, acc);
@@ -834,8 +730,8 @@ hipError_t launch_collide_off(float4 *force, const float4 *sPos, const float4 *s
                               const KP &kp, hipStream_t st) {
     if (n == 0) return hipSuccess;
     const bool oneLayer = kp.e.stencil == NW_STENCIL_2D || kp.p.gridSize.z == 1;
-    const bool ldsOk = oneLayer && kp.p.gridSize.x >= 3 && sCell != nullptr;
-    const bool lds = ldsOk && kp.e.collideKernel != NW_COLLIDE_GLOBAL;
+    if (!oneLayer || kp.p.gridSize.x < 3) return launch_collide_layers(force, sPos, sVel, sTan, sIdx, off, sCell, n, kp, st);
+    const bool lds = kp.e.collideKernel != NW_COLLIDE_GLOBAL;
     const bool wca = kp.e.pairPotential == NW_PAIR_WCA;
     const bool tan = !wca || kp.p.activity != 0.0f;
     // sorted beads per LDS workgroup: 128, 256 or 512 (512 only for the WCA

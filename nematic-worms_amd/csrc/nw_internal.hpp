@@ -64,9 +64,6 @@ hipError_t launch_fill_u32(uint32_t *p, uint32_t value, uint64_t n, hipStream_t 
 hipError_t launch_reorder(uint32_t *cellStart, uint32_t *cellEnd, float4 *sPos, float4 *sVel, float4 *sTan,
                           const uint32_t *hash, const uint32_t *index, const float4 *pos, const float4 *vel,
                           const float4 *tan, uint32_t n, uint32_t numCells, hipStream_t st);
-hipError_t launch_collide_filaments(float4 *force, const float4 *sPos, const float4 *sVel, const float4 *sTan,
-                                    const uint32_t *sIdx, const uint32_t *cellStart, const uint32_t *cellEnd,
-                                    uint32_t n, uint32_t numCells, const KP &kp, hipStream_t st);
 hipError_t launch_filament_forces(float4 *force, float4 *tangent, const float4 *pos, uint32_t numFilaments,
                                   const KP &kp, hipStream_t st);
 hipError_t launch_langevin(float4 *force, const float4 *vel, float stddev, uint32_t n, uint64_t seed,
@@ -83,6 +80,16 @@ hipError_t launch_collide_solvent(const float4 *pos, float4 *vel, const float4 *
 hipError_t launch_reverse_filaments(float4 *force, float4 *forceOld, float4 *vel, float4 *pos,
                                     uint32_t numFilaments, uint64_t seed, uint64_t offset, const KP &kp,
                                     hipStream_t st);
+
+// ---- nw_pairs.hip ----
+// pair forces over the reference's cell tables
+hipError_t launch_collide_filaments(float4 *force, const float4 *sPos, const float4 *sVel, const float4 *sTan,
+                                    const uint32_t *sIdx, const uint32_t *cellStart, const uint32_t *cellEnd,
+                                    uint32_t n, const KP &kp, hipStream_t st);
+// and over CSR offsets (the fused steps' stencils of several layers)
+hipError_t launch_collide_layers(float4 *force, const float4 *sPos, const float4 *sVel, const float4 *sTan,
+                                 const uint32_t *sIdx, const uint32_t *off, const uint32_t *sCell, uint32_t n,
+                                 const KP &kp, hipStream_t st);
 
 // ---- nw_sort.hip ----
 // Scratch sized for n keys / `bins` bins is grown by the caller (ensure_sort_scratch).

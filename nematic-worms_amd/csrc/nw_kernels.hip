@@ -110,99 +110,6 @@ __global__ __launch_bounds__(kBlock) void k_reorder(uint32_t *__restrict__ cellS
 }
 
 // ===========================================================================
-// Pair forces (collideFilamentsKernel :694-744, collideCell :492-556,
-// collideParticles :427-462, bondHookean :466-473, extensileForce :477-487).
-//
-// The 27 reference offsets are folded per axis into distinct wrapped cells
-// with multiplicities (a grid one cell deep in z visits that layer 3 times
-// upstream: multiplicity 3).  A cell row y..z is scanned as one contiguous
-// run of the sorted arrays when its three x-cells are consecutive hashes.
-// ===========================================================================
-template <int MODE>  // 0: reference DEM/bond/extensile, 1: WCA (+extensile)
-__global__ __launch_bounds__(kBlock) void k_collide(float4 *__restrict__ force, const float4 *__restrict__ sPos,
-                                                    const float4 *__restrict__ sVel,
-                                                    const float4 *__restrict__ sTan,
-                                                    const uint32_t *__restrict__ sIdx,
-                                                    const uint32_t *__restrict__ cellStart,
-                                                    const uint32_t *__restrict__ cellEnd, uint32_t n, KP kp) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const SimParams &p = kp.p;
-    const f3 r = mk(sPos[i]);
-    const bool useVel = MODE == 0;
-    const bool useTan = MODE == 0 || p.activity != 0.0f;
-    const f3 v = useVel ? mk(sVel[i]) : mk(0.f, 0.f, 0.f);
-    const f3 t = useTan ? mk(sTan[i]) : mk(0.f, 0.f, 0.f);
-    const uint32_t myIdx = sIdx[i];
-    uint32_t fil, ch;
-    worm_of(kp, myIdx, fil, ch);
-
-    const int gx = cell_coord(r.x, p.origin.x, p.cellSize.x);
-    const int gy = cell_coord(r.y, p.origin.y, p.cellSize.y);
-    const int gz = cell_coord(r.z, p.origin.z, p.cellSize.z);
-    const bool twoD = kp.e.stencil == NW_STENCIL_2D;
-    const AxisCells ax = axis_cells(gx, p.gridSize.x, false);
-    const AxisCells ay = axis_cells(gy, p.gridSize.y, false);
-    const AxisCells az = axis_cells(gz, p.gridSize.z, twoD);
-    const float rc2 = kp.e.wcaCutoff * kp.e.wcaCutoff;
-
-    // the neighbour cells by selects over scalars (a runtime index into the
-    // AxisCells arrays would put them in scratch memory)
-    const int cx0 = ax.c[0], cx1 = ax.c[1], cx2 = ax.c[2], cy0 = ay.c[0], cy1 = ay.c[1], cy2 = ay.c[2];
-    const int cz0 = az.c[0], cz1 = az.c[1], cz2 = az.c[2];
-    const float wx0 = ax.w[0], wx1 = ax.w[1], wx2 = ax.w[2], wy0 = ay.w[0], wy1 = ay.w[1], wy2 = ay.w[2];
-    const float wz0 = az.w[0], wz1 = az.w[1], wz2 = az.w[2];
-    f3 force_acc = mk(0.f, 0.f, 0.f);
-    for (int zi = 0; zi < az.n; ++zi) {
-        const int cz = zi == 0 ? cz0 : (zi == 1 ? cz1 : cz2);
-        const float wz = zi == 0 ? wz0 : (zi == 1 ? wz1 : wz2);
-        for (int yi = 0; yi < ay.n; ++yi) {
-            const int cy = yi == 0 ? cy0 : (yi == 1 ? cy1 : cy2);
-            const float wy = yi == 0 ? wy0 : (yi == 1 ? wy1 : wy2);
-            const uint32_t rowBase = (uint32_t(cz) * p.gridSize.y + uint32_t(cy)) * p.gridSize.x;
-            for (int xi = 0; xi < ax.n; ++xi) {
-                const float wgt = wz * wy * (xi == 0 ? wx0 : (xi == 1 ? wx1 : wx2));
-                const uint32_t h = rowBase + uint32_t(xi == 0 ? cx0 : (xi == 1 ? cx1 : cx2));
-                const uint32_t start = cellStart[h];
-                if (start == 0xffffffffu) continue;
-                const uint32_t end = cellEnd[h];
-                f3 fc = mk(0.f, 0.f, 0.f);
-                for (uint32_t j = start; j < end; ++j) {
-                    if (j == i) continue;
-                    const f3 r2 = mk(sPos[j]);
-                    const uint32_t idx2 = sIdx[j];
-                    uint32_t fil2, ch2;
-                    worm_of(kp, idx2, fil2, ch2);
-                    const bool same = fil == fil2;
-                    if (MODE == 0) {
-                        const f3 v2 = mk(sVel[j]);
-                        if (same && ((ch + 1u == ch2) || (ch - 1u == ch2))) {
-                            fc += bond_hookean(p, r, r2, p.bondSpringK, p.bondSpringL);
-                        } else {
-                            fc += dem_force(p, r, r2, v, v2);
-                        }
-                    } else {
-                        if (!same) fc += wca_force(p, kp.e, r, r2, rc2);
-                    }
-                    if (useTan && !same) {
-                        const f3 t2 = mk(sTan[j]);
-                        fc += extensile_force(p, r, r2, t, t2, p.activity);
-                    }
-                }
-                if (wgt == 1.0f) force_acc += fc;
-                else force_acc += wgt * fc;
-            }
-        }
-    }
-    float4 F = force[myIdx];
-    F.x += force_acc.x;
-    F.y += force_acc.y;
-    F.z += force_acc.z;
-    F.w += 0.0f;
-    force[myIdx] = F;
-}
-
-// ===========================================================================
 // Bonded forces (filamentKernel :751-818).  One bead per lane; whole worms
 // are packed into each 64-lane wavefront (floor(64/n) worms, the remaining
 // lanes idle) and chain neighbours come from cross-lane shuffles instead of
@@ -441,20 +348,6 @@ hipError_t launch_reorder(uint32_t *cellStart, uint32_t *cellEnd, float4 *sPos, 
     if (e != hipSuccess || n == 0) return e;
     hipLaunchKernelGGL(k_reorder, dim3(grid_for(n)), dim3(kBlock), 0, st, cellStart, cellEnd, sPos, sVel, sTan, hash,
                        index, pos, vel, tan, n, numCells);
-    return hipGetLastError();
-}
-
-hipError_t launch_collide_filaments(float4 *force, const float4 *sPos, const float4 *sVel, const float4 *sTan,
-                                    const uint32_t *sIdx, const uint32_t *cellStart, const uint32_t *cellEnd,
-                                    uint32_t n, uint32_t numCells, const KP &kp, hipStream_t st) {
-    (void)numCells;
-    if (n == 0) return hipSuccess;
-    if (kp.e.pairPotential == NW_PAIR_WCA)
-        hipLaunchKernelGGL(k_collide<1>, dim3(grid_for(n)), dim3(kBlock), 0, st, force, sPos, sVel, sTan, sIdx,
-                           cellStart, cellEnd, n, kp);
-    else
-        hipLaunchKernelGGL(k_collide<0>, dim3(grid_for(n)), dim3(kBlock), 0, st, force, sPos, sVel, sTan, sIdx,
-                           cellStart, cellEnd, n, kp);
     return hipGetLastError();
 }
 

@@ -70,33 +70,8 @@ struct AxisCells {
     int n;
 };
 
-__device__ __forceinline__ AxisCells axis_cells(int g, uint32_t G, bool onlyCentre) {
-    AxisCells a;
-    if (onlyCentre) {
-        a.c[0] = wrap_mod(g, G);
-        a.w[0] = 1.0f;
-        a.n = 1;
-        return a;
-    }
-    const int m = wrap_mod(g - 1, G), c = wrap_mod(g, G), p = wrap_mod(g + 1, G);
-    if (G >= 3) {
-        a.c[0] = m; a.c[1] = c; a.c[2] = p;
-        a.w[0] = a.w[1] = a.w[2] = 1.0f;
-        a.n = 3;
-    } else if (G == 2) {
-        // offsets -1 and +1 land on the same cell
-        a.c[0] = m; a.w[0] = 2.0f;
-        a.c[1] = c; a.w[1] = 1.0f;
-        a.n = 2;
-    } else {
-        a.c[0] = c; a.w[0] = 3.0f;
-        a.n = 1;
-    }
-    return a;
-}
-
-// axis_cells of a coordinate already in [0, G): the neighbours wrap by
-// selects (the same cells as wrap_mod gives)
+// The distinct cells around coordinate g in [0, G) and how often the
+// reference's three offsets land on each; the neighbours wrap by selects
 __device__ __forceinline__ AxisCells axis_cells_in(int g, uint32_t G, bool onlyCentre) {
     AxisCells a = {{g, g, g}, {0.f, 0.f, 0.f}, 0};  // unused entries: the centre cell, weight 0
     if (onlyCentre) {
@@ -122,37 +97,6 @@ __device__ __forceinline__ AxisCells axis_cells_in(int g, uint32_t G, bool onlyC
     return a;
 }
 
-// DEM soft sphere (collideParticles)
-__device__ __forceinline__ f3 dem_force(const SimParams &p, f3 rA, f3 rB, f3 vA, f3 vB) {
-    const f3 rel = min_image_pair(p, rA, rB);
-    const float dist = length(rel);
-    const float cd = p.particleRadius + p.particleRadius;
-    f3 force = mk(0.f, 0.f, 0.f);
-    if (dist < cd) {
-        const f3 nrm = rel / dist;
-        const f3 relVel = vB - vA;
-        const f3 tanVel = relVel - (dot(relVel, nrm) * nrm);
-        force = -p.spring * (cd - dist) * nrm;
-        force += p.damping * relVel;
-        force += p.shear * tanVel;
-    }
-    return force;
-}
-
-__device__ __forceinline__ f3 bond_hookean(const SimParams &p, f3 rA, f3 rB, float k, float L) {
-    const f3 rel = min_image_pair(p, rA, rB);
-    const float dist = length(rel);
-    const f3 nrm = rel / dist;
-    return -k * (L - dist) * nrm;
-}
-
-__device__ __forceinline__ f3 extensile_force(const SimParams &p, f3 rA, f3 rB, f3 tA, f3 tB, float A) {
-    const f3 rel = min_image_pair(p, rA, rB);
-    const float dist = length(rel);
-    if (dot(tA, tB) < -0.5f) return -A * (tA - tB) / (2.0f * dist);
-    return mk(0.f, 0.f, 0.f);
-}
-
 // 24 eps (2 s^12/r^14 - s^6/r^8) at rr = r^2, with the hardware reciprocal
 // (1 ulp): the force is a product of powers of 1/r^2
 __device__ __forceinline__ float wca_mag(const NWExtParams &e, float rr) {
@@ -160,14 +104,6 @@ __device__ __forceinline__ float wca_mag(const NWExtParams &e, float rr) {
     const float s2 = e.wcaSigma * e.wcaSigma * inv2;
     const float s6 = s2 * s2 * s2;
     return 24.0f * e.wcaEpsilon * inv2 * s6 * (2.0f * s6 - 1.0f);
-}
-
-// WCA-LJ force on A from B: F_A = -24 eps (2 s^12/r^14 - s^6/r^8) (rB - rA), r < rc
-__device__ __forceinline__ f3 wca_force(const SimParams &p, const NWExtParams &e, f3 rA, f3 rB, float rc2) {
-    const f3 rel = min_image_pair(p, rA, rB);
-    const float rr = dot(rel, rel);
-    if (rr < rc2) return -wca_mag(e, rr) * rel;
-    return mk(0.f, 0.f, 0.f);
 }
 
 // ---------------------------------------------------------------------------
