@@ -216,7 +216,7 @@ void nwRadixSortPairs(uint *dGridParticleHash, uint *dGridParticleIndex,
    SimParams.reverseProbability > 0), langevinThermostat (when `langevin`),
    filamentForces, calcHash, sortParticles, reorderDataAndFindCellStart and
    collideFilaments -- in the order ParticleSystem::update issues them
-   (simulation/particleSystem.cpp:257-330) -- in four launches, for worms of
+   (simulation/particleSystem.cpp:257-330) -- in two to four launches, for worms of
    1..64 beads.  No counterpart in the reference.  Draws advance the generator
    exactly as the separate calls do.  On return gridParticleIndex holds the
    bead ids in stable cell order, sortedPos (and sortedVel / sortedTangent,
@@ -527,7 +527,8 @@ uint nwGetDeviceFlags(int clear);
    "integrate", "langevin", "filament", "hash", "sort", "reorder", "collide",
    "srd_hash", "srd_sort", "srd_reorder", "srd_com", "srd_thermo",
    "srd_collide", "srd_stream", "reverse"; of the fused steps: "md_front",
-   "md_tiles" (the sort's first level), "md_sort", "md_collide",
+   "md_tiles" (the sort's first level), "md_sort", "md_collide" (a small
+   system's order and pair forces are one launch, under "md_collide"),
    "srdf_tiles", "srdf_cells", "srdf_rotate"; of the batched step's kernels
    (launched directly, not from a replayed graph): "batch_front",
    "batch_tiles", "batch_sort", "batch_collide", and "batch_step" around a

@@ -671,6 +671,15 @@ static bool fused_md(const KP &kp, float *pos, float *vel, float *force, float *
         TimedScope ts(fixed ? noTimer : "md_front", s.stream, true);
         NW_HIP_R(launch_md_front(a, kp, s.stream), false);
     }
+    RowsPlan rows;
+    if (rows_plan(N, kp, rows)) {
+        // a small system: the cell order and the pair forces in one launch
+        TimedScope ts(fixed ? noTimer : "md_collide", s.stream, true);
+        NW_HIP_R(launch_rows(rows, a.hash, a.pos, swapForces ? a.forceOld : a.force, gridParticleIndex, sc.off,
+                             sc.sortedCell, reinterpret_cast<float4 *>(sortedPos), uint32_t(N), kp, s.stream), false);
+        s.lastHashPtr = nullptr;
+        return true;
+    }
     {
         TimedScope ts(fixed ? noTimer : "md_tiles", s.stream, true);
         NW_HIP_R(launch_hash_tiles(a.hash, bp, base, s.stream), false);

@@ -939,7 +939,7 @@ hipError_t ensure_bucket_scratch(BucketScratch &s, const BucketPlan &bp) {
 
 // LDS beyond 64 KiB is granted per kernel, once (outside any graph capture:
 // the first launch of a size runs directly)
-static hipError_t grant_lds(const void *fn, size_t lds) {
+hipError_t grant_lds(const void *fn, size_t lds) {
     static std::vector<std::pair<const void *, size_t>> granted;
     if (lds <= 65536) return hipSuccess;
     for (auto &g : granted)

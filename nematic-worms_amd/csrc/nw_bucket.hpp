@@ -146,6 +146,19 @@ hipError_t launch_collide_off(float4 *force, const float4 *sPos, const float4 *s
                               const uint32_t *sIdx, const uint32_t *off, const uint32_t *sortedCell, uint32_t n,
                               const KP &kp, hipStream_t st);
 
+// Cell order and WCA pair forces of a small one-layer system in one launch
+// (nw_rows.hip): workgroups owning `rows` grid rows each, `cap` staged beads,
+// `cells` cells of the staged rows.
+struct RowsPlan {
+    uint32_t rows, blocks, cap, cells, lds;
+};
+// whether the launch takes this system, and its shape
+bool rows_plan(uint64_t N, const KP &kp, RowsPlan &out);
+hipError_t launch_rows(const RowsPlan &pl, const uint32_t *hash, const float4 *pos, float4 *force, uint32_t *ids,
+                       uint32_t *off, uint32_t *sCell, float4 *sPos, uint32_t N, const KP &kp, hipStream_t st);
+// LDS beyond 64 KiB, granted per kernel once
+hipError_t grant_lds(const void *fn, size_t lds);
+
 // ---------------------------------------------------------------------------
 // batched replicas (the fused MD step over many independent systems).  A
 // device table of R records is followed by the R records' waveOffset values,
@@ -284,8 +297,9 @@ __device__ __forceinline__ void block_excl_scan(uint32_t *a, uint32_t m, uint32_
     const uint32_t incl = wave_scan_add(s);
     if (lane == 63u) wsum[wid] = incl;
     __syncthreads();
-    uint32_t run = incl - s;
-    for (uint32_t w = 0; w < wid; ++w) run += wsum[w];
+    // the waves' sums scanned by every wave (one LDS read, no serial loop)
+    const uint32_t ws = wave_scan_add(lane < T / 64 ? wsum[lane] : 0u);
+    uint32_t run = incl - s + (wid ? uint32_t(__builtin_amdgcn_readlane(int(ws), int(__builtin_amdgcn_readfirstlane(wid)) - 1)) : 0u);
     for (uint32_t k = 0; k < per; ++k) {
         if (b0 + k < m) {
             const uint32_t v = a[b0 + k];
@@ -295,11 +309,7 @@ __device__ __forceinline__ void block_excl_scan(uint32_t *a, uint32_t m, uint32_
             run += v;
         }
     }
-    if (threadIdx.x == T - 1) {
-        uint32_t tot = 0;
-        for (uint32_t w = 0; w < T / 64; ++w) tot += wsum[w];
-        a[m] = tot;
-    }
+    if (threadIdx.x == T - 1) a[m] = wave_last_lane(ws);
     __syncthreads();
 }
 

@@ -325,21 +325,12 @@ struct RowsLds {
 };
 
 // One candidate of the LDS walk.  The WCA term alone is evaluated for every
-// candidate and masked afterwards (no branch): a skipped one (the bead's own worm, or at
-// or beyond the cutoff, or a non-finite position) adds +0, as the branching
-// form does, which leaves the accumulator unchanged -- it starts at +0, and
-// an FP32 sum is -0 only when both of its terms are.
+// candidate and masked afterwards (no branch)
 template <int MODE, bool TAN, bool UNIT>
 __device__ __forceinline__ void lds_pair(const KP &kp, const Owner<MODE, TAN> &o, float rc2, float wt, f3 &acc,
                                          const float4 &P, const float4 &V, const float4 &T) {
     if (MODE == 1 && !TAN) {
-        const f3 rel = min_image_pair(kp.p, o.r, mk(P));
-        const float rr = dot(rel, rel);
-        const bool hit = __float_as_uint(P.w) != o.fil && rr < rc2;
-        const f3 f = -wca_mag(kp.e, rr) * rel;
-        const uint32_t m = hit ? 0xffffffffu : 0u;
-        const f3 t = mk(__uint_as_float(__float_as_uint(f.x) & m), __uint_as_float(__float_as_uint(f.y) & m),
-                        __uint_as_float(__float_as_uint(f.z) & m));
+        const f3 t = wca_term_masked(kp, o.r, o.fil, rc2, P);
         acc += UNIT ? t : wt * t;
     } else {
         add_pair<MODE, TAN, UNIT>(kp, o, rc2, wt, acc, mk(P), __float_as_uint(P.w),

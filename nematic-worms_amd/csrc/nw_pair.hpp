@@ -57,6 +57,21 @@ __device__ __forceinline__ void add_pair(const KP &kp, const Owner<MODE, TAN> &o
     }
 }
 
+// The WCA term of a bead at r of worm fil with the staged record P (position,
+// worm in w), evaluated without a branch and masked: a candidate of the bead's
+// own worm, at or beyond the cutoff or at a non-finite position gives +0,
+// which leaves an accumulator that starts at +0 unchanged (an FP32 sum is -0
+// only when both of its terms are)
+__device__ __forceinline__ f3 wca_term_masked(const KP &kp, f3 r, uint32_t fil, float rc2, const float4 &P) {
+    const f3 rel = min_image_pair(kp.p, r, mk(P));
+    const float rr = dot(rel, rel);
+    const bool hit = __float_as_uint(P.w) != fil && rr < rc2;
+    const f3 f = -wca_mag(kp.e, rr) * rel;
+    const uint32_t m = hit ? 0xffffffffu : 0u;
+    return mk(__uint_as_float(__float_as_uint(f.x) & m), __uint_as_float(__float_as_uint(f.y) & m),
+              __uint_as_float(__float_as_uint(f.z) & m));
+}
+
 template <int MODE, bool TAN>
 __device__ __forceinline__ Owner<MODE, TAN> load_owner(const KP &kp, uint32_t i, uint32_t me,
                                                        const float4 *__restrict__ sPos,

@@ -232,7 +232,8 @@ extern "C" int nwAutotuneFused(float *pos, float *vel, float *force, float *forc
                 t.pairStage = stage;
                 c.push_back(t);
             }
-        search(c, {"md_collide"}, false);
+        // with the sort: a small system's built-in choice does both in one launch
+        search(c, {"md_tiles", "md_sort", "md_collide"}, false);
     }
     if (numSolvent) {
         std::vector<NWTuning> c;
