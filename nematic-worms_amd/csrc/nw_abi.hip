@@ -65,6 +65,7 @@ struct State {
         std::vector<SortRep> sort;  // every replica's own sort plan
         SortRep *sortDev = nullptr;
         BatchSortPlan sortPlan;
+        RowsPlan rows{};  // blocks > 0: order and pairs in one launch
         // the step as graphs: [0] force -> forceOld, [1] the buffers' roles
         // exchanged (double-buffered forces, when no replica reverses)
         hipGraphExec_t exec[2] = {nullptr, nullptr};
@@ -1024,6 +1025,7 @@ void nwBatchSetReplicas(const NWReplicaParams *reps, uint numReplicas) {
     if (b.mode == 0) b.tan = true;
     if (numReplicas == 0) b.tan = false, b.unit = true;
     b.steps = 0;
+    (void)rows_plan_batch(b.reps.data(), numReplicas, b.rows);
     if (b.dev) (void)hipFree(b.dev);
     b.dev = nullptr;
     if (numReplicas) {
@@ -1031,12 +1033,13 @@ void nwBatchSetReplicas(const NWReplicaParams *reps, uint numReplicas) {
         // kernels' replica lookups bisect those)
         static_assert(sizeof(BatchRep) % alignof(uint32_t) == 0, "offsets follow the records");
         const size_t recBytes = sizeof(BatchRep) * numReplicas;
-        std::vector<unsigned char> table(recBytes + 2 * sizeof(uint32_t) * numReplicas);
+        std::vector<unsigned char> table(recBytes + 3 * sizeof(uint32_t) * numReplicas);
         memcpy(table.data(), b.reps.data(), recBytes);
         uint32_t *off = reinterpret_cast<uint32_t *>(table.data() + recBytes);
         for (uint r = 0; r < numReplicas; ++r) {
             off[r] = b.reps[r].waveOffset;
             off[numReplicas + r] = b.reps[r].blockOffset;
+            off[2 * numReplicas + r] = b.reps[r].rowBlock;
         }
         NW_HIP(hipMalloc(&b.dev, table.size()));
         NW_HIP(hipMemcpy(b.dev, table.data(), table.size(), hipMemcpyHostToDevice));
@@ -1079,6 +1082,10 @@ static hipError_t batch_step(State::Batch &b, const BatchArrays &a, const float4
     {
         TimedScope ts(timed ? "batch_front" : "", st, true);
         if ((e = launch_md_front_batch(a, b.dev, b.R, b.waves, b.stepCtr, dt, st)) != hipSuccess) return e;
+    }
+    if (b.rows.blocks) {
+        TimedScope ts(timed ? "batch_collide" : "", st, true);
+        return launch_rows_batch(b.rows, a, b.dev, b.R, b.stepCtr, st);
     }
     {
         TimedScope ts(timed ? "batch_tiles" : "", st, true);
@@ -1544,6 +1551,7 @@ static hipError_t batch_step_into(State::Batch &b, const BatchArrays &a, float d
     sc.sortedCell = a.sCell;
     hipError_t e;
     if ((e = launch_md_front_batch(a, b.dev, b.R, b.waves, b.stepCtr, dt, st)) != hipSuccess) return e;
+    if (b.rows.blocks) return launch_rows_batch(b.rows, a, b.dev, b.R, b.stepCtr, st);
     if ((e = launch_hash_tiles_batch(a.hash, b.sortDev, b.R, b.sortPlan, b.scratch, st)) != hipSuccess) return e;
     if ((e = launch_md_cells_batch(b.sortDev, b.R, b.sortPlan, sc, a.ids, a.pos, nullptr, nullptr, a.sPos, nullptr,
                                    nullptr, st)) != hipSuccess)

@@ -162,8 +162,9 @@ hipError_t grant_lds(const void *fn, size_t lds);
 // ---------------------------------------------------------------------------
 // batched replicas (the fused MD step over many independent systems).  A
 // device table of R records is followed by the R records' waveOffset values,
-// then their blockOffset values, packed (replica_of_wave / replica_of_block
-// read those); nwBatchSetReplicas builds it so.
+// then their blockOffset and their rowBlock values, packed (replica_of_wave /
+// replica_of_block / replica_of_row_block read those); nwBatchSetReplicas
+// builds it so.
 // ---------------------------------------------------------------------------
 struct BatchRep {
     KP kp;                 // the replica's parameters (box, grid, worms, force constants)
@@ -179,11 +180,14 @@ struct BatchRep {
     float lgvGamma;        // the Langevin gamma
     int32_t langevin;
     uint32_t numBeads;     // numFilaments x filamentSize
+    uint32_t rows;         // grid rows of a workgroup of the one-launch order and pairs
+    uint32_t rowBlock;     // its first workgroup
 };
 
 // the replica of a front wavefront / pair workgroup of a batched launch.
 // The device table holds the R records, then their wavefront offsets, then
-// their workgroup offsets, packed (ascending): the bisection reads 4 bytes per
+// their workgroup offsets of the two pair kernels, packed (ascending): the
+// bisection reads 4 bytes per
 // replica that stay in the scalar cache rather than one record's line per step.
 __device__ __forceinline__ uint32_t replica_of_offset(const uint32_t *__restrict__ off, uint32_t R, uint32_t v) {
     uint32_t lo = 0, hi = R;
@@ -199,6 +203,9 @@ __device__ __forceinline__ uint32_t replica_of_wave(const BatchRep *__restrict__
 }
 __device__ __forceinline__ uint32_t replica_of_block(const BatchRep *__restrict__ reps, uint32_t R, uint32_t blk) {
     return replica_of_offset(reinterpret_cast<const uint32_t *>(reps + R) + R, R, blk);
+}
+__device__ __forceinline__ uint32_t replica_of_row_block(const BatchRep *__restrict__ reps, uint32_t R, uint32_t blk) {
+    return replica_of_offset(reinterpret_cast<const uint32_t *>(reps + R) + 2u * R, R, blk);
 }
 
 // The batched sort: every replica sorted against its own plan (tiles of
@@ -266,6 +273,14 @@ struct BatchArrays {
     uint32_t *sCell;  // cell of every sorted slot
     float4 *sPos, *sVel, *sTan;
 };
+
+// Cell order and pair forces of a batch of small replicas in one launch
+// (nw_rows.hip): the replicas' rows and rowBlock, and the launch's shape;
+// false (out.blocks 0) when the batch takes the sort and the pair kernel.
+bool rows_plan_batch(BatchRep *reps, uint32_t R, RowsPlan &out);
+// the last kernel of a batched step: advances *stepCtr
+hipError_t launch_rows_batch(const RowsPlan &pl, const BatchArrays &a, const BatchRep *reps, uint32_t R,
+                             uint64_t *stepCtr, hipStream_t st);
 
 // exchanges the contents of two float4 arrays of n records
 hipError_t launch_swap4(float4 *a, float4 *b, uint64_t n, hipStream_t st);

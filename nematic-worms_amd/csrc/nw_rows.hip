@@ -337,6 +337,22 @@ __global__ __launch_bounds__(kRowsBlock) void k_rows(RowsArgs a, uint32_t N, uin
     rows_body<kRowsBlock>(kp, a, N, 0u, 0u, 0u, b * rows, rows, cap, maxCells, smem);
 }
 
+// the same of every replica of a batch: a workgroup belongs to one replica
+__global__ __launch_bounds__(kRowsBlock) void k_rows_batch(BatchArrays a, const BatchRep *__restrict__ reps,
+                                                           uint32_t R, uint32_t cap, uint32_t maxCells,
+                                                           uint64_t *__restrict__ stepCtr) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    // the step's last kernel advances the step counter the next front reads
+    if (blockIdx.x == 0 && threadIdx.x == 0) stepCtr[0] = stepCtr[0] + 1u;
+    const uint32_t b = xcd_contiguous(blockIdx.x, gridDim.x);
+    const BatchRep &rep = reps[__builtin_amdgcn_readfirstlane(replica_of_row_block(reps, R, b))];
+    const uint32_t b0 = rep.beadOffset, c0 = rep.cellOffset;
+    const RowsArgs x{a.hash + b0,    a.pos + b0, (a.swapForces ? a.forceOld : a.force) + b0, a.ids + b0,
+                     a.off + c0,     a.sCell + b0, a.sPos + b0};
+    rows_body<kRowsBlock>(rep.kp, x, rep.numBeads, b0, c0, b0, (b - rep.rowBlock) * rep.rows, rep.rows, cap, maxCells,
+                          smem);
+}
+
 // ---------------------------------------------------------------------------
 // plan and launcher
 // ---------------------------------------------------------------------------
@@ -348,26 +364,82 @@ constexpr uint64_t kRowsMaxBeads = 131072;
 constexpr uint32_t kRowsMaxBlocks = 256;  // one round of the CUs: 64,000 beads over 291 rows take 23.0 us by single rows, 16.0 by pairs
 constexpr uint32_t kRowsMaxOwn = 768;     // beads of a workgroup on average: three rounds of its quads
 
-bool rows_plan(uint64_t N, const KP &kp, RowsPlan &out) {
+// whether the launch computes a system's pair term at all
+static bool rows_term(const KP &kp) {
     const SimParams &p = kp.p;
+    return kp.e.pairPotential == NW_PAIR_WCA && p.activity == 0.0f && kp.e.stencil == NW_STENCIL_2D &&
+           kp.e.collideKernel == NW_COLLIDE_AUTO && p.gridSize.z == 1 && p.gridSize.x >= 3 && p.gridSize.y >= 3;
+}
+
+// beads staged by a workgroup of `rows` rows: two and a half times the
+// average, since rows fill to at most about the close packing of their cells
+static uint32_t rows_cap(uint64_t N, uint32_t Gy, uint32_t rows) {
+    return std::max(1024u, (uint32_t(2.5 * double(N) / Gy * (rows + 2u)) + 255u) & ~255u);
+}
+
+static bool rows_fits(RowsPlan &pl) {
+    pl.lds = rows_layout(pl.cap, pl.cells).total;
+    return pl.cells <= 8192u && pl.cap <= 8192u && pl.lds <= 150u * 1024u;
+}
+
+bool rows_plan(uint64_t N, const KP &kp, RowsPlan &out) {
     const Tuning &t = tuning();
-    const uint32_t Gx = p.gridSize.x, Gy = p.gridSize.y;
-    if (kp.e.pairPotential != NW_PAIR_WCA || p.activity != 0.0f || kp.e.stencil != NW_STENCIL_2D ||
-        kp.e.collideKernel != NW_COLLIDE_AUTO || p.gridSize.z != 1 || Gx < 3 || Gy < 3)
-        return false;
+    const uint32_t Gx = kp.p.gridSize.x, Gy = kp.p.gridSize.y;
+    if (!rows_term(kp)) return false;
     // a launch shape asked of the sort or the pair kernel is theirs
     if (t.mdTileItems || t.mdMembers || t.pairBlock || t.pairStage) return false;
     if (N == 0 || N > kRowsMaxBeads) return false;
     out.rows = std::min((Gy + kRowsMaxBlocks - 1u) / kRowsMaxBlocks, Gy - 2u);
     out.blocks = (Gy + out.rows - 1u) / out.rows;
-    const double perRow = double(N) / Gy;
-    if (perRow * out.rows > double(kRowsMaxOwn)) return false;
+    if (double(N) / Gy * out.rows > double(kRowsMaxOwn)) return false;
     out.cells = (out.rows + 2u) * Gx;
-    // two and a half times the average: rows fill to at most about the close
-    // packing of their cells
-    out.cap = std::max(1024u, (uint32_t(2.5 * perRow * (out.rows + 2u)) + 255u) & ~255u);
-    out.lds = rows_layout(out.cap, out.cells).total;
-    return out.cells <= 8192u && out.lds <= 150u * 1024u;
+    out.cap = rows_cap(N, Gy, out.rows);
+    return rows_fits(out);
+}
+
+// The batch takes the launch when its workgroups are done sooner than the sort
+// and the pair kernel.  Measured with one size of replica throughout (us, sort
+// + pairs / this launch): 16 x 8,000 beads 24.6 / 11.0, 64 x 8,000 35.5 / 26.6,
+// 128 x 8,000 47.8 / 48.1, 256 x 2,000 35.0 / 24.6, 16 x 12,000 25.7 / 13.5, 64
+// x 12,000 42.4 / 35.1, 16 x 30,000 33.3 / 30.4, 64 x 30,000 72.4 / 95.1, 16 x
+// 60,000 45.4 / 61.9: the sort and the pairs take some 22 us and 26 us a
+// million beads, 256 workgroups here 8 us and 1 us for every 10,000 beads of
+// their replica.
+bool rows_plan_batch(BatchRep *reps, uint32_t R, RowsPlan &out) {
+    out = RowsPlan{};
+    uint64_t rows = 0;
+    for (uint32_t r = 0; r < R; ++r) {
+        if (!rows_term(reps[r].kp)) return false;
+        rows += reps[r].kp.p.gridSize.y;
+    }
+    RowsPlan pl{};
+    const uint32_t per = uint32_t((rows + kRowsMaxBlocks - 1u) / kRowsMaxBlocks);
+    double here = 0.0, beads = 0.0;
+    for (uint32_t r = 0; r < R; ++r) {
+        BatchRep &q = reps[r];
+        const uint32_t Gx = q.kp.p.gridSize.x, Gy = q.kp.p.gridSize.y;
+        const double perRow = std::max(1.0, double(q.numBeads) / Gy);
+        if (perRow > double(kRowsMaxOwn)) return false;
+        q.rows = std::max(1u, std::min({per, uint32_t(kRowsMaxOwn / perRow), Gy - 2u}));
+        q.rowBlock = pl.blocks;
+        const uint32_t blocks = (Gy + q.rows - 1u) / q.rows;
+        pl.blocks += blocks;
+        pl.cells = std::max(pl.cells, (q.rows + 2u) * Gx);
+        pl.cap = std::max(pl.cap, rows_cap(q.numBeads, Gy, q.rows));
+        here += blocks * (8.0 + 1e-4 * q.numBeads) / kRowsMaxBlocks;
+        beads += q.numBeads;
+    }
+    if (!pl.blocks || here > 22.0 + 26e-6 * beads || !rows_fits(pl)) return false;
+    out = pl;
+    return true;
+}
+
+hipError_t launch_rows_batch(const RowsPlan &pl, const BatchArrays &a, const BatchRep *reps, uint32_t R,
+                             uint64_t *stepCtr, hipStream_t st) {
+    const hipError_t e = grant_lds(reinterpret_cast<const void *>(&k_rows_batch), pl.lds);
+    if (e != hipSuccess) return e;
+    NW_LAUNCH(k_rows_batch, dim3(pl.blocks), dim3(kRowsBlock), pl.lds, st, a, reps, R, pl.cap, pl.cells, stepCtr);
+    return hipGetLastError();
 }
 
 hipError_t launch_rows(const RowsPlan &pl, const uint32_t *hash, const float4 *pos, float4 *force, uint32_t *ids,

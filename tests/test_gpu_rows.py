@@ -65,3 +65,43 @@ def test_one_launch_equals_sort_and_pairs(lib, grid, W, n, shift, squeeze):
     b = step(lib, p, e, state, NWTuning(mdMembers=512), shift)
     for name, x, y in zip(("pos", "vel", "force", "forceOld", "tangent", "hash", "ids", "sortedPos"), a, b):
         assert np.array_equal(x, y), (name, int((x != y).sum()))
+
+
+@pytest.mark.parametrize("sizes", [
+    [(1, 1, 3), (5, 7, 3), (40, 16, 31), (3, 5, 4), (333, 7, 64), (17, 12, 300)],  # uneven, offsets of every residue
+    [(20, 9, 12)] * 40,                                                            # more rows than workgroups wanted
+])
+def test_batch_one_launch_equals_sort_and_pairs(lib, sizes):
+    """Replicas (worms, beads per worm, cells a side) stepped together: the built-in choice against the sort and the
+    pair kernel (collideKernel set), forces, positions, cell order and sorted records bit for bit."""
+    rng = np.random.default_rng([29, len(sizes)])
+    reps, pos, vel, force = (abi.NWReplicaParams * len(sizes))(), [], [], []
+    for r, (W, n, G) in enumerate(sizes):
+        p = sim_params(grid=(G, G, 1), cell=1.2, W=W, n=n, bondSpringL=0.8, activity=0.0)
+        q = random_worms(p, rng, twod=True)
+        f = random_forces(rng, W * n, 0.5)
+        f[:, 3] = 0
+        reps[r].params, reps[r].seed, reps[r].offset, reps[r].langevin = p, 7 + r, 3, 1
+        reps[r].langevinGamma, reps[r].langevinKbT = p.gamma, 0.1
+        pos.append(q[0])
+        vel.append(q[1])
+        force.append(f)
+    arrays = [np.concatenate(x) for x in (pos, vel, force, force[::-1], force)]
+    N = len(arrays[0])
+    got = []
+    for kern in (abi.NW_COLLIDE_AUTO, abi.NW_COLLIDE_LDS):
+        for r in range(len(sizes)):
+            reps[r].ext = ext_params(pairPotential=abi.NW_PAIR_WCA, bondedMode=abi.NW_BONDED_CHAIN, driveForce=1.0,
+                                     stencil=abi.NW_STENCIL_2D, collideKernel=kern)
+        lib.nwBatchSetReplicas(reps, len(sizes))
+        d = [DeviceArray.from_numpy(lib, a) for a in arrays]
+        i, sp = DeviceArray(lib, 4 * N), DeviceArray(lib, 16 * N)
+        for graph in (0, 1):
+            lib.nwBatchMdStep(*[x.p for x in d], i.p, sp.p, None, None, 1e-4, 3, graph)
+        lib.threadSync()
+        assert lib.nwGetLastError() == 0
+        got.append([x.download(np.uint32, (N, 4)) for x in d] + [i.download(np.uint32, (N,)),
+                                                                 sp.download(np.uint32, (N, 4))])
+    lib.nwBatchSetReplicas(None, 0)
+    for name, x, y in zip(("pos", "vel", "force", "forceOld", "tangent", "ids", "sortedPos"), *got):
+        assert np.array_equal(x, y), name
