@@ -1812,24 +1812,16 @@ void nwBatchPolarSpeedGrad(const float *pos, const float *vel, float *dPdPos, fl
     State &s = S();
     State::Batch &b = s.batch;
     NW_REQUIRE(pos != nullptr && vel != nullptr && P != nullptr, "nwBatchPolarSpeedGrad: NULL argument");
-    for (uint32_t r = 0; r < b.R; ++r) {
-        const BatchRep &rep = b.reps[r];
-        const size_t o = size_t(rep.beadOffset) * 4;
-        NWObservables obs;
-        observe_kp(rep.kp, pos + o, vel + o, rep.kp.p.numFilaments, &obs);
-        P[r] = obs.polarSpeed;
-        if (!dPdPos) continue;
-        if (obs.beads > 0) {
-            NW_HIP(launch_polar_speed_grad(reinterpret_cast<const float4 *>(pos + o),
-                                           reinterpret_cast<const float4 *>(vel + o), rep.kp.p.numFilaments,
-                                           1.0 / obs.beads, reinterpret_cast<float4 *>(dPdPos + o),
-                                           dPdVel ? reinterpret_cast<float4 *>(dPdVel + o) : nullptr, rep.kp,
-                                           s.stream));
-        } else {
-            NW_HIP(hipMemsetAsync(dPdPos + o, 0, size_t(rep.numBeads) * 16, s.stream));
-            if (dPdVel) NW_HIP(hipMemsetAsync(dPdVel + o, 0, size_t(rep.numBeads) * 16, s.stream));
-        }
+    if (b.R == 0) {
+        NW_HIP(hipStreamSynchronize(s.stream));
+        return;
     }
+    NW_REQUIRE(grow(s.obsPartial, s.obsCap, uint64_t(b.waves) + b.R), "nwBatchPolarSpeedGrad: out of device memory");
+    double *out = s.obsPartial + b.waves;
+    NW_HIP(launch_polar_speed_batch(reinterpret_cast<const float4 *>(pos), reinterpret_cast<const float4 *>(vel),
+                                    b.dev, b.R, b.waves, s.obsPartial, out, reinterpret_cast<float4 *>(dPdPos),
+                                    reinterpret_cast<float4 *>(dPdVel), s.stream));
+    NW_HIP(hipMemcpyAsync(P, out, size_t(b.R) * sizeof(double), hipMemcpyDeviceToHost, s.stream));
     NW_HIP(hipStreamSynchronize(s.stream));
 }
 

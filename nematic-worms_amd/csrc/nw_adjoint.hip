@@ -464,6 +464,77 @@ __global__ __launch_bounds__(kBlock) void k_polar_speed_grad(const float4 *__res
     if (dVel) dVel[m.bead] = f4(scale * t, 0.0f);
 }
 
+// The polar speed of every replica of a batch in one launch: a wavefront of
+// the batched front kernel writes its share of the FP64 sum of v . t (bead
+// tangents in FP64, as the order parameters take them) to sums[wave] and, dPos
+// given, its beads' gradients as above, scaled by 1 over the replica's beads.
+__global__ __launch_bounds__(kBlock) void k_polar_speed_batch(const float4 *__restrict__ pos,
+                                                              const float4 *__restrict__ vel,
+                                                              const BatchRep *__restrict__ reps, uint32_t R,
+                                                              uint32_t waves, double *__restrict__ sums,
+                                                              float4 *__restrict__ dPos, float4 *__restrict__ dVel) {
+    const uint32_t wave = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    if (wave >= waves) return;
+    const BatchRep &rep = reps[__builtin_amdgcn_readfirstlane(replica_of_wave(reps, R, wave))];
+    const KP &kp = rep.kp;
+    const SimParams &p = kp.p;
+    const uint32_t n = p.filamentSize, b0 = rep.beadOffset;
+    const WaveWorm m = wave_worm_at(wave - rep.waveOffset, n, p.numFilaments);
+    const f3 r = mk(load4_or_zero(pos + b0, m.bead, m.active));
+    const f3 v = mk(load4_or_zero(vel + b0, m.bead, m.active));
+    const f3 rn = shfl_down3(r, 1), rp = shfl_up3(r, 1);
+    const float scale = float(1.0 / double(rep.numBeads));
+    f3 g = mk(0.f, 0.f, 0.f), t = g;
+    double s = 0.0;
+    if (m.active && n >= 2u) {
+        const f3 d = min_image(p, m.pp == 0u ? r : rp, m.pp + 1u == n ? r : rn);
+        const double dx = d.x, dy = d.y, dz = d.z;
+        const double inv = 1.0 / sqrt(dx * dx + dy * dy + dz * dz);
+        s = double(v.x) * (dx * inv) + double(v.y) * (dy * inv) + double(v.z) * (dz * inv);
+        const float len = sqrtf(dot(d, d));
+        t = d / len;
+        g = (scale / len) * (v - t * dot(t, v));
+    }
+    s = wave_sum_d(s);
+    if (m.lane == 0u) sums[wave] = s;
+    if (!dPos) return;
+    const f3 gPrev = shfl_up3(g, 1), gNext = shfl_down3(g, 1);
+    if (!m.active) return;
+    f3 o = mk(0.f, 0.f, 0.f);
+    if (n >= 2u) {
+        if (m.pp >= 1u) o += gPrev;
+        if (m.pp + 1u < n) o -= gNext;
+        if (m.pp == 0u) o -= g;
+        if (m.pp + 1u == n) o += g;
+    }
+    dPos[b0 + m.bead] = f4(o, 0.0f);
+    if (dVel) dVel[b0 + m.bead] = f4(scale * t, 0.0f);
+}
+
+// out[r] = the sum of replica r's wavefronts over its beads, in a fixed order
+__global__ __launch_bounds__(64) void k_polar_speed_total(const double *__restrict__ sums,
+                                                          const BatchRep *__restrict__ reps, uint32_t R,
+                                                          uint32_t waves, double *__restrict__ out) {
+    const uint32_t r = blockIdx.x;
+    const uint32_t lo = reps[r].waveOffset, hi = r + 1 < R ? reps[r + 1].waveOffset : waves;
+    double s = 0.0;
+    for (uint32_t w = lo + threadIdx.x; w < hi; w += 64u) s += sums[w];
+    s = wave_sum_d(s);
+    const bool tangents = reps[r].numBeads > 0u && reps[r].kp.p.filamentSize >= 2u;
+    if (threadIdx.x == 0u) out[r] = tangents ? s / double(reps[r].numBeads) : 0.0;
+}
+
+hipError_t launch_polar_speed_batch(const float4 *pos, const float4 *vel, const BatchRep *reps, uint32_t R,
+                                    uint32_t waves, double *sums, double *out, float4 *dPos, float4 *dVel,
+                                    hipStream_t st) {
+    if (R == 0) return hipSuccess;
+    if (waves)
+        hipLaunchKernelGGL(k_polar_speed_batch, dim3(grid_for(uint64_t(waves) * 64u)), dim3(kBlock), 0, st, pos, vel,
+                           reps, R, waves, sums, dPos, dVel);
+    hipLaunchKernelGGL(k_polar_speed_total, dim3(R), dim3(64), 0, st, sums, reps, R, waves, out);
+    return hipGetLastError();
+}
+
 // out[k] += sum over rows of partial[row][k]: thread t adds the entries
 // t, t + kTotalBlock, ... of the row-major table (all of parameter
 // t mod kAdjParams) in order, then a fixed tree over the threads of each

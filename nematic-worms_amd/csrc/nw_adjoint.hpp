@@ -39,6 +39,12 @@ hipError_t launch_srd_adj(const uint32_t *ids, const uint32_t *off, const uint32
 // scale * d(sum of v . t)/d(r, v) of the polar speed (dVel may be NULL)
 hipError_t launch_polar_speed_grad(const float4 *pos, const float4 *vel, uint32_t W, double scale, float4 *dPos,
                                    float4 *dVel, const KP &kp, hipStream_t st);
+// polar speed of every replica into out[R] and, dPos (dVel) given, its
+// gradient with respect to the beads' positions (velocities); sums: one
+// double per front wavefront
+hipError_t launch_polar_speed_batch(const float4 *pos, const float4 *vel, const BatchRep *reps, uint32_t R,
+                                    uint32_t waves, double *sums, double *out, float4 *dPos, float4 *dVel,
+                                    hipStream_t st);
 // one adjoint step of every replica of a batch (a: concatenated arrays,
 // off over the concatenated cells, ids global; the replicas' own W,
 // Langevin and Philox from reps; a.partial: one row per front wavefront,
