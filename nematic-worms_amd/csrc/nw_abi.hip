@@ -1363,9 +1363,10 @@ void nwAdjointBackward(const float *dLdPos, const float *dLdVel, double grad[4])
     NW_REQUIRE(dLdPos != nullptr && grad != nullptr, "nwAdjointBackward: NULL argument");
     const uint64_t N = A.N, K = A.K;
     NW_REQUIRE(ensure_segment(A), "nwAdjointBackward: out of device memory");
-    const uint64_t rowsPerStep = adj_step_blocks(A.W, A.kp.p.filamentSize);
-    NW_REQUIRE(grow(A.partial, A.capPartial, K * rowsPerStep * kAdjParams), "nwAdjointBackward: out of memory");
+    const uint64_t rows = adj_step_rows(A.W, A.kp.p.filamentSize);
+    NW_REQUIRE(grow(A.partial, A.capPartial, rows * kAdjParams), "nwAdjointBackward: out of memory");
     if (!A.grad) NW_HIP(hipMalloc(&A.grad, kAdjParams * sizeof(double)));
+    NW_HIP(hipMemsetAsync(A.partial, 0, rows * kAdjParams * sizeof(double), s.stream));
     NW_HIP(hipMemsetAsync(A.grad, 0, kAdjParams * sizeof(double), s.stream));
     const uint64_t NT = A.NT, stride = 2 * NT + 2 * N;
     const size_t bytes = N * sizeof(float4);
@@ -1442,7 +1443,6 @@ void nwAdjointBackward(const float *dLdPos, const float *dLdVel, double grad[4])
                                       A.collCom + q * A.Cs, A.wVel, lv, A.cellSum, A.N, uint32_t(NT), A.Cs, A.cosA,
                                       A.sinA, A.rotBeads, s.stream));
             }
-            double *part = A.partial + uint64_t(j) * rowsPerStep * kAdjParams;
             AdjStepArgs as;
             as.pos = A.segPos + uint64_t(j + 1) * N;
             as.vel = A.segVel + uint64_t(j + 1) * N;
@@ -1454,7 +1454,7 @@ void nwAdjointBackward(const float *dLdPos, const float *dLdVel, double grad[4])
             as.lr = lr;
             as.lv = lv;
             as.lG = lG;
-            as.partial = part;
+            as.partial = A.partial;
             as.W = A.W;
             as.langevin = A.langevin;
             as.lgvStd = A.lgvStd;
@@ -1468,8 +1468,8 @@ void nwAdjointBackward(const float *dLdPos, const float *dLdVel, double grad[4])
             }
             cur = 1 - cur;
         }
-        NW_HIP(launch_adj_total(A.partial, uint64_t(len) * rowsPerStep, A.grad, s.stream));
     }
+    NW_HIP(launch_adj_total(A.partial, rows, A.grad, s.stream));
     s.offset = A.endOffset;  // the generator continues after the forward run
     NW_HIP(hipMemcpyAsync(grad, A.grad, kAdjParams * sizeof(double), hipMemcpyDeviceToHost, s.stream));
     NW_HIP(hipStreamSynchronize(s.stream));

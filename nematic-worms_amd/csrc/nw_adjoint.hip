@@ -73,44 +73,206 @@ __device__ __forceinline__ double wave_sum_d(double v) {
     return v;
 }
 
-// the workgroup's FP64 partials (kAdjParams of them) into out[blockIdx]
-__device__ __forceinline__ void block_partials(double (&acc)[kAdjParams], double *__restrict__ out) {
-    __shared__ double ls[kBlock / 64][kAdjParams];
-#pragma unroll
-    for (int k = 0; k < kAdjParams; ++k) {
-        const double s = wave_sum_d(acc[k]);
-        if ((threadIdx.x & 63u) == 0u) ls[threadIdx.x >> 6][k] = s;
-    }
-    __syncthreads();
-    if (threadIdx.x < kAdjParams) {
-        double s = 0.0;
-        for (int w = 0; w < kBlock / 64; ++w) s += ls[w][threadIdx.x];
-        out[uint64_t(blockIdx.x) * kAdjParams + threadIdx.x] = s;
-    }
-}
-
 // ---------------------------------------------------------------------------
-// One adjoint step, whole worms per wavefront (bead order):
+// One adjoint step of the whole worms of one front wavefront (at most 64
+// beads):
 //   bonded:  Rb = (dB/dr')^T lF by dual numbers through the forward bending
 //            and bond expressions (chain neighbours by shuffles), the drive's
 //            transpose product written out; kappa, f_a, gamma partials
 //   pairs:   Rp = sum_j w H_ij (lF_i - lF_j), H = f I + 2 f' d d^T for
 //            F_i = -f(|d|^2) d, d = r_j - r_i, over the forward step's cell
 //            lists of r' (the bead's cell recomputed as the forward hashed
-//            it; w the stencil weight of the row); epsilon partial
+//            it; w the stencil weight of the row), the terms added in list
+//            order; epsilon partial
 //   update:  R = lr + Rb + Rp, V = lv - gamma lF + dt R, then the new
 //            (lr, lv, lF, lG) of the bead (lF into the other buffer: the
 //            neighbours still read the old one)
+// A bead's candidates are a chain of loads (cell bounds, id and position,
+// adjoint).  In a large system the wavefronts cover it and a bead takes one
+// lane for everything: 800,000 beads 62 us, 64 replicas of 12,000 59 us.  A
+// small one gives a CU two wavefronts, each waiting on four such chains in a
+// row: there four lanes share a bead's candidates, and the bonded part runs
+// beside them in a wavefront of its own.
 // ---------------------------------------------------------------------------
-// The lanes m of one system: a's bead arrays (pos, vel, lF, lFout, lr, lv,
-// lG) and off start at the system's first bead and cell; ids and sPos are the
+// The pairs of bead first + b of a group (b < beads), by lane q of its four: Rp
+// (in every lane) and the lane's share of the epsilon partial.  a's bead arrays
+// and off start at the system's first bead and cell; ids and sPos are the
 // step's sorted slots, whose ids exceed the system's bead index by idBase.
-__device__ __forceinline__ void adj_step_lanes(const AdjStepArgs &a, const KP &kp, const WaveWorm &m,
-                                               uint32_t idBase, double (&acc)[kAdjParams]) {
+__device__ __forceinline__ f3 adj_pairs_quad(const AdjStepArgs &a, const KP &kp, uint32_t first, uint32_t b,
+                                             uint32_t q, uint32_t beads, uint32_t idBase, double &eps) {
+    const SimParams &p = kp.p;
+    f3 Rp = mk(0.f, 0.f, 0.f);
+    if (b < beads) {
+        const uint32_t me = first + b;
+        const f3 rv = mk(load4(a.pos, me)), lam = mk(load4(a.lF, me));
+        uint32_t fil, ch;
+        worm_of(kp, me, fil, ch);
+        const uint32_t Gx = p.gridSize.x, Gy = p.gridSize.y;
+        const int gx = wrap_mod(cell_coord(rv.x, p.origin.x, p.cellSize.x), Gx);
+        const int gy = wrap_mod(cell_coord(rv.y, p.origin.y, p.cellSize.y), Gy);
+        const int gz = p.gridSize.z > 1u ? wrap_mod(cell_coord(rv.z, p.origin.z, p.cellSize.z), p.gridSize.z) : 0;
+        const AxisCells ay = axis_cells_in(gy, Gy, false);
+        const float wz = kp.e.stencil == NW_STENCIL_2D ? 1.0f : axis_cells_in(gz, p.gridSize.z, false).w[0];
+        const float rc2 = kp.e.wcaCutoff * kp.e.wcaCutoff;
+        const float eps24 = 24.0f * kp.e.wcaEpsilon, s2c = kp.e.wcaSigma * kp.e.wcaSigma;
+        // the candidates in stencil order: two pieces a row (its three cells,
+        // across the periodic wrap), piece k at [pre[k], pre[k + 1]) of the
+        // list and from sorted slot d[k] + pre[k] on
+        const bool mid = gx >= 1 && gx + 1 < int(Gx), left = gx == 0;
+        uint32_t pre[7], d[6];
+        float w[3];
+        pre[0] = 0u;
+#pragma unroll
+        for (int yi = 0; yi < 3; ++yi) {
+            const bool use = yi < ay.n;
+            w[yi] = wz * ay.w[yi];
+            const uint32_t base = (uint32_t(gz) * Gy + uint32_t(ay.c[yi])) * Gx;
+            const uint32_t a0 = a.off[mid ? base + gx - 1 : (left ? base + Gx - 1 : base + Gx - 2)];
+            const uint32_t a1 = a.off[mid ? base + gx + 2 : base + Gx];
+            const uint32_t b0 = a.off[base], b1 = a.off[mid ? base : (left ? base + 2 : base + 1)];
+            d[2 * yi] = a0 - pre[2 * yi];
+            pre[2 * yi + 1] = pre[2 * yi] + (use ? a1 - a0 : 0u);
+            d[2 * yi + 1] = b0 - pre[2 * yi + 1];
+            pre[2 * yi + 2] = pre[2 * yi + 1] + (use ? b1 - b0 : 0u);
+        }
+        const uint32_t K = pre[6];
+        for (uint32_t t0 = 0; t0 < K; t0 += 4u * kAdjBatch) {
+            // kAdjBatch candidates of the lane, their loads in flight
+            // together; past the list the last one again, masked
+            uint32_t I[kAdjBatch];
+            float4 Q[kAdjBatch], LF[kAdjBatch];
+            float W[kAdjBatch];
+#pragma unroll
+            for (int u = 0; u < kAdjBatch; ++u) {
+                const uint32_t t = min(t0 + 4u * uint32_t(u) + q, K - 1u);
+                uint32_t j = d[5];
+#pragma unroll
+                for (int k = 4; k >= 0; --k) j = t < pre[k + 1] ? d[k] : j;
+                j += t;
+                W[u] = t < pre[2] ? w[0] : (t < pre[4] ? w[1] : w[2]);
+                I[u] = a.ids[j] - idBase;
+                Q[u] = load4(a.sPos, j);
+            }
+#pragma unroll
+            for (int u = 0; u < kAdjBatch; ++u) LF[u] = load4(a.lF, I[u]);
+#pragma unroll
+            for (int u = 0; u < kAdjBatch; ++u) {
+                if (t0 + 4u * uint32_t(u) >= K) break;
+                const bool listed = t0 + 4u * uint32_t(u) + q < K;
+                uint32_t fil2, ch2;
+                worm_of(kp, I[u], fil2, ch2);
+                const f3 x = min_image_pair(p, rv, mk(Q[u]));
+                const float rr = dot(x, x);
+                const bool hit = listed && fil2 != fil && rr < rc2;
+                const float uu = __builtin_amdgcn_rcpf(rr);
+                const float s6 = s2c * uu * (s2c * uu) * (s2c * uu);
+                const float f = eps24 * uu * s6 * (2.0f * s6 - 1.0f);
+                const float fp = -eps24 * uu * uu * s6 * (14.0f * s6 - 4.0f);  // df / d(r^2)
+                const f3 dl = lam - mk(LF[u]);                                  // lF_i - lF_j
+                const f3 t = W[u] * (f * dl + (2.0f * fp * dot(x, dl)) * x);    // w H dl
+                const uint32_t m = hit ? 0xffffffffu : 0u;
+                add_quad(Rp, mk(__uint_as_float(__float_as_uint(t.x) & m), __uint_as_float(__float_as_uint(t.y) & m),
+                                __uint_as_float(__float_as_uint(t.z) & m)));
+                if (hit) eps += double(W[u]) * double(dot(lam, x)) * double(f);
+            }
+        }
+    }
+    return Rp;
+}
+
+// The same by the bead's own lane of its front wavefront (bead rv of worm fil
+// with adjoint lam)
+__device__ __forceinline__ f3 adj_pairs_lane(const AdjStepArgs &a, const KP &kp, f3 rv, f3 lam, uint32_t fil,
+                                             uint32_t idBase, double &epsPart) {
+    const SimParams &p = kp.p;
+    f3 Rp = mk(0.f, 0.f, 0.f);
+    // WCA pairs over the cell lists of r'
+    const uint32_t Gx = p.gridSize.x, Gy = p.gridSize.y;
+    const int gx = wrap_mod(cell_coord(rv.x, p.origin.x, p.cellSize.x), Gx);
+    const int gy = wrap_mod(cell_coord(rv.y, p.origin.y, p.cellSize.y), Gy);
+    const int gz = wrap_mod(cell_coord(rv.z, p.origin.z, p.cellSize.z), p.gridSize.z);
+    const AxisCells ay = axis_cells_in(gy, Gy, false);
+    const float wz = kp.e.stencil == NW_STENCIL_2D ? 1.0f : axis_cells_in(gz, p.gridSize.z, false).w[0];
+    const float rc2 = kp.e.wcaCutoff * kp.e.wcaCutoff;
+    const float eps = kp.e.wcaEpsilon, s2c = kp.e.wcaSigma * kp.e.wcaSigma;
+    // the six candidate runs (two per stencil row, the row's three cells
+    // with the periodic wrap), flattened; candidates in groups of
+    // kAdjBatch with all their loads in flight together (every slot of a
+    // run holds a bead of this system, so a group past the last candidate
+    // reloads the last one and discards it)
+    uint32_t ps[6], pl[6];
+    float pw[6];
+#pragma unroll
+    for (int yi = 0; yi < 3; ++yi) {
+        ps[2 * yi] = pl[2 * yi] = ps[2 * yi + 1] = pl[2 * yi + 1] = 0u;
+        pw[2 * yi] = pw[2 * yi + 1] = 0.0f;
+        if (yi < ay.n) {
+            const uint32_t base = (uint32_t(gz) * Gy + uint32_t(ay.c[yi])) * Gx;
+            const bool mid = gx >= 1 && gx + 1 < int(Gx), left = gx == 0;
+            const uint32_t ia0 = mid ? base + gx - 1 : (left ? base + Gx - 1 : base + Gx - 2);
+            const uint32_t ia1 = mid ? base + gx + 2 : base + Gx;
+            const uint32_t ib1 = mid ? base : (left ? base + 2 : base + 1);
+            const uint32_t a0 = a.off[ia0], a1 = a.off[ia1], b0 = a.off[base], b1 = a.off[ib1];
+            ps[2 * yi] = a0;
+            pl[2 * yi] = a1 - a0;
+            ps[2 * yi + 1] = b0;
+            pl[2 * yi + 1] = b1 - b0;
+            pw[2 * yi] = pw[2 * yi + 1] = wz * ay.w[yi];
+        }
+    }
+    uint32_t pre[7];
+    pre[0] = 0u;
+#pragma unroll
+    for (int k = 0; k < 6; ++k) pre[k + 1] = pre[k] + pl[k];
+    const uint32_t K = pre[6];
+    for (uint32_t t0 = 0; t0 < K; t0 += kAdjBatch) {
+        uint32_t I[kAdjBatch];
+        float4 Q[kAdjBatch], LF[kAdjBatch];
+        float W[kAdjBatch];
+#pragma unroll
+        for (int u = 0; u < kAdjBatch; ++u) {
+            const uint32_t t = min(t0 + uint32_t(u), K - 1u);
+            uint32_t j = 0u;
+            float w = 0.0f;
+#pragma unroll
+            for (int k = 0; k < 6; ++k) {
+                if (t >= pre[k] && t < pre[k + 1]) {
+                    j = ps[k] + (t - pre[k]);
+                    w = pw[k];
+                }
+            }
+            I[u] = a.ids[j] - idBase;
+            Q[u] = a.sPos[j];
+            W[u] = w;
+        }
+#pragma unroll
+        for (int u = 0; u < kAdjBatch; ++u) LF[u] = a.lF[I[u]];
+#pragma unroll
+        for (int u = 0; u < kAdjBatch; ++u) {
+            if (t0 + uint32_t(u) >= K) continue;
+            uint32_t fil2, ch2;
+            worm_of(kp, I[u], fil2, ch2);
+            if (fil2 == fil) continue;
+            const f3 d = min_image_pair(p, rv, mk(Q[u]));
+            const float rr = dot(d, d);
+            if (!(rr < rc2)) continue;
+            const float uu = __builtin_amdgcn_rcpf(rr);
+            const float s6 = s2c * uu * (s2c * uu) * (s2c * uu);
+            const float f = 24.0f * eps * uu * s6 * (2.0f * s6 - 1.0f);
+            const float fp = -24.0f * eps * uu * uu * s6 * (14.0f * s6 - 4.0f);  // df / d(r^2)
+            const f3 dl = lam - mk(LF[u]);                                       // lF_i - lF_j
+            Rp += W[u] * (f * dl + (2.0f * fp * dot(d, dl)) * d);                // w H dl
+            epsPart += double(W[u]) * double(dot(lam, d)) * double(f);
+        }
+    }
+    return Rp;
+}
+
+// The bonded part: lane m's R and its parameter partials
+__device__ __forceinline__ f3 adj_bonded(const AdjStepArgs &a, const KP &kp, const WaveWorm &m, f3 rv, f3 lam,
+                                         double (&acc)[kAdjParams]) {
     const SimParams &p = kp.p;
     const uint32_t n = p.filamentSize;
-    const f3 rv = mk(load4_or_zero(a.pos, m.bead, m.active));
-    const f3 lam = mk(load4_or_zero(a.lF, m.bead, m.active));
     const d3 r = {rv, lam};
     const uint32_t pp = m.pp;
 
@@ -156,142 +318,137 @@ __device__ __forceinline__ void adj_step_lanes(const AdjStepArgs &a, const KP &k
     if (pp >= 1u) bond = bond - fbPrev;
     if (pp + 1u < n) bond = bond + fb;
 
+    f3 R = bend.t + bond.t;
+    if (!m.active) return R;
+    if (pp + 1u < n) R -= driveT;
+    if (pp >= 1u) R += driveFromPrev;
+    // parameter partials lF . dF/dtheta (F the force this step produced)
+    if (pp + 1u < n) acc[kAdjDrive] = double(dot(lam, that));
+    if (p.bondBendingK != 0.0f) acc[kAdjKappa] = double(dot(lam, bend.v)) / double(p.bondBendingK);
+    if (a.langevin) {
+        const f3 v = mk(load4(a.vel, m.bead));
+        const u4 b = philox_block(a.seed, a.offLgv + m.bead);
+        float z0, z1, z2, z3;
+        box_muller(b.x, b.y, z0, z1);
+        box_muller(b.z, b.w, z2, z3);
+        (void)z3;
+        const f3 xi = mk(z0 * a.lgvStd + 0.0f, z1 * a.lgvStd + 0.0f, z2 * a.lgvStd + 0.0f);
+        // F_lgv = -gamma v + sigma(gamma) z, d sigma / d gamma = sigma / (2 gamma)
+        acc[kAdjGamma] = -double(dot(lam, v)) + double(dot(lam, xi)) / (2.0 * double(a.gamma));
+    }
+    return R;
+}
+
+// the adjoint of the step for lane m's bead from its bonded and pair parts
+__device__ __forceinline__ void adj_update(const AdjStepArgs &a, const WaveWorm &m, f3 lam, f3 R, f3 Rp, f3 lr,
+                                           f3 lv, f3 lG) {
+    const f3 Rt = lr + R + Rp;
+    // the drag -gamma v' is part of F' only with the Langevin thermostat on
+    const f3 V = lv - (a.langevin ? a.gamma : 0.0f) * lam + a.dt * Rt;
+    a.lr[m.bead] = f4(Rt, 0.0f);
+    a.lv[m.bead] = f4(V, 0.0f);
+    a.lFout[m.bead] = f4(lG + (0.5f * a.dt * a.dt) * Rt + (0.5f * a.dt) * V, 0.0f);
+    a.lG[m.bead] = f4((0.5f * a.dt) * V, 0.0f);
+}
+
+// Front wavefront `wave` of one system, by five wavefronts (QUADS: four lanes a
+// bead for the pairs, beside the bonded wavefront) or by one (a bead a lane
+// does both parts); row: its FP64 partials, added to
+template <bool QUADS>
+__device__ __forceinline__ void adj_group(const AdjStepArgs &a, const KP &kp, uint32_t wave, uint32_t idBase,
+                                          double *__restrict__ row) {
+    const uint32_t n = kp.p.filamentSize;
+    const WaveWorm m = wave_worm_at(wave, n, a.W);
+    const bool bonded = !QUADS || threadIdx.x >= 256u;  // the last wavefront
+    f3 rv = mk(0.f, 0.f, 0.f), lam = rv, R = rv, Rp = rv, lr = rv, lv = rv, lG = rv;
+    double acc[kAdjParams] = {0.0, 0.0, 0.0, 0.0}, eps = 0.0, mine = 0.0;
+    if (bonded) {
+        if (m.lane < uint32_t(kAdjParams)) mine = row[m.lane];  // lane k keeps partial k
+        rv = mk(load4_or_zero(a.pos, m.bead, m.active));
+        lam = mk(load4_or_zero(a.lF, m.bead, m.active));
+        if (QUADS) {  // in flight under the bonded part
+            lr = mk(load4_or_zero(a.lr, m.bead, m.active));
+            lv = mk(load4_or_zero(a.lv, m.bead, m.active));
+            lG = mk(load4_or_zero(a.lG, m.bead, m.active));
+        }
+        R = adj_bonded(a, kp, m, rv, lam, acc);
+    }
+    if constexpr (QUADS) {
+        __shared__ float lp[3][64];
+        __shared__ double le[4];
+        if (!bonded) {
+            const uint32_t w0 = wave * (64u / n), beads = (min(w0 + 64u / n, a.W) - w0) * n;
+            const uint32_t b = threadIdx.x >> 2, q = threadIdx.x & 3u;
+            Rp = adj_pairs_quad(a, kp, w0 * n, b, q, beads, idBase, eps);
+            if (q == 0u) {
+                lp[0][b] = Rp.x;
+                lp[1][b] = Rp.y;
+                lp[2][b] = Rp.z;
+            }
+            eps = wave_sum_d(eps);
+            if (m.lane == 0u) le[threadIdx.x >> 6] = eps;
+        }
+        __syncthreads();
+        if (!bonded) return;
+        Rp = mk(lp[0][m.lane], lp[1][m.lane], lp[2][m.lane]);
+        eps = m.lane == 0u ? le[0] + le[1] + le[2] + le[3] : 0.0;
+    } else if (m.active) {
+        Rp = adj_pairs_lane(a, kp, rv, lam, m.worm, idBase, eps);
+        lr = mk(load4(a.lr, m.bead));
+        lv = mk(load4(a.lv, m.bead));
+        lG = mk(load4(a.lG, m.bead));
+    }
     if (m.active) {
-        f3 R = bend.t + bond.t;
-        if (pp + 1u < n) R -= driveT;
-        if (pp >= 1u) R += driveFromPrev;
-        // parameter partials lF . dF/dtheta (F the force this step produced)
-        if (pp + 1u < n) acc[kAdjDrive] = double(dot(lam, that));
-        if (p.bondBendingK != 0.0f) acc[kAdjKappa] = double(dot(lam, bend.v)) / double(p.bondBendingK);
-        if (a.langevin) {
-            const f3 v = mk(load4(a.vel, m.bead));
-            const u4 b = philox_block(a.seed, a.offLgv + m.bead);
-            float z0, z1, z2, z3;
-            box_muller(b.x, b.y, z0, z1);
-            box_muller(b.z, b.w, z2, z3);
-            (void)z3;
-            const f3 xi = mk(z0 * a.lgvStd + 0.0f, z1 * a.lgvStd + 0.0f, z2 * a.lgvStd + 0.0f);
-            // F_lgv = -gamma v + sigma(gamma) z, d sigma / d gamma = sigma / (2 gamma)
-            acc[kAdjGamma] = -double(dot(lam, v)) + double(dot(lam, xi)) / (2.0 * double(a.gamma));
-        }
-
-        // WCA pairs over the cell lists of r'
-        const uint32_t me = m.bead;
-        const uint32_t Gx = p.gridSize.x, Gy = p.gridSize.y;
-        const int gx = wrap_mod(cell_coord(rv.x, p.origin.x, p.cellSize.x), Gx);
-        const int gy = wrap_mod(cell_coord(rv.y, p.origin.y, p.cellSize.y), Gy);
-        const int gz = wrap_mod(cell_coord(rv.z, p.origin.z, p.cellSize.z), p.gridSize.z);
-        const AxisCells ay = axis_cells_in(gy, Gy, false);
-        const float wz = kp.e.stencil == NW_STENCIL_2D ? 1.0f : axis_cells_in(gz, p.gridSize.z, false).w[0];
-        const float rc2 = kp.e.wcaCutoff * kp.e.wcaCutoff;
-        const float eps = kp.e.wcaEpsilon, s2c = kp.e.wcaSigma * kp.e.wcaSigma;
-        const uint32_t fil = m.worm;
-        f3 Rp = mk(0.f, 0.f, 0.f);
-        double epsPart = 0.0;
-        // the six candidate runs (two per stencil row, the row's three cells
-        // with the periodic wrap), flattened; candidates in groups of
-        // kAdjBatch with all their loads in flight together (every slot of a
-        // run holds a bead of this system, so a group past the last candidate
-        // reloads the last one and discards it)
-        uint32_t ps[6], pl[6];
-        float pw[6];
-#pragma unroll
-        for (int yi = 0; yi < 3; ++yi) {
-            ps[2 * yi] = pl[2 * yi] = ps[2 * yi + 1] = pl[2 * yi + 1] = 0u;
-            pw[2 * yi] = pw[2 * yi + 1] = 0.0f;
-            if (yi < ay.n) {
-                const uint32_t base = (uint32_t(gz) * Gy + uint32_t(ay.c[yi])) * Gx;
-                const bool mid = gx >= 1 && gx + 1 < int(Gx), left = gx == 0;
-                const uint32_t ia0 = mid ? base + gx - 1 : (left ? base + Gx - 1 : base + Gx - 2);
-                const uint32_t ia1 = mid ? base + gx + 2 : base + Gx;
-                const uint32_t ib1 = mid ? base : (left ? base + 2 : base + 1);
-                const uint32_t a0 = a.off[ia0], a1 = a.off[ia1], b0 = a.off[base], b1 = a.off[ib1];
-                ps[2 * yi] = a0;
-                pl[2 * yi] = a1 - a0;
-                ps[2 * yi + 1] = b0;
-                pl[2 * yi + 1] = b1 - b0;
-                pw[2 * yi] = pw[2 * yi + 1] = wz * ay.w[yi];
-            }
-        }
-        uint32_t pre[7];
-        pre[0] = 0u;
-#pragma unroll
-        for (int k = 0; k < 6; ++k) pre[k + 1] = pre[k] + pl[k];
-        const uint32_t K = pre[6];
-        for (uint32_t t0 = 0; t0 < K; t0 += kAdjBatch) {
-            uint32_t I[kAdjBatch];
-            float4 Q[kAdjBatch], LF[kAdjBatch];
-            float W[kAdjBatch];
-#pragma unroll
-            for (int u = 0; u < kAdjBatch; ++u) {
-                const uint32_t t = min(t0 + uint32_t(u), K - 1u);
-                uint32_t j = 0u;
-                float w = 0.0f;
-#pragma unroll
-                for (int k = 0; k < 6; ++k) {
-                    if (t >= pre[k] && t < pre[k + 1]) {
-                        j = ps[k] + (t - pre[k]);
-                        w = pw[k];
-                    }
-                }
-                I[u] = a.ids[j] - idBase;
-                Q[u] = a.sPos[j];
-                W[u] = w;
-            }
-#pragma unroll
-            for (int u = 0; u < kAdjBatch; ++u) LF[u] = a.lF[I[u]];
-#pragma unroll
-            for (int u = 0; u < kAdjBatch; ++u) {
-                if (t0 + uint32_t(u) >= K) continue;
-                uint32_t fil2, ch2;
-                worm_of(kp, I[u], fil2, ch2);
-                if (fil2 == fil) continue;
-                const f3 d = min_image_pair(p, rv, mk(Q[u]));
-                const float rr = dot(d, d);
-                if (!(rr < rc2)) continue;
-                const float uu = __builtin_amdgcn_rcpf(rr);
-                const float s6 = s2c * uu * (s2c * uu) * (s2c * uu);
-                const float f = 24.0f * eps * uu * s6 * (2.0f * s6 - 1.0f);
-                const float fp = -24.0f * eps * uu * uu * s6 * (14.0f * s6 - 4.0f);  // df / d(r^2)
-                const f3 dl = lam - mk(LF[u]);                                       // lF_i - lF_j
-                Rp += W[u] * (f * dl + (2.0f * fp * dot(d, dl)) * d);                // w H dl
-                epsPart += double(W[u]) * double(dot(lam, d)) * double(f);
-            }
-        }
-        acc[kAdjEpsilon] = -epsPart / double(eps);  // F is linear in epsilon
-        (void)me;
-
-        // adjoint of the step for this bead
-        const f3 Rt = mk(load4(a.lr, m.bead)) + R + Rp;
+        const f3 Rt = lr + R + Rp;
         // the drag -gamma v' is part of F' only with the Langevin thermostat on
-        const f3 V = mk(load4(a.lv, m.bead)) - (a.langevin ? a.gamma : 0.0f) * lam + a.dt * Rt;
-        const f3 lG = mk(load4(a.lG, m.bead));
+        const f3 V = lv - (a.langevin ? a.gamma : 0.0f) * lam + a.dt * Rt;
         a.lr[m.bead] = f4(Rt, 0.0f);
         a.lv[m.bead] = f4(V, 0.0f);
         a.lFout[m.bead] = f4(lG + (0.5f * a.dt * a.dt) * Rt + (0.5f * a.dt) * V, 0.0f);
         a.lG[m.bead] = f4((0.5f * a.dt) * V, 0.0f);
     }
+    acc[kAdjEpsilon] = -eps / double(kp.e.wcaEpsilon);  // F is linear in epsilon
+    double total = 0.0;
+#pragma unroll
+    for (int k = 0; k < kAdjParams; ++k) {
+        const double t = wave_sum_d(acc[k]);
+        total = m.lane == uint32_t(k) ? t : total;
+    }
+    if (m.lane < uint32_t(kAdjParams)) row[m.lane] = mine + total;
 }
 
-__global__ __launch_bounds__(kBlock) void k_adj_step(AdjStepArgs a, KP kp) {
-    const WaveWorm m = wave_worm(kp.p.filamentSize, a.W);
-    double acc[kAdjParams] = {0.0, 0.0, 0.0, 0.0};
-    adj_step_lanes(a, kp, m, 0u, acc);
-    block_partials(acc, a.partial);  // every thread, once (a workgroup barrier inside)
+// Front wavefronts up to which four lanes share a bead: 500 (32,000 beads) 8.1
+// against 13.4 us with a bead a lane, 300 (worms of 37) 7.4 against 9.5, 2,000
+// 25.6 against 17.2 (the pair part's set-up four times over is issue there).
+constexpr uint32_t kAdjQuadWaves = 1024;
+
+// threads of a workgroup, and its front wavefronts (contiguous runs per XCD:
+// the beads of neighbouring worms of a replica share cell lists)
+template <bool QUADS>
+constexpr int kAdjBlock = QUADS ? 320 : kBlock;
+template <bool QUADS>
+__device__ __forceinline__ uint32_t adj_wave() {
+    const uint32_t g = xcd_contiguous(blockIdx.x, gridDim.x);
+    return QUADS ? g : __builtin_amdgcn_readfirstlane(g * (kBlock / 64) + (threadIdx.x >> 6));
+}
+
+template <bool QUADS>
+__global__ __launch_bounds__(kAdjBlock<QUADS>) void k_adj_step(AdjStepArgs a, uint32_t waves, KP kp) {
+    const uint32_t wave = adj_wave<QUADS>();
+    if (wave >= waves) return;
+    adj_group<QUADS>(a, kp, wave, 0u, a.partial + uint64_t(wave) * kAdjParams);
 }
 
 // One adjoint step of every replica of a batch (a: the concatenated arrays;
-// the wavefronts of the batched front kernel).  Each wavefront adds its FP64
-// partials to its own row of a.partial (one row of kAdjParams per
-// wavefront, accumulated over the steps in step order).
-__global__ __launch_bounds__(kBlock) void k_adj_step_batch(AdjStepArgs a0, const BatchRep *__restrict__ reps,
-                                                           uint32_t R, uint32_t waves, uint64_t step) {
-    const uint32_t wave = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+// the wavefronts of the batched front kernel).
+template <bool QUADS>
+__global__ __launch_bounds__(kAdjBlock<QUADS>) void k_adj_step_batch(AdjStepArgs a0, const BatchRep *__restrict__ reps,
+                                                                     uint32_t R, uint32_t waves, uint64_t step) {
+    const uint32_t wave = adj_wave<QUADS>();
     if (wave >= waves) return;
     const uint32_t r = __builtin_amdgcn_readfirstlane(replica_of_wave(reps, R, wave));
     const BatchRep &rep = reps[r];
     const KP &kp = rep.kp;
-    const WaveWorm m = wave_worm_at(wave - rep.waveOffset, kp.p.filamentSize, kp.p.numFilaments);
     AdjStepArgs a = a0;
     const uint32_t b0 = rep.beadOffset;
     a.pos += b0;
@@ -308,13 +465,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_step_batch(AdjStepArgs a0, const
     a.gamma = kp.p.gamma;
     a.seed = rep.seed;
     a.offLgv = rep.rngBase + step * rep.rngStride + rep.revBlocks;
-    double acc[kAdjParams] = {0.0, 0.0, 0.0, 0.0};
-    adj_step_lanes(a, kp, m, b0, acc);
-#pragma unroll
-    for (int k = 0; k < kAdjParams; ++k) {
-        const double t = wave_sum_d(acc[k]);
-        if ((threadIdx.x & 63u) == 0u) a0.partial[uint64_t(wave) * kAdjParams + k] += t;
-    }
+    adj_group<QUADS>(a, kp, wave - rep.waveOffset, b0, a0.partial + uint64_t(wave) * kAdjParams);
 }
 
 // out[r][k] = sum of the rows of replica r's wavefronts, in a fixed order
@@ -563,15 +714,24 @@ __global__ __launch_bounds__(kTotalBlock) void k_adj_total(const double *__restr
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-uint32_t adj_step_blocks(uint32_t W, uint32_t n) {
+// workgroups of the kernels with a bead a lane
+static uint32_t adj_step_blocks(uint32_t W, uint32_t n) {
     const uint32_t wpw = 64u / n;
     return grid_for(((uint64_t(W) + wpw - 1) / wpw) * 64u);
 }
 
+uint32_t adj_step_rows(uint32_t W, uint32_t n) {
+    const uint32_t wpw = 64u / n;
+    return (W + wpw - 1u) / wpw;
+}
+
 hipError_t launch_adj_step(const AdjStepArgs &a, const KP &kp, hipStream_t st) {
-    const uint32_t blocks = adj_step_blocks(a.W, kp.p.filamentSize);
+    const uint32_t blocks = adj_step_rows(a.W, kp.p.filamentSize);
     if (!blocks) return hipSuccess;
-    NW_LAUNCH(k_adj_step, dim3(blocks), dim3(kBlock), 0, st, a, kp);
+    if (blocks <= kAdjQuadWaves)
+        NW_LAUNCH(k_adj_step<true>, dim3(blocks), dim3(kAdjBlock<true>), 0, st, a, blocks, kp);
+    else
+        NW_LAUNCH(k_adj_step<false>, dim3((blocks + 3u) / 4u), dim3(kAdjBlock<false>), 0, st, a, blocks, kp);
     return hipGetLastError();
 }
 
@@ -607,8 +767,11 @@ hipError_t launch_polar_speed_grad(const float4 *pos, const float4 *vel, uint32_
 hipError_t launch_adj_step_batch(const AdjStepArgs &a, const BatchRep *reps, uint32_t R, uint32_t waves,
                                  uint64_t step, hipStream_t st) {
     if (waves == 0) return hipSuccess;
-    NW_LAUNCH(k_adj_step_batch, dim3(grid_for(uint64_t(waves) * 64u)), dim3(kBlock), 0, st, a, reps, R,
-                       waves, step);
+    if (waves <= kAdjQuadWaves)
+        NW_LAUNCH(k_adj_step_batch<true>, dim3(waves), dim3(kAdjBlock<true>), 0, st, a, reps, R, waves, step);
+    else
+        NW_LAUNCH(k_adj_step_batch<false>, dim3((waves + 3u) / 4u), dim3(kAdjBlock<false>), 0, st, a, reps, R, waves,
+                  step);
     return hipGetLastError();
 }
 

@@ -16,14 +16,15 @@ struct AdjStepArgs {
     const float4 *lF;               // adjoint of the step's force
     float4 *lFout;                  // adjoint of the previous force (the other buffer)
     float4 *lr, *lv, *lG;           // updated in place
-    double *partial;                // out: one row of kAdjParams per workgroup
+    double *partial;                // one row of kAdjParams per workgroup, added to
     uint32_t W;
     int langevin;
     float lgvStd, gamma, dt;
     uint64_t seed, offLgv;          // the step's Langevin draws
 };
 
-uint32_t adj_step_blocks(uint32_t W, uint32_t n);
+// workgroups of a step (one per front wavefront): rows of partial
+uint32_t adj_step_rows(uint32_t W, uint32_t n);
 hipError_t launch_adj_step(const AdjStepArgs &a, const KP &kp, hipStream_t st);
 // d S / d r of the bond-tangent nematic order: e the unit eigenvector of the
 // largest eigenvalue of <1.5 b b - 0.5 I>, scale = 3 / bonds
@@ -47,8 +48,7 @@ hipError_t launch_polar_speed_batch(const float4 *pos, const float4 *vel, const 
                                     hipStream_t st);
 // one adjoint step of every replica of a batch (a: concatenated arrays,
 // off over the concatenated cells, ids global; the replicas' own W,
-// Langevin and Philox from reps; a.partial: one row per front wavefront,
-// added to)
+// Langevin and Philox from reps)
 hipError_t launch_adj_step_batch(const AdjStepArgs &a, const BatchRep *reps, uint32_t R, uint32_t waves,
                                  uint64_t step, hipStream_t st);
 // out[r][k] = the sum of replica r's wavefront rows

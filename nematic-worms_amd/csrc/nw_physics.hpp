@@ -116,6 +116,20 @@ __device__ __forceinline__ f3 shfl_up3(f3 a, int d) {
     return mk(__shfl_up(a.x, d, 64), __shfl_up(a.y, d, 64), __shfl_up(a.z, d, 64));
 }
 
+// x of lane I of this lane's quad
+template <int I>
+__device__ __forceinline__ float quad_lane(float x) {
+    constexpr int ctrl = I | I << 2 | I << 4 | I << 6;  // quad_perm
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), ctrl, 0xf, 0xf, true));
+}
+// acc + the four lanes' terms, lane 0's first
+__device__ __forceinline__ void add_quad(f3 &acc, f3 t) {
+    acc += mk(quad_lane<0>(t.x), quad_lane<0>(t.y), quad_lane<0>(t.z));
+    acc += mk(quad_lane<1>(t.x), quad_lane<1>(t.y), quad_lane<1>(t.z));
+    acc += mk(quad_lane<2>(t.x), quad_lane<2>(t.y), quad_lane<2>(t.z));
+    acc += mk(quad_lane<3>(t.x), quad_lane<3>(t.y), quad_lane<3>(t.z));
+}
+
 // ---------------------------------------------------------------------------
 // Whole worms packed per 64-lane wavefront: floor(64/n) worms per wave, bead
 // p of worm w on lane (w mod wpw) * n + p, the remaining lanes idle.

@@ -54,20 +54,6 @@ __host__ __device__ inline RowsLayout rows_layout(uint32_t cap, uint32_t cells) 
     return L;
 }
 
-// x of lane I of this lane's quad
-template <int I>
-__device__ __forceinline__ float quad_lane(float x) {
-    constexpr int ctrl = I | I << 2 | I << 4 | I << 6;  // quad_perm
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), ctrl, 0xf, 0xf, true));
-}
-// acc + the four lanes' terms, lane 0's first
-__device__ __forceinline__ void add_quad(f3 &acc, f3 t) {
-    acc += mk(quad_lane<0>(t.x), quad_lane<0>(t.y), quad_lane<0>(t.z));
-    acc += mk(quad_lane<1>(t.x), quad_lane<1>(t.y), quad_lane<1>(t.z));
-    acc += mk(quad_lane<2>(t.x), quad_lane<2>(t.y), quad_lane<2>(t.z));
-    acc += mk(quad_lane<3>(t.x), quad_lane<3>(t.y), quad_lane<3>(t.z));
-}
-
 // the three stencil cells of x in stencil order: an inner cell's neighbours
 // in one piece, an edge cell's in two (x = 0: Gx - 1, then 0 and 1; x = Gx -
 // 1: Gx - 2 and Gx - 1, then 0), as [a0, a1) and [b0, b1) within a row
