@@ -49,6 +49,7 @@ def test_one_lane_equals_four(nwlib, W, n, G, copies):
         one = [DeviceArray.from_numpy(lib, x) for x in (pos[r], vel[r], *[np.zeros_like(pos[r])] * 3)]
         lib.nwAdjointForward(*[x.p for x in one], W, dt, 2.0, 100.0, 1, steps, K)
         h = (ctypes.c_double * 4)()
-        lib.nwAdjointBackward(DeviceArray.from_numpy(lib, lp[r]).p, None, h)
+        dl1 = DeviceArray.from_numpy(lib, lp[r])
+        lib.nwAdjointBackward(dl1.p, None, h)
         assert np.allclose(got[r], np.array(h), rtol=1e-9, atol=0), (r, got[r], list(h))
     lib.nwBatchSetReplicas(None, 0)
