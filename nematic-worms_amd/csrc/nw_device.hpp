@@ -250,8 +250,13 @@ __device__ __forceinline__ uint32_t srd_hash(const SimParams &p, const SolventPa
 // --------------------------------------------------------------------------
 struct u4 { uint32_t x, y, z, w; };
 
-__host__ __device__ __forceinline__ uint32_t mulhi32(uint32_t a, uint32_t b) {
-    return uint32_t((uint64_t(a) * uint64_t(b)) >> 32);
+// a ^ b ^ c, one three-input operation on the device
+__host__ __device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+#else
+    return a ^ b ^ c;
+#endif
 }
 
 __host__ __device__ __forceinline__ u4 philox4x32_10(u4 c, uint32_t k0, uint32_t k1) {
@@ -259,9 +264,10 @@ __host__ __device__ __forceinline__ u4 philox4x32_10(u4 c, uint32_t k0, uint32_t
     const uint32_t W0 = 0x9E3779B9u, W1 = 0xBB67AE85u;
 #pragma unroll
     for (int r = 0; r < 10; ++r) {
-        const uint32_t hi0 = mulhi32(M0, c.x), lo0 = M0 * c.x;
-        const uint32_t hi1 = mulhi32(M1, c.z), lo1 = M1 * c.z;
-        c = u4{hi1 ^ c.y ^ k0, lo1, hi0 ^ c.w ^ k1, lo0};
+        // both halves of a product by one 64-bit multiply-add (the 32-bit
+        // multiplies are a quarter of the rate each)
+        const uint64_t p0 = uint64_t(M0) * c.x, p1 = uint64_t(M1) * c.z;
+        c = u4{xor3(uint32_t(p1 >> 32), c.y, k0), uint32_t(p1), xor3(uint32_t(p0 >> 32), c.w, k1), uint32_t(p0)};
         k0 += W0;
         k1 += W1;
     }

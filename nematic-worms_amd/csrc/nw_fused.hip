@@ -40,6 +40,15 @@ __device__ __forceinline__ FrontLane md_front_lane(const KP &kp, const WaveWorm 
     const uint32_t b = m.active ? m.bead : 0u;
     const v4 Pl = reinterpret_cast<const v4 *>(pos)[b], Vl = reinterpret_cast<const v4 *>(vel)[b];
     const v4 Fl = reinterpret_cast<const v4 *>(force)[b], FOl = reinterpret_cast<const v4 *>(forceOld)[b];
+    // The step's parameters in scalar registers, read together here: a
+    // replica's lie in memory, and each one read where it is first used was a
+    // scalar load waited for by itself, some fifteen in a row (a batch of 16
+    // replicas of 8,000 beads: 10.4 us without, 9.4 with).
+    asm volatile("" ::"s"(p.origin.x), "s"(p.origin.y), "s"(p.origin.z), "s"(p.boxSize.x), "s"(p.boxSize.y),
+                 "s"(p.boxSize.z), "s"(p.boundaryX), "s"(p.boundaryY), "s"(p.boundaryZ), "s"(p.gridSize.x),
+                 "s"(p.gridSize.y), "s"(p.gridSize.z), "s"(p.cellSize.x), "s"(p.cellSize.y), "s"(p.bondSpringK),
+                 "s"(p.bondSpringL), "s"(p.bondBendingK), "s"(p.reverseProbability), "s"(p.gamma),
+                 "s"(kp.e.driveForce), "s"(kp.e.bondedMode));
     // the random draws depend on the bead alone: formed while the loads are
     // in flight
     const bool rev = p.reverseProbability > 0.0f && m.active &&

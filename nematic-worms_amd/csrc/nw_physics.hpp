@@ -45,7 +45,18 @@ __device__ __forceinline__ void noslip_wall(f3 &pos, int axis, f3 &vel, f3 dr, f
     }
 }
 
+// periodic_bc without a branch
+__device__ __forceinline__ float periodic_select(float r, float L0, float L) {
+    return r < L0 ? r + L : (r > L + L0 ? r - L : r);
+}
+
 __device__ __forceinline__ void apply_boundaries(const SimParams &p, f3 &pos, f3 &vel, f3 dr, float R) {
+    // a box periodic on every axis (PERIODIC is 0): no branch of the lanes
+    if ((p.boundaryX | p.boundaryY | p.boundaryZ) == PERIODIC) {
+        pos = mk(periodic_select(pos.x, p.origin.x, p.boxSize.x), periodic_select(pos.y, p.origin.y, p.boxSize.y),
+                 periodic_select(pos.z, p.origin.z, p.boxSize.z));
+        return;
+    }
     if (p.boundaryX == PERIODIC) periodic_bc(pos.x, p.origin.x, p.boxSize.x);
     else if (p.boundaryX == WALL) damped_wall(pos.x, vel.x, p.boundaryDamping, p.origin.x, p.boxSize.x, R);
     else if (p.boundaryX == WALL_NO_SLIP)
@@ -179,22 +190,22 @@ __device__ __forceinline__ bool bonded_lane(const KP &kp, f3 r, uint32_t pp, f3 
     const SimParams &p = kp.p;
     const uint32_t n = p.filamentSize;
     const f3 rn1 = shfl_down3(r, 1);
-    const f3 rn2 = shfl_down3(r, 2);
-    const f3 rp1 = shfl_up3(r, 1);
+    // the bond (pp, pp + 1) and its length, once; the bond (pp + 1, pp + 2) is
+    // the next lane's, the same values from the same positions.
+    // min_image_pair: min_image's value, the wrap tests only when some lane's
+    // chain spans half the box
+    const f3 r_ij = min_image_pair(p, r, rn1);
+    const float dd = dot(r_ij, r_ij), d_ij = sqrtf(dd);
+    const f3 r_jk = shfl_down3(r_ij, 1);
+    const float dd_jk = __shfl_down(dd, 1, 64), d_jk = __shfl_down(d_ij, 1, 64);
 
     f3 fi = mk(0.f, 0.f, 0.f), fj = fi, fk = fi;
     const bool hasTriple = n >= 3 && pp + 2u < n;
     if (hasTriple) {
-        // min_image_pair: min_image's value, the wrap tests only when some
-        // lane's chain spans half the box
-        const f3 r_ij = min_image_pair(p, r, rn1);
-        const f3 r_jk = min_image_pair(p, rn1, rn2);
-        const float d_ij = length(r_ij);
-        const float d_jk = length(r_jk);
         const float d_ij_jk = dot(r_ij, r_jk);
         const float A = p.bondBendingK / (d_ij * d_jk);
-        const f3 B = r_ij * d_ij_jk / dot(r_ij, r_ij);
-        const f3 C = r_jk * d_ij_jk / dot(r_jk, r_jk);
+        const f3 B = r_ij * d_ij_jk / dd;
+        const f3 C = r_jk * d_ij_jk / dd_jk;
         fi = -A * (r_jk - B);
         fk = -A * (C - r_ij);
         fj = mk(-fi.x - fk.x, -fi.y - fk.y, -fi.z - fk.z);
@@ -205,10 +216,8 @@ __device__ __forceinline__ bool bonded_lane(const KP &kp, f3 r, uint32_t pp, f3 
     const bool chain = kp.e.bondedMode == NW_BONDED_CHAIN;
     f3 fb = mk(0.f, 0.f, 0.f), drive = fb;
     if (chain && pp + 1u < n) {
-        const f3 d = min_image_pair(p, r, rn1);
-        const float len = length(d);
-        fb = (p.bondSpringK * (len - p.bondSpringL) / len) * d;
-        drive = (kp.e.driveForce / len) * d;
+        fb = (p.bondSpringK * (d_ij - p.bondSpringL) / d_ij) * r_ij;
+        drive = (kp.e.driveForce / d_ij) * r_ij;
     }
     const f3 fb_prev = shfl_up3(fb, 1);
 
@@ -223,6 +232,7 @@ __device__ __forceinline__ bool bonded_lane(const KP &kp, f3 r, uint32_t pp, f3 
         }
     }
     if (n < 3 || !wantTan) return false;
+    const f3 rp1 = shfl_up3(r, 1);
     if (pp == 0u) tg = tangent_of(p, r, rn1);
     else if (pp + 1u < n) tg = tangent_of(p, rp1, rn1);
     else {
