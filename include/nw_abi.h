@@ -369,7 +369,7 @@ void nwBatchLayout(uint *beadOffset, uint *cellOffset);
 /* `steps` fused MD steps of every replica over the concatenated arrays
    (sortedVel / sortedTangent may be NULL as in nwFusedMdStep).  useGraph:
    after one direct step, the step is captured once as a hipGraph (per
-   argument set) and replayed. */
+   argument set) and replayed; the call's last step is direct. */
 void nwBatchMdStep(float *pos, float *vel, float *force, float *forceOld, float *tangent,
                    uint *gridParticleIndex, float *sortedPos, float *sortedVel, float *sortedTangent,
                    float deltaTime, uint steps, int useGraph);
