@@ -10,7 +10,7 @@
 //             writes the prefix as one row of P, then its (cell, id) pairs
 //             grouped by bucket into its pair region (staged in LDS and
 //             written out coalesced when the tile fits)
-//   level 2   (k_bucket_cells) a workgroup per bucket, buckets mapped to
+//   level 2   (k_md_cells, k_srd_cells) a workgroup per bucket, buckets mapped to
 //             XCDs in contiguous runs so neighbours share L2 lines of P: the
 //             column sum of P at the bucket is its first sorted slot, the
 //             column differences are its segments in the tiles' regions; the
@@ -22,6 +22,7 @@
 //             rotates about its cell's momentum, solvent streams
 // Results are deterministic and equal to a stable sort by cell.
 #include <algorithm>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -66,12 +67,19 @@ Tuning &tuning() {
     return t;
 }
 
+// Bucket population the MD sort aims at: two buckets a CU of a system up to
+// 786,000 beads, but no fewer than 512 beads (its second level at 1,536 / 512
+// a bucket: 229,000 beads 7.9 / 6.5 us, 96,000 with three records 10.4 / 6.6;
+// at 256 7.2 and 6.6), 1,536 from there (800,000: 12.0 us, at 512 13.5: more
+// prefix rows to read).
+static uint32_t md_members(uint64_t n) { return uint32_t(std::min<uint64_t>(std::max<uint64_t>(n / 512u, 512u), 1536u)); }
+
 BucketPlan fused_plan(uint64_t n, uint64_t cells, bool srd) {
     const Tuning &t = tuning();
     const uint32_t items = srd ? t.srdTileItems : t.mdTileItems;
     const uint32_t members = srd ? t.srdMembers : t.mdMembers;
-    const BucketPlan bp = make_bucket_plan(n, cells, items, members ? members : 1536u);
-    if ((items || members) && *bucket_plan_problem(bp)) return make_bucket_plan(n, cells, 0);
+    const BucketPlan bp = make_bucket_plan(n, cells, items, members ? members : (srd ? 1536u : md_members(n)));
+    if ((items || members) && *bucket_plan_problem(bp)) return make_bucket_plan(n, cells, 0, srd ? 1536u : md_members(n));
     return bp;
 }
 
@@ -97,7 +105,8 @@ __host__ __device__ inline CellsLayout cells_layout(const BucketPlan &bp, bool s
     uint32_t o = 0;
     L.wsum = o; o += align16(4u * 2u * (kCellsBlockMax / 64));
     L.cnt = o;  o += align16(4u * (nc + 1));
-    L.cur = o;  o += align16(4u * nc);
+    // MD: the placement cursors of an unstaged bucket, or a staged one's ids in order
+    L.cur = o;  o += align16(srd ? 4u * nc : max(4u * nc, 4u * cap));
     L.lid = o;  o += align16(4u * cap);
     L.lcell = o; if (!srd) o += align16(2u * cap);
     // segment tables (the staged members themselves wait in registers)
@@ -347,61 +356,6 @@ __device__ __forceinline__ uint32_t seg_of(const uint32_t *segStart, uint32_t ti
 }
 
 
-// MD level 2, staged bucket of m members: ids, cells and the gathered
-// records of the sorted slots, in groups of G members per thread with the
-// gathers of a group in flight together; past the last member a thread
-// handles member m - 1 again (the same values to the same addresses)
-template <bool POS, bool VEL, bool TAN, int BLOCK, int G>
-__device__ __forceinline__ void md_gather_group(const CellsArgs &o, const uint32_t *lid, const uint16_t *lcell,
-                                                uint32_t sb, uint32_t cell0, uint32_t m, uint32_t j0) {
-    // records moved as plain 4-vectors (register values, never a copy of a
-    // float4 object through memory)
-    typedef float v4 __attribute__((ext_vector_type(4)));
-    const v4 *pos = reinterpret_cast<const v4 *>(o.pos), *vel = reinterpret_cast<const v4 *>(o.vel),
-             *tan = reinterpret_cast<const v4 *>(o.tan);
-    v4 *sPos = reinterpret_cast<v4 *>(o.sPos), *sVel = reinterpret_cast<v4 *>(o.sVel),
-       *sTan = reinterpret_cast<v4 *>(o.sTan);
-    const uint32_t tid = threadIdx.x;
-    uint32_t *out = o.ids + sb;
-    {
-        uint32_t k[G], id[G];
-        v4 P[G], V[G], Tn[G];
-#pragma unroll
-        for (int j = 0; j < G; ++j) {
-            k[j] = min(tid + (j0 + uint32_t(j)) * BLOCK, m - 1u);
-            id[j] = lid[k[j]];
-        }
-#pragma unroll
-        for (int j = 0; j < G; ++j) {
-            if (POS) P[j] = pos[id[j]];
-            if (VEL) V[j] = vel[id[j]];
-            if (TAN) Tn[j] = tan[id[j]];
-        }
-#pragma unroll
-        for (int j = 0; j < G; ++j) {
-            out[k[j]] = id[j];
-            o.cellOf[sb + k[j]] = o.cellBase + cell0 + uint32_t(lcell[k[j]]);
-            if (POS) sPos[sb + k[j]] = P[j];
-            if (VEL) sVel[sb + k[j]] = V[j];
-            if (TAN) sTan[sb + k[j]] = Tn[j];
-        }
-    }
-}
-
-template <bool POS, bool VEL, bool TAN, int BLOCK, int CAP>
-__device__ __forceinline__ void md_gather_staged(const CellsArgs &o, const uint32_t *lid, const uint16_t *lcell,
-                                                 uint32_t sb, uint32_t cell0, uint32_t m) {
-    // groups of two members, a group's gathers in flight together (groups of
-    // four measured about 0.4 us slower per launch at 800k beads)
-    constexpr int PER = CAP / BLOCK, G = PER < 2 ? PER : 2;
-#pragma unroll
-    for (int g = 0; g < PER; g += G)
-        if (m > uint32_t(g) * BLOCK) md_gather_group<POS, VEL, TAN, BLOCK, G>(o, lid, lcell, sb, cell0, m, g);
-}
-
-// Bucket b of one system (see CellsArgs for the bases of a replica), BLOCK
-// threads; a bucket of at most CAP members is staged in LDS, each thread
-// holding at most PER = CAP / BLOCK of them.
 // Ascending sort of N values in registers (N a power of two): Batcher's
 // odd-even merge network (63 compare-exchanges for 16 against the bitonic
 // network's 80), every compare-exchange at a compile-time position
@@ -559,37 +513,22 @@ __device__ __forceinline__ void fill_tile_of(uint16_t *tileOf, uint32_t *wsum) {
     __syncthreads();
 }
 
-template <bool SRD, int BLOCK, int CAP = int(kBucketCap)>
-__device__ __forceinline__ void bucket_cells_body(const CellsArgs &o, const BucketPlan &bp, uint32_t b,
-                                                  unsigned char *smem) {
-    constexpr int PER = CAP / BLOCK;
-    static_assert(PER * BLOCK == CAP, "the staged members are PER per thread");
-    const CellsLayout L = cells_layout(bp, SRD, CAP);
-    uint32_t *wsum = reinterpret_cast<uint32_t *>(smem + L.wsum);
-    uint32_t *cnt = reinterpret_cast<uint32_t *>(smem + L.cnt);
-    uint32_t *cur = reinterpret_cast<uint32_t *>(smem + L.cur);
-    uint32_t *lid = reinterpret_cast<uint32_t *>(smem + L.lid);
-    uint16_t *lcell = reinterpret_cast<uint16_t *>(smem + L.lcell);
-    uint32_t *segStart = reinterpret_cast<uint32_t *>(smem + L.segStart);
-    uint32_t *segBase = reinterpret_cast<uint32_t *>(smem + L.segBase);
-    uint16_t *tileOf = reinterpret_cast<uint16_t *>(smem + L.tileOf);
-
-    const uint32_t B1 = bp.buckets + 1;
-    const uint32_t tid = threadIdx.x, bd = blockDim.x;
-    const uint32_t cell0 = b << bp.shift;
-    const uint32_t nc = min(1u << bp.shift, bp.cells - cell0);
-    // cleared here, under the barriers of the segment pass: the cell counts
-    // and the member tile marks (tileOf, CAP entries over lid)
-    for (uint32_t c = tid; c < nc; c += bd) cnt[c] = 0u;
-    for (uint32_t k = tid; k < uint32_t(CAP) / 2u; k += bd) reinterpret_cast<uint32_t *>(tileOf)[k] = 0u;
-
-    // segments of this bucket in every tile; first sorted slot.  With tile
-    // ranges, only the tiles whose members reach this bucket have their row
-    // read: a tile wholly below it contributes all its members to the slot,
-    // one wholly above none.
-    uint32_t part = 0;
-    for (uint32_t t = tid; t < bp.tiles; t += bd) {
-        uint32_t lo = 0u, len = 0u;
+// The segments of bucket b in the tiles' regions: segBase[t] the segment's
+// start within tile t's region, segStart[t] the bucket member it begins with
+// and, in tileOf (cleared), the tile at the first slot of every nonempty one.
+// Returns the bucket's first sorted slot, m its members.  With tile ranges,
+// only the tiles whose members reach this bucket have their row read: a tile
+// wholly below it contributes all its members to the slot, one wholly above
+// none.  Up to BLOCK tiles (a million beads), one tile a thread: both sums in
+// one pass of register scans and one barrier.
+template <int BLOCK, int CAP>
+__device__ __forceinline__ uint32_t bucket_segments(const CellsArgs &o, const BucketPlan &bp, uint32_t b,
+                                                    uint32_t *segStart, uint32_t *segBase, uint16_t *tileOf,
+                                                    uint32_t *wsum, uint32_t &m) {
+    constexpr uint32_t NW = BLOCK / 64;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wid = tid >> 6, B1 = bp.buckets + 1;
+    const auto segment = [&](uint32_t t, uint32_t &lo, uint32_t &len) {
+        lo = len = 0u;
         bool read = true;
         if (o.tileRange) {
             const uint32_t r0 = o.tileRange[2u * t], r1 = o.tileRange[2u * t + 1u];
@@ -601,17 +540,240 @@ __device__ __forceinline__ void bucket_cells_body(const CellsArgs &o, const Buck
             lo = row[0];
             len = row[1] - lo;
         }
+    };
+    if (bp.tiles <= uint32_t(BLOCK)) {
+        uint32_t lo = 0u, len = 0u;
+        if (tid < bp.tiles) segment(tid, lo, len);
+        const uint32_t sl = wave_scan_add(len), sp = wave_scan_add(lo);
+        if (lane == 63u) {
+            wsum[wid] = sl;
+            wsum[NW + wid] = sp;
+        }
+        __syncthreads();
+        const uint32_t ws = wave_scan_add(lane < 2u * NW ? wsum[lane] : 0u);
+        m = uint32_t(__builtin_amdgcn_readlane(int(ws), int(NW) - 1));
+        const uint32_t before =
+            wid ? uint32_t(__builtin_amdgcn_readlane(int(ws), int(__builtin_amdgcn_readfirstlane(wid)) - 1)) : 0u;
+        if (tid < bp.tiles) {
+            const uint32_t at = before + sl - len;
+            segStart[tid] = at;
+            segBase[tid] = lo;
+            if (len != 0u && at < uint32_t(CAP)) tileOf[at] = uint16_t(tid);
+        }
+        __syncthreads();
+        return uint32_t(__builtin_amdgcn_readlane(int(ws), 2 * int(NW) - 1)) - m;
+    }
+    uint32_t part = 0;
+    for (uint32_t t = tid; t < bp.tiles; t += BLOCK) {
+        uint32_t lo, len;
+        segment(t, lo, len);
         segBase[t] = lo;
         segStart[t] = len;
         part += lo;
     }
     part = wave_scan_add(part);
-    if ((tid & 63u) == 63u) wsum[BLOCK / 64 + (tid >> 6)] = part;  // upper half of wsum
+    if (lane == 63u) wsum[NW + wid] = part;  // upper half of wsum
     __syncthreads();
     uint32_t sb = 0;
-    for (uint32_t w = 0; w < BLOCK / 64; ++w) sb += wsum[BLOCK / 64 + w];
+    for (uint32_t w = 0; w < NW; ++w) sb += wsum[NW + w];
     block_excl_scan<false, true>(segStart, bp.tiles, wsum, nullptr, tileOf, uint32_t(CAP));
-    const uint32_t m = segStart[bp.tiles];
+    m = segStart[bp.tiles];
+    return sb;
+}
+
+// Exclusive prefix of the nc cell counts in LDS in place (zero up to the next
+// multiple of four; nc at most 2048), cnt[nc] = m their sum: four consecutive
+// cells a thread and round, one 16-byte read and write each.  (One cell after
+// another at a stride of eight cells a thread, every read met its bank
+// fifteen times over: 1.4 us of a bucket's 8.5.)
+template <int BLOCK>
+__device__ __forceinline__ void scan_cells(uint32_t *cnt, uint32_t nc, uint32_t m, uint32_t *wsum) {
+    constexpr uint32_t NW = BLOCK / 64, R = BLOCK >= 512 ? 1u : 2048u / (4u * BLOCK);
+    typedef uint32_t w4 __attribute__((ext_vector_type(4)));
+    w4 *c4 = reinterpret_cast<w4 *>(cnt);
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wid = tid >> 6;
+    w4 v[R];
+    uint32_t s[R], incl[R];
+#pragma unroll
+    for (uint32_t r = 0; r < R; ++r) {
+        const uint32_t i = r * BLOCK + tid;
+        v[r] = 4u * i < nc ? c4[i] : w4{0u, 0u, 0u, 0u};
+        s[r] = v[r].x + v[r].y + v[r].z + v[r].w;
+        incl[r] = wave_scan_add(s[r]);
+        if (lane == 63u) wsum[r * NW + wid] = incl[r];
+    }
+    __syncthreads();
+    const uint32_t ws = wave_scan_add(lane < R * NW ? wsum[lane] : 0u);
+#pragma unroll
+    for (uint32_t r = 0; r < R; ++r) {
+        const uint32_t i = r * BLOCK + tid, w = __builtin_amdgcn_readfirstlane(r * NW + wid);
+        const uint32_t a = incl[r] - s[r] + (w ? uint32_t(__builtin_amdgcn_readlane(int(ws), int(w) - 1)) : 0u);
+        if (4u * i < nc) c4[i] = w4{a, a + v[r].x, a + v[r].x + v[r].y, a + v[r].x + v[r].y + v[r].z};
+    }
+    if (tid == 0u) cnt[nc] = m;  // nc no multiple of four: what the last vector holds there
+    __syncthreads();
+}
+
+// what the MD sort gathers beside the ids and cells
+enum : int { kGatherPos = 1, kGatherVel = 2, kGatherTan = 4 };
+
+// MD, bucket b of one system (see CellsArgs for the bases of a replica),
+// BLOCK threads; a bucket of at most CAP members is staged in LDS, each
+// thread holding at most PER = CAP / BLOCK of them from their load to the
+// store of their records.
+// A bucket is one chain of loads, LDS passes and barriers, and with three
+// buckets or fewer on a CU their length is the kernel's time.  So a member's
+// records are fetched as soon as its id is known and wait in registers; the
+// count of its cell hands it its place; and its rank among the ids of its
+// cell (the order of a stable sort by cell) is counted by the member itself,
+// where one thread a cell ran through up to eight cells' insertion sorts one
+// after another.  Before and after: 229,000 beads 11.4 us, 6.6; 96,000 with
+// three records a bead 14.0, 6.8; 30,000 (order only) 10.8, 5.1; 800,000
+// 13.8, 11.0; 21.9 million in a batch, bound by memory, 278, 264.
+template <int GATHER, int BLOCK, int CAP>
+__device__ __forceinline__ void md_cells_body(const CellsArgs &o, const BucketPlan &bp, uint32_t b,
+                                              unsigned char *smem) {
+    constexpr int PER = CAP / BLOCK;
+    static_assert(PER * BLOCK == CAP, "the staged members are PER per thread");
+    constexpr bool POS = GATHER & kGatherPos, VEL = GATHER & kGatherVel, TAN = GATHER & kGatherTan;
+    // records moved as plain 4-vectors (register values, never a copy of a
+    // float4 object through memory)
+    typedef float v4 __attribute__((ext_vector_type(4)));
+    const CellsLayout L = cells_layout(bp, false, CAP);
+    uint32_t *wsum = reinterpret_cast<uint32_t *>(smem + L.wsum);
+    uint32_t *cnt = reinterpret_cast<uint32_t *>(smem + L.cnt);
+    uint32_t *cur = reinterpret_cast<uint32_t *>(smem + L.cur);
+    uint32_t *lid = reinterpret_cast<uint32_t *>(smem + L.lid);
+    uint16_t *lcell = reinterpret_cast<uint16_t *>(smem + L.lcell);
+    uint32_t *segStart = reinterpret_cast<uint32_t *>(smem + L.segStart);
+    uint32_t *segBase = reinterpret_cast<uint32_t *>(smem + L.segBase);
+    uint16_t *tileOf = reinterpret_cast<uint16_t *>(smem + L.tileOf);
+
+    const uint32_t tid = threadIdx.x;
+    const uint32_t cell0 = b << bp.shift;
+    const uint32_t nc = min(1u << bp.shift, bp.cells - cell0);
+    // cleared here, under the barriers of the segment pass: the cell counts
+    // and the member tile marks (tileOf, CAP entries over lid)
+    for (uint32_t c = tid; c < ((nc + 3u) & ~3u); c += BLOCK) cnt[c] = 0u;
+    for (uint32_t k = tid; k < uint32_t(CAP) / 2u; k += BLOCK) reinterpret_cast<uint32_t *>(tileOf)[k] = 0u;
+    uint32_t m;
+    const uint32_t sb = bucket_segments<BLOCK, CAP>(o, bp, b, segStart, segBase, tileOf, wsum, m);
+    const uint64_t T = bp.tileItems;
+    uint32_t *out = o.ids + sb;
+
+    if (m <= uint32_t(CAP)) {
+        uint2 q[PER];
+        uint32_t rk[PER];
+        v4 P[POS ? PER : 1], V[VEL ? PER : 1], Tn[TAN ? PER : 1];
+        if (m) {
+            fill_tile_of<BLOCK, PER>(tileOf, wsum);
+            // every load of the thread's members in flight before the first
+            // use (indices past the last member load the last member again,
+            // unused)
+#pragma unroll
+            for (int j = 0; j < PER; ++j) {
+                const uint32_t k = min(tid + uint32_t(j) * BLOCK, m - 1u);
+                const uint32_t t = tileOf[k];
+                q[j] = unpack_pair(o.pairs[uint64_t(t) * T + segBase[t] + (k - segStart[t])], o.idBase + t * uint32_t(T));
+            }
+#pragma unroll
+            for (int j = 0; j < PER; ++j) {
+                if (POS) P[j] = reinterpret_cast<const v4 *>(o.pos)[q[j].y];
+                if (VEL) V[j] = reinterpret_cast<const v4 *>(o.vel)[q[j].y];
+                if (TAN) Tn[j] = reinterpret_cast<const v4 *>(o.tan)[q[j].y];
+            }
+#pragma unroll
+            for (int j = 0; j < PER; ++j)
+                if (tid + uint32_t(j) * BLOCK < m) rk[j] = atomicAdd(&cnt[q[j].x], 1u);
+        }
+        __syncthreads();
+        scan_cells<BLOCK>(cnt, nc, m, wsum);
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            if (tid + uint32_t(j) * BLOCK < m) {
+                const uint32_t slot = cnt[q[j].x] + rk[j];
+                lid[slot] = q[j].y;
+                lcell[slot] = uint16_t(q[j].x);
+            }
+        }
+        for (uint32_t c = tid; c < nc; c += BLOCK) o.off[cell0 + c] = o.slotBase + sb + cnt[c];
+        if (tid == 0u && cell0 + nc == bp.cells) o.off[bp.cells] = o.slotBase + bp.n;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            if (tid + uint32_t(j) * BLOCK < m) {
+                const uint32_t a = cnt[q[j].x], z = cnt[q[j].x + 1u];
+                uint32_t r = a;
+                for (uint32_t u = a; u < z; ++u) r += lid[u] < q[j].y ? 1u : 0u;
+                cur[r] = q[j].y;
+                if (POS) reinterpret_cast<v4 *>(o.sPos)[sb + r] = P[j];
+                if (VEL) reinterpret_cast<v4 *>(o.sVel)[sb + r] = V[j];
+                if (TAN) reinterpret_cast<v4 *>(o.sTan)[sb + r] = Tn[j];
+            }
+        }
+        __syncthreads();
+        for (uint32_t k = tid; k < m; k += BLOCK) {
+            out[k] = cur[k];
+            o.cellOf[sb + k] = o.cellBase + cell0 + uint32_t(lcell[k]);
+        }
+        return;
+    }
+
+    // more members than the stage: through memory
+    for (uint32_t k = tid; k < m; k += BLOCK) {
+        const uint32_t t = seg_of(segStart, bp.tiles, k);
+        atomicAdd(&cnt[o.pairs[uint64_t(t) * T + segBase[t] + (k - segStart[t])] >> kPairIdBits], 1u);
+    }
+    __syncthreads();
+    block_excl_scan<true>(cnt, nc, wsum, cur);
+    for (uint32_t k = tid; k < m; k += BLOCK) {
+        const uint32_t t = seg_of(segStart, bp.tiles, k);
+        const uint2 q =
+            unpack_pair(o.pairs[uint64_t(t) * T + segBase[t] + (k - segStart[t])], o.idBase + t * uint32_t(T));
+        out[atomicAdd(&cur[q.x], 1u)] = q.y;
+    }
+    __syncthreads();
+    for (uint32_t c = tid; c < nc; c += BLOCK) {
+        const uint32_t a = cnt[c], z = cnt[c + 1];
+        sort_cell_ids<1>(out, a, z);
+        o.off[cell0 + c] = o.slotBase + sb + a;
+    }
+    if (tid == 0 && cell0 + nc == bp.cells) o.off[bp.cells] = o.slotBase + bp.n;
+    __syncthreads();
+    for (uint32_t k = tid; k < m; k += BLOCK) {
+        const uint32_t id = out[k];
+        o.cellOf[sb + k] = o.cellBase + cell0 + seg_of(cnt, nc, k);
+        if (POS) o.sPos[sb + k] = o.pos[id];
+        if (VEL) o.sVel[sb + k] = o.vel[id];
+        if (TAN) o.sTan[sb + k] = o.tan[id];
+    }
+}
+
+// SRD, bucket b; staged as the MD sort's
+template <int BLOCK, int CAP = int(kBucketCap)>
+__device__ __forceinline__ void srd_cells_body(const CellsArgs &o, const BucketPlan &bp, uint32_t b,
+                                                  unsigned char *smem) {
+    constexpr int PER = CAP / BLOCK;
+    static_assert(PER * BLOCK == CAP, "the staged members are PER per thread");
+    const CellsLayout L = cells_layout(bp, true, CAP);
+    uint32_t *wsum = reinterpret_cast<uint32_t *>(smem + L.wsum);
+    uint32_t *cnt = reinterpret_cast<uint32_t *>(smem + L.cnt);
+    uint32_t *cur = reinterpret_cast<uint32_t *>(smem + L.cur);
+    uint32_t *lid = reinterpret_cast<uint32_t *>(smem + L.lid);
+    uint32_t *segStart = reinterpret_cast<uint32_t *>(smem + L.segStart);
+    uint32_t *segBase = reinterpret_cast<uint32_t *>(smem + L.segBase);
+    uint16_t *tileOf = reinterpret_cast<uint16_t *>(smem + L.tileOf);
+
+    const uint32_t tid = threadIdx.x, bd = blockDim.x;
+    const uint32_t cell0 = b << bp.shift;
+    const uint32_t nc = min(1u << bp.shift, bp.cells - cell0);
+    // cleared here, under the barriers of the segment pass: the cell counts
+    // and the member tile marks (tileOf, CAP entries over lid)
+    for (uint32_t c = tid; c < nc; c += bd) cnt[c] = 0u;
+    for (uint32_t k = tid; k < uint32_t(CAP) / 2u; k += bd) reinterpret_cast<uint32_t *>(tileOf)[k] = 0u;
+
+    uint32_t m;
+    const uint32_t sb = bucket_segments<BLOCK, CAP>(o, bp, b, segStart, segBase, tileOf, wsum, m);
 
     const bool staged = m <= uint32_t(CAP);
     const uint64_t T = bp.tileItems;
@@ -652,7 +814,6 @@ __device__ __forceinline__ void bucket_cells_body(const CellsArgs &o, const Buck
                 const uint32_t lc = q[j].x;
                 const uint32_t slot = atomicAdd(&cur[lc], 1u);
                 lid[slot] = q[j].y;
-                if (!SRD) lcell[slot] = uint16_t(lc);
             }
         }
     } else {
@@ -667,7 +828,7 @@ __device__ __forceinline__ void bucket_cells_body(const CellsArgs &o, const Buck
     // SRD, one system: the cells' rotation signs, one Philox block per four
     // cells (uniform_at's draws) computed once -- by the first wave for a
     // bucket of up to 256 cells -- into cur, free after the placement
-    if (SRD && !o.srdReps) {
+    if (!o.srdReps) {
         const uint32_t b0 = cell0 >> 2, nb = ((cell0 + nc - 1u) >> 2) - b0 + 1u;
         for (uint32_t t = tid; t < nb; t += bd) {
             const u4 r = philox_block(o.seed, o.offset + b0 + t);
@@ -680,38 +841,17 @@ __device__ __forceinline__ void bucket_cells_body(const CellsArgs &o, const Buck
         }
     }
     // every cell in ascending id order; CSR offsets.  SRD cells hold ~6
-    // particles (a network of 16 takes all but the rare crowded ones); MD
-    // cells hold ~1 bead.  The two storages take separate calls so that the
-    // staged ids are read as LDS, not through a generic pointer.
+    // particles (a network of 16 takes all but the rare crowded ones).  The
+    // two storages take separate calls so that the staged ids are read as
+    // LDS, not through a generic pointer.
     for (uint32_t c = tid; c < nc; c += bd) {
         const uint32_t a = cnt[c], z = cnt[c + 1];
-        if (staged) sort_cell_ids<SRD ? 16 : 1>(lid, a, z);
-        else sort_cell_ids<SRD ? 16 : 1>(out, a, z);
+        if (staged) sort_cell_ids<16>(lid, a, z);
+        else sort_cell_ids<16>(out, a, z);
         o.off[cell0 + c] = o.slotBase + sb + a;
     }
     if (tid == 0 && cell0 + nc == bp.cells) o.off[bp.cells] = o.slotBase + bp.n;
     __syncthreads();
-
-    if (!SRD) {
-        if (staged) {
-            if (!o.sPos) md_gather_staged<false, false, false, BLOCK, CAP>(o, lid, lcell, sb, cell0, m);
-            else if (o.sVel && o.sTan) md_gather_staged<true, true, true, BLOCK, CAP>(o, lid, lcell, sb, cell0, m);
-            else if (o.sVel) md_gather_staged<true, true, false, BLOCK, CAP>(o, lid, lcell, sb, cell0, m);
-            else if (o.sTan) md_gather_staged<true, false, true, BLOCK, CAP>(o, lid, lcell, sb, cell0, m);
-            else md_gather_staged<true, false, false, BLOCK, CAP>(o, lid, lcell, sb, cell0, m);
-            return;
-        }
-        for (uint32_t k = tid; k < m; k += bd) {
-            const uint32_t id = out[k];
-            o.cellOf[sb + k] = o.cellBase + cell0 + seg_of(cnt, nc, k);
-            if (o.sPos) {
-                o.sPos[sb + k] = o.pos[id];
-                if (o.sVel) o.sVel[sb + k] = o.vel[id];
-                if (o.sTan) o.sTan[sb + k] = o.tan[id];
-            }
-        }
-        return;
-    }
 
     // SRD: the sorted ids out.  The cell sums below read the velocities from
     // memory by id (with the solvent in cell order those reads are near
@@ -747,17 +887,23 @@ __device__ __forceinline__ void bucket_cells_body(const CellsArgs &o, const Buck
     }
 }
 
-template <bool SRD, int BLOCK>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_bucket_cells(CellsArgs o, BucketPlan bp) {
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_srd_cells(CellsArgs o, BucketPlan bp) {
     extern __shared__ __align__(16) unsigned char smem[];
-    bucket_cells_body<SRD, BLOCK>(o, bp, xcd_contiguous(blockIdx.x, gridDim.x), smem);
+    srd_cells_body<BLOCK>(o, bp, xcd_contiguous(blockIdx.x, gridDim.x), smem);
+}
+
+template <int GATHER, int BLOCK, int CAP>
+__global__ __launch_bounds__(BLOCK) void k_md_cells(CellsArgs o, BucketPlan bp) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    md_cells_body<GATHER, BLOCK, CAP>(o, bp, xcd_contiguous(blockIdx.x, gridDim.x), smem);
 }
 
 // level 2 of the batched sort: every replica's buckets in one launch; the
 // arrays are offset to the replica's first bead and cell, the bead ids in the
 // pairs are global
-template <int BLOCK, int CAP>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_bucket_cells_batch(CellsArgs a, const SortRep *__restrict__ reps,
+template <int GATHER, int BLOCK, int CAP>
+__global__ __launch_bounds__(BLOCK) void k_md_cells_batch(CellsArgs a, const SortRep *__restrict__ reps,
                                                               uint32_t R) {
     extern __shared__ __align__(16) unsigned char smem[];
     const uint32_t v = xcd_contiguous(blockIdx.x, gridDim.x);
@@ -768,13 +914,13 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(7, 8))) v
     o.ids = a.ids + r.beadOffset;
     o.off = a.off + r.cellOffset;
     o.cellOf = a.cellOf + r.beadOffset;
-    if (o.sPos) o.sPos = a.sPos + r.beadOffset;
-    if (o.sVel) o.sVel = a.sVel + r.beadOffset;
-    if (o.sTan) o.sTan = a.sTan + r.beadOffset;
+    if (GATHER & kGatherPos) o.sPos = a.sPos + r.beadOffset;
+    if (GATHER & kGatherVel) o.sVel = a.sVel + r.beadOffset;
+    if (GATHER & kGatherTan) o.sTan = a.sTan + r.beadOffset;
     o.cellBase = r.cellOffset;
     o.slotBase = r.beadOffset;
     o.idBase = r.beadOffset;
-    bucket_cells_body<false, BLOCK, CAP>(o, plan_of(r), v - r.bucketOff, smem);
+    md_cells_body<GATHER, BLOCK, CAP>(o, plan_of(r), v - r.bucketOff, smem);
 }
 
 // ---------------------------------------------------------------------------
@@ -1105,6 +1251,16 @@ hipError_t launch_hash_tiles_batch(const uint32_t *hash, const SortRep *reps, ui
     return hipGetLastError();
 }
 
+// go(std::integral_constant<int, G>) for the records that the arguments gather
+template <typename F>
+static void md_gather_dispatch(const CellsArgs &o, const F &go) {
+    if (!o.sPos) go(std::integral_constant<int, 0>{});
+    else if (o.sVel && o.sTan) go(std::integral_constant<int, kGatherPos | kGatherVel | kGatherTan>{});
+    else if (o.sVel) go(std::integral_constant<int, kGatherPos | kGatherVel>{});
+    else if (o.sTan) go(std::integral_constant<int, kGatherPos | kGatherTan>{});
+    else go(std::integral_constant<int, kGatherPos>{});
+}
+
 hipError_t launch_md_cells_batch(const SortRep *reps, uint32_t R, const BatchSortPlan &tot, BucketScratch &s,
                                  uint32_t *ids, const float4 *pos, const float4 *vel, const float4 *tan, float4 *sPos,
                                  float4 *sVel, float4 *sTan, hipStream_t st) {
@@ -1122,12 +1278,17 @@ hipError_t launch_md_cells_batch(const SortRep *reps, uint32_t R, const BatchSor
     o.sVel = sVel;
     o.sTan = sTan;
     const CellsLayout L = batch_cells_layout(tot);
-    const void *fn = reinterpret_cast<const void *>(&k_bucket_cells_batch<kMdCellsBlock, int(kBatchBucketCap)>);
-    const hipError_t e = grant_lds(fn, L.total);
-    if (e != hipSuccess) return e;
-    NW_LAUNCH((k_bucket_cells_batch<kMdCellsBlock, int(kBatchBucketCap)>), dim3(tot.buckets),
-                       dim3(kMdCellsBlock), L.total, st, o, reps, R);
-    return hipGetLastError();
+    hipError_t e = hipSuccess;
+    const auto go = [&](auto g) {
+        constexpr int G = decltype(g)::value;
+        e = grant_lds(reinterpret_cast<const void *>(&k_md_cells_batch<G, kBatchCellsBlock, int(kBatchBucketCap)>), L.total);
+        if (e != hipSuccess) return;
+        NW_LAUNCH((k_md_cells_batch<G, kBatchCellsBlock, int(kBatchBucketCap)>), dim3(tot.buckets), dim3(kBatchCellsBlock),
+                  L.total, st, o, reps, R);
+        e = hipGetLastError();
+    };
+    md_gather_dispatch(o, go);
+    return e;
 }
 
 __global__ __launch_bounds__(kBlock) void k_solvent_keys(const float4 *__restrict__ pos, uint32_t N, uint32_t Ns,
@@ -1182,7 +1343,7 @@ __global__ __launch_bounds__(kBlock) void k_sort_finish(uint32_t *__restrict__ k
 hipError_t bucket_sort_pairs(uint32_t *keys, uint32_t *vals, uint32_t n, uint32_t bound, BucketScratch &s,
                              hipStream_t st) {
     if (n == 0) return hipSuccess;
-    const BucketPlan bp = make_bucket_plan(n, bound, 0);
+    const BucketPlan bp = make_bucket_plan(n, bound, 0, md_members(n));
     if (*bucket_plan_problem(bp)) return hipErrorNotSupported;
     hipError_t e;
     if ((e = ensure_bucket_scratch(s, bp)) != hipSuccess) return e;
@@ -1212,9 +1373,17 @@ hipError_t launch_md_cells(const BucketPlan &bp, BucketScratch &s, uint32_t *ids
     o.sPos = sPos;
     o.sVel = sVel;
     o.sTan = sTan;
-    const CellsLayout L = cells_layout(bp, false);
-    NW_LAUNCH((k_bucket_cells<false, kMdCellsBlock>), dim3(bp.buckets), dim3(kMdCellsBlock), L.total, st, o,
-                       bp);
+    const auto go = [&](auto g) {
+        constexpr int G = decltype(g)::value;
+        // the smaller stage where twice the average bucket fits it
+        if (uint64_t(bp.n) * 2u <= uint64_t(bp.buckets) * kMdSmallCap)
+            NW_LAUNCH((k_md_cells<G, int(kMdSmallCap) / kMdCellsPer, int(kMdSmallCap)>), dim3(bp.buckets),
+                      dim3(kMdSmallCap / kMdCellsPer), cells_layout(bp, false, kMdSmallCap).total, st, o, bp);
+        else
+            NW_LAUNCH((k_md_cells<G, int(kBucketCap) / kMdCellsPer, int(kBucketCap)>), dim3(bp.buckets),
+                      dim3(kBucketCap / kMdCellsPer), cells_layout(bp, false).total, st, o, bp);
+    };
+    md_gather_dispatch(o, go);
     return hipGetLastError();
 }
 
@@ -1236,7 +1405,7 @@ hipError_t launch_srd_cells(const BucketPlan &bp, BucketScratch &s, uint32_t *id
     o.seed = seed;
     o.offset = offset;
     const CellsLayout L = cells_layout(bp, true);
-    NW_LAUNCH((k_bucket_cells<true, kSrdCellsBlock>), dim3(bp.buckets), dim3(kSrdCellsBlock), L.total, st,
+    NW_LAUNCH((k_srd_cells<kSrdCellsBlock>), dim3(bp.buckets), dim3(kSrdCellsBlock), L.total, st,
                        o, bp);
     return hipGetLastError();
 }
@@ -1259,7 +1428,7 @@ hipError_t launch_srd_cells_batch(const BucketPlan &bp, BucketScratch &s, uint32
     o.srdR = R;
     o.collision = collision;
     const CellsLayout L = cells_layout(bp, true);
-    NW_LAUNCH((k_bucket_cells<true, kSrdCellsBlock>), dim3(bp.buckets), dim3(kSrdCellsBlock), L.total, st, o, bp);
+    NW_LAUNCH((k_srd_cells<kSrdCellsBlock>), dim3(bp.buckets), dim3(kSrdCellsBlock), L.total, st, o, bp);
     return hipGetLastError();
 }
 

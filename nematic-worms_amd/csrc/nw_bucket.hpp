@@ -23,6 +23,7 @@ struct BucketPlan {
 };
 
 constexpr uint32_t kBucketCap = 2048;     // bucket members staged in LDS (more: global-memory path)
+constexpr uint32_t kMdSmallCap = 1024;    // the MD sort's smaller stage
 constexpr uint32_t kMaxTiles = 4096;      // level-2 segment tables in LDS
 constexpr uint32_t kMaxBuckets = 32767;   // level-1 LDS histogram (128 KiB of the 160 KiB)
 constexpr uint64_t kMaxMatrix = 1ull << 24;  // entries of P
@@ -38,7 +39,12 @@ __host__ __device__ inline uint32_t pack_pair(uint32_t cellInBucket, uint32_t id
 __host__ __device__ inline uint2 unpack_pair(uint32_t p, uint32_t tileFirstId) {
     return make_uint2(p >> kPairIdBits, tileFirstId + (p & ((1u << kPairIdBits) - 1u)));
 }
-constexpr int kMdCellsBlock = 256;        // level-2 workgroup, MD sort
+// staged members a thread of the MD sort's level 2 (256 threads with the
+// smaller stage, 512 with the larger: 11.0 us for 800,000 beads, with 256
+// 11.4; the smaller stage with 512 the same for one system, but a batch of 21.9
+// million beads 329 us against 264)
+constexpr int kMdCellsPer = 4;
+constexpr int kBatchCellsBlock = 256;     // level-2 workgroup of a batch
 constexpr int kSrdCellsBlock = 256;       // level-2 workgroup, SRD sort
 constexpr int kCellsBlockMax = 1024;
 constexpr int kPairBlock = 256;           // sorted beads per LDS pair-kernel workgroup
