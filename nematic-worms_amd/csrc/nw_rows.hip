@@ -343,10 +343,10 @@ __global__ __launch_bounds__(kRowsBlock) void k_rows_batch(BatchArrays a, const 
 // plan and launcher
 // ---------------------------------------------------------------------------
 // Every workgroup reads every bead's cell, so the launch wins while that read
-// is short: sort + pairs 23.2 -> 7.7 us at 8,000 beads, 23.4 -> 8.7 at 16,000,
-// 26.8 -> 10.9 at 32,000, 22.8 -> 16.0 at 64,000, 24.1 -> 20.4 at 96,000, 24.7
-// -> 23.9 at 128,000 (and two launches fewer), 24.1 -> 31 at 192,000.
-constexpr uint64_t kRowsMaxBeads = 131072;
+// is short.  A whole step with the sort and the pair kernel / with this launch:
+// 25.7 / 12.4 us at 6,400 beads, 26.5 / 15.4 at 32,000, 27.1 / 20.7 at 64,000,
+// 28.3 / 25.4 at 96,000, 28.7 / 27.5 at 112,000, 29.0 / 29.8 at 128,000.
+constexpr uint64_t kRowsMaxBeads = 114688;
 constexpr uint32_t kRowsMaxBlocks = 256;  // one round of the CUs: 64,000 beads over 291 rows take 23.0 us by single rows, 16.0 by pairs
 constexpr uint32_t kRowsMaxOwn = 768;     // beads of a workgroup on average: three rounds of its quads
 
@@ -384,13 +384,13 @@ bool rows_plan(uint64_t N, const KP &kp, RowsPlan &out) {
 }
 
 // The batch takes the launch when its workgroups are done sooner than the sort
-// and the pair kernel.  Measured with one size of replica throughout (us, sort
-// + pairs / this launch): 16 x 8,000 beads 24.6 / 11.0, 64 x 8,000 35.5 / 26.6,
-// 128 x 8,000 47.8 / 48.1, 256 x 2,000 35.0 / 24.6, 16 x 12,000 25.7 / 13.5, 64
-// x 12,000 42.4 / 35.1, 16 x 30,000 33.3 / 30.4, 64 x 30,000 72.4 / 95.1, 16 x
-// 60,000 45.4 / 61.9: the sort and the pairs take some 22 us and 26 us a
-// million beads, 256 workgroups here 8 us and 1 us for every 10,000 beads of
-// their replica.
+// and the pair kernel.  Measured with one size of replica throughout (us a
+// step, sort + pairs / this launch): 16 x 1,100 beads 30.4 / 17.0, 16 x 8,600
+// 35.5 / 24.4, 64 x 7,700 52.6 / 47.5, 64 x 4,100 43.8 / 34.2, 128 x 4,000 54.3
+// / 46.4, 256 x 2,000 56.4 / 49.1, 16 x 30,000 52.3 / 48.8; the launch alone
+// loses at 64 x 30,000 (95 us) and 16 x 60,000 (62).  The sort and the pairs
+// take some 19 us and 26 us a million beads, 256 workgroups here 8 us and 1 us
+// for every 10,000 beads of their replica.
 bool rows_plan_batch(BatchRep *reps, uint32_t R, RowsPlan &out) {
     out = RowsPlan{};
     uint64_t rows = 0;
@@ -415,7 +415,7 @@ bool rows_plan_batch(BatchRep *reps, uint32_t R, RowsPlan &out) {
         here += blocks * (8.0 + 1e-4 * q.numBeads) / kRowsMaxBlocks;
         beads += q.numBeads;
     }
-    if (!pl.blocks || here > 22.0 + 26e-6 * beads || !rows_fits(pl)) return false;
+    if (!pl.blocks || here > 19.0 + 26e-6 * beads || !rows_fits(pl)) return false;
     out = pl;
     return true;
 }
