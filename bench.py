@@ -86,7 +86,7 @@ SINGLE_KERNEL = {"integrate", "langevin", "filament", "hash", "collide", "srd_co
 
 # kernel behind each single-kernel family of the fused path (the names that
 # rocprofv3 reports), for the HBM traffic measured by its counters
-FAMILY_KERNEL = {"srdf_cells": "k_srd_cells<256>", "srdf_rotate": "k_srd_rotate"}
+FAMILY_KERNEL = {"srdf_rotate": "k_srd_rotate"}
 
 
 def dispatched_kernel(family, w):
@@ -103,6 +103,9 @@ def dispatched_kernel(family, w):
     if family == "md_sort":
         # the smaller stage where twice the average bucket fits it
         return "k_md_cells<1, 256, 1024>" if 2 * w["N"] <= 1024 * w["md_plan"][1] else "k_md_cells<1, 512, 2048>"
+    if family == "srdf_cells":
+        # the larger sorting network above seven particles a cell
+        return f"k_srd_cells<256, {32 if w['NT'] > 7 * w['Cs'] else 16}>"
     if family == "md_tiles":
         items = w["md_plan"][2]
         shapes = {1024: "4, 256", 2048: "8, 256", 4096: "4, 1024", 8192: "8, 1024", 16384: "16, 1024"}

@@ -420,9 +420,10 @@ __device__ __forceinline__ void sort_cell_ids(uint32_t *arr, uint32_t a, uint32_
 // registers for both sums (a cell holds ~6 particles); the rest are read
 // kSumTail at a time in each sum.  Slots past z load the last particle
 // again, unused.
+template <uint32_t kSumHead>
 __device__ __forceinline__ void srd_cell_sums(const CellsArgs &o, const uint32_t *ids, uint32_t a, uint32_t z,
                                               f3 &mom, float &lambda) {
-    constexpr uint32_t kSumHead = 8, kSumTail = 4;
+    constexpr uint32_t kSumTail = 4;
     uint32_t I[kSumHead];
 #pragma unroll
     for (uint32_t k = 0; k < kSumHead; ++k) I[k] = ids[min(a + k, z - 1u)];
@@ -527,23 +528,30 @@ __device__ __forceinline__ uint32_t bucket_segments(const CellsArgs &o, const Bu
                                                     uint32_t *wsum, uint32_t &m) {
     constexpr uint32_t NW = BLOCK / 64;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wid = tid >> 6, B1 = bp.buckets + 1;
-    const auto segment = [&](uint32_t t, uint32_t &lo, uint32_t &len) {
-        lo = len = 0u;
-        bool read = true;
-        if (o.tileRange) {
-            const uint32_t r0 = o.tileRange[2u * t], r1 = o.tileRange[2u * t + 1u];
-            read = b >= r0 && b <= r1;
-            if (b > r1) lo = min(bp.tileItems, bp.n - t * bp.tileItems);
+    // tile t's buckets, its prefix at this one and (raw) at the next
+    typedef uint32_t w2 __attribute__((ext_vector_type(2)));
+    const auto range = [&](uint32_t t) {
+        return o.tileRange ? reinterpret_cast<const w2 *>(o.tileRange)[t] : w2{0u, ~0u};
+    };
+    const auto row = [&](uint32_t t, w2 g, uint32_t &lo, uint32_t &hi) {
+        lo = hi = 0u;
+        if (b >= g.x && b <= g.y) {
+            const uint32_t *p = o.P + uint64_t(t) * B1 + b;
+            lo = p[0];
+            hi = p[1];
         }
-        if (read) {
-            const uint32_t *row = o.P + uint64_t(t) * B1 + b;
-            lo = row[0];
-            len = row[1] - lo;
-        }
+    };
+    const auto settle = [&](uint32_t t, w2 g, uint32_t &lo, uint32_t &len) {
+        len -= lo;
+        if (b > g.y) lo = min(bp.tileItems, bp.n - t * bp.tileItems);
     };
     if (bp.tiles <= uint32_t(BLOCK)) {
         uint32_t lo = 0u, len = 0u;
-        if (tid < bp.tiles) segment(tid, lo, len);
+        if (tid < bp.tiles) {
+            const w2 g = range(tid);
+            row(tid, g, lo, len);
+            settle(tid, g, lo, len);
+        }
         const uint32_t sl = wave_scan_add(len), sp = wave_scan_add(lo);
         if (lane == 63u) {
             wsum[wid] = sl;
@@ -564,12 +572,28 @@ __device__ __forceinline__ uint32_t bucket_segments(const CellsArgs &o, const Bu
         return uint32_t(__builtin_amdgcn_readlane(int(ws), 2 * int(NW) - 1)) - m;
     }
     uint32_t part = 0;
-    for (uint32_t t = tid; t < bp.tiles; t += BLOCK) {
-        uint32_t lo, len;
-        segment(t, lo, len);
-        segBase[t] = lo;
-        segStart[t] = len;
-        part += lo;
+    // the ranges, then the rows, of several tiles a thread in flight together
+    constexpr uint32_t R = 3;
+    for (uint32_t t0 = tid; t0 < bp.tiles; t0 += R * BLOCK) {
+        w2 g[R];
+        uint32_t lo[R], len[R];
+#pragma unroll
+        for (uint32_t k = 0; k < R; ++k) {
+            const uint32_t t = t0 + k * BLOCK;
+            g[k] = t < bp.tiles ? range(t) : w2{~0u, 0u};
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < R; ++k) row(t0 + k * BLOCK, g[k], lo[k], len[k]);
+#pragma unroll
+        for (uint32_t k = 0; k < R; ++k) {
+            const uint32_t t = t0 + k * BLOCK;
+            if (t < bp.tiles) {
+                settle(t, g[k], lo[k], len[k]);
+                segBase[t] = lo[k];
+                segStart[t] = len[k];
+                part += lo[k];
+            }
+        }
     }
     part = wave_scan_add(part);
     if (lane == 63u) wsum[NW + wid] = part;  // upper half of wsum
@@ -750,7 +774,7 @@ __device__ __forceinline__ void md_cells_body(const CellsArgs &o, const BucketPl
 }
 
 // SRD, bucket b; staged as the MD sort's
-template <int BLOCK, int CAP = int(kBucketCap)>
+template <int BLOCK, int NET, int CAP = int(kBucketCap)>
 __device__ __forceinline__ void srd_cells_body(const CellsArgs &o, const BucketPlan &bp, uint32_t b,
                                                   unsigned char *smem) {
     constexpr int PER = CAP / BLOCK;
@@ -769,7 +793,7 @@ __device__ __forceinline__ void srd_cells_body(const CellsArgs &o, const BucketP
     const uint32_t nc = min(1u << bp.shift, bp.cells - cell0);
     // cleared here, under the barriers of the segment pass: the cell counts
     // and the member tile marks (tileOf, CAP entries over lid)
-    for (uint32_t c = tid; c < nc; c += bd) cnt[c] = 0u;
+    for (uint32_t c = tid; c < ((nc + 3u) & ~3u); c += bd) cnt[c] = 0u;
     for (uint32_t k = tid; k < uint32_t(CAP) / 2u; k += bd) reinterpret_cast<uint32_t *>(tileOf)[k] = 0u;
 
     uint32_t m;
@@ -794,7 +818,8 @@ __device__ __forceinline__ void srd_cells_body(const CellsArgs &o, const BucketP
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
             const uint32_t k = tid + uint32_t(j) * BLOCK;
-            if (k < m) atomicAdd(&cnt[q[j].x], 1u);
+            // its place in the cell's run of arrivals beside the cell (both below 2^11)
+            if (k < m) q[j].x |= atomicAdd(&cnt[q[j].x], 1u) << 16;
         }
     } else if (!staged) {
         for (uint32_t k = tid; k < m; k += bd) {
@@ -803,7 +828,8 @@ __device__ __forceinline__ void srd_cells_body(const CellsArgs &o, const BucketP
         }
     }
     __syncthreads();
-    block_excl_scan<true>(cnt, nc, wsum, cur);
+    if (staged) scan_cells<BLOCK>(cnt, nc, m, wsum);
+    else block_excl_scan<true>(cnt, nc, wsum, cur);
 
     uint32_t *out = o.ids + sb;
     if (staged) {
@@ -811,9 +837,7 @@ __device__ __forceinline__ void srd_cells_body(const CellsArgs &o, const BucketP
         for (int j = 0; j < PER; ++j) {
             const uint32_t k = tid + uint32_t(j) * BLOCK;
             if (k < m) {
-                const uint32_t lc = q[j].x;
-                const uint32_t slot = atomicAdd(&cur[lc], 1u);
-                lid[slot] = q[j].y;
+                lid[cnt[q[j].x & 0xffffu] + (q[j].x >> 16)] = q[j].y;
             }
         }
     } else {
@@ -846,8 +870,8 @@ __device__ __forceinline__ void srd_cells_body(const CellsArgs &o, const BucketP
     // LDS, not through a generic pointer.
     for (uint32_t c = tid; c < nc; c += bd) {
         const uint32_t a = cnt[c], z = cnt[c + 1];
-        if (staged) sort_cell_ids<16>(lid, a, z);
-        else sort_cell_ids<16>(out, a, z);
+        if (staged) sort_cell_ids<NET>(lid, a, z);
+        else sort_cell_ids<NET>(out, a, z);
         o.off[cell0 + c] = o.slotBase + sb + a;
     }
     if (tid == 0 && cell0 + nc == bp.cells) o.off[bp.cells] = o.slotBase + bp.n;
@@ -870,7 +894,7 @@ __device__ __forceinline__ void srd_cells_body(const CellsArgs &o, const BucketP
         if (a != z) {
             // one instance for both storages, through a generic pointer (two
             // instances specialised to LDS and global memory measured slower)
-            srd_cell_sums(o, staged ? lid : out, a, z, mom, lambda);
+            srd_cell_sums<NET / 2>(o, staged ? lid : out, a, z, mom, lambda);
         }
         const uint32_t cell = cell0 + c;
         bool up;
@@ -887,10 +911,10 @@ __device__ __forceinline__ void srd_cells_body(const CellsArgs &o, const BucketP
     }
 }
 
-template <int BLOCK>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_srd_cells(CellsArgs o, BucketPlan bp) {
+template <int BLOCK, int NET>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(NET > 16 ? 4 : 8, 8))) void k_srd_cells(CellsArgs o, BucketPlan bp) {
     extern __shared__ __align__(16) unsigned char smem[];
-    srd_cells_body<BLOCK>(o, bp, xcd_contiguous(blockIdx.x, gridDim.x), smem);
+    srd_cells_body<BLOCK, NET>(o, bp, xcd_contiguous(blockIdx.x, gridDim.x), smem);
 }
 
 template <int GATHER, int BLOCK, int CAP>
@@ -1387,6 +1411,20 @@ hipError_t launch_md_cells(const BucketPlan &bp, BucketScratch &s, uint32_t *ids
     return hipGetLastError();
 }
 
+// The network takes a cell whose ids fit it, the sums load half as many
+// velocities together: 32 and 16 where cells hold more than seven particles on
+// average (a million particles of ten a cell in random order: 28.3 us, with 16
+// and 8 30.4: above sixteen the sort is by insertion, and every four velocities
+// past the first batch are another round trip).
+static hipError_t launch_srd_buckets(const CellsArgs &o, const BucketPlan &bp, hipStream_t st) {
+    const CellsLayout L = cells_layout(bp, true);
+    if (uint64_t(bp.n) > 7u * uint64_t(bp.cells))
+        NW_LAUNCH((k_srd_cells<kSrdCellsBlock, 32>), dim3(bp.buckets), dim3(kSrdCellsBlock), L.total, st, o, bp);
+    else
+        NW_LAUNCH((k_srd_cells<kSrdCellsBlock, 16>), dim3(bp.buckets), dim3(kSrdCellsBlock), L.total, st, o, bp);
+    return hipGetLastError();
+}
+
 hipError_t launch_srd_cells(const BucketPlan &bp, BucketScratch &s, uint32_t *ids, const float4 *vel, float4 *com,
                             int iso, uint64_t seed, uint64_t offset, const KP &kp, hipStream_t st) {
     if (bp.n == 0) return hipSuccess;
@@ -1404,10 +1442,7 @@ hipError_t launch_srd_cells(const BucketPlan &bp, BucketScratch &s, uint32_t *id
     o.kbT = kp.s.kbT;
     o.seed = seed;
     o.offset = offset;
-    const CellsLayout L = cells_layout(bp, true);
-    NW_LAUNCH((k_srd_cells<kSrdCellsBlock>), dim3(bp.buckets), dim3(kSrdCellsBlock), L.total, st,
-                       o, bp);
-    return hipGetLastError();
+    return launch_srd_buckets(o, bp, st);
 }
 
 hipError_t launch_srd_cells_batch(const BucketPlan &bp, BucketScratch &s, uint32_t *ids, const float4 *vel,
@@ -1427,9 +1462,7 @@ hipError_t launch_srd_cells_batch(const BucketPlan &bp, BucketScratch &s, uint32
     o.srdReps = reps;
     o.srdR = R;
     o.collision = collision;
-    const CellsLayout L = cells_layout(bp, true);
-    NW_LAUNCH((k_srd_cells<kSrdCellsBlock>), dim3(bp.buckets), dim3(kSrdCellsBlock), L.total, st, o, bp);
-    return hipGetLastError();
+    return launch_srd_buckets(o, bp, st);
 }
 
 hipError_t launch_srd_hash_batch(const float4 *pos, uint32_t *hash, const SrdRep *reps, uint32_t R, uint32_t Nb,
