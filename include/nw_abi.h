@@ -403,7 +403,8 @@ void nwBatchSolventLayout(uint *solventOffset, uint *srdCellOffset);
 /* `steps` nwFusedMdStep steps from (pos, vel, force, forceOld), in place,
    with the SimParams / NWExtParams of the last setParameters /
    nwSetExtParameters; the state and generator offset are checkpointed every
-   checkpointEvery steps for nwAdjointBackward.  langevinGamma must equal
+   checkpointEvery steps for nwAdjointBackward, whose segment store (up to 4
+   GiB) takes the states of the last segment right away.  langevinGamma must equal
    SimParams.gamma when langevin is on. */
 void nwAdjointForward(float *pos, float *vel, float *force, float *forceOld, float *tangent, uint numFilaments,
                       float deltaTime, float langevinGamma, float langevinKbT, int langevin, uint steps,
@@ -424,7 +425,8 @@ void nwAdjointForwardSrd(float *pos, float *vel, float *force, float *forceOld, 
                          uint checkpointEvery);
 /* The adjoint of the last nwAdjointForward run, backwards from dLdPos /
    dLdVel (adjoints of the final positions / velocities, device float4 per
-   bead; dLdVel may be NULL): every segment is recomputed from its checkpoint
+   bead; dLdVel may be NULL): every segment but the one that the forward
+   run left is recomputed from its checkpoint
    with the Philox noise replayed, then swept backwards.  grad[4] receives
    d loss / d theta.  The generator is left where the forward run left it.
    Synchronises. */

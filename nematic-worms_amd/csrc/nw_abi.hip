@@ -97,7 +97,11 @@ struct State {
         float4 *collCom = nullptr, *cellSum = nullptr, *wPos = nullptr, *wVel = nullptr;
         uint64_t capCollHash = 0, capCollIds = 0, capCollOff = 0, capCollCom = 0, capCellSum = 0, capWPos = 0,
                  capWVel = 0;
-        // one segment: states after every step and the cell lists of every step
+        // one segment: states after every step and the cell lists of every
+        // step; held: the segment they are of, as the forward run or the
+        // backward pass left them (-1: none)
+        int held = -1;
+        std::vector<uint64_t> lgvOff;  // its steps' generator offsets
         float4 *segPos = nullptr, *segVel = nullptr, *segSPos = nullptr, *work = nullptr, *lam = nullptr;
         uint32_t *segIds = nullptr, *segOff = nullptr, *segCell = nullptr;
         double *partial = nullptr, *grad = nullptr;
@@ -124,6 +128,7 @@ struct State {
         float dt = 0.f;
         float4 *ckpt = nullptr;   // checkpoints x (2 NT + 2 N): pos, vel, force, forceOld
         float *shifts = nullptr;  // collisions x R x 3 grid shifts
+        int held = -1;            // the segment in the store below, as Adjoint's
         float4 *segPos = nullptr, *segVel = nullptr, *segSPos = nullptr, *work = nullptr, *lam = nullptr;
         float4 *wPos = nullptr, *wVel = nullptr, *collCom = nullptr, *cellSum = nullptr;
         uint32_t *segIds = nullptr, *segOff = nullptr, *hash = nullptr, *sCell = nullptr;
@@ -623,7 +628,8 @@ static bool fused_md(const KP &kp, float *pos, float *vel, float *force, float *
                      uint *gridParticleHash, uint *gridParticleIndex, float *sortedPos, float *sortedVel,
                      float *sortedTangent, float deltaTime, float langevinGamma, float langevinKbT, int langevin,
                      uint numFilaments, uint32_t *offOut, uint32_t *cellOut, const float *posIn = nullptr,
-                     const float *velIn = nullptr, bool swapForces = false, const BucketScratch *fixed = nullptr) {
+                     const float *velIn = nullptr, bool swapForces = false, const BucketScratch *fixed = nullptr,
+                     float4 *keepPos = nullptr, float4 *keepVel = nullptr) {
     State &s = S();
     const uint32_t n = kp.p.filamentSize;
     NW_REQUIRE_R(n >= 1 && n <= 64, false, "nwFusedMdStep: worms of %u beads (1..64 supported)", n);
@@ -658,6 +664,8 @@ static bool fused_md(const KP &kp, float *pos, float *vel, float *force, float *
     a.tangent = reinterpret_cast<float4 *>(tangent);
     a.posIn = reinterpret_cast<const float4 *>(posIn);
     a.velIn = reinterpret_cast<const float4 *>(velIn);
+    a.keepPos = keepPos;
+    a.keepVel = keepVel;
     a.hash = gridParticleHash ? gridParticleHash : base.hash;
     a.dt = deltaTime;
     a.W = numFilaments;
@@ -1249,6 +1257,28 @@ static KP collision_kp(const State::Adjoint &A, uint32_t c) {
     return kp;
 }
 
+static bool ensure_segment(State::Adjoint &A) {
+    const uint64_t N = A.N, K = A.K, NT = A.NT;
+    if (!(grow(A.segPos, A.capPos, (K + 1) * N) && grow(A.segVel, A.capVel, (K + 1) * N) &&
+          grow(A.segSPos, A.capSPos, K * N) && grow(A.segIds, A.capIds, std::max(K * N, NT)) &&
+          grow(A.segOff, A.capOff, K * (uint64_t(A.C) + 2)) && grow(A.segCell, A.capCell, K * N) &&
+          grow(A.work, A.capWork, 2 * N) && grow(A.lam, A.capLam, 4 * N + NT)))
+        return false;
+    if (!A.srd) return true;
+    // at most this many collisions in a segment of K steps
+    const uint64_t cpS = (K + A.gap - 1) / A.gap + 1;
+    return grow(A.collHash, A.capCollHash, cpS * NT) && grow(A.collIds, A.capCollIds, cpS * NT) &&
+           grow(A.collOff, A.capCollOff, cpS * (uint64_t(A.Cs) + 2)) &&
+           grow(A.collCom, A.capCollCom, cpS * A.Cs) && grow(A.cellSum, A.capCellSum, A.Cs) &&
+           grow(A.wPos, A.capWPos, NT) && grow(A.wVel, A.capWVel, NT);
+}
+
+// The forward run leaves its last segment in the segment store, which the
+// backward pass then need not recompute, when the store (allocated by the
+// backward pass in any case) takes at most this much: a forward run alone does
+// not claim more.
+constexpr uint64_t kHoldBytes = 4ull << 30;
+
 // The forward run of nwAdjointForward / nwAdjointForwardSrd (srd: numSolvent,
 // gap and shifts set in A by the caller, A.srd true).
 static void adjoint_forward(float *pos, float *vel, float *force, float *forceOld, float *tangent,
@@ -1299,6 +1329,14 @@ static void adjoint_forward(float *pos, float *vel, float *force, float *forceOl
     A.seed = s.seed;
     const uint32_t nck = (steps + checkpointEvery - 1) / checkpointEvery;
     const uint64_t NT = A.NT, stride = 2 * NT + 2 * N;
+    const uint64_t K = checkpointEvery;
+    const uint64_t perStep = 56 * N + 4 * C + 8 + (A.srd ? (8 * NT + 20 * uint64_t(A.Cs)) / A.gap : 0);
+    A.held = -1;
+    bool hold = K <= kHoldBytes / perStep;
+    if (hold && !ensure_segment(A)) {
+        (void)hipGetLastError();  // no room for it: the run goes on without
+        hold = false;
+    }
     NW_REQUIRE(grow(A.ckpt, A.capCkpt, uint64_t(nck) * stride) && grow(A.segSPos, A.capSPos, N) &&
                    grow(A.segIds, A.capIds, NT),
                "nwAdjointForward: out of device memory");
@@ -1306,6 +1344,8 @@ static void adjoint_forward(float *pos, float *vel, float *force, float *forceOl
         NW_REQUIRE(grow(A.collCom, A.capCollCom, A.Cs) && grow(A.collHash, A.capCollHash, NT),
                    "nwAdjointForwardSrd: out of device memory");
     A.ckptOffset.assign(nck, 0);
+    A.lgvOff.assign(hold ? std::min<uint64_t>(K, steps) : 0, 0);
+    uint64_t slots = 0;  // collisions kept
     const size_t bytesT = NT * sizeof(float4), bytes = N * sizeof(float4);
     for (uint32_t k = 0; k < steps; ++k) {
         if (k % checkpointEvery == 0) {
@@ -1317,17 +1357,27 @@ static void adjoint_forward(float *pos, float *vel, float *force, float *forceOl
                        "nwAdjointForward: checkpoint copy failed");
             A.ckptOffset[c] = s.offset;
         }
-        // sorted positions and ids go to the segment store (scratch here)
-        // the pair term reads no tangents: the run's last step stores them
-        if (!fused_md(kp, pos, vel, force, forceOld, k + 1 == steps ? tangent : nullptr, nullptr, A.segIds, reinterpret_cast<float *>(A.segSPos),
-                      nullptr, nullptr, deltaTime, langevinGamma, langevinKbT, langevin, numFilaments, nullptr,
-                      nullptr))
+        // the last segment's states and cell lists into their slots; before it
+        // the store's first slots are scratch.  The pair term reads no
+        // tangents: the run's last step stores them
+        const bool keep = hold && k / K == nck - 1u;
+        const uint64_t j = keep ? k % K : 0;
+        if (keep) A.lgvOff[j] = s.offset;
+        if (!fused_md(kp, pos, vel, force, forceOld, k + 1 == steps ? tangent : nullptr, nullptr, A.segIds + j * N,
+                      reinterpret_cast<float *>(A.segSPos + j * N), nullptr, nullptr, deltaTime, langevinGamma,
+                      langevinKbT, langevin, numFilaments, keep ? A.segOff + j * (C + 2) : nullptr,
+                      keep ? A.segCell + j * N : nullptr, nullptr, nullptr, false, nullptr,
+                      keep ? A.segPos + (j + 1) * N : nullptr, keep ? A.segVel + (j + 1) * N : nullptr))
             return;
-        if (A.srd && k % A.gap == 0 &&
-            !fused_srd(collision_kp(A, k / A.gap), pos, vel, reinterpret_cast<float *>(A.collCom), A.collHash,
-                       A.segIds, nullptr, deltaTime * float(A.gap), uint32_t(N), A.Ns, 0))
-            return;
+        if (A.srd && k % A.gap == 0) {
+            const uint64_t u = keep ? slots++ : 0;
+            if (!fused_srd(collision_kp(A, k / A.gap), pos, vel, reinterpret_cast<float *>(A.collCom + u * A.Cs),
+                           A.collHash + u * NT, keep ? A.collIds + u * NT : A.segIds,
+                           keep ? A.collOff + u * (A.Cs + 2) : nullptr, deltaTime * float(A.gap), uint32_t(N), A.Ns, 0))
+                return;
+        }
     }
+    if (hold) A.held = int(nck) - 1;
     A.endOffset = s.offset;
     A.ready = true;
 }
@@ -1360,22 +1410,6 @@ void nwAdjointForwardSrd(float *pos, float *vel, float *force, float *forceOld, 
                     checkpointEvery);
 }
 
-static bool ensure_segment(State::Adjoint &A) {
-    const uint64_t N = A.N, K = A.K, NT = A.NT;
-    if (!(grow(A.segPos, A.capPos, (K + 1) * N) && grow(A.segVel, A.capVel, (K + 1) * N) &&
-          grow(A.segSPos, A.capSPos, K * N) && grow(A.segIds, A.capIds, std::max(K * N, NT)) &&
-          grow(A.segOff, A.capOff, K * (uint64_t(A.C) + 2)) && grow(A.segCell, A.capCell, K * N) &&
-          grow(A.work, A.capWork, 2 * N) && grow(A.lam, A.capLam, 4 * N + NT)))
-        return false;
-    if (!A.srd) return true;
-    // at most this many collisions in a segment of K steps
-    const uint64_t cpS = (K + A.gap - 1) / A.gap + 1;
-    return grow(A.collHash, A.capCollHash, cpS * NT) && grow(A.collIds, A.capCollIds, cpS * NT) &&
-           grow(A.collOff, A.capCollOff, cpS * (uint64_t(A.Cs) + 2)) &&
-           grow(A.collCom, A.capCollCom, cpS * A.Cs) && grow(A.cellSum, A.capCellSum, A.Cs) &&
-           grow(A.wPos, A.capWPos, NT) && grow(A.wVel, A.capWVel, NT);
-}
-
 void nwAdjointBackward(const float *dLdPos, const float *dLdVel, double grad[4]) {
     NW_INIT();
     State &s = S();
@@ -1401,66 +1435,62 @@ void nwAdjointBackward(const float *dLdPos, const float *dLdVel, double grad[4])
     int cur = 0;
     float4 *F = A.work, *G = A.work + N;
     const uint32_t nck = (A.steps + A.K - 1) / A.K;
-    std::vector<uint64_t> lgvOff(K);
+    A.lgvOff.resize(std::min<uint64_t>(K, A.steps));
     std::vector<int> collSlot(K);  // the collision store slot of each step of the segment, -1: none
     for (int c = int(nck) - 1; c >= 0; --c) {
         const uint32_t s0 = uint32_t(c) * A.K, len = std::min<uint32_t>(A.K, A.steps - s0);
         const float4 *ck = A.ckpt + uint64_t(c) * stride;
-        NW_HIP(hipMemcpyAsync(A.segPos, ck, bytes, hipMemcpyDeviceToDevice, s.stream));
-        NW_HIP(hipMemcpyAsync(A.segVel, ck + NT, bytes, hipMemcpyDeviceToDevice, s.stream));
-        NW_HIP(hipMemcpyAsync(F, ck + 2 * NT, bytes, hipMemcpyDeviceToDevice, s.stream));
-        NW_HIP(hipMemcpyAsync(G, ck + 2 * NT + N, bytes, hipMemcpyDeviceToDevice, s.stream));
-        if (A.srd) {
-            NW_HIP(hipMemcpyAsync(A.wPos, ck, NT * sizeof(float4), hipMemcpyDeviceToDevice, s.stream));
-            NW_HIP(hipMemcpyAsync(A.wVel, ck + NT, NT * sizeof(float4), hipMemcpyDeviceToDevice, s.stream));
+        // recompute the segment, keeping every step's state and cell lists,
+        // unless the forward run left them
+        const bool have = A.held == c;
+        if (!have) {
+            A.held = -1;
+            if (A.srd) {
+                NW_HIP(hipMemcpyAsync(A.wPos, ck, NT * sizeof(float4), hipMemcpyDeviceToDevice, s.stream));
+                NW_HIP(hipMemcpyAsync(A.wVel, ck + NT, NT * sizeof(float4), hipMemcpyDeviceToDevice, s.stream));
+            } else {
+                NW_HIP(hipMemcpyAsync(A.segPos, ck, bytes, hipMemcpyDeviceToDevice, s.stream));
+                NW_HIP(hipMemcpyAsync(A.segVel, ck + NT, bytes, hipMemcpyDeviceToDevice, s.stream));
+            }
+            NW_HIP(hipMemcpyAsync(F, ck + 2 * NT, bytes, hipMemcpyDeviceToDevice, s.stream));
+            NW_HIP(hipMemcpyAsync(G, ck + 2 * NT + N, bytes, hipMemcpyDeviceToDevice, s.stream));
+            s.offset = A.ckptOffset[c];
         }
-        // recompute the segment, keeping every step's state and cell lists
-        s.offset = A.ckptOffset[c];
         int slots = 0;
         for (uint32_t j = 0; j < len; ++j) {
-            // step j reads slot j and writes slot j + 1
+            const uint32_t k = s0 + j;
+            collSlot[j] = A.srd && k % A.gap == 0 ? slots++ : -1;
+            if (have) continue;
+            // step j reads slot j and writes slot j + 1; with the solvent the
+            // full state steps in place and the slots take the beads' copies
             float4 *pj = A.segPos + uint64_t(j + 1) * N, *vj = A.segVel + uint64_t(j + 1) * N;
-            lgvOff[j] = s.offset;
-            collSlot[j] = -1;
-            if (A.srd) {
-                // the full state steps in place; the beads' copies fill the slots
-                if (!fused_md(A.kp, reinterpret_cast<float *>(A.wPos), reinterpret_cast<float *>(A.wVel),
-                              reinterpret_cast<float *>(F), reinterpret_cast<float *>(G), nullptr, nullptr, A.segIds + uint64_t(j) * N,
-                              reinterpret_cast<float *>(A.segSPos + uint64_t(j) * N), nullptr, nullptr, A.dt, A.gamma,
-                              A.kT, A.langevin, A.W, A.segOff + uint64_t(j) * (A.C + 2),
-                              A.segCell + uint64_t(j) * N, nullptr, nullptr))
-                    return;
-                NW_HIP(hipMemcpyAsync(pj, A.wPos, bytes, hipMemcpyDeviceToDevice, s.stream));
-                NW_HIP(hipMemcpyAsync(vj, A.wVel, bytes, hipMemcpyDeviceToDevice, s.stream));
-                const uint32_t k = s0 + j;
-                if (k % A.gap == 0) {
-                    const int q = slots++;
-                    collSlot[j] = q;
-                    if (!fused_srd(collision_kp(A, k / A.gap), reinterpret_cast<float *>(A.wPos),
-                                   reinterpret_cast<float *>(A.wVel),
-                                   reinterpret_cast<float *>(A.collCom + uint64_t(q) * A.Cs),
-                                   A.collHash + uint64_t(q) * NT, A.collIds + uint64_t(q) * NT,
-                                   A.collOff + uint64_t(q) * (A.Cs + 2), A.dt * float(A.gap), A.N, A.Ns, 0))
-                        return;
-                }
-                continue;
-            }
-            if (!fused_md(A.kp, reinterpret_cast<float *>(pj), reinterpret_cast<float *>(vj),
-                          reinterpret_cast<float *>(F), reinterpret_cast<float *>(G), nullptr, nullptr,
-                          A.segIds + uint64_t(j) * N, reinterpret_cast<float *>(A.segSPos + uint64_t(j) * N),
-                          nullptr, nullptr, A.dt, A.gamma, A.kT, A.langevin, A.W,
-                          A.segOff + uint64_t(j) * (A.C + 2), A.segCell + uint64_t(j) * N,
-                          reinterpret_cast<const float *>(A.segPos + uint64_t(j) * N),
-                          reinterpret_cast<const float *>(A.segVel + uint64_t(j) * N)))
+            float4 *p = A.srd ? A.wPos : pj, *v = A.srd ? A.wVel : vj;
+            A.lgvOff[j] = s.offset;
+            if (!fused_md(A.kp, reinterpret_cast<float *>(p), reinterpret_cast<float *>(v), reinterpret_cast<float *>(F),
+                          reinterpret_cast<float *>(G), nullptr, nullptr, A.segIds + uint64_t(j) * N,
+                          reinterpret_cast<float *>(A.segSPos + uint64_t(j) * N), nullptr, nullptr, A.dt, A.gamma, A.kT,
+                          A.langevin, A.W, A.segOff + uint64_t(j) * (A.C + 2), A.segCell + uint64_t(j) * N,
+                          A.srd ? nullptr : reinterpret_cast<const float *>(pj - N),
+                          A.srd ? nullptr : reinterpret_cast<const float *>(vj - N), false, nullptr,
+                          A.srd ? pj : nullptr, A.srd ? vj : nullptr))
                 return;
+            if (collSlot[j] >= 0) {
+                const uint64_t q = uint64_t(collSlot[j]);
+                if (!fused_srd(collision_kp(A, k / A.gap), reinterpret_cast<float *>(A.wPos),
+                               reinterpret_cast<float *>(A.wVel), reinterpret_cast<float *>(A.collCom + q * A.Cs),
+                               A.collHash + q * NT, A.collIds + q * NT, A.collOff + q * (A.Cs + 2),
+                               A.dt * float(A.gap), A.N, A.Ns, 0))
+                    return;
+            }
         }
+        A.held = c;
         // the adjoint through the segment, last step first
         for (int j = int(len) - 1; j >= 0; --j) {
             if (collSlot[j] >= 0) {
                 // the step's collision came after its MD part: undo it first
                 const uint64_t q = uint64_t(collSlot[j]);
                 NW_HIP(launch_srd_adj(A.collIds + q * NT, A.collOff + q * (A.Cs + 2), A.collHash + q * NT,
-                                      A.collCom + q * A.Cs, A.wVel, lv, A.cellSum, A.N, uint32_t(NT), A.Cs, A.cosA,
+                                      A.collCom + q * A.Cs, ck + NT, lv, A.cellSum, A.N, uint32_t(NT), A.Cs, A.cosA,
                                       A.sinA, A.rotBeads, s.stream));
             }
             AdjStepArgs as;
@@ -1481,7 +1511,7 @@ void nwAdjointBackward(const float *dLdPos, const float *dLdVel, double grad[4])
             as.gamma = A.gamma;
             as.dt = A.dt;
             as.seed = A.seed;
-            as.offLgv = lgvOff[j];
+            as.offLgv = A.lgvOff[j];
             {
                 TimedScope ts("adj_step", s.stream, true);
                 NW_HIP(launch_adj_step(as, A.kp, s.stream));
@@ -1618,6 +1648,28 @@ void nwBatchSrdStep(float *pos, float *vel, float *solventCellCOM, uint *gridPar
                               q.shift, deltaTime);
 }
 
+static bool ensure_batch_segment(State::BatchAdjoint &A) {
+    const uint64_t N = A.N, K = A.K, NT = A.NT;
+    if (!(grow(A.segPos, A.capPos, (K + 1) * N) && grow(A.segVel, A.capVel, (K + 1) * N) &&
+          grow(A.segSPos, A.capSPos, K * N) && grow(A.segIds, A.capIds, K * N) &&
+          grow(A.segOff, A.capOff, K * (uint64_t(A.C) + 2)) && grow(A.work, A.capWork, 2 * N) &&
+          grow(A.lam, A.capLam, 4 * N + NT) && grow(A.wPos, A.capWPos, NT) && grow(A.wVel, A.capWVel, NT) &&
+          grow(A.partial, A.capPartial, uint64_t(A.waves) * kAdjParams) &&
+          grow(A.grad, A.capGrad, uint64_t(A.R) * kAdjParams)))
+        return false;
+    if (!A.srd) return true;
+    const uint64_t cpS = (K + A.gap - 1) / A.gap + 1;  // collisions in a segment, at most
+    return grow(A.collHash, A.capCollHash, cpS * NT) && grow(A.collIds, A.capCollIds, cpS * NT) &&
+           grow(A.collOff, A.capCollOff, cpS * (uint64_t(A.Cs) + 2)) &&
+           grow(A.collCom, A.capCollCom, cpS * A.Cs) && grow(A.cellSum, A.capCellSum, A.Cs);
+}
+
+static bool batch_langevin(const State::Batch &b) {
+    bool lgv = false;
+    for (const BatchRep &q : b.reps) lgv = lgv || q.langevin != 0;
+    return lgv;
+}
+
 void nwBatchAdjointForward(float *pos, float *vel, float *force, float *forceOld, float *tangent, float deltaTime,
                            uint srdGap, const float *srdShifts, uint steps, uint checkpointEvery) {
     NW_INIT();
@@ -1662,6 +1714,15 @@ void nwBatchAdjointForward(float *pos, float *vel, float *force, float *forceOld
     A.ctr0 = b.steps;
     const uint32_t nck = (steps + checkpointEvery - 1) / checkpointEvery;
     const uint64_t stride = 2 * NT + 2 * N;
+    // the last segment stays in the store (see kHoldBytes)
+    const uint64_t K = checkpointEvery;
+    const uint64_t perStep = 52 * N + 4 * C + 8 + (srd ? (8 * NT + 20 * Cs) / srdGap : 0);
+    A.held = -1;
+    bool hold = K <= kHoldBytes / perStep;
+    if (hold && !ensure_batch_segment(A)) {
+        (void)hipGetLastError();  // no room for it: the run goes on without
+        hold = false;
+    }
     NW_REQUIRE(grow(A.ckpt, A.capCkpt, uint64_t(nck) * stride) && grow(A.hash, A.capHash, NT) &&
                    grow(A.sCell, A.capSCell, N) && grow(A.segIds, A.capIds, N) && grow(A.segSPos, A.capSPos, N) &&
                    grow(A.segOff, A.capOff, C + 2),
@@ -1680,10 +1741,10 @@ void nwBatchAdjointForward(float *pos, float *vel, float *force, float *forceOld
     a.force = reinterpret_cast<float4 *>(force);
     a.forceOld = reinterpret_cast<float4 *>(forceOld);
     a.hash = A.hash;
-    a.ids = A.segIds;
-    a.off = A.segOff;
     a.sCell = A.sCell;
-    a.sPos = A.segSPos;
+    // the step velocities are read only for the Langevin partials
+    const bool lgv = batch_langevin(b);
+    uint64_t slots = 0;  // collisions kept
     const size_t bytesT = NT * sizeof(float4), bytes = N * sizeof(float4);
     for (uint32_t k = 0; k < steps; ++k) {
         if (k % checkpointEvery == 0) {
@@ -1693,8 +1754,17 @@ void nwBatchAdjointForward(float *pos, float *vel, float *force, float *forceOld
                            copy_d2d(ck + 2 * NT + N, forceOld, bytes, s.stream),
                        "nwBatchAdjointForward: checkpoint copy failed");
         }
+        const bool keep = hold && k / K == nck - 1u;
+        const uint64_t j = keep ? k % K : 0;
         {
             TimedScope ts("batch_adj_fwd_md", s.stream);
+            // the last segment into its slots; before it the store's first
+            // slots are scratch
+            a.ids = A.segIds + j * N;
+            a.off = A.segOff + j * (C + 2);
+            a.sPos = A.segSPos + j * N;
+            a.keepPos = keep ? A.segPos + (j + 1) * N : nullptr;
+            a.keepVel = keep && lgv ? A.segVel + (j + 1) * N : nullptr;
             // the pair term reads no tangents: the run's last step stores them
             if (k + 1 == steps) a.tangent = reinterpret_cast<float4 *>(tangent);
             NW_HIP(batch_step_into(b, a, deltaTime, s.stream));
@@ -1703,28 +1773,15 @@ void nwBatchAdjointForward(float *pos, float *vel, float *force, float *forceOld
         if (srd && k % srdGap == 0) {
             TimedScope ts("batch_adj_fwd_srd", s.stream);
             const uint32_t c = k / srdGap;
-            if (!batch_srd_collision(s, c, a.pos, a.vel, A.collHash, A.collIds, A.collOff, A.collCom,
-                                     A.shifts + uint64_t(c) * b.R * 3, deltaTime * float(srdGap)))
+            const uint64_t u = keep ? slots++ : 0;
+            if (!batch_srd_collision(s, c, a.pos, a.vel, A.collHash + u * NT, A.collIds + u * NT,
+                                     A.collOff + u * (Cs + 2), A.collCom + u * Cs, A.shifts + uint64_t(c) * b.R * 3,
+                                     deltaTime * float(srdGap)))
                 return;
         }
     }
+    if (hold) A.held = int(nck) - 1;
     A.ready = true;
-}
-
-static bool ensure_batch_segment(State::BatchAdjoint &A) {
-    const uint64_t N = A.N, K = A.K, NT = A.NT;
-    if (!(grow(A.segPos, A.capPos, (K + 1) * N) && grow(A.segVel, A.capVel, (K + 1) * N) &&
-          grow(A.segSPos, A.capSPos, K * N) && grow(A.segIds, A.capIds, K * N) &&
-          grow(A.segOff, A.capOff, K * (uint64_t(A.C) + 2)) && grow(A.work, A.capWork, 2 * N) &&
-          grow(A.lam, A.capLam, 4 * N + NT) && grow(A.wPos, A.capWPos, NT) && grow(A.wVel, A.capWVel, NT) &&
-          grow(A.partial, A.capPartial, uint64_t(A.waves) * kAdjParams) &&
-          grow(A.grad, A.capGrad, uint64_t(A.R) * kAdjParams)))
-        return false;
-    if (!A.srd) return true;
-    const uint64_t cpS = (K + A.gap - 1) / A.gap + 1;  // collisions in a segment, at most
-    return grow(A.collHash, A.capCollHash, cpS * NT) && grow(A.collIds, A.capCollIds, cpS * NT) &&
-           grow(A.collOff, A.capCollOff, cpS * (uint64_t(A.Cs) + 2)) &&
-           grow(A.collCom, A.capCollCom, cpS * A.Cs) && grow(A.cellSum, A.capCellSum, A.Cs);
 }
 
 void nwBatchAdjointBackward(const float *dLdPos, const float *dLdVel, double *grad) {
@@ -1751,20 +1808,27 @@ void nwBatchAdjointBackward(const float *dLdPos, const float *dLdVel, double *gr
     const uint32_t nck = (A.steps + A.K - 1) / A.K;
     std::vector<int> collSlot(K);
     // the step velocities are read only for the Langevin partials
-    bool lgv = false;
-    for (uint32_t r = 0; r < b.R; ++r) lgv = lgv || b.reps[r].langevin != 0;
+    const bool lgv = batch_langevin(b);
     for (int c = int(nck) - 1; c >= 0; --c) {
         const uint32_t s0 = uint32_t(c) * A.K, len = std::min<uint32_t>(A.K, A.steps - s0);
         const float4 *ck = A.ckpt + uint64_t(c) * stride;
-        NW_HIP(hipMemcpyAsync(A.wPos, ck, NT * sizeof(float4), hipMemcpyDeviceToDevice, s.stream));
-        NW_HIP(hipMemcpyAsync(A.wVel, ck + NT, NT * sizeof(float4), hipMemcpyDeviceToDevice, s.stream));
-        NW_HIP(hipMemcpyAsync(F, ck + 2 * NT, bytes, hipMemcpyDeviceToDevice, s.stream));
-        NW_HIP(hipMemcpyAsync(G, ck + 2 * NT + N, bytes, hipMemcpyDeviceToDevice, s.stream));
-        NW_HIP(launch_set_step(b.stepCtr, A.ctr0 + s0, s.stream));
-        // recompute the segment: the full state in place, every step's bead
-        // state and cell lists and every collision's cells kept
+        // recompute the segment unless the forward run left it: the full state
+        // in place, every step's bead state and cell lists and every
+        // collision's cells kept
+        const bool have = A.held == c;
+        if (!have) {
+            A.held = -1;
+            NW_HIP(hipMemcpyAsync(A.wPos, ck, NT * sizeof(float4), hipMemcpyDeviceToDevice, s.stream));
+            NW_HIP(hipMemcpyAsync(A.wVel, ck + NT, NT * sizeof(float4), hipMemcpyDeviceToDevice, s.stream));
+            NW_HIP(hipMemcpyAsync(F, ck + 2 * NT, bytes, hipMemcpyDeviceToDevice, s.stream));
+            NW_HIP(hipMemcpyAsync(G, ck + 2 * NT + N, bytes, hipMemcpyDeviceToDevice, s.stream));
+            NW_HIP(launch_set_step(b.stepCtr, A.ctr0 + s0, s.stream));
+        }
         int slots = 0;
         for (uint32_t j = 0; j < len; ++j) {
+            const uint32_t k = s0 + j;
+            collSlot[j] = A.srd && k % A.gap == 0 ? slots++ : -1;
+            if (have) continue;
             BatchArrays a{};
             a.pos = A.wPos;
             a.vel = A.wVel;
@@ -1775,29 +1839,24 @@ void nwBatchAdjointBackward(const float *dLdPos, const float *dLdVel, double *gr
             a.off = A.segOff + uint64_t(j) * (C + 2);
             a.sCell = A.sCell;
             a.sPos = A.segSPos + uint64_t(j) * N;
+            a.keepPos = A.segPos + uint64_t(j + 1) * N;
+            a.keepVel = lgv ? A.segVel + uint64_t(j + 1) * N : nullptr;
             NW_HIP(batch_step_into(b, a, A.dt, s.stream));
-            NW_HIP(hipMemcpyAsync(A.segPos + uint64_t(j + 1) * N, A.wPos, bytes, hipMemcpyDeviceToDevice, s.stream));
-            if (lgv)
-                NW_HIP(hipMemcpyAsync(A.segVel + uint64_t(j + 1) * N, A.wVel, bytes, hipMemcpyDeviceToDevice,
-                                      s.stream));
-            collSlot[j] = -1;
-            const uint32_t k = s0 + j;
-            if (A.srd && k % A.gap == 0) {
-                const int sl = slots++;
-                collSlot[j] = sl;
-                const uint64_t u = uint64_t(sl);
+            if (collSlot[j] >= 0) {
+                const uint64_t u = uint64_t(collSlot[j]);
                 if (!batch_srd_collision(s, k / A.gap, A.wPos, A.wVel, A.collHash + u * NT, A.collIds + u * NT,
                                          A.collOff + u * (A.Cs + 2), A.collCom + u * A.Cs,
                                          A.shifts + uint64_t(k / A.gap) * A.R * 3, A.dt * float(A.gap)))
                     return;
             }
         }
+        A.held = c;
         // the adjoint through the segment, last step first
         for (int j = int(len) - 1; j >= 0; --j) {
             if (collSlot[j] >= 0) {
                 const uint64_t u = uint64_t(collSlot[j]);
                 NW_HIP(launch_srd_adj(A.collIds + u * NT, A.collOff + u * (A.Cs + 2), A.collHash + u * NT,
-                                      A.collCom + u * A.Cs, A.wVel, lv, A.cellSum, A.N, uint32_t(NT), A.Cs, q.cosA,
+                                      A.collCom + u * A.Cs, ck + NT, lv, A.cellSum, A.N, uint32_t(NT), A.Cs, q.cosA,
                                       q.sinA, q.rotBeads, s.stream));
             }
             AdjStepArgs as{};

@@ -89,6 +89,7 @@ hipError_t ensure_bucket_scratch(BucketScratch &s, const BucketPlan &bp);
 struct MdFrontArgs {
     float4 *pos, *vel, *force, *forceOld, *tangent;
     const float4 *posIn, *velIn;  // the step's input state when not pos / vel (NULL: in place)
+    float4 *keepPos, *keepVel;    // the new state once more (NULL: not)
     uint32_t *hash;               // out: the cell of every bead
     float dt, lgvStd;
     int langevin;
@@ -270,6 +271,7 @@ hipError_t launch_srd_rotate_batch(const uint32_t *hash, const float4 *com, floa
 
 struct BatchArrays {
     float4 *pos, *vel, *force, *forceOld, *tangent;
+    float4 *keepPos, *keepVel;  // the new state once more (NULL: not)
     // nonzero: the new force goes to forceOld's buffer (pairs add there too)
     // and force's buffer is left as the old force (no replica reverses)
     int swapForces;

@@ -142,8 +142,11 @@ __global__ __launch_bounds__(BLOCK) void k_md_front(MdFrontArgs a, KP kp) {
     const FrontLane o = md_front_lane(kp, m, a.posIn ? a.posIn : a.pos, a.velIn ? a.velIn : a.vel, a.force,
                                       a.forceOld, a.dt, a.lgvStd, a.langevin, a.seed, a.offRev, a.offLgv,
                                       a.tangent != nullptr);
-    if (m.active)
+    if (m.active) {
         a.hash[m.bead] = md_front_store(kp, m, o, a.pos, a.vel, a.force, a.forceOld, a.tangent, a.swapForces != 0);
+        if (a.keepPos) a.keepPos[m.bead] = f4(o.r, o.pw);
+        if (a.keepVel) a.keepVel[m.bead] = f4(o.v, o.vw);
+    }
 }
 
 // The tangents of the worms' beads from their positions, as the front's
@@ -678,6 +681,8 @@ __global__ __launch_bounds__(kBlock) void k_md_front_batch(BatchArrays a, const 
         const uint32_t h = md_front_store(kp, m, o, pos, vel, force, forceOld,
                                           a.tangent ? a.tangent + rep.beadOffset : nullptr, a.swapForces != 0);
         a.hash[rep.beadOffset + m.bead] = rep.cellOffset + h;
+        if (a.keepPos) a.keepPos[rep.beadOffset + m.bead] = f4(o.r, o.pw);
+        if (a.keepVel) a.keepVel[rep.beadOffset + m.bead] = f4(o.v, o.vw);
     }
 }
 
