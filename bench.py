@@ -171,8 +171,8 @@ def fused_plan(n, cells, filament_size):
 def batched_form(args):
     """256 independent replicas (worms U[500, 8000] x U{10..30} beads, area
     fraction 0.3, f_a log-uniform [0.1, 10], kappa U[1, 20], Langevin gamma 2,
-    kT 0.1, dt 1e-3): aggregate bead-steps/s of the batched step replayed as a
-    hipGraph, and of the same replicas one launch sequence per replica."""
+    kT 0.1, dt 1e-3): aggregate bead-steps/s of the batched step, and of the
+    same replicas one launch sequence per replica."""
     from nwamd import replicas, system
     specs = replicas.replica_specs_config2(args.replicas)
     rs = replicas.ReplicaSet(specs, replicas.worm_physics(gamma=2.0, kT=0.1, fdt=True))
@@ -184,7 +184,7 @@ def batched_form(args):
                              ("one_per_launch", replicas.NW_REPLICAS_ONE_PER_LAUNCH, args.one_per_launch_steps)):
         if steps <= 0:
             continue
-        rs.update(args.dt, max(2, steps // 10), form)  # warm-up (the graph is captured here)
+        rs.update(args.dt, max(2, steps // 10), form)  # warm-up
         rs.sync()
         t0 = time.perf_counter()
         rs.update(args.dt, steps, form)
@@ -194,9 +194,8 @@ def batched_form(args):
                         ms_per_step=round(el / steps * 1e3, 4))
     if "graph" in out and "one_per_launch" in out:
         out["speedup"] = round(out["graph"]["value"] / out["one_per_launch"]["value"], 2)
-    # the kernels the graph replays, launched directly for a few steps with
-    # events on their dispatch packets: per-kernel durations, the roofline of
-    # the longest
+    # a few more steps with events on the kernels' dispatch packets: per-kernel
+    # durations, the roofline of the longest
     import ctypes
 
     import numpy as np
@@ -456,8 +455,7 @@ def main():
     ap.add_argument("--replicas", type=int, default=256, help="replicas of the batched form")
     ap.add_argument("--batched-steps", type=int, default=200, help="timed steps of the batched form (0: skip)")
     ap.add_argument("--batched-no-graph", action="store_true",
-                    help="launch the batched step's kernels directly instead of replaying the captured graph "
-                         "(for counter passes of a profiler)")
+                    help="the batched step's NW_REPLICAS_LAUNCHES form (the same launches as the default)")
     ap.add_argument("--one-per-launch-steps", type=int, default=20,
                     help="timed steps of the replicas one launch sequence each (0: skip)")
     ap.add_argument("--adjoint-steps", type=int, default=2000,

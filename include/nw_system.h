@@ -102,7 +102,7 @@ typedef struct NWReplicaPhysics {
 } NWReplicaPhysics;
 
 enum {
-    NW_REPLICAS_GRAPH = 0,          /* batched step, captured once as a hipGraph and replayed */
+    NW_REPLICAS_GRAPH = 0,          /* batched step (nwBatchMdStep with useGraph: the same launches) */
     NW_REPLICAS_LAUNCHES = 1,       /* batched step, launched kernel by kernel */
     NW_REPLICAS_ONE_PER_LAUNCH = 2  /* every replica through its own nwFusedMdStep per step */
 };

@@ -66,11 +66,6 @@ struct State {
         SortRep *sortDev = nullptr;
         BatchSortPlan sortPlan;
         RowsPlan rows{};  // blocks > 0: order and pairs in one launch
-        // the step as graphs: [0] force -> forceOld, [1] the buffers' roles
-        // exchanged (double-buffered forces, when no replica reverses)
-        hipGraphExec_t exec[2] = {nullptr, nullptr};
-        hipGraph_t graph[2] = {nullptr, nullptr};
-        std::vector<uintptr_t> key;  // arguments the graphs were captured with
         bool swap = false;
     } batch;
     // adjoint of the fused MD step: checkpoints of the last nwAdjointForward
@@ -963,22 +958,11 @@ static void observe_kp(const KP &kp, const float *pos, const float *vel, uint nu
 // ---------------------------------------------------------------------------
 // batched replicas
 // ---------------------------------------------------------------------------
-static void batch_drop_graph(State::Batch &b) {
-    for (int k = 0; k < 2; ++k) {
-        if (b.exec[k]) (void)hipGraphExecDestroy(b.exec[k]);
-        if (b.graph[k]) (void)hipGraphDestroy(b.graph[k]);
-        b.exec[k] = nullptr;
-        b.graph[k] = nullptr;
-    }
-    b.key.clear();
-}
-
 void nwBatchSetReplicas(const NWReplicaParams *reps, uint numReplicas) {
     NW_INIT();
     State &s = S();
     State::Batch &b = s.batch;
     NW_REQUIRE(numReplicas == 0 || reps != nullptr, "nwBatchSetReplicas: NULL replicas");
-    batch_drop_graph(b);
     s.bsol.R = 0;  // a new batch has no solvent until nwBatchSetSolvent
     s.badj.ready = false;
     b.reps.assign(numReplicas, BatchRep{});
@@ -1082,36 +1066,35 @@ void nwBatchRngState(uint replica, uint64_t *offset) {
 }
 
 // the launches of one batched step
-// (timed: each kernel may carry the events of its timer family -- never
-// while the stream is being captured into a graph)
 static hipError_t batch_step(State::Batch &b, const BatchArrays &a, const float4 *vel, const float4 *tan,
-                             float4 *sVel, float4 *sTan, float dt, hipStream_t st, bool timed = false) {
+                             float4 *sVel, float4 *sTan, float dt, hipStream_t st) {
     hipError_t e;
     {
-        TimedScope ts(timed ? "batch_front" : "", st, true);
+        TimedScope ts("batch_front", st, true);
         if ((e = launch_md_front_batch(a, b.dev, b.R, b.waves, b.stepCtr, dt, st)) != hipSuccess) return e;
     }
     if (b.rows.blocks) {
-        TimedScope ts(timed ? "batch_collide" : "", st, true);
+        TimedScope ts("batch_collide", st, true);
         return launch_rows_batch(b.rows, a, b.dev, b.R, b.stepCtr, st);
     }
     {
-        TimedScope ts(timed ? "batch_tiles" : "", st, true);
+        TimedScope ts("batch_tiles", st, true);
         if ((e = launch_hash_tiles_batch(a.hash, b.sortDev, b.R, b.sortPlan, b.scratch, st)) != hipSuccess) return e;
     }
     {
-        TimedScope ts(timed ? "batch_sort" : "", st, true);
+        TimedScope ts("batch_sort", st, true);
         if ((e = launch_md_cells_batch(b.sortDev, b.R, b.sortPlan, b.scratch, a.ids, a.pos, vel, tan, a.sPos, sVel,
                                        sTan, st)) != hipSuccess)
             return e;
     }
-    TimedScope ts(timed ? "batch_collide" : "", st, true);
+    TimedScope ts("batch_collide", st, true);
     return launch_collide_batch(a, b.dev, b.R, b.blocks, b.mode, b.tan, b.unit, b.stepCtr, st);
 }
 
 void nwBatchMdStep(float *pos, float *vel, float *force, float *forceOld, float *tangent, uint *gridParticleIndex,
                    float *sortedPos, float *sortedVel, float *sortedTangent, float deltaTime, uint steps,
                    int useGraph) {
+    (void)useGraph;  // see nw_abi.h
     NW_INIT();
     State &s = S();
     State::Batch &b = s.batch;
@@ -1136,11 +1119,6 @@ void nwBatchMdStep(float *pos, float *vel, float *force, float *forceOld, float 
     a.sTan = b.tan ? reinterpret_cast<float4 *>(sortedTangent) : nullptr;
     const float4 *gv = b.mode == 0 ? a.vel : nullptr;
     const float4 *gt = b.tan ? a.tangent : nullptr;
-    uint32_t dtBits;
-    std::memcpy(&dtBits, &deltaTime, 4);
-    const std::vector<uintptr_t> key = {uintptr_t(pos), uintptr_t(vel), uintptr_t(force), uintptr_t(forceOld),
-                                        uintptr_t(tangent), uintptr_t(gridParticleIndex), uintptr_t(sortedPos),
-                                        uintptr_t(sortedVel), uintptr_t(sortedTangent), uintptr_t(dtBits)};
     // double-buffered forces: phase 0 reads force and writes the new force
     // into forceOld's buffer, phase 1 the other way round.  The call's last
     // step puts everything where the caller reads it: it stores the tangents
@@ -1153,70 +1131,23 @@ void nwBatchMdStep(float *pos, float *vel, float *force, float *forceOld, float 
     ar[1].force = a.forceOld;
     ar[1].forceOld = a.force;
     int ph = 0;
-    uint done = 0;
-    const auto direct_step = [&]() {
+    for (uint done = 0; done < steps; ++done) {
         BatchArrays x = ar[ph];
         if (done + 1 == steps) {
             x.tangent = a.tangent;
             if (ph == 0) x.swapForces = 0;
         }
-        return batch_step(b, x, gv, gt, a.sVel, a.sTan, deltaTime, s.stream, true);
-    };
-    // after `done` steps and a failure: the force arrays' contents in the
-    // caller's roles and the tangents of the positions reached
-    const auto settle = [&]() {
-        if (ph == 1) (void)launch_swap4(a.force, a.forceOld, b.N, s.stream);
-        for (uint32_t r = 0; !b.tan && done > 0 && r < b.R; ++r) {
-            const BatchRep &q = b.reps[r];
-            (void)launch_filament_tangents(a.pos + q.beadOffset, a.tangent + q.beadOffset, q.kp.p.numFilaments, q.kp,
-                                           s.stream);
-        }
-    };
-    if (useGraph && steps > 1 && (!b.exec[0] || b.key != key)) {
-        // one direct step first (scratch and kernel attributes are set up
-        // outside the capture), then capture the step (the phases that the
-        // steps before the last take)
-        batch_drop_graph(b);
-        NW_HIP(direct_step());
-        ++done;
-        ++b.steps;
-        if (b.swap) ph = 1;
-        if (done + 1 < steps) {
-            hipError_t e = hipSuccess;
-            for (int k = 0; k < (b.swap ? 2 : 1) && e == hipSuccess; ++k) {
-                if ((e = hipStreamBeginCapture(s.stream, hipStreamCaptureModeThreadLocal)) != hipSuccess) break;
-                const hipError_t e1 = batch_step(b, ar[k], gv, gt, a.sVel, a.sTan, deltaTime, s.stream);
-                hipGraph_t g = nullptr;
-                const hipError_t e2 = hipStreamEndCapture(s.stream, &g);
-                e = e1 != hipSuccess ? e1 : e2;
-                if (e != hipSuccess) break;
-                b.graph[k] = g;
-                e = hipGraphInstantiate(&b.exec[k], g, nullptr, nullptr, 0);
-            }
-            if (e != hipSuccess) {
-                // as in the replay loop below: the contents go back to the
-                // caller's roles before the error is reported
-                batch_drop_graph(b);
-                settle();
-                fail(__FILE__, __LINE__, int(e), "nwBatchMdStep: graph capture failed: HIP error %d (%s)", int(e),
-                     hipGetErrorString(e));
-                return;
-            }
-            b.key = key;
-        }
-    }
-    for (; done < steps; ++done) {
-        hipError_t e = hipSuccess;
-        if (useGraph && done + 1 < steps) {
-            TimedScope ts("batch_step", s.stream);
-            e = hipGraphLaunch(b.exec[ph], s.stream);
-        } else {
-            e = direct_step();
-        }
+        const hipError_t e = batch_step(b, x, gv, gt, a.sVel, a.sTan, deltaTime, s.stream);
         if (e != hipSuccess) {
-            // report the failing step; what the steps before it reached is
-            // the caller's
-            settle();
+            // what the steps before it reached is the caller's: the force
+            // arrays' contents in their roles and the tangents; then report
+            // the failing step
+            if (ph == 1) (void)launch_swap4(a.force, a.forceOld, b.N, s.stream);
+            for (uint32_t r = 0; !b.tan && done > 0 && r < b.R; ++r) {
+                const BatchRep &q = b.reps[r];
+                (void)launch_filament_tangents(a.pos + q.beadOffset, a.tangent + q.beadOffset, q.kp.p.numFilaments,
+                                               q.kp, s.stream);
+            }
             fail(__FILE__, __LINE__, int(e), "nwBatchMdStep: step %u of %u failed: HIP error %d (%s)", done, steps,
                  int(e), hipGetErrorString(e));
             return;
