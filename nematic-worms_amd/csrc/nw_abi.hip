@@ -57,6 +57,8 @@ struct State {
         std::vector<uint32_t> beadOff, cellOff;
         BatchRep *dev = nullptr;
         uint64_t *stepCtr = nullptr;
+        unsigned char *table = nullptr;  // holds stepCtr, dev and sortDev
+        size_t capTable = 0;
         uint32_t R = 0, N = 0, cells = 0, waves = 0, blocks = 0;
         int mode = 1;
         bool tan = false, unit = true;
@@ -106,7 +108,9 @@ struct State {
     // SRD solvent of the batch (nwBatchSetSolvent)
     struct BatchSolvent {
         std::vector<SrdRep> reps;
-        SrdRep *dev = nullptr;
+        SrdRep *dev = nullptr;  // in table
+        unsigned char *table = nullptr;
+        size_t capTable = 0;
         std::vector<uint32_t> solvOff, cellOff;  // R + 1 each: first solvent particle, first SRD cell
         uint32_t R = 0, Ns = 0, cells = 0;
         float cosA = 0.f, sinA = 0.f;
@@ -958,6 +962,23 @@ static void observe_kp(const KP &kp, const float *pos, const float *vel, uint nu
 // ---------------------------------------------------------------------------
 // batched replicas
 // ---------------------------------------------------------------------------
+// A replica table to the device, into the buffer that is there when it is large
+// enough (a batch is set anew for every evaluation of an objective; two frees,
+// two allocations and four copies took 52 us, one copy 28).  Waits for kernels
+// that may still read the table before, on any stream, as freeing it did.
+static hipError_t upload_table(unsigned char *&dev, size_t &cap, const void *src, size_t bytes) {
+    hipError_t e = hipDeviceSynchronize();
+    if (e != hipSuccess) return e;
+    if (bytes > cap || bytes < cap / 4) {
+        if (dev) (void)hipFree(dev);
+        dev = nullptr;
+        cap = 0;
+        if ((e = hipMalloc(&dev, bytes)) != hipSuccess) return e;
+        cap = bytes;
+    }
+    return hipMemcpy(dev, src, bytes, hipMemcpyHostToDevice);
+}
+
 void nwBatchSetReplicas(const NWReplicaParams *reps, uint numReplicas) {
     NW_INIT();
     State &s = S();
@@ -1018,35 +1039,34 @@ void nwBatchSetReplicas(const NWReplicaParams *reps, uint numReplicas) {
     if (numReplicas == 0) b.tan = false, b.unit = true;
     b.steps = 0;
     (void)rows_plan_batch(b.reps.data(), numReplicas, b.rows);
-    if (b.dev) (void)hipFree(b.dev);
-    b.dev = nullptr;
-    if (numReplicas) {
-        // the records, then their wavefront and workgroup offsets packed (the
-        // kernels' replica lookups bisect those)
-        static_assert(sizeof(BatchRep) % alignof(uint32_t) == 0, "offsets follow the records");
-        const size_t recBytes = sizeof(BatchRep) * numReplicas;
-        std::vector<unsigned char> table(recBytes + 3 * sizeof(uint32_t) * numReplicas);
-        memcpy(table.data(), b.reps.data(), recBytes);
-        uint32_t *off = reinterpret_cast<uint32_t *>(table.data() + recBytes);
-        for (uint r = 0; r < numReplicas; ++r) {
-            off[r] = b.reps[r].waveOffset;
-            off[numReplicas + r] = b.reps[r].blockOffset;
-            off[2 * numReplicas + r] = b.reps[r].rowBlock;
-        }
-        NW_HIP(hipMalloc(&b.dev, table.size()));
-        NW_HIP(hipMemcpy(b.dev, table.data(), table.size(), hipMemcpyHostToDevice));
-    }
-    if (!b.stepCtr) NW_HIP(hipMalloc(&b.stepCtr, sizeof(uint64_t)));
-    NW_HIP(hipMemset(b.stepCtr, 0, sizeof(uint64_t)));
     b.sort.assign(numReplicas, SortRep{});
     b.sortPlan = BatchSortPlan{};
-    if (b.sortDev) (void)hipFree(b.sortDev);
+    const char *why = "";
+    if (N) why = make_sort_reps(b.beadOff.data(), b.cellOff.data(), numReplicas, b.sort.data(), b.sortPlan);
+    // one buffer, one copy: the step counter, the records, then their
+    // wavefront and workgroup offsets packed (the kernels' replica lookups
+    // bisect those), then the sort's records
+    static_assert(sizeof(BatchRep) % alignof(uint32_t) == 0, "offsets follow the records");
+    const size_t recAt = 16, offAt = recAt + sizeof(BatchRep) * numReplicas,
+                 sortAt = (offAt + 3 * sizeof(uint32_t) * numReplicas + 15) & ~size_t(15);
+    std::vector<unsigned char> table(sortAt + sizeof(SortRep) * numReplicas, 0);
+    memcpy(table.data() + recAt, b.reps.data(), offAt - recAt);
+    memcpy(table.data() + sortAt, b.sort.data(), table.size() - sortAt);
+    uint32_t *off = reinterpret_cast<uint32_t *>(table.data() + offAt);
+    for (uint r = 0; r < numReplicas; ++r) {
+        off[r] = b.reps[r].waveOffset;
+        off[numReplicas + r] = b.reps[r].blockOffset;
+        off[2 * numReplicas + r] = b.reps[r].rowBlock;
+    }
+    b.dev = nullptr;
     b.sortDev = nullptr;
+    b.stepCtr = nullptr;
+    NW_HIP(upload_table(b.table, b.capTable, table.data(), table.size()));
+    b.stepCtr = reinterpret_cast<uint64_t *>(b.table);
+    if (numReplicas) b.dev = reinterpret_cast<BatchRep *>(b.table + recAt);
     if (N) {
-        const char *why = make_sort_reps(b.beadOff.data(), b.cellOff.data(), numReplicas, b.sort.data(), b.sortPlan);
         NW_REQUIRE(!*why, "nwBatchSetReplicas: %s", why);
-        NW_HIP(hipMalloc(&b.sortDev, sizeof(SortRep) * numReplicas));
-        NW_HIP(hipMemcpy(b.sortDev, b.sort.data(), sizeof(SortRep) * numReplicas, hipMemcpyHostToDevice));
+        b.sortDev = reinterpret_cast<SortRep *>(b.table + sortAt);
         NW_HIP(ensure_batch_sort_scratch(b.scratch, b.sortPlan));
     }
 }
@@ -1467,7 +1487,6 @@ void nwBatchSetSolvent(const NWReplicaSolvent *solvent, uint numReplicas) {
     s.badj.ready = false;
     q.R = q.Ns = q.cells = 0;
     q.reps.clear();
-    if (q.dev) (void)hipFree(q.dev);
     q.dev = nullptr;
     if (numReplicas == 0) return;
     NW_REQUIRE(solvent != nullptr && numReplicas == b.R,
@@ -1510,8 +1529,8 @@ void nwBatchSetSolvent(const NWReplicaSolvent *solvent, uint numReplicas) {
     q.cosA = float(std::cos(double(alpha)));
     q.sinA = float(std::sin(double(alpha)));
     q.rotBeads = rot;
-    NW_HIP(hipMalloc(&q.dev, sizeof(SrdRep) * numReplicas));
-    NW_HIP(hipMemcpy(q.dev, q.reps.data(), sizeof(SrdRep) * numReplicas, hipMemcpyHostToDevice));
+    NW_HIP(upload_table(q.table, q.capTable, q.reps.data(), sizeof(SrdRep) * numReplicas));
+    q.dev = reinterpret_cast<SrdRep *>(q.table);
     q.R = numReplicas;
 }
 
