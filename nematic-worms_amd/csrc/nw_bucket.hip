@@ -124,6 +124,13 @@ __host__ __device__ constexpr uint32_t staged_stage_words(uint32_t B1, uint32_t 
     return (B1 + TB / 64 + 2 + 3) & ~3u;
 }
 
+// words that level 1 copies beside reading the keys (from NULL: none): the
+// values of a key-value sort, which level 2 writes in order over the originals
+struct TileCopy {
+    const uint32_t *from;
+    uint32_t *to;
+};
+
 // ---------------------------------------------------------------------------
 // level 1 as a kernel of its own: the cell of every particle (SRD: from the
 // position, written to hash; otherwise read from hash), tile histogram, P
@@ -133,7 +140,7 @@ template <bool FROM_POS>
 __global__ __launch_bounds__(kTileBlock) void k_tiles(const float4 *__restrict__ pos, uint32_t *__restrict__ hash,
                                                       uint32_t *__restrict__ pairs, uint32_t *__restrict__ P,
                                                       uint32_t *__restrict__ range,
-                                                      BucketPlan bp, KP kp) {
+                                                      BucketPlan bp, KP kp, TileCopy cp) {
     // the whole row is written: the full bucket range
     if (range && threadIdx.x == 0) {
         range[2u * blockIdx.x] = 0u;
@@ -154,6 +161,7 @@ __global__ __launch_bounds__(kTileBlock) void k_tiles(const float4 *__restrict__
             hash[i] = h;
         } else {
             h = min(hash[i], bp.cells - 1u);  // a key outside the grid sorts as its last cell
+            if (cp.from) cp.to[i] = cp.from[i];
         }
         atomicAdd(&lh[h >> bp.shift], 1u);
     }
@@ -182,7 +190,7 @@ template <bool FROM_POS, int ITEMS, int TB = kTileBlock>
 __device__ __forceinline__ void tiles_staged_body(const float4 *__restrict__ pos, uint32_t *__restrict__ hash,
                                                   uint32_t *__restrict__ pairs, uint32_t *__restrict__ P,
                                                   uint32_t *__restrict__ range, const BucketPlan &bp, const KP &kp,
-                                                  uint32_t t, uint32_t cellBase, uint32_t *lh) {
+                                                  uint32_t t, uint32_t cellBase, uint32_t *lh, TileCopy cp = {}) {
     const uint32_t B1 = bp.buckets + 1;
     uint32_t *wsum = lh + B1;
     uint32_t *brng = wsum + TB / 64;  // the tile's first and last bucket
@@ -195,7 +203,11 @@ __device__ __forceinline__ void tiles_staged_body(const float4 *__restrict__ pos
     __syncthreads();
     const uint32_t i0 = t * bp.tileItems;
     const uint32_t i1 = min(i0 + bp.tileItems, bp.n);
-    uint32_t h[ITEMS], rk[ITEMS];
+    uint32_t h[ITEMS], rk[ITEMS], v[ITEMS];
+    if (!FROM_POS && cp.from) {
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) v[k] = cp.from[min(i0 + uint32_t(k) * TB + threadIdx.x, i1 - 1u)];
+    }
     const SrdGrid g = srd_grid(kp.s, mk(kp.s.randOffset.x, kp.s.randOffset.y, kp.s.randOffset.z));
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
@@ -246,6 +258,7 @@ __device__ __forceinline__ void tiles_staged_body(const float4 *__restrict__ pos
 #pragma unroll
     for (int k = 0; k < ITEMS; ++k) {
         const uint32_t i = i0 + uint32_t(k) * TB + threadIdx.x;
+        if (!FROM_POS && cp.from && i < i1) cp.to[i] = v[k];
         if (i < i1) stage[lh[h[k] >> bp.shift] + rk[k]] = pack_pair(h[k] & ((1u << bp.shift) - 1u), i - i0);
     }
     __syncthreads();
@@ -257,9 +270,10 @@ template <bool FROM_POS, int ITEMS, int TB = kTileBlock>
 __global__ __launch_bounds__(TB) void k_tiles_staged(const float4 *__restrict__ pos,
                                                              uint32_t *__restrict__ hash,
                                                              uint32_t *__restrict__ pairs, uint32_t *__restrict__ P,
-                                                             uint32_t *__restrict__ range, BucketPlan bp, KP kp) {
+                                                             uint32_t *__restrict__ range, BucketPlan bp, KP kp,
+                                                             TileCopy cp) {
     extern __shared__ __align__(16) uint32_t lh[];
-    tiles_staged_body<FROM_POS, ITEMS, TB>(pos, hash, pairs, P, range, bp, kp, blockIdx.x, 0u, lh);
+    tiles_staged_body<FROM_POS, ITEMS, TB>(pos, hash, pairs, P, range, bp, kp, blockIdx.x, 0u, lh, cp);
 }
 
 // the replica that owns item v of a launch over all replicas (offsets
@@ -321,6 +335,10 @@ struct CellsArgs {
     // MD gathers (sPos NULL: none)
     const float4 *pos, *vel, *tan;
     float4 *sPos, *sVel, *sTan;
+    // the values of a key-value sort (NULL: none) and where they go in order;
+    // ids is scratch then
+    const uint32_t *val;
+    uint32_t *sVal;
     // SRD cell sums
     const float4 *srdVel;
     float4 *com;
@@ -639,7 +657,8 @@ __device__ __forceinline__ void scan_cells(uint32_t *cnt, uint32_t nc, uint32_t 
 }
 
 // what the MD sort gathers beside the ids and cells
-enum : int { kGatherPos = 1, kGatherVel = 2, kGatherTan = 4 };
+// (kGatherVal: instead of the ids, the values of a key-value sort)
+enum : int { kGatherPos = 1, kGatherVel = 2, kGatherTan = 4, kGatherVal = 8 };
 
 // MD, bucket b of one system (see CellsArgs for the bases of a replica),
 // BLOCK threads; a bucket of at most CAP members is staged in LDS, each
@@ -659,7 +678,8 @@ __device__ __forceinline__ void md_cells_body(const CellsArgs &o, const BucketPl
                                               unsigned char *smem) {
     constexpr int PER = CAP / BLOCK;
     static_assert(PER * BLOCK == CAP, "the staged members are PER per thread");
-    constexpr bool POS = GATHER & kGatherPos, VEL = GATHER & kGatherVel, TAN = GATHER & kGatherTan;
+    constexpr bool POS = GATHER & kGatherPos, VEL = GATHER & kGatherVel, TAN = GATHER & kGatherTan,
+                   VAL = GATHER & kGatherVal;
     // records moved as plain 4-vectors (register values, never a copy of a
     // float4 object through memory)
     typedef float v4 __attribute__((ext_vector_type(4)));
@@ -689,6 +709,7 @@ __device__ __forceinline__ void md_cells_body(const CellsArgs &o, const BucketPl
         uint2 q[PER];
         uint32_t rk[PER];
         v4 P[POS ? PER : 1], V[VEL ? PER : 1], Tn[TAN ? PER : 1];
+        uint32_t X[VAL ? PER : 1];
         if (m) {
             fill_tile_of<BLOCK, PER>(tileOf, wsum);
             // every load of the thread's members in flight before the first
@@ -705,6 +726,7 @@ __device__ __forceinline__ void md_cells_body(const CellsArgs &o, const BucketPl
                 if (POS) P[j] = reinterpret_cast<const v4 *>(o.pos)[q[j].y];
                 if (VEL) V[j] = reinterpret_cast<const v4 *>(o.vel)[q[j].y];
                 if (TAN) Tn[j] = reinterpret_cast<const v4 *>(o.tan)[q[j].y];
+                if (VAL) X[j] = o.val[q[j].y];
             }
 #pragma unroll
             for (int j = 0; j < PER; ++j)
@@ -729,7 +751,7 @@ __device__ __forceinline__ void md_cells_body(const CellsArgs &o, const BucketPl
                 const uint32_t a = cnt[q[j].x], z = cnt[q[j].x + 1u];
                 uint32_t r = a;
                 for (uint32_t u = a; u < z; ++u) r += lid[u] < q[j].y ? 1u : 0u;
-                cur[r] = q[j].y;
+                cur[r] = VAL ? X[j] : q[j].y;
                 if (POS) reinterpret_cast<v4 *>(o.sPos)[sb + r] = P[j];
                 if (VEL) reinterpret_cast<v4 *>(o.sVel)[sb + r] = V[j];
                 if (TAN) reinterpret_cast<v4 *>(o.sTan)[sb + r] = Tn[j];
@@ -737,7 +759,7 @@ __device__ __forceinline__ void md_cells_body(const CellsArgs &o, const BucketPl
         }
         __syncthreads();
         for (uint32_t k = tid; k < m; k += BLOCK) {
-            out[k] = cur[k];
+            (VAL ? o.sVal + sb : out)[k] = cur[k];
             o.cellOf[sb + k] = o.cellBase + cell0 + uint32_t(lcell[k]);
         }
         return;
@@ -770,6 +792,7 @@ __device__ __forceinline__ void md_cells_body(const CellsArgs &o, const BucketPl
         if (POS) o.sPos[sb + k] = o.pos[id];
         if (VEL) o.sVel[sb + k] = o.vel[id];
         if (TAN) o.sTan[sb + k] = o.tan[id];
+        if (VAL) o.sVal[sb + k] = o.val[id];
     }
 }
 
@@ -1121,7 +1144,7 @@ hipError_t grant_lds(const void *fn, size_t lds) {
 
 template <bool FROM_POS, int ITEMS, int TB = kTileBlock>
 static hipError_t launch_staged(const float4 *pos, uint32_t *hash, const BucketPlan &bp, BucketScratch &s,
-                                const KP &kp, uint32_t *range, hipStream_t st) {
+                                const KP &kp, uint32_t *range, TileCopy cp, hipStream_t st) {
     static_assert(ITEMS * TB == 1024 || ITEMS * TB == 2048 || ITEMS * TB == 4096 || ITEMS * TB == 8192 ||
                       ITEMS * TB == 16384,
                   "tile size");
@@ -1131,7 +1154,7 @@ static hipError_t launch_staged(const float4 *pos, uint32_t *hash, const BucketP
     hipError_t e = grant_lds(fn, lds);
     if (e != hipSuccess) return e;
     NW_LAUNCH((k_tiles_staged<FROM_POS, ITEMS, TB>), dim3(bp.tiles), dim3(TB), lds, st, pos, hash, s.pairs, s.P,
-              range, bp, kp);
+              range, bp, kp, cp);
     return hipGetLastError();
 }
 
@@ -1140,26 +1163,26 @@ static hipError_t launch_staged(const float4 *pos, uint32_t *hash, const BucketP
 // ranges: record every tile's bucket range and write only that part of its
 // P row (the cells pass must then read them: o.tileRange)
 static hipError_t launch_tiles(bool fromPos, const float4 *pos, uint32_t *hash, const BucketPlan &bp,
-                               BucketScratch &s, const KP &kp, bool ranges, hipStream_t st) {
+                               BucketScratch &s, const KP &kp, bool ranges, hipStream_t st, TileCopy cp = {}) {
     if (bp.n == 0) return hipSuccess;
     uint32_t *range = ranges ? s.tileRange : nullptr;
     const size_t stagedLds = size_t(staged_stage_words(bp.buckets + 1, kTileBlock)) * 4 + size_t(bp.tileItems) * 4;
     if (stagedLds <= 160 * 1024) {
         // small tiles (more workgroups for a chip of 256 CUs) as 256 threads
-        if (!fromPos && bp.tileItems == 1024) return launch_staged<false, 4, 256>(pos, hash, bp, s, kp, range, st);
-        if (!fromPos && bp.tileItems == 2048) return launch_staged<false, 8, 256>(pos, hash, bp, s, kp, range, st);
+        if (!fromPos && bp.tileItems == 1024) return launch_staged<false, 4, 256>(pos, hash, bp, s, kp, range, cp, st);
+        if (!fromPos && bp.tileItems == 2048) return launch_staged<false, 8, 256>(pos, hash, bp, s, kp, range, cp, st);
         if (bp.tileItems == 4 * kTileBlock)
-            return fromPos ? launch_staged<true, 4>(pos, hash, bp, s, kp, range, st)
-                           : launch_staged<false, 4>(pos, hash, bp, s, kp, range, st);
+            return fromPos ? launch_staged<true, 4>(pos, hash, bp, s, kp, range, cp, st)
+                           : launch_staged<false, 4>(pos, hash, bp, s, kp, range, cp, st);
         // the SRD tiles of 8192 as 512 threads x 16: three workgroups per CU
         // by LDS and registers against two of 1024 threads (SRD workload:
         // 708 tiles in one round, 35 -> 33 us)
         if (bp.tileItems == 8 * kTileBlock)
-            return fromPos ? launch_staged<true, 16, 512>(pos, hash, bp, s, kp, range, st)
-                           : launch_staged<false, 8>(pos, hash, bp, s, kp, range, st);
+            return fromPos ? launch_staged<true, 16, 512>(pos, hash, bp, s, kp, range, cp, st)
+                           : launch_staged<false, 8>(pos, hash, bp, s, kp, range, cp, st);
         if (bp.tileItems == 16 * kTileBlock)
-            return fromPos ? launch_staged<true, 16>(pos, hash, bp, s, kp, range, st)
-                           : launch_staged<false, 16>(pos, hash, bp, s, kp, range, st);
+            return fromPos ? launch_staged<true, 16>(pos, hash, bp, s, kp, range, cp, st)
+                           : launch_staged<false, 16>(pos, hash, bp, s, kp, range, cp, st);
     }
     const size_t lds = (size_t(bp.buckets) + 1 + kTileBlock / 64) * sizeof(uint32_t);
     const void *fn = fromPos ? reinterpret_cast<const void *>(&k_tiles<true>)
@@ -1168,10 +1191,10 @@ static hipError_t launch_tiles(bool fromPos, const float4 *pos, uint32_t *hash, 
     if (e != hipSuccess) return e;
     if (fromPos)
         NW_LAUNCH(k_tiles<true>, dim3(bp.tiles), dim3(kTileBlock), lds, st, pos, hash, s.pairs, s.P, range,
-                  bp, kp);
+                  bp, kp, cp);
     else
         NW_LAUNCH(k_tiles<false>, dim3(bp.tiles), dim3(kTileBlock), lds, st, pos, hash, s.pairs, s.P, range,
-                  bp, kp);
+                  bp, kp, cp);
     return hipGetLastError();
 }
 
@@ -1278,7 +1301,8 @@ hipError_t launch_hash_tiles_batch(const uint32_t *hash, const SortRep *reps, ui
 // go(std::integral_constant<int, G>) for the records that the arguments gather
 template <typename F>
 static void md_gather_dispatch(const CellsArgs &o, const F &go) {
-    if (!o.sPos) go(std::integral_constant<int, 0>{});
+    if (o.sVal) go(std::integral_constant<int, kGatherVal>{});
+    else if (!o.sPos) go(std::integral_constant<int, 0>{});
     else if (o.sVel && o.sTan) go(std::integral_constant<int, kGatherPos | kGatherVel | kGatherTan>{});
     else if (o.sVel) go(std::integral_constant<int, kGatherPos | kGatherVel>{});
     else if (o.sTan) go(std::integral_constant<int, kGatherPos | kGatherTan>{});
@@ -1353,15 +1377,19 @@ hipError_t launch_solvent_gather(const float4 *pos, const float4 *vel, const uin
     return hipGetLastError();
 }
 
-// keys[k] = cell of slot k, vals[k] = the value of the particle in slot k
-__global__ __launch_bounds__(kBlock) void k_sort_finish(uint32_t *__restrict__ keys, uint32_t *__restrict__ vals,
-                                                        const uint32_t *__restrict__ pos,
-                                                        const uint32_t *__restrict__ cell,
-                                                        const uint32_t *__restrict__ valsIn, uint32_t n) {
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    keys[k] = cell[k];
-    vals[k] = valsIn[pos[k]];
+static hipError_t launch_md_buckets(const CellsArgs &o, const BucketPlan &bp, hipStream_t st) {
+    const auto go = [&](auto g) {
+        constexpr int G = decltype(g)::value;
+        // the smaller stage where twice the average bucket fits it
+        if (uint64_t(bp.n) * 2u <= uint64_t(bp.buckets) * kMdSmallCap)
+            NW_LAUNCH((k_md_cells<G, int(kMdSmallCap) / kMdCellsPer, int(kMdSmallCap)>), dim3(bp.buckets),
+                      dim3(kMdSmallCap / kMdCellsPer), cells_layout(bp, false, kMdSmallCap).total, st, o, bp);
+        else
+            NW_LAUNCH((k_md_cells<G, int(kBucketCap) / kMdCellsPer, int(kBucketCap)>), dim3(bp.buckets),
+                      dim3(kBucketCap / kMdCellsPer), cells_layout(bp, false).total, st, o, bp);
+    };
+    md_gather_dispatch(o, go);
+    return hipGetLastError();
 }
 
 hipError_t bucket_sort_pairs(uint32_t *keys, uint32_t *vals, uint32_t n, uint32_t bound, BucketScratch &s,
@@ -1371,14 +1399,19 @@ hipError_t bucket_sort_pairs(uint32_t *keys, uint32_t *vals, uint32_t n, uint32_
     if (*bucket_plan_problem(bp)) return hipErrorNotSupported;
     hipError_t e;
     if ((e = ensure_bucket_scratch(s, bp)) != hipSuccess) return e;
-    if ((e = hipMemcpyAsync(s.aux, vals, size_t(n) * 4, hipMemcpyDeviceToDevice, st)) != hipSuccess) return e;
-    if ((e = launch_hash_tiles(keys, bp, s, st)) != hipSuccess) return e;
-    // sorted positions into s.hash (free here: the keys come from the caller)
-    if ((e = launch_md_cells(bp, s, s.hash, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, st)) != hipSuccess)
-        return e;
-    hipLaunchKernelGGL(k_sort_finish, dim3(grid_for(n)), dim3(kBlock), 0, st, keys, vals, s.hash, s.sortedCell, s.aux,
-                       n);
-    return hipGetLastError();
+    // level 1 copies the values; level 2 writes the keys and the values in
+    // order over the originals (a copy and a gather launched before and after:
+    // 30,000 particles 16.5 us and two launches more, against 11.0)
+    if ((e = launch_tiles(false, nullptr, keys, bp, s, KP{}, false, st, TileCopy{vals, s.aux})) != hipSuccess) return e;
+    CellsArgs o{};
+    o.pairs = s.pairs;
+    o.P = s.P;
+    o.ids = s.hash;  // free here: the keys come from the caller
+    o.off = s.off;
+    o.cellOf = keys;
+    o.val = s.aux;
+    o.sVal = vals;
+    return launch_md_buckets(o, bp, st);
 }
 
 hipError_t launch_md_cells(const BucketPlan &bp, BucketScratch &s, uint32_t *ids, const float4 *pos,
@@ -1397,18 +1430,7 @@ hipError_t launch_md_cells(const BucketPlan &bp, BucketScratch &s, uint32_t *ids
     o.sPos = sPos;
     o.sVel = sVel;
     o.sTan = sTan;
-    const auto go = [&](auto g) {
-        constexpr int G = decltype(g)::value;
-        // the smaller stage where twice the average bucket fits it
-        if (uint64_t(bp.n) * 2u <= uint64_t(bp.buckets) * kMdSmallCap)
-            NW_LAUNCH((k_md_cells<G, int(kMdSmallCap) / kMdCellsPer, int(kMdSmallCap)>), dim3(bp.buckets),
-                      dim3(kMdSmallCap / kMdCellsPer), cells_layout(bp, false, kMdSmallCap).total, st, o, bp);
-        else
-            NW_LAUNCH((k_md_cells<G, int(kBucketCap) / kMdCellsPer, int(kBucketCap)>), dim3(bp.buckets),
-                      dim3(kBucketCap / kMdCellsPer), cells_layout(bp, false).total, st, o, bp);
-    };
-    md_gather_dispatch(o, go);
-    return hipGetLastError();
+    return launch_md_buckets(o, bp, st);
 }
 
 // The network takes a cell whose ids fit it, the sums load half as many
