@@ -643,8 +643,13 @@ static bool fused_md(const KP &kp, float *pos, float *vel, float *force, float *
     NW_REQUIRE_R(!needTan || tangent != nullptr, false,
                  "nwFusedMdStep: tangent is NULL but the pair term reads tangents");
     if (N == 0) return true;
-    const BucketPlan bp = fused_plan(N, cells, false);
+    BucketPlan bp = fused_plan(N, cells, false);
     NW_REQUIRE_R(!*bucket_plan_problem(bp), false, "nwFusedMdStep: %s", bucket_plan_problem(bp));
+    RowsPlan rows;
+    const bool oneLaunch = rows_plan(N, kp, rows);
+    uint32_t frontBlock = 0;
+    // (the fixed scratch is carved for the sort's own tiles)
+    const bool frontTiles = !oneLaunch && !fixed && front_tiles_plan(numFilaments, n, bp, frontBlock);
     if (!fixed) NW_HIP_R(ensure_bucket_scratch(s.bucket, bp), false);
     BucketScratch base = fixed ? *fixed : s.bucket;
     BucketScratch sc = base;
@@ -665,7 +670,7 @@ static bool fused_md(const KP &kp, float *pos, float *vel, float *force, float *
     a.velIn = reinterpret_cast<const float4 *>(velIn);
     a.keepPos = keepPos;
     a.keepVel = keepVel;
-    a.hash = gridParticleHash ? gridParticleHash : base.hash;
+    a.hash = gridParticleHash || frontTiles ? gridParticleHash : base.hash;
     a.dt = deltaTime;
     a.W = numFilaments;
     a.seed = s.seed;
@@ -677,10 +682,10 @@ static bool fused_md(const KP &kp, float *pos, float *vel, float *force, float *
     if (langevin) s.offset += N;
     {
         TimedScope ts(fixed ? noTimer : "md_front", s.stream, true);
-        NW_HIP_R(launch_md_front(a, kp, s.stream), false);
+        if (frontTiles) NW_HIP_R(launch_md_front_tiles(a, kp, bp, frontBlock, base, s.stream), false);
+        else NW_HIP_R(launch_md_front(a, kp, s.stream), false);
     }
-    RowsPlan rows;
-    if (rows_plan(N, kp, rows)) {
+    if (oneLaunch) {
         // a small system: the cell order and the pair forces in one launch
         TimedScope ts(fixed ? noTimer : "md_collide", s.stream, true);
         NW_HIP_R(launch_rows(rows, a.hash, a.pos, swapForces ? a.forceOld : a.force, gridParticleIndex, sc.off,
@@ -688,7 +693,7 @@ static bool fused_md(const KP &kp, float *pos, float *vel, float *force, float *
         s.lastHashPtr = nullptr;
         return true;
     }
-    {
+    if (!frontTiles) {
         TimedScope ts(fixed ? noTimer : "md_tiles", s.stream, true);
         NW_HIP_R(launch_hash_tiles(a.hash, bp, base, s.stream), false);
     }

@@ -118,12 +118,6 @@ __host__ __device__ inline CellsLayout cells_layout(const BucketPlan &bp, bool s
 }
 
 
-// words of a staged level-1 tile's LDS before its pair stage: the bucket
-// counts (B1), the scan's wave sums, the tile's bucket range (2), aligned to 4
-__host__ __device__ constexpr uint32_t staged_stage_words(uint32_t B1, uint32_t TB) {
-    return (B1 + TB / 64 + 2 + 3) & ~3u;
-}
-
 // words that level 1 copies beside reading the keys (from NULL: none): the
 // values of a key-value sort, which level 2 writes in order over the originals
 struct TileCopy {

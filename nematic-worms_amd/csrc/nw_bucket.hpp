@@ -110,6 +110,12 @@ struct FrontLane {
 // integrate + reversal + Langevin + bonded + tangent + MD cell (a.tangent
 // NULL: no tangents stored)
 hipError_t launch_md_front(const MdFrontArgs &a, const KP &kp, hipStream_t st);
+// The front with the sort's first level in the same launch: bp gets the front's
+// tiles (a workgroup's worms), block its threads; false when the system keeps
+// the two launches.  a.hash may be NULL (the cells are not stored).
+bool front_tiles_plan(uint32_t W, uint32_t n, BucketPlan &bp, uint32_t &block);
+hipError_t launch_md_front_tiles(const MdFrontArgs &a, const KP &kp, const BucketPlan &bp, uint32_t block,
+                                 BucketScratch &s, hipStream_t st);
 // the tangents the front stores, from the positions (worms of 1..64 beads)
 hipError_t launch_filament_tangents(const float4 *pos, float4 *tangent, uint32_t W, const KP &kp, hipStream_t st);
 // level 1 over precomputed cells
@@ -334,6 +340,12 @@ __device__ __forceinline__ void block_excl_scan(uint32_t *a, uint32_t m, uint32_
     }
     if (threadIdx.x == T - 1) a[m] = wave_last_lane(ws);
     __syncthreads();
+}
+
+// words of a staged level-1 tile's LDS before its pair stage: the bucket
+// counts (B1), the scan's wave sums, the tile's bucket range (2), aligned to 4
+__host__ __device__ constexpr uint32_t staged_stage_words(uint32_t B1, uint32_t TB) {
+    return (B1 + TB / 64 + 2 + 3) & ~3u;
 }
 
 }  // namespace nw

@@ -149,6 +149,41 @@ __global__ __launch_bounds__(BLOCK) void k_md_front(MdFrontArgs a, KP kp) {
     }
 }
 
+// The front of a workgroup's worms and the sort's first level over them (their
+// beads are consecutive: one tile of its own size): the cells stay in
+// registers, and the tile's launch, a chain of loads and barriers of 5 us
+// however small the system, is its last four barriers here.
+template <int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_md_front_tiles(MdFrontArgs a, KP kp, BucketPlan bp,
+                                                          uint32_t *__restrict__ pairs, uint32_t *__restrict__ P) {
+    extern __shared__ __align__(16) uint32_t lh[];
+    const uint32_t B1 = bp.buckets + 1, i0 = blockIdx.x * bp.tileItems;
+    uint32_t *wsum = lh + B1, *stage = lh + staged_stage_words(B1, BLOCK);
+    for (uint32_t b = threadIdx.x; b < B1; b += BLOCK) lh[b] = 0u;
+    const WaveWorm m = wave_worm(kp.p.filamentSize, a.W);
+    const FrontLane o = md_front_lane(kp, m, a.posIn ? a.posIn : a.pos, a.velIn ? a.velIn : a.vel, a.force,
+                                      a.forceOld, a.dt, a.lgvStd, a.langevin, a.seed, a.offRev, a.offLgv,
+                                      a.tangent != nullptr);
+    uint32_t h = 0u, rk = 0u;
+    if (m.active) {
+        h = md_front_store(kp, m, o, a.pos, a.vel, a.force, a.forceOld, a.tangent, a.swapForces != 0);
+        if (a.hash) a.hash[m.bead] = h;
+        if (a.keepPos) a.keepPos[m.bead] = f4(o.r, o.pw);
+        if (a.keepVel) a.keepVel[m.bead] = f4(o.v, o.vw);
+        h = min(h, bp.cells - 1u);
+    }
+    __syncthreads();
+    if (m.active) rk = atomicAdd(&lh[h >> bp.shift], 1u);
+    __syncthreads();
+    block_excl_scan(lh, bp.buckets, wsum);
+    uint32_t *row = P + uint64_t(blockIdx.x) * B1;
+    for (uint32_t b = threadIdx.x; b < B1; b += BLOCK) row[b] = lh[b];
+    if (m.active) stage[lh[h >> bp.shift] + rk] = pack_pair(h & ((1u << bp.shift) - 1u), m.bead - i0);
+    __syncthreads();
+    const uint32_t cnt = min(bp.tileItems, bp.n - i0);
+    for (uint32_t k = threadIdx.x; k < cnt; k += BLOCK) pairs[i0 + k] = stage[k];
+}
+
 // The tangents of the worms' beads from their positions, as the front's
 // bonded_lane writes them (the same arithmetic on the same values: bit for
 // bit), for a caller whose fused steps skipped them.
@@ -718,6 +753,35 @@ hipError_t launch_md_front(const MdFrontArgs &a, const KP &kp, hipStream_t st) {
         case 1024: NW_LAUNCH(k_md_front<1024>, dim3(grid_for(threads, 1024)), dim3(1024), 0, st, a, kp); break;
         default: NW_LAUNCH(k_md_front<kBlock>, dim3(grid_for(threads)), dim3(kBlock), 0, st, a, kp); break;
     }
+    return hipGetLastError();
+}
+
+// Up to 4,096 wavefronts of worms, one round of the CUs by workgroups of up to
+// 1,024 threads, and 4,096 buckets.  A step with one launch / two: 10,000 beads
+// of the 3D soft spheres 19.6 / 23.4 us, 48,000 26.3 / 29.8, 96,000 38.8 / 42.7,
+// 125,000 49.2 / 51.9, 161,000 WCA beads (3,491 wavefronts) 27.0 / 29.5; 195,000
+// (4,239) 35.6 / 31.5, and with workgroups of 512 there 32.3.
+bool front_tiles_plan(uint32_t W, uint32_t n, BucketPlan &bp, uint32_t &block) {
+    const Tuning &t = tuning();
+    const uint32_t wpw = 64u / n, waves = (W + wpw - 1u) / wpw;
+    // a tile or a front workgroup asked for is a launch of its own
+    if (t.mdTileItems || t.frontBlock || waves > 4096u || bp.buckets > 4096u) return false;
+    BucketPlan q = bp;
+    block = waves > 2048u ? 1024u : 512u;
+    q.tileItems = block / 64u * wpw * n;
+    q.tiles = (bp.n + q.tileItems - 1u) / q.tileItems;
+    if (*bucket_plan_problem(q)) return false;
+    bp = q;
+    return true;
+}
+
+hipError_t launch_md_front_tiles(const MdFrontArgs &a, const KP &kp, const BucketPlan &bp, uint32_t block,
+                                 BucketScratch &s, hipStream_t st) {
+    const size_t lds = size_t(staged_stage_words(bp.buckets + 1u, block) + bp.tileItems) * sizeof(uint32_t);
+    if (block == 1024u)
+        NW_LAUNCH(k_md_front_tiles<1024>, dim3(bp.tiles), dim3(1024), lds, st, a, kp, bp, s.pairs, s.P);
+    else
+        NW_LAUNCH(k_md_front_tiles<512>, dim3(bp.tiles), dim3(512), lds, st, a, kp, bp, s.pairs, s.P);
     return hipGetLastError();
 }
 

@@ -344,9 +344,9 @@ __global__ __launch_bounds__(kRowsBlock) void k_rows_batch(BatchArrays a, const 
 // ---------------------------------------------------------------------------
 // Every workgroup reads every bead's cell, so the launch wins while that read
 // is short.  A whole step with the sort and the pair kernel / with this launch:
-// 25.7 / 12.4 us at 6,400 beads, 26.5 / 15.4 at 32,000, 27.1 / 20.7 at 64,000,
-// 28.3 / 25.4 at 96,000, 28.7 / 27.5 at 112,000, 29.0 / 29.8 at 128,000.
-constexpr uint64_t kRowsMaxBeads = 114688;
+// 21.1 / 12.0 us at 6,400 beads, 21.5 / 15.1 at 32,000, 22.0 / 20.8 at 64,000,
+// 21.3 / 22.3 at 69,000, 22.5 / 23.4 at 80,000, 23.4 / 27.5 at 112,000.
+constexpr uint64_t kRowsMaxBeads = 65536;
 constexpr uint32_t kRowsMaxBlocks = 256;  // one round of the CUs: 64,000 beads over 291 rows take 23.0 us by single rows, 16.0 by pairs
 constexpr uint32_t kRowsMaxOwn = 768;     // beads of a workgroup on average: three rounds of its quads
 

@@ -207,7 +207,8 @@ extern "C" int nwAutotuneFused(float *pos, float *vel, float *force, float *forc
             t.frontBlock = fb;
             c.push_back(t);
         }
-        search(c, {"md_front"}, false);
+        // with the sort's first level, which a small system's built-in front does itself
+        search(c, {"md_front", "md_tiles", "md_sort"}, false);
     }
     {
         std::vector<NWTuning> c;
@@ -220,7 +221,7 @@ extern "C" int nwAutotuneFused(float *pos, float *vel, float *force, float *forc
                 if (nwGetLastError() == 0 && plan_is(N, C, n, items)) c.push_back(t);
             }
         nwSetTuning(&best);
-        search(c, {"md_tiles", "md_sort"}, false);
+        search(c, {"md_front", "md_tiles", "md_sort"}, false);
     }
     {
         // the pair workgroup and its stage (0: pairBlock + 128 per row)
