@@ -670,6 +670,7 @@ static bool fused_md(const KP &kp, float *pos, float *vel, float *force, float *
     a.velIn = reinterpret_cast<const float4 *>(velIn);
     a.keepPos = keepPos;
     a.keepVel = keepVel;
+    a.wormRows = oneLaunch ? base.pairs : nullptr;  // the sort's, which is not launched
     a.hash = gridParticleHash || frontTiles ? gridParticleHash : base.hash;
     a.dt = deltaTime;
     a.W = numFilaments;
@@ -688,7 +689,7 @@ static bool fused_md(const KP &kp, float *pos, float *vel, float *force, float *
     if (oneLaunch) {
         // a small system: the cell order and the pair forces in one launch
         TimedScope ts(fixed ? noTimer : "md_collide", s.stream, true);
-        NW_HIP_R(launch_rows(rows, a.hash, a.pos, swapForces ? a.forceOld : a.force, gridParticleIndex, sc.off,
+        NW_HIP_R(launch_rows(rows, a.hash, a.wormRows, a.pos, swapForces ? a.forceOld : a.force, gridParticleIndex, sc.off,
                              sc.sortedCell, reinterpret_cast<float4 *>(sortedPos), uint32_t(N), kp, s.stream), false);
         s.lastHashPtr = nullptr;
         return true;
@@ -1136,6 +1137,7 @@ void nwBatchMdStep(float *pos, float *vel, float *force, float *forceOld, float 
     a.tangent = reinterpret_cast<float4 *>(tangent);
     a.swapForces = b.swap ? 1 : 0;
     a.hash = b.scratch.hash;
+    a.wormRows = b.rows.blocks ? b.scratch.pairs : nullptr;  // the sort's, which is not launched
     a.ids = gridParticleIndex;
     a.off = b.scratch.off;
     a.sCell = b.scratch.sortedCell;
@@ -1696,6 +1698,7 @@ void nwBatchAdjointForward(float *pos, float *vel, float *force, float *forceOld
     a.force = reinterpret_cast<float4 *>(force);
     a.forceOld = reinterpret_cast<float4 *>(forceOld);
     a.hash = A.hash;
+    a.wormRows = b.rows.blocks ? b.scratch.pairs : nullptr;
     a.sCell = A.sCell;
     // the step velocities are read only for the Langevin partials
     const bool lgv = batch_langevin(b);
@@ -1790,6 +1793,7 @@ void nwBatchAdjointBackward(const float *dLdPos, const float *dLdVel, double *gr
             a.force = F;
             a.forceOld = G;
             a.hash = A.hash;
+            a.wormRows = b.rows.blocks ? b.scratch.pairs : nullptr;
             a.ids = A.segIds + uint64_t(j) * N;
             a.off = A.segOff + uint64_t(j) * (C + 2);
             a.sCell = A.sCell;

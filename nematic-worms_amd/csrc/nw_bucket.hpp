@@ -90,6 +90,7 @@ struct MdFrontArgs {
     float4 *pos, *vel, *force, *forceOld, *tangent;
     const float4 *posIn, *velIn;  // the step's input state when not pos / vel (NULL: in place)
     float4 *keepPos, *keepVel;    // the new state once more (NULL: not)
+    uint32_t *wormRows;           // out: every worm's rows of cells (worm_rows_word; NULL: not)
     uint32_t *hash;               // out: the cell of every bead
     float dt, lgvStd;
     int langevin;
@@ -113,6 +114,7 @@ hipError_t launch_md_front(const MdFrontArgs &a, const KP &kp, hipStream_t st);
 // The front with the sort's first level in the same launch: bp gets the front's
 // tiles (a workgroup's worms), block its threads; false when the system keeps
 // the two launches.  a.hash may be NULL (the cells are not stored).
+constexpr uint32_t kFrontTilesWaves = 4096;
 bool front_tiles_plan(uint32_t W, uint32_t n, BucketPlan &bp, uint32_t &block);
 hipError_t launch_md_front_tiles(const MdFrontArgs &a, const KP &kp, const BucketPlan &bp, uint32_t block,
                                  BucketScratch &s, hipStream_t st);
@@ -167,7 +169,7 @@ struct RowsPlan {
 };
 // whether the launch takes this system, and its shape
 bool rows_plan(uint64_t N, const KP &kp, RowsPlan &out);
-hipError_t launch_rows(const RowsPlan &pl, const uint32_t *hash, const float4 *pos, float4 *force, uint32_t *ids,
+hipError_t launch_rows(const RowsPlan &pl, const uint32_t *hash, const uint32_t *wormRows, const float4 *pos, float4 *force, uint32_t *ids,
                        uint32_t *off, uint32_t *sCell, float4 *sPos, uint32_t N, const KP &kp, hipStream_t st);
 // LDS beyond 64 KiB, granted per kernel once
 hipError_t grant_lds(const void *fn, size_t lds);
@@ -278,6 +280,7 @@ hipError_t launch_srd_rotate_batch(const uint32_t *hash, const float4 *com, floa
 struct BatchArrays {
     float4 *pos, *vel, *force, *forceOld, *tangent;
     float4 *keepPos, *keepVel;  // the new state once more (NULL: not)
+    uint32_t *wormRows;         // every worm's rows of cells, from its replica's first bead on (NULL: not)
     // nonzero: the new force goes to forceOld's buffer (pairs add there too)
     // and force's buffer is left as the old force (no replica reverses)
     int swapForces;

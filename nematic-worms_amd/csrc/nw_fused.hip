@@ -142,10 +142,16 @@ __global__ __launch_bounds__(BLOCK) void k_md_front(MdFrontArgs a, KP kp) {
     const FrontLane o = md_front_lane(kp, m, a.posIn ? a.posIn : a.pos, a.velIn ? a.velIn : a.vel, a.force,
                                       a.forceOld, a.dt, a.lgvStd, a.langevin, a.seed, a.offRev, a.offLgv,
                                       a.tangent != nullptr);
+    uint32_t h = 0u;
     if (m.active) {
-        a.hash[m.bead] = md_front_store(kp, m, o, a.pos, a.vel, a.force, a.forceOld, a.tangent, a.swapForces != 0);
+        h = md_front_store(kp, m, o, a.pos, a.vel, a.force, a.forceOld, a.tangent, a.swapForces != 0);
+        a.hash[m.bead] = h;
         if (a.keepPos) a.keepPos[m.bead] = f4(o.r, o.pw);
         if (a.keepVel) a.keepVel[m.bead] = f4(o.v, o.vw);
+    }
+    if (a.wormRows) {
+        const uint32_t w = worm_rows_word(div_exact(h, kp.gxMagic, kp.p.gridSize.x), m.pp, kp.p.filamentSize);
+        if (m.active && m.pp == 0u) a.wormRows[m.worm] = w;
     }
 }
 
@@ -712,12 +718,17 @@ __global__ __launch_bounds__(kBlock) void k_md_front_batch(BatchArrays a, const 
     float4 *force = a.force + rep.beadOffset, *forceOld = a.forceOld + rep.beadOffset;
     const FrontLane o = md_front_lane(kp, m, pos, vel, force, forceOld, dt, rep.lgvStd, rep.langevin, rep.seed,
                                       offRev, offLgv, a.tangent != nullptr);
+    uint32_t h = 0u;
     if (m.active) {
-        const uint32_t h = md_front_store(kp, m, o, pos, vel, force, forceOld,
-                                          a.tangent ? a.tangent + rep.beadOffset : nullptr, a.swapForces != 0);
+        h = md_front_store(kp, m, o, pos, vel, force, forceOld, a.tangent ? a.tangent + rep.beadOffset : nullptr,
+                           a.swapForces != 0);
         a.hash[rep.beadOffset + m.bead] = rep.cellOffset + h;
         if (a.keepPos) a.keepPos[rep.beadOffset + m.bead] = f4(o.r, o.pw);
         if (a.keepVel) a.keepVel[rep.beadOffset + m.bead] = f4(o.v, o.vw);
+    }
+    if (a.wormRows) {
+        const uint32_t w = worm_rows_word(div_exact(h, kp.gxMagic, kp.p.gridSize.x), m.pp, kp.p.filamentSize);
+        if (m.active && m.pp == 0u) a.wormRows[rep.beadOffset + m.worm] = w;
     }
 }
 
@@ -765,7 +776,7 @@ bool front_tiles_plan(uint32_t W, uint32_t n, BucketPlan &bp, uint32_t &block) {
     const Tuning &t = tuning();
     const uint32_t wpw = 64u / n, waves = (W + wpw - 1u) / wpw;
     // a tile or a front workgroup asked for is a launch of its own
-    if (t.mdTileItems || t.frontBlock || waves > 4096u || bp.buckets > 4096u) return false;
+    if (t.mdTileItems || t.frontBlock || waves > kFrontTilesWaves || bp.buckets > 4096u) return false;
     BucketPlan q = bp;
     block = waves > 2048u ? 1024u : 512u;
     q.tileItems = block / 64u * wpw * n;

@@ -127,6 +127,20 @@ __device__ __forceinline__ f3 shfl_up3(f3 a, int d) {
     return mk(__shfl_up(a.x, d, 64), __shfl_up(a.y, d, 64), __shfl_up(a.z, d, 64));
 }
 
+// The least and the greatest of y (below 2^16) over the lanes of a worm of n
+// beads, as (2^16 - 1 - least) << 16 | greatest, in its first lane (pp the
+// lane's bead in the worm)
+__device__ __forceinline__ uint32_t worm_rows_word(uint32_t y, uint32_t pp, uint32_t n) {
+    typedef uint16_t w2 __attribute__((ext_vector_type(2)));
+    uint32_t w = (0xffffu - y) << 16 | y;
+    for (uint32_t d = 1; d < n; d <<= 1) {
+        const uint32_t x = __shfl_down(w, d, 64);
+        if (pp + d < n)
+            w = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(w2, w), __builtin_bit_cast(w2, x)));
+    }
+    return w;
+}
+
 // x of lane I of this lane's quad
 template <int I>
 __device__ __forceinline__ float quad_lane(float x) {

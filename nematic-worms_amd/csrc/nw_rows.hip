@@ -4,15 +4,16 @@
 // The two-level cell sort and the pair pass are three launches, each a chain
 // of dependent phases on a mostly idle chip when the system has some ten
 // thousand beads: 5.9 + 8.7 + 12.2 us at 32,000 beads.  Here a workgroup owns
-// `rows` consecutive rows of a one-layer grid.  It reads the cell of every bead
-// (a few hundred KB, from L2), keeps the beads of its rows and of the row on
-// either side -- one interval of cells modulo the grid, so the wrap in y needs
+// `rows` consecutive rows of a one-layer grid.  It reads the rows of cells that
+// every worm spans (one word a worm, left by the front), lists the worms that
+// may have a bead in its rows or in the row on either side and keeps those
+// beads -- one interval of cells modulo the grid, so the wrap in y needs
 // no case of its own and whole rows hold the wrap in x -- orders them in LDS
 // by (cell, id), counts the beads of the rows before its own (its first sorted
 // slot), writes its part of the order and evaluates its beads' pairs from LDS.
-// Nothing passes between workgroups.  At 32,000 beads the launch takes 10.9 us:
-// 4.3 the read of the cells (issue: some four VALU a cell in 16 wavefronts),
-// 2.9 the order, 1.7 the pairs, the rest the dispatch.
+// Nothing passes between workgroups.  At 32,000 beads the launch takes 8.5 us
+// (11.7 reading every bead's cell): 1.3 the worms, 2 the order, 1.5 the pairs,
+// the rest the dispatch and barriers.
 //
 // The pairs: four lanes a bead, lane q evaluating candidates q, q + 4, ... of
 // the flattened list, their terms added in list order by quad broadcasts: the
@@ -24,12 +25,13 @@
 
 namespace nw {
 
-// threads of a workgroup: 1024 read the cells of 32,000 beads in 3.4 us, 512 in
-// 5.6, 256 in 10.5 (kernel 10.9 / 14.1 / 21.8 us; at 4,000 beads 6.6 / 6.8 / 7.5)
+// threads of a workgroup: 1024 against 512 and 256, 32,000 beads 10.9 / 14.1 / 21.8
+// us and 4,000 6.6 / 6.8 / 7.5 (as measured with every bead's cell read)
 constexpr int kRowsBlock = 1024;
 
 struct RowsArgs {
-    const uint32_t *hash;  // cell of every bead, bead order
+    const uint32_t *hash;   // cell of every bead, bead order
+    const uint32_t *worms;  // rows of every worm (worm_rows_word)
     const float4 *pos;
     float4 *force;
     uint32_t *ids, *off, *sCell;
@@ -43,7 +45,7 @@ struct RowsLayout {
 __host__ __device__ inline RowsLayout rows_layout(uint32_t cap, uint32_t cells) {
     RowsLayout L;
     uint32_t o = 0;
-    L.pos = o;   o += 16u * cap;  // while the beads are collected: their groups of four
+    L.pos = o;   o += 16u * cap;  // while the beads are collected: their worms
     L.lid = o;   o += 4u * cap;
     L.lcell = o; o += 2u * cap;
     o = (o + 15u) & ~15u;
@@ -129,12 +131,12 @@ __device__ __forceinline__ void rows_body(const KP &kp, const RowsArgs &a, uint3
                                           uint32_t cap, uint32_t maxCells, unsigned char *smem) {
     const RowsLayout L = rows_layout(cap, maxCells);
     float4 *lpos = reinterpret_cast<float4 *>(smem + L.pos);
-    uint32_t *group = reinterpret_cast<uint32_t *>(smem + L.pos);  // until the positions come: 4 cap words
+    uint32_t *list = reinterpret_cast<uint32_t *>(smem + L.pos);  // until the positions come: 4 cap words
     uint32_t *lid = reinterpret_cast<uint32_t *>(smem + L.lid);
     uint16_t *lcell = reinterpret_cast<uint16_t *>(smem + L.lcell);
     uint32_t *cnt = reinterpret_cast<uint32_t *>(smem + L.cnt);
     uint32_t *cur = reinterpret_cast<uint32_t *>(smem + L.cur);
-    uint32_t *wsum = reinterpret_cast<uint32_t *>(smem + L.wsum);  // 16 scan sums, 16 counts below, groups
+    uint32_t *wsum = reinterpret_cast<uint32_t *>(smem + L.wsum);  // 16 scan sums, 16 counts below, worms
 
     const uint32_t Gx = kp.p.gridSize.x, Gy = kp.p.gridSize.y, C = Gx * Gy;
     const uint32_t own = min(rows, Gy - y0);
@@ -145,91 +147,76 @@ __device__ __forceinline__ void rows_body(const KP &kp, const RowsArgs &a, uint3
     if (t == 0) wsum[32] = 0u;
     __syncthreads();
 
-    // Every bead's cell: below the own rows (counted) and, in groups of four
-    // words, whether one lies in the staged rows (its local cell is the
-    // distance from the first staged cell).  16-byte loads from the first
-    // aligned word, eight a thread in flight; a wavefront lists its groups
-    // with a staged bead by one append.  The words before the first whole
-    // group are group `quads`, those after the last one quads + 1.
-    // the staged cells: nA from hLo on and, past the grid's end, the first nB
+    // Every worm's rows, which the front left: a worm wholly below the own rows
+    // has all its beads counted there, one that may have a bead in the staged
+    // rows is listed (a wavefront's by one append), any other is passed over.
+    // The own rows' first row lies between two staged ones, or is the grid's
+    // first with no row below: a worm on both sides of it is listed.
+    const uint32_t n = kp.p.filamentSize, W = div_exact(N, kp.fdivMagic, n);
+    const uint32_t yLo = y0 == 0u ? Gy - 1u : y0 - 1u;
+    const uint32_t rA = min(own + 2u, Gy - yLo), rB = own + 2u - rA;  // staged: rA rows from yLo on, the first rB
+    uint32_t below = 0;
+    auto look = [&](uint32_t w, uint32_t x) {
+        const uint32_t lo = 0xffffu - (x >> 16), hi = x & 0xffffu;
+        const bool hit = w < W && ((hi >= yLo && lo < yLo + rA) || lo < rB);
+        below += w < W && !hit && hi < y0 ? n : 0u;
+        const uint64_t hits = __ballot(hit);
+        if (hits) {
+            uint32_t at = 0;
+            if ((t & 63u) == 0u) at = atomicAdd(&wsum[32], uint32_t(__popcll(hits)));
+            at = __builtin_amdgcn_readfirstlane(at) +
+                 __builtin_amdgcn_mbcnt_hi(uint32_t(hits >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(hits), 0u));
+            if (hit && at < 4u * cap) list[at] = w;
+        }
+    };
+    constexpr uint32_t U = 8;  // a thread's worms in flight together
+    for (uint32_t w0 = 0; w0 < W; w0 += U * T) {
+        uint32_t x[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u)
+            if (w0 + u * T < W) x[u] = a.worms[min(w0 + u * T + t, W - 1u)];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u)
+            if (w0 + u * T < W) look(w0 + u * T + t, x[u]);
+    }
+    __syncthreads();
+    // the cells of the listed worms' beads (of every bead when the list is too
+    // short), the first kWords a thread held from here to the placement
     const uint32_t nA = min(nc, C - hLo), nB = nc - nA;
-    auto local = [&](uint32_t h) {
+    auto local = [&](uint32_t h) {  // the distance from the first staged cell
         const uint32_t d = h - hLo;
         return d < nA ? d : (h < nB ? nA + h : ~0u);
     };
-    const uint32_t head = min((4u - (uint32_t(reinterpret_cast<uintptr_t>(a.hash)) >> 2 & 3u)) & 3u, N);
-    const uint32_t quads = (N - head) / 4u, rest = head + 4u * quads;
-    const uint4 *h4 = reinterpret_cast<const uint4 *>(a.hash + head);
-    uint32_t below = 0;
-    // one group: whether it holds a staged bead
-    auto look = [&](const uint4 &x) {
-        const uint32_t h0 = x.x - cellBase, h1 = x.y - cellBase, h2 = x.z - cellBase, h3 = x.w - cellBase;
-        below += h0 < hOwn ? 1u : 0u;
-        below += h1 < hOwn ? 1u : 0u;
-        below += h2 < hOwn ? 1u : 0u;
-        below += h3 < hOwn ? 1u : 0u;
-        const uint32_t d = min(min(h0 - hLo, h1 - hLo), min(h2 - hLo, h3 - hLo));
-        return d < nA || min(min(h0, h1), min(h2, h3)) < nB;
+    const bool listed = wsum[32] <= 4u * cap;
+    const uint32_t words = listed ? wsum[32] * n : N;
+    auto bead_of = [&](uint32_t k) {
+        uint32_t w, q;
+        worm_of(kp, k, w, q);
+        return listed ? list[w] * n + q : k;
     };
-    // (the whole wavefront) lists the groups q + T b of the bits b of hit
-    auto list = [&](uint32_t hit, uint32_t q) {
-        if (!__any(hit != 0u)) return;
-        const uint32_t n = uint32_t(__popc(hit)), incl = wave_scan_add(n);
-        uint32_t at = 0;
-        if ((t & 63u) == 63u) at = atomicAdd(&wsum[32], incl);
-        at = wave_last_lane(at) + incl - n;
-        for (; hit; hit &= hit - 1u, ++at)
-            if (at < 4u * cap) group[at] = q + uint32_t(__builtin_ctz(hit)) * T;
+    if (!listed) below = 0u;
+    constexpr uint32_t kWords = 4;
+    uint32_t idk[kWords], hk[kWords];
+#pragma unroll
+    for (uint32_t j = 0; j < kWords; ++j) {
+        const uint32_t k = t + j * T;
+        idk[j] = k < words ? bead_of(k) : N;
+        hk[j] = idk[j] < N ? a.hash[idk[j]] - cellBase : ~0u;
+    }
+    auto count = [&](uint32_t h, bool on) {
+        below += on && h < hOwn ? 1u : 0u;
+        const uint32_t d = on ? local(h) : ~0u;
+        if (d < nc) atomicAdd(&cnt[d], 1u);
+        return d;
     };
-    constexpr uint32_t U = 8;
-    const uint32_t whole = quads / T;  // rounds in which every thread has a group
-    for (uint32_t r = 0; r < whole; r += U) {
-        uint4 x[U];
 #pragma unroll
-        for (uint32_t u = 0; u < U; ++u)
-            if (r + u < whole) x[u] = h4[(r + u) * T + t];
-        uint32_t hit = 0;
-#pragma unroll
-        for (uint32_t u = 0; u < U; ++u)
-            if (r + u < whole) hit |= look(x[u]) ? 1u << u : 0u;
-        list(hit, r * T + t);
-    }
-    if (whole * T < quads) {
-        const uint32_t q = whole * T + t;
-        uint32_t hit = 0;
-        if (q < quads) hit = look(h4[q]) ? 1u : 0u;
-        list(hit, q);
-    }
-    if (t < head + (N - rest)) {
-        below += a.hash[t < head ? t : rest + (t - head)] - cellBase < hOwn ? 1u : 0u;
-        if (t == 0) {
-            const uint32_t at = atomicAdd(&wsum[32], 2u);
-            if (at < 4u * cap) group[at] = quads;
-            if (at + 1u < 4u * cap) group[at + 1u] = quads + 1u;
-        }
-    }
+    for (uint32_t j = 0; j < kWords; ++j) hk[j] = count(hk[j], idk[j] < N);
+    for (uint32_t k = t + kWords * T; k < words; k += T) (void)count(a.hash[bead_of(k)] - cellBase, true);
     below = wave_scan_add(below);
     if ((t & 63u) == 63u) wsum[16u + (t >> 6)] = below;
     __syncthreads();
-    const uint32_t slotBase = slotAdd + wave_last_lane(wave_scan_add((t & 63u) < uint32_t(T / 64) ? wsum[16u + (t & 63u)] : 0u));
-    const uint32_t words = 4u * wsum[32];
-    // word k of the listed groups: its bead, or N (group quads: the words
-    // before the first whole group, quads + 1: those after the last)
-    auto bead_of = [&](uint32_t k) {
-        const uint32_t g = group[k >> 2], i = k & 3u;
-        if (g < quads) return head + 4u * g + i;
-        return g == quads ? (i < head ? i : N) : min(rest + i, N);
-    };
-    const bool listed = words <= 16u * cap;
-    uint32_t id0 = N, d0 = ~0u;  // the thread's first word
-    for (uint32_t k = t; k < (listed ? words : N); k += T) {
-        const uint32_t id = listed ? bead_of(k) : k;
-        const uint32_t d = id < N ? local(a.hash[id] - cellBase) : ~0u;
-        if (d < nc) atomicAdd(&cnt[d], 1u);
-        if (k == t) id0 = id, d0 = d;
-    }
-    __syncthreads();
     block_excl_scan<true>(cnt, nc, wsum, cur);
+    const uint32_t slotBase = slotAdd + wave_last_lane(wave_scan_add((t & 63u) < uint32_t(T / 64) ? wsum[16u + (t & 63u)] : 0u));
     const uint32_t m = cnt[nc];  // staged beads
     const uint32_t s0 = cnt[Gx], s1 = cnt[(own + 1u) * Gx];  // the own beads' staged slots
     // CSR offsets of the own cells
@@ -239,14 +226,18 @@ __device__ __forceinline__ void rows_body(const KP &kp, const RowsArgs &a, uint3
         rows_unstaged(kp, a, N, idBase, cellBase, slotBase - slotAdd, y0, own, cnt);
         return;
     }
-    for (uint32_t k = t; k < words; k += T) {
-        const uint32_t id = k == t ? id0 : bead_of(k);
-        const uint32_t d = k == t ? d0 : (id < N ? local(a.hash[id] - cellBase) : ~0u);
+    auto place = [&](uint32_t id, uint32_t d) {
         if (d < nc) {
             const uint32_t s = atomicAdd(&cur[d], 1u);
             lid[s] = id;
             lcell[s] = uint16_t(d);
         }
+    };
+#pragma unroll
+    for (uint32_t j = 0; j < kWords; ++j) place(idk[j], hk[j]);
+    for (uint32_t k = t + kWords * T; k < words; k += T) {
+        const uint32_t id = bead_of(k);
+        place(id, local(a.hash[id] - cellBase));
     }
     __syncthreads();
     // a cell's beads in ascending id (MD cells hold about one)
@@ -333,7 +324,7 @@ __global__ __launch_bounds__(kRowsBlock) void k_rows_batch(BatchArrays a, const 
     const uint32_t b = xcd_contiguous(blockIdx.x, gridDim.x);
     const BatchRep &rep = reps[__builtin_amdgcn_readfirstlane(replica_of_row_block(reps, R, b))];
     const uint32_t b0 = rep.beadOffset, c0 = rep.cellOffset;
-    const RowsArgs x{a.hash + b0,    a.pos + b0, (a.swapForces ? a.forceOld : a.force) + b0, a.ids + b0,
+    const RowsArgs x{a.hash + b0, a.wormRows + b0, a.pos + b0, (a.swapForces ? a.forceOld : a.force) + b0, a.ids + b0,
                      a.off + c0,     a.sCell + b0, a.sPos + b0};
     rows_body<kRowsBlock>(rep.kp, x, rep.numBeads, b0, c0, b0, (b - rep.rowBlock) * rep.rows, rep.rows, cap, maxCells,
                           smem);
@@ -342,19 +333,25 @@ __global__ __launch_bounds__(kRowsBlock) void k_rows_batch(BatchArrays a, const 
 // ---------------------------------------------------------------------------
 // plan and launcher
 // ---------------------------------------------------------------------------
-// Every workgroup reads every bead's cell, so the launch wins while that read
-// is short.  A whole step with the sort and the pair kernel / with this launch:
-// 21.1 / 12.0 us at 6,400 beads, 21.5 / 15.1 at 32,000, 22.0 / 20.8 at 64,000,
-// 21.3 / 22.3 at 69,000, 22.5 / 23.4 at 80,000, 23.4 / 27.5 at 112,000.
-constexpr uint64_t kRowsMaxBeads = 65536;
+// A step with the sort and the pair kernel / with this launch, worms of 16: 21.5
+// / 13.0 us at 32,000 beads, 22.1 / 16.0 at 64,000, 25.0 / 19.9 at 128,000, 27.7
+// / 24.2 at 192,000, 28.5 / 29.2 at 224,000; where the front and the sort's first
+// level are two launches (front_tiles_plan: more than 4,096 wavefronts), worms
+// of 23: 33.3 / 28.8 at 195,000 and 34.5 / 30.5 at 229,000.
+constexpr uint64_t kRowsMaxBeads = 204800, kRowsMaxBeadsTwo = 240000;
+// every workgroup reads every worm's rows: 22.8 / 20.4 us with 20,000 worms of
+// three, 23.1 / 24.8 with 30,000; of five 22.7 / 19.6 with 15,000, 26.9 / 28.1
+// with 30,000
+constexpr uint64_t kRowsMaxWorms = 24576;
 constexpr uint32_t kRowsMaxBlocks = 256;  // one round of the CUs: 64,000 beads over 291 rows take 23.0 us by single rows, 16.0 by pairs
-constexpr uint32_t kRowsMaxOwn = 768;     // beads of a workgroup on average: three rounds of its quads
+constexpr uint32_t kRowsMaxOwn = 1280;    // beads of a workgroup on average: five rounds of its quads
 
 // whether the launch computes a system's pair term at all
 static bool rows_term(const KP &kp) {
     const SimParams &p = kp.p;
     return kp.e.pairPotential == NW_PAIR_WCA && p.activity == 0.0f && kp.e.stencil == NW_STENCIL_2D &&
-           kp.e.collideKernel == NW_COLLIDE_AUTO && p.gridSize.z == 1 && p.gridSize.x >= 3 && p.gridSize.y >= 3;
+           kp.e.collideKernel == NW_COLLIDE_AUTO && p.gridSize.z == 1 && p.gridSize.x >= 3 && p.gridSize.y >= 3 &&
+           p.gridSize.y < 65536u;  // a row in 16 bits
 }
 
 // beads staged by a workgroup of `rows` rows: two and a half times the
@@ -374,7 +371,8 @@ bool rows_plan(uint64_t N, const KP &kp, RowsPlan &out) {
     if (!rows_term(kp)) return false;
     // a launch shape asked of the sort or the pair kernel is theirs
     if (t.mdTileItems || t.mdMembers || t.pairBlock || t.pairStage) return false;
-    if (N == 0 || N > kRowsMaxBeads) return false;
+    const uint32_t n = kp.p.filamentSize, waves = uint32_t((N / n + 64u / n - 1u) / (64u / n));
+    if (N == 0 || N / n > kRowsMaxWorms || N > (waves > kFrontTilesWaves ? kRowsMaxBeadsTwo : kRowsMaxBeads)) return false;
     out.rows = std::min((Gy + kRowsMaxBlocks - 1u) / kRowsMaxBlocks, Gy - 2u);
     out.blocks = (Gy + out.rows - 1u) / out.rows;
     if (double(N) / Gy * out.rows > double(kRowsMaxOwn)) return false;
@@ -383,14 +381,13 @@ bool rows_plan(uint64_t N, const KP &kp, RowsPlan &out) {
     return rows_fits(out);
 }
 
-// The batch takes the launch when its workgroups are done sooner than the sort
-// and the pair kernel.  Measured with one size of replica throughout (us a
-// step, sort + pairs / this launch): 16 x 1,100 beads 30.4 / 17.0, 16 x 8,600
-// 35.5 / 24.4, 64 x 7,700 52.6 / 47.5, 64 x 4,100 43.8 / 34.2, 128 x 4,000 54.3
-// / 46.4, 256 x 2,000 56.4 / 49.1, 16 x 30,000 52.3 / 48.8; the launch alone
-// loses at 64 x 30,000 (95 us) and 16 x 60,000 (62).  The sort and the pairs
-// take some 19 us and 26 us a million beads, 256 workgroups here 8 us and 1 us
-// for every 10,000 beads of their replica.
+// The batch takes the launch up to 480,000 beads.  A step (us, sort + pairs / this
+// launch): 16 x 1,100 beads 27.8 / 13.5, 16 x 8,600 34.3 / 20.5, 32 x 8,100 40.2
+// / 33.1, 64 x 7,700 52.4 / 48.1, 16 x 29,700 49.7 / 48.3, 128 x 4,000 53.9 / 48.5,
+// 256 x 2,000 55.5 / 55.3; past it 96 x 8,000 63.6 / 69.0, 8 x 79,500 55.4 / 66.9.
+constexpr uint64_t kRowsMaxBatchBeads = 480000;
+constexpr double kRowsBatchOwn = 768.0, kRowsBatchOwnOne = 1024.0;  // beads of a workgroup on average
+
 bool rows_plan_batch(BatchRep *reps, uint32_t R, RowsPlan &out) {
     out = RowsPlan{};
     uint64_t rows = 0;
@@ -400,22 +397,31 @@ bool rows_plan_batch(BatchRep *reps, uint32_t R, RowsPlan &out) {
     }
     RowsPlan pl{};
     const uint32_t per = uint32_t((rows + kRowsMaxBlocks - 1u) / kRowsMaxBlocks);
-    double here = 0.0, beads = 0.0;
+    // the rows of a workgroup of replica q with at most maxOwn beads on average
+    const auto rows_of = [&](const BatchRep &q, double maxOwn) {
+        const double perRow = std::max(1.0, double(q.numBeads) / q.kp.p.gridSize.y);
+        return std::max(1u, std::min({per, uint32_t(maxOwn / perRow), q.kp.p.gridSize.y - 2u}));
+    };
+    // a batch that one more round of quads fits into one round of the CUs
+    // takes it (16 x 12,000 beads by six rows, 288 workgroups, 21.6 us, by
+    // seven, 256, 14.8)
+    uint64_t one = 0;
+    for (uint32_t r = 0; r < R; ++r) one += (reps[r].kp.p.gridSize.y + rows_of(reps[r], kRowsBatchOwnOne) - 1u) / rows_of(reps[r], kRowsBatchOwnOne);
+    const double maxOwn = one <= kRowsMaxBlocks ? kRowsBatchOwnOne : kRowsBatchOwn;
+    uint64_t beads = 0;
     for (uint32_t r = 0; r < R; ++r) {
         BatchRep &q = reps[r];
         const uint32_t Gx = q.kp.p.gridSize.x, Gy = q.kp.p.gridSize.y;
-        const double perRow = std::max(1.0, double(q.numBeads) / Gy);
-        if (perRow > double(kRowsMaxOwn)) return false;
-        q.rows = std::max(1u, std::min({per, uint32_t(kRowsMaxOwn / perRow), Gy - 2u}));
+        if (double(q.numBeads) / Gy > kRowsBatchOwn || q.kp.p.numFilaments > kRowsMaxWorms) return false;
+        q.rows = rows_of(q, maxOwn);
         q.rowBlock = pl.blocks;
         const uint32_t blocks = (Gy + q.rows - 1u) / q.rows;
         pl.blocks += blocks;
         pl.cells = std::max(pl.cells, (q.rows + 2u) * Gx);
         pl.cap = std::max(pl.cap, rows_cap(q.numBeads, Gy, q.rows));
-        here += blocks * (8.0 + 1e-4 * q.numBeads) / kRowsMaxBlocks;
         beads += q.numBeads;
     }
-    if (!pl.blocks || here > 19.0 + 26e-6 * beads || !rows_fits(pl)) return false;
+    if (!pl.blocks || beads > kRowsMaxBatchBeads || !rows_fits(pl)) return false;
     out = pl;
     return true;
 }
@@ -428,9 +434,9 @@ hipError_t launch_rows_batch(const RowsPlan &pl, const BatchArrays &a, const Bat
     return hipGetLastError();
 }
 
-hipError_t launch_rows(const RowsPlan &pl, const uint32_t *hash, const float4 *pos, float4 *force, uint32_t *ids,
+hipError_t launch_rows(const RowsPlan &pl, const uint32_t *hash, const uint32_t *wormRows, const float4 *pos, float4 *force, uint32_t *ids,
                        uint32_t *off, uint32_t *sCell, float4 *sPos, uint32_t N, const KP &kp, hipStream_t st) {
-    const RowsArgs a{hash, pos, force, ids, off, sCell, sPos};
+    const RowsArgs a{hash, wormRows, pos, force, ids, off, sCell, sPos};
     const hipError_t e = grant_lds(reinterpret_cast<const void *>(&k_rows), pl.lds);
     if (e != hipSuccess) return e;
     NW_LAUNCH(k_rows, dim3(pl.blocks), dim3(kRowsBlock), pl.lds, st, a, N, pl.rows, pl.cap, pl.cells, kp);
