@@ -121,6 +121,72 @@ __device__ __forceinline__ void rows_unstaged(const KP &kp, const RowsArgs &a, u
     }
 }
 
+// own beads above which a bead takes one lane instead of four: 229,000 beads
+// (1,140 a workgroup) 19.1 -> 16.2 us, 192,000 (770) 16.5 -> 14.7, 16 replicas of
+// 8,600 (570) 12.9 -> 10.6; 64,000 (440) 11.6 -> 11.0
+constexpr uint32_t kRowsLaneBeads = 400;
+
+// The pair forces of the staged beads s0 .. s1, LANES (1 or 4) lanes a bead:
+// lane q evaluates candidates q, q + LANES, ... of the flattened list, the
+// terms added in list order either way.  Four lanes shorten a bead's chain,
+// one costs half the instructions a candidate.
+template <int T, int LANES>
+__device__ __forceinline__ void rows_pairs(const KP &kp, const RowsArgs &a, const uint32_t *lid, const float4 *lpos,
+                                           const uint16_t *lcell, const uint32_t *cnt, uint32_t s0, uint32_t s1) {
+    const uint32_t Gx = kp.p.gridSize.x, t = threadIdx.x, lane = t % LANES;
+    const float rc2 = kp.e.wcaCutoff * kp.e.wcaCutoff;
+    for (uint32_t s = s0 + t / LANES; s < s1; s += T / LANES) {
+        const uint32_t me = lid[s];
+        const float4 F = load4(a.force, me);
+        const float4 O = lpos[s];
+        const f3 r = mk(O);
+        const uint32_t fil = __float_as_uint(O.w), c = lcell[s];
+        const uint32_t ly = div_exact(c, kp.gxMagic, Gx), x = c - ly * Gx, row = (ly - 1u) * Gx;
+        uint32_t a0, a1, b0, b1;
+        row_pieces(x, Gx, a0, a1, b0, b1);
+        // pieces k of slots pre[k] .. pre[k + 1] of the list, at slot t + d[k]
+        uint32_t pre[7], d[6];
+        pre[0] = 0u;
+#pragma unroll
+        for (int y = 0; y < 3; ++y) {
+            const uint32_t R = row + uint32_t(y) * Gx;
+            const uint32_t p0 = cnt[R + a0], p1 = cnt[R + a1], q0 = cnt[R], q1 = cnt[R + b1];
+            d[2 * y] = p0 - pre[2 * y];
+            pre[2 * y + 1] = pre[2 * y] + (p1 - p0);
+            d[2 * y + 1] = q0 - pre[2 * y + 1];
+            pre[2 * y + 2] = pre[2 * y + 1] + (q1 - q0);
+        }
+        const uint32_t K = pre[6];
+        f3 acc = mk(0.f, 0.f, 0.f);
+        if (LANES == 1) {
+            // without an edge bead in the wavefront every second piece is empty
+            if (__any(b1 != 0u)) {
+                for (uint32_t i = 0; i < K; ++i) {
+                    uint32_t j = d[5];
+#pragma unroll
+                    for (int k = 4; k >= 0; --k) j = i < pre[k + 1] ? d[k] : j;
+                    acc += wca_term_masked(kp, r, fil, rc2, lpos[i + j]);
+                }
+            } else {
+                for (uint32_t i = 0; i < K; ++i) {
+                    const uint32_t j = i < pre[1] ? d[0] : (i < pre[3] ? d[2] : d[4]);
+                    acc += wca_term_masked(kp, r, fil, rc2, lpos[i + j]);
+                }
+            }
+        } else {
+            for (uint32_t i = lane; i - lane < K; i += 4u) {
+                uint32_t j = d[5];
+#pragma unroll
+                for (int k = 4; k >= 0; --k) j = i < pre[k + 1] ? d[k] : j;
+                const bool on = i < K;
+                // past the list: the bead itself, masked by its worm
+                add_quad(acc, wca_term_masked(kp, r, fil, rc2, lpos[on ? i + j : s]));
+            }
+        }
+        if (lane == 0u) a.force[me] = make_float4(F.x + acc.x, F.y + acc.y, F.z + acc.z, F.w + 0.0f);
+    }
+}
+
 // Rows [y0, y0 + rows) of one system: N beads whose arrays hash, pos, force
 // start at its first bead; ids, sCell and sPos (indexed by sorted slot) and
 // off (by cell) at its own first entries; bead ids, cells and slots of the
@@ -270,41 +336,8 @@ __device__ __forceinline__ void rows_body(const KP &kp, const RowsArgs &a, uint3
     }
     __syncthreads();
 
-    const float rc2 = kp.e.wcaCutoff * kp.e.wcaCutoff;
-    const uint32_t lane = t & 3u;
-    for (uint32_t s = s0 + t / 4u; s < s1; s += T / 4u) {
-        const uint32_t me = lid[s];
-        const float4 F = load4(a.force, me);
-        const float4 O = lpos[s];
-        const f3 r = mk(O);
-        const uint32_t fil = __float_as_uint(O.w), c = lcell[s];
-        const uint32_t ly = div_exact(c, kp.gxMagic, Gx), x = c - ly * Gx, row = (ly - 1u) * Gx;
-        uint32_t a0, a1, b0, b1;
-        row_pieces(x, Gx, a0, a1, b0, b1);
-        // pieces k of slots pre[k] .. pre[k + 1] of the list, at slot t + d[k]
-        uint32_t pre[7], d[6];
-        pre[0] = 0u;
-#pragma unroll
-        for (int y = 0; y < 3; ++y) {
-            const uint32_t R = row + uint32_t(y) * Gx;
-            const uint32_t p0 = cnt[R + a0], p1 = cnt[R + a1], q0 = cnt[R], q1 = cnt[R + b1];
-            d[2 * y] = p0 - pre[2 * y];
-            pre[2 * y + 1] = pre[2 * y] + (p1 - p0);
-            d[2 * y + 1] = q0 - pre[2 * y + 1];
-            pre[2 * y + 2] = pre[2 * y + 1] + (q1 - q0);
-        }
-        const uint32_t K = pre[6];
-        f3 acc = mk(0.f, 0.f, 0.f);
-        for (uint32_t i = lane; i - lane < K; i += 4u) {
-            uint32_t j = d[5];
-#pragma unroll
-            for (int k = 4; k >= 0; --k) j = i < pre[k + 1] ? d[k] : j;
-            const bool on = i < K;
-            float4 P = lpos[on ? i + j : s];  // past the list: the bead itself, masked by its worm
-            add_quad(acc, wca_term_masked(kp, r, fil, rc2, P));
-        }
-        if (lane == 0u) a.force[me] = make_float4(F.x + acc.x, F.y + acc.y, F.z + acc.z, F.w + 0.0f);
-    }
+    if (s1 - s0 > kRowsLaneBeads) rows_pairs<T, 1>(kp, a, lid, lpos, lcell, cnt, s0, s1);
+    else rows_pairs<T, 4>(kp, a, lid, lpos, lcell, cnt, s0, s1);
 }
 
 __global__ __launch_bounds__(kRowsBlock) void k_rows(RowsArgs a, uint32_t N, uint32_t rows, uint32_t cap,
@@ -335,16 +368,17 @@ __global__ __launch_bounds__(kRowsBlock) void k_rows_batch(BatchArrays a, const 
 // ---------------------------------------------------------------------------
 // A step with the sort and the pair kernel / with this launch, worms of 16: 21.5
 // / 13.0 us at 32,000 beads, 22.1 / 16.0 at 64,000, 25.0 / 19.9 at 128,000, 27.7
-// / 24.2 at 192,000, 28.5 / 29.2 at 224,000; where the front and the sort's first
-// level are two launches (front_tiles_plan: more than 4,096 wavefronts), worms
-// of 23: 33.3 / 28.8 at 195,000 and 34.5 / 30.5 at 229,000.
-constexpr uint64_t kRowsMaxBeads = 204800, kRowsMaxBeadsTwo = 240000;
+// / 22.6 at 192,000, 28.9 / 27.5 at 256,000, 33.1 / 33.6 at 288,000; where the
+// front and the sort's first level are two launches (front_tiles_plan: more than
+// 4,096 wavefronts), worms of 23: 32.9 / 27.9 at 229,000, 35.8 / 31.4 at 298,000,
+// 39.0 / 38.8 at 344,000.
+constexpr uint64_t kRowsMaxBeads = 262144, kRowsMaxBeadsTwo = 300000;
 // every workgroup reads every worm's rows: 22.8 / 20.4 us with 20,000 worms of
 // three, 23.1 / 24.8 with 30,000; of five 22.7 / 19.6 with 15,000, 26.9 / 28.1
 // with 30,000
 constexpr uint64_t kRowsMaxWorms = 24576;
 constexpr uint32_t kRowsMaxBlocks = 256;  // one round of the CUs: 64,000 beads over 291 rows take 23.0 us by single rows, 16.0 by pairs
-constexpr uint32_t kRowsMaxOwn = 1280;    // beads of a workgroup on average: five rounds of its quads
+constexpr uint32_t kRowsMaxOwn = 1408;    // beads of a workgroup on average, which its stage and its rounds allow
 
 // whether the launch computes a system's pair term at all
 static bool rows_term(const KP &kp) {
@@ -381,45 +415,39 @@ bool rows_plan(uint64_t N, const KP &kp, RowsPlan &out) {
     return rows_fits(out);
 }
 
-// The batch takes the launch up to 480,000 beads.  A step (us, sort + pairs / this
-// launch): 16 x 1,100 beads 27.8 / 13.5, 16 x 8,600 34.3 / 20.5, 32 x 8,100 40.2
-// / 33.1, 64 x 7,700 52.4 / 48.1, 16 x 29,700 49.7 / 48.3, 128 x 4,000 53.9 / 48.5,
-// 256 x 2,000 55.5 / 55.3; past it 96 x 8,000 63.6 / 69.0, 8 x 79,500 55.4 / 66.9.
-constexpr uint64_t kRowsMaxBatchBeads = 480000;
-constexpr double kRowsBatchOwn = 768.0, kRowsBatchOwnOne = 1024.0;  // beads of a workgroup on average
+// The batch takes the launch up to 700,000 beads in replicas of up to 100,000.  A
+// step (us, sort + pairs / this launch): 16 x 1,100 beads 27.8 / 13.5, 48 x 8,100
+// 46 / 40, 64 x 7,700 51 / 44, 80 x 8,500 59 / 55, 16 x 29,700 49 / 44, 8 x 79,500 55
+// / 50, 128 x 4,000 53 / 44, 256 x 2,000 55 / 49; past it 128 x 8,100 76 / 75, 6 x
+// 127,000 57 / 61, 2 x 180,000 39 / 42.
+constexpr uint64_t kRowsMaxBatchBeads = 700000, kRowsMaxReplicaBeads = 100000;
 
 bool rows_plan_batch(BatchRep *reps, uint32_t R, RowsPlan &out) {
     out = RowsPlan{};
-    uint64_t rows = 0;
+    uint64_t rows = 0, beads = 0;
     for (uint32_t r = 0; r < R; ++r) {
         if (!rows_term(reps[r].kp)) return false;
         rows += reps[r].kp.p.gridSize.y;
+        beads += reps[r].numBeads;
     }
     RowsPlan pl{};
     const uint32_t per = uint32_t((rows + kRowsMaxBlocks - 1u) / kRowsMaxBlocks);
-    // the rows of a workgroup of replica q with at most maxOwn beads on average
-    const auto rows_of = [&](const BatchRep &q, double maxOwn) {
-        const double perRow = std::max(1.0, double(q.numBeads) / q.kp.p.gridSize.y);
-        return std::max(1u, std::min({per, uint32_t(maxOwn / perRow), q.kp.p.gridSize.y - 2u}));
-    };
-    // a batch that one more round of quads fits into one round of the CUs
-    // takes it (16 x 12,000 beads by six rows, 288 workgroups, 21.6 us, by
-    // seven, 256, 14.8)
-    uint64_t one = 0;
-    for (uint32_t r = 0; r < R; ++r) one += (reps[r].kp.p.gridSize.y + rows_of(reps[r], kRowsBatchOwnOne) - 1u) / rows_of(reps[r], kRowsBatchOwnOne);
-    const double maxOwn = one <= kRowsMaxBlocks ? kRowsBatchOwnOne : kRowsBatchOwn;
-    uint64_t beads = 0;
+    // beads of a workgroup: somewhat more than an even share of a round of the
+    // CUs, so that a replica denser than the rest is cut finer (16 of 800 to
+    // 24,000 beads: 576 us a pass with 1,408 throughout, 565 with its 768)
+    const double own = std::min(std::max(1.25 * double(beads) / kRowsMaxBlocks, 768.0), double(kRowsMaxOwn));
     for (uint32_t r = 0; r < R; ++r) {
         BatchRep &q = reps[r];
         const uint32_t Gx = q.kp.p.gridSize.x, Gy = q.kp.p.gridSize.y;
-        if (double(q.numBeads) / Gy > kRowsBatchOwn || q.kp.p.numFilaments > kRowsMaxWorms) return false;
-        q.rows = rows_of(q, maxOwn);
+        const double perRow = std::max(1.0, double(q.numBeads) / Gy);
+        if (perRow > own || q.numBeads > kRowsMaxReplicaBeads || q.kp.p.numFilaments > kRowsMaxWorms)
+            return false;
+        q.rows = std::max(1u, std::min({per, uint32_t(own / perRow), Gy - 2u}));
         q.rowBlock = pl.blocks;
         const uint32_t blocks = (Gy + q.rows - 1u) / q.rows;
         pl.blocks += blocks;
         pl.cells = std::max(pl.cells, (q.rows + 2u) * Gx);
         pl.cap = std::max(pl.cap, rows_cap(q.numBeads, Gy, q.rows));
-        beads += q.numBeads;
     }
     if (!pl.blocks || beads > kRowsMaxBatchBeads || !rows_fits(pl)) return false;
     out = pl;
