@@ -293,7 +293,7 @@ __device__ __forceinline__ void add_layer_global(const KP &kp, const Owner<MODE,
             if (t0 + uint32_t(u) < K) {
                 uint32_t fil2, ch2;
                 worm_of(kp, I[u] - beadBase, fil2, ch2);
-                add_pair<MODE, TAN>(kp, o, rc2, W[u], acc, mk(P[u]), fil2, ch2,
+                add_pair<MODE, TAN>(kp, o, rc2, W[u], acc, mk(P[u]), pair_who(o, fil2, ch2),
                                     MODE == 0 ? mk(V[u]) : mk(0.f, 0.f, 0.f), TAN ? mk(T[u]) : mk(0.f, 0.f, 0.f));
             }
         }
@@ -386,8 +386,8 @@ __device__ __forceinline__ void lds_pair(const KP &kp, const Owner<MODE, TAN> &o
         const f3 t = wca_term_masked(kp, o.r, o.fil, rc2, P);
         acc += UNIT ? t : wt * t;
     } else {
-        add_pair<MODE, TAN, UNIT>(kp, o, rc2, wt, acc, mk(P), __float_as_uint(P.w),
-                                  MODE == 0 ? __float_as_uint(V.w) : 0u, MODE == 0 ? mk(V) : mk(0.f, 0.f, 0.f),
+        add_pair<MODE, TAN, UNIT>(kp, o, rc2, wt, acc, mk(P),
+                                  pair_who(o, __float_as_uint(P.w), MODE == 0 ? __float_as_uint(V.w) : 0u), MODE == 0 ? mk(V) : mk(0.f, 0.f, 0.f),
                                   TAN ? mk(T) : mk(0.f, 0.f, 0.f));
     }
 }

@@ -14,6 +14,18 @@ struct Owner {
     uint32_t fil, ch;
 };
 
+// whose a candidate is: the owner itself, of the owner's worm, its chain
+// neighbour
+struct PairWho {
+    bool self, same, bonded;
+};
+// of the candidate in worm fil2 at place ch2 of its chain
+template <int MODE, bool TAN>
+__device__ __forceinline__ PairWho pair_who(const Owner<MODE, TAN> &o, uint32_t fil2, uint32_t ch2) {
+    const bool same = o.fil == fil2;
+    return {same && ch2 == o.ch, same, same && (o.ch + 1u == ch2 || o.ch - 1u == ch2)};
+}
+
 // One candidate's terms, MODE 0: the chain bond (bondHookean
 // particles_kernel_impl.cuh:466-473) between chain neighbours, else the soft
 // sphere (collideParticles :427-462); MODE 1: WCA between different worms;
@@ -25,16 +37,15 @@ struct Owner {
 // on the way to a component stays what three divisions made it.
 template <int MODE, bool TAN, bool UNIT = false>
 __device__ __forceinline__ void add_pair(const KP &kp, const Owner<MODE, TAN> &o, float rc2, float w, f3 &acc,
-                                         f3 r2, uint32_t fil2, uint32_t ch2, f3 v2, f3 t2) {
+                                         f3 r2, PairWho who, f3 v2, f3 t2) {
     const SimParams &p = kp.p;
-    const bool same = o.fil == fil2;
-    if (MODE == 0 ? (same && ch2 == o.ch) : same) return;
+    if (MODE == 0 ? who.self : who.same) return;
     const f3 rel = min_image_pair(p, o.r, r2);
     const float rr = dot(rel, rel);
     f3 t = mk(0.f, 0.f, 0.f);
     if (MODE == 0) {
         const float dist = sqrtf(rr);
-        if (same && ((o.ch + 1u == ch2) || (o.ch - 1u == ch2))) {
+        if (who.bonded) {
             t = (-p.bondSpringK * (p.bondSpringL - dist) / dist) * rel;
         } else {
             const float cd = p.particleRadius + p.particleRadius;
@@ -50,7 +61,7 @@ __device__ __forceinline__ void add_pair(const KP &kp, const Owner<MODE, TAN> &o
         if (rr < rc2) t = -wca_mag(kp.e, rr) * rel;
     }
     acc += UNIT ? t : w * t;
-    if (TAN && !same) {
+    if (TAN && !who.same) {
         f3 x = mk(0.f, 0.f, 0.f);
         if (dot(o.t, t2) < -0.5f) x = (-p.activity / (2.0f * sqrtf(rr))) * (o.t - t2);
         acc += UNIT ? x : w * x;

@@ -8,9 +8,9 @@
 // share a bead: each looks up its share of the cells, the lanes' counts are
 // scanned, and the bead's candidates are written to one LDS list, from which
 // the S lanes take them in turn.  The lanes' sums are added in a fixed order.
-// Measured at 96,000 beads, 64 x 64 x 32 cells: 86 -> 25 us against one lane a
+// Measured at 96,000 beads, 64 x 64 x 32 cells: 86 -> 23.7 us against one lane a
 // bead (22,600 instructions of unrolled walk, nine divisions a candidate); at
-// 30,000 beads through the reference's tables 80 -> 14 us.  What bounds it now
+// 30,000 beads through the reference's tables 80 -> 12.8 us.  What bounds it now
 // is the issue of some 1,000 VALU a wavefront (8 beads), a fifth of them exact
 // square roots and quotients.
 #include "nw_internal.hpp"
@@ -74,7 +74,8 @@ __global__ __launch_bounds__(kBlock) void k_pair_list(float4 *__restrict__ force
     // through the sorted slots row by row); one beyond an
     // axis's distinct cells counts nothing.  Every load is unconditional and
     // in bounds (an unused entry of AxisCells holds the centre).
-    uint32_t a[PER], len[PER], total = 0;
+    uint32_t a[PER], end[PER], len[PER], total = 0;
+    bool use[PER];
     float wt[PER];
 #pragma unroll
     for (uint32_t j = 0; j < PER; ++j) {
@@ -84,21 +85,24 @@ __global__ __launch_bounds__(kBlock) void k_pair_list(float4 *__restrict__ force
         const int cy = yi == 0 ? ay.c[0] : (yi == 1 ? ay.c[1] : ay.c[2]);
         const int cz = zi == 0 ? az.c[0] : (zi == 1 ? az.c[1] : az.c[2]);
         const uint32_t h = (uint32_t(cz) * p.gridSize.y + uint32_t(cy)) * p.gridSize.x + uint32_t(cx);
-        const bool use = own && k < 27u && int(xi) < ax.n && int(yi) < ay.n && int(zi) < az.n;
-        uint32_t b;
-        if (CSR) {
-            a[j] = cells.off[h];
-            b = cells.off[h + 1u];
-        } else {
-            a[j] = cells.start[h];
-            b = a[j] == 0xffffffffu ? a[j] : cells.end[h];
-        }
-        len[j] = use && b > a[j] ? b - a[j] : 0u;
+        use[j] = own && k < 27u && int(xi) < ax.n && int(yi) < ay.n && int(zi) < az.n;
+        // (an empty cell's entry of `end` holds what it held, unused)
+        a[j] = CSR ? cells.off[h] : cells.start[h];
+        end[j] = CSR ? cells.off[h + 1u] : cells.end[h];
         if (!UNIT) {
             wt[j] = (zi == 0 ? az.w[0] : (zi == 1 ? az.w[1] : az.w[2])) *
                     (yi == 0 ? ay.w[0] : (yi == 1 ? ay.w[1] : ay.w[2])) *
                     (xi == 0 ? ax.w[0] : (xi == 1 ? ax.w[1] : ax.w[2]));
         }
+    }
+    // the ends loaded beside the starts, not behind a branch on each (30,000
+    // beads by the tables: 14.4 us with it, 12.8 without)
+#pragma unroll
+    for (uint32_t j = 0; j < PER; ++j) asm volatile("" ::"v"(end[j]));
+#pragma unroll
+    for (uint32_t j = 0; j < PER; ++j) {
+        const bool any = use[j] && (CSR || a[j] != 0xffffffffu);
+        len[j] = any && end[j] > a[j] ? end[j] - a[j] : 0u;
         total += len[j];
     }
     uint32_t K;
@@ -129,9 +133,10 @@ __global__ __launch_bounds__(kBlock) void k_pair_list(float4 *__restrict__ force
             float4 V0{}, T0{};
             if (MODE == 0) V0 = load4(sVel, j0);
             if (TAN) T0 = load4(sTan, j0);
-            uint32_t fil, ch;
-            worm_of(kp, I0, fil, ch);
-            add_pair<MODE, TAN, UNIT>(kp, o, rc2, UNIT ? 1.0f : listW[g][t], acc, mk(P0), fil, ch, mk(V0), mk(T0));
+            // by the bead ids alone: the owner's worm starts at me - o.ch
+            const bool same = I0 - (me - o.ch) < p.filamentSize;
+            const PairWho who{I0 == me, same, same && (I0 + 1u == me || I0 - 1u == me)};
+            add_pair<MODE, TAN, UNIT>(kp, o, rc2, UNIT ? 1.0f : listW[g][t], acc, mk(P0), who, mk(V0), mk(T0));
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
