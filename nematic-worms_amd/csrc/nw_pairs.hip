@@ -10,7 +10,7 @@
 // the S lanes take them in turn.  The lanes' sums are added in a fixed order.
 // Measured at 96,000 beads, 64 x 64 x 32 cells: 86 -> 23.7 us against one lane a
 // bead (22,600 instructions of unrolled walk, nine divisions a candidate); at
-// 30,000 beads through the reference's tables 80 -> 12.8 us.  What bounds it now
+// 30,000 beads through the reference's tables 80 -> 12.5 us.  What bounds it now
 // is the issue of some 1,000 VALU a wavefront (8 beads), a fifth of them exact
 // square roots and quotients.
 #include "nw_internal.hpp"
@@ -40,14 +40,15 @@ __device__ __forceinline__ uint32_t group_scan(uint32_t v, uint32_t s, uint32_t 
     return x - v;
 }
 
-template <int MODE, bool TAN, bool UNIT, bool CSR, int S>
+// CELLS: the stencil's cells, 9 of one layer or 27
+template <int MODE, bool TAN, bool UNIT, bool CSR, int S, int CELLS>
 __global__ __launch_bounds__(kBlock) void k_pair_list(float4 *__restrict__ force, const float4 *__restrict__ sPos,
                                                       const float4 *__restrict__ sVel,
                                                       const float4 *__restrict__ sTan,
                                                       const uint32_t *__restrict__ sIdx, PairCells cells,
                                                       const uint32_t *__restrict__ sCell, uint32_t n, KP kp) {
     constexpr uint32_t G = kBlock / S;           // beads of a workgroup
-    constexpr uint32_t PER = (27 + S - 1) / S;   // cells of a lane
+    constexpr uint32_t PER = (CELLS + S - 1) / S;  // cells of a lane
     __shared__ uint32_t list[G][kListCap];
     __shared__ float listW[UNIT ? 1 : G][UNIT ? 1 : kListCap];
     const SimParams &p = kp.p;
@@ -70,7 +71,7 @@ __global__ __launch_bounds__(kBlock) void k_pair_list(float4 *__restrict__ force
     const AxisCells ay = axis_cells_in(gy, p.gridSize.y, false);
     const AxisCells az = axis_cells_in(gz, p.gridSize.z, kp.e.stencil == NW_STENCIL_2D);
 
-    // The lane's cells, PER in a row of the 27 (x fastest, so the list runs
+    // The lane's cells, PER in a row of them (x fastest, so the list runs
     // through the sorted slots row by row); one beyond an
     // axis's distinct cells counts nothing.  Every load is unconditional and
     // in bounds (an unused entry of AxisCells holds the centre).
@@ -79,13 +80,13 @@ __global__ __launch_bounds__(kBlock) void k_pair_list(float4 *__restrict__ force
     float wt[PER];
 #pragma unroll
     for (uint32_t j = 0; j < PER; ++j) {
-        const uint32_t k = s * PER + j, kc = min(k, 26u);
-        const uint32_t zi = kc / 9u, yi = kc / 3u % 3u, xi = kc % 3u;
+        const uint32_t k = s * PER + j, kc = min(k, uint32_t(CELLS) - 1u);
+        const uint32_t zi = CELLS == 9 ? 0u : kc / 9u, yi = kc / 3u % 3u, xi = kc % 3u;
         const int cx = xi == 0 ? ax.c[0] : (xi == 1 ? ax.c[1] : ax.c[2]);
         const int cy = yi == 0 ? ay.c[0] : (yi == 1 ? ay.c[1] : ay.c[2]);
         const int cz = zi == 0 ? az.c[0] : (zi == 1 ? az.c[1] : az.c[2]);
         const uint32_t h = (uint32_t(cz) * p.gridSize.y + uint32_t(cy)) * p.gridSize.x + uint32_t(cx);
-        use[j] = own && k < 27u && int(xi) < ax.n && int(yi) < ay.n && int(zi) < az.n;
+        use[j] = own && k < uint32_t(CELLS) && int(xi) < ax.n && int(yi) < ay.n && int(zi) < az.n;
         // (an empty cell's entry of `end` holds what it held, unused)
         a[j] = CSR ? cells.off[h] : cells.start[h];
         end[j] = CSR ? cells.off[h + 1u] : cells.end[h];
@@ -152,18 +153,17 @@ __global__ __launch_bounds__(kBlock) void k_pair_list(float4 *__restrict__ force
     }
 }
 
-// Lanes a bead: 8.  96,000 beads of the reference's physics in 64 x 64 x 32
-// cells (CSR): 29.9 / 27.4 / 31.3 / 38.2 us with 4 / 8 / 16 / 32 lanes (first
-// form of the kernel, now 25.0); 30,000 beads by the reference's tables: 18.6
-// / 13.4 / 14.4 / 16.3 us.
-constexpr int kPairLanes = 8;
+// Lanes a bead: 8 while that fills the chip, 4 beyond, where the lanes' lookups
+// and sums are work (through the tables, us with 8 / 4 / 2 lanes): 27 cells, 96,000
+// beads of the soft spheres 27 / 29 / 41, 800,000 160 / 152 / 200, WCA in three
+// dimensions 110 / 93 / 135; 9 cells, 10,000 WCA beads 6.7 with 8, 800,000 70 / 52 /
+// 74; soft spheres in one layer, 800,000, 100 / 115 / 170: 8 throughout.
+constexpr uint32_t kPairFewBeads = 200000;
 
-template <bool CSR>
-static hipError_t launch_list(float4 *force, const float4 *sPos, const float4 *sVel, const float4 *sTan,
-                               const uint32_t *sIdx, const PairCells &c, const uint32_t *sCell, uint32_t n,
-                               const KP &kp, hipStream_t st) {
-    if (n == 0) return hipSuccess;
-    constexpr int S = kPairLanes;
+template <bool CSR, int S, int CELLS>
+static void launch_list_of(float4 *force, const float4 *sPos, const float4 *sVel, const float4 *sTan,
+                           const uint32_t *sIdx, const PairCells &c, const uint32_t *sCell, uint32_t n, const KP &kp,
+                           hipStream_t st) {
     const bool wca = kp.e.pairPotential == NW_PAIR_WCA;
     const bool tan = !wca || kp.p.activity != 0.0f;
     // every distinct cell counts once when no axis folds its offsets
@@ -171,7 +171,7 @@ static hipError_t launch_list(float4 *force, const float4 *sPos, const float4 *s
                       (kp.e.stencil == NW_STENCIL_2D || kp.p.gridSize.z >= 3);
     const dim3 grid(grid_for(uint64_t(n) * S)), block(kBlock);
 #define NW_LIST(M, T, U) \
-    NW_LAUNCH((k_pair_list<M, T, U, CSR, S>), grid, block, 0, st, force, sPos, sVel, sTan, sIdx, c, sCell, n, kp)
+    NW_LAUNCH((k_pair_list<M, T, U, CSR, S, CELLS>), grid, block, 0, st, force, sPos, sVel, sTan, sIdx, c, sCell, n, kp)
     if (unit) {
         if (!wca) NW_LIST(0, true, true);
         else if (tan) NW_LIST(1, true, true);
@@ -182,6 +182,23 @@ static hipError_t launch_list(float4 *force, const float4 *sPos, const float4 *s
         else NW_LIST(1, false, false);
     }
 #undef NW_LIST
+}
+
+template <bool CSR>
+static hipError_t launch_list(float4 *force, const float4 *sPos, const float4 *sVel, const float4 *sTan,
+                              const uint32_t *sIdx, const PairCells &c, const uint32_t *sCell, uint32_t n,
+                              const KP &kp, hipStream_t st) {
+    if (n == 0) return hipSuccess;
+    const bool few = n <= kPairFewBeads, oneLayer = kp.e.stencil == NW_STENCIL_2D || kp.p.gridSize.z == 1;
+#define NW_LIST_OF(S, CELLS) launch_list_of<CSR, S, CELLS>(force, sPos, sVel, sTan, sIdx, c, sCell, n, kp, st)
+    if (oneLayer) {
+        if (few || kp.e.pairPotential != NW_PAIR_WCA) NW_LIST_OF(8, 9);
+        else NW_LIST_OF(4, 9);
+    } else {
+        if (few) NW_LIST_OF(8, 27);
+        else NW_LIST_OF(4, 27);
+    }
+#undef NW_LIST_OF
     return hipGetLastError();
 }
 
