@@ -369,7 +369,7 @@ void nwBatchLayout(uint *beadOffset, uint *cellOffset);
 /* `steps` fused MD steps of every replica over the concatenated arrays
    (sortedVel / sortedTangent may be NULL as in nwFusedMdStep).  useGraph
    changes nothing: the step is two to four launches, and replaying them as a
-   captured hipGraph took 9 to 33 % longer (20 steps of 16 replicas of 8,600
+   captured hipGraph took 2 to 35 % longer (20 steps of 16 replicas of 8,600
    beads 498 us, launched 423; of two replicas of 360 339 and 252). */
 void nwBatchMdStep(float *pos, float *vel, float *force, float *forceOld, float *tangent,
                    uint *gridParticleIndex, float *sortedPos, float *sortedVel, float *sortedTangent,
@@ -530,7 +530,8 @@ uint nwGetDeviceFlags(int clear);
    "integrate", "langevin", "filament", "hash", "sort", "reorder", "collide",
    "srd_hash", "srd_sort", "srd_reorder", "srd_com", "srd_thermo",
    "srd_collide", "srd_stream", "reverse"; of the fused steps: "md_front",
-   "md_tiles" (the sort's first level), "md_sort", "md_collide" (a small
+   "md_tiles" (the sort's first level; under "md_front" where a mid-sized
+   system's front and first level are one launch), "md_sort", "md_collide" (a small
    system's order and pair forces are one launch, under "md_collide"),
    "srdf_tiles", "srdf_cells", "srdf_rotate"; of the batched step's kernels:
    "batch_front", "batch_tiles", "batch_sort", "batch_collide"; of the adjoint

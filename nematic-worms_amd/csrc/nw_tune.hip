@@ -4,10 +4,11 @@
 // nwFusedSrdStep) under each candidate NWTuning, reads the per-kernel timers
 // (HIP events on the kernels' dispatch packets) and keeps the fastest choice
 // of every knob.  The knobs act on different kernels, so they are searched
-// one kernel at a time: the front's workgroup size on the front, the MD
-// sort's tile and bucket sizes jointly on its two levels, the pair kernel's
-// workgroup size on the pair kernel, the SRD sort's tile and bucket sizes on
-// the collision's two sort levels.  Choices are cached in a text file, one
+// one kernel at a time: the front's workgroup size and the MD sort's tile and
+// bucket sizes on the front and the sort's two levels together (mid-sized
+// systems run the first two as one launch), the pair kernel's workgroup size
+// on the pair kernel, the SRD sort's tile and bucket sizes on the collision's
+// two sort levels.  Choices are cached in a text file, one
 // line per device and system size.
 #include <hip/hip_runtime.h>
 #include <sys/stat.h>
