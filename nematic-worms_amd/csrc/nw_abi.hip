@@ -1198,6 +1198,13 @@ static bool grow(T *&p, uint64_t &cap, uint64_t need) {
     cap = need;
     return true;
 }
+
+template <typename T>
+static void drop(T *&p, uint64_t &cap) {
+    if (p) (void)hipFree(p);
+    p = nullptr;
+    cap = 0;
+}
 }
 
 static bool copy_d2d(void *dst, const void *src, size_t bytes, hipStream_t st) {
@@ -1229,6 +1236,16 @@ static bool ensure_segment(State::Adjoint &A) {
            grow(A.collOff, A.capCollOff, cpS * (uint64_t(A.Cs) + 2)) &&
            grow(A.collCom, A.capCollCom, cpS * A.Cs) && grow(A.cellSum, A.capCellSum, A.Cs) &&
            grow(A.wPos, A.capWPos, NT) && grow(A.wVel, A.capWVel, NT);
+}
+
+// gives the segment store back, where a forward run that would have kept its
+// last segment does not fit with it
+static void drop_segment(State::Adjoint &A) {
+    drop(A.segPos, A.capPos), drop(A.segVel, A.capVel), drop(A.segSPos, A.capSPos), drop(A.segIds, A.capIds);
+    drop(A.segOff, A.capOff), drop(A.segCell, A.capCell), drop(A.work, A.capWork), drop(A.lam, A.capLam);
+    drop(A.collHash, A.capCollHash), drop(A.collIds, A.capCollIds), drop(A.collOff, A.capCollOff);
+    drop(A.collCom, A.capCollCom), drop(A.cellSum, A.capCellSum), drop(A.wPos, A.capWPos), drop(A.wVel, A.capWVel);
+    (void)hipGetLastError();
 }
 
 // The forward run leaves its last segment in the segment store, which the
@@ -1291,16 +1308,16 @@ static void adjoint_forward(float *pos, float *vel, float *force, float *forceOl
     const uint64_t perStep = 56 * N + 4 * C + 8 + (A.srd ? (8 * NT + 20 * uint64_t(A.Cs)) / A.gap : 0);
     A.held = -1;
     bool hold = K <= kHoldBytes / perStep;
-    if (hold && !ensure_segment(A)) {
-        (void)hipGetLastError();  // no room for it: the run goes on without
+    const auto room = [&] {
+        return grow(A.ckpt, A.capCkpt, uint64_t(nck) * stride) && grow(A.segSPos, A.capSPos, N) &&
+               grow(A.segIds, A.capIds, NT) &&
+               (!A.srd || (grow(A.collCom, A.capCollCom, A.Cs) && grow(A.collHash, A.capCollHash, NT)));
+    };
+    if (hold && !(ensure_segment(A) && room())) {
+        drop_segment(A);  // no room for it: the run goes on without
         hold = false;
     }
-    NW_REQUIRE(grow(A.ckpt, A.capCkpt, uint64_t(nck) * stride) && grow(A.segSPos, A.capSPos, N) &&
-                   grow(A.segIds, A.capIds, NT),
-               "nwAdjointForward: out of device memory");
-    if (A.srd)
-        NW_REQUIRE(grow(A.collCom, A.capCollCom, A.Cs) && grow(A.collHash, A.capCollHash, NT),
-                   "nwAdjointForwardSrd: out of device memory");
+    NW_REQUIRE(room(), "nwAdjointForward: out of device memory");
     A.ckptOffset.assign(nck, 0);
     A.lgvOff.assign(hold ? std::min<uint64_t>(K, steps) : 0, 0);
     uint64_t slots = 0;  // collisions kept
@@ -1621,6 +1638,15 @@ static bool ensure_batch_segment(State::BatchAdjoint &A) {
            grow(A.collCom, A.capCollCom, cpS * A.Cs) && grow(A.cellSum, A.capCellSum, A.Cs);
 }
 
+static void drop_batch_segment(State::BatchAdjoint &A) {
+    drop(A.segPos, A.capPos), drop(A.segVel, A.capVel), drop(A.segSPos, A.capSPos), drop(A.segIds, A.capIds);
+    drop(A.segOff, A.capOff), drop(A.work, A.capWork), drop(A.lam, A.capLam);
+    drop(A.wPos, A.capWPos), drop(A.wVel, A.capWVel), drop(A.collHash, A.capCollHash);
+    drop(A.collIds, A.capCollIds), drop(A.collOff, A.capCollOff), drop(A.collCom, A.capCollCom);
+    drop(A.cellSum, A.capCellSum);
+    (void)hipGetLastError();
+}
+
 static bool batch_langevin(const State::Batch &b) {
     bool lgv = false;
     for (const BatchRep &q : b.reps) lgv = lgv || q.langevin != 0;
@@ -1676,20 +1702,21 @@ void nwBatchAdjointForward(float *pos, float *vel, float *force, float *forceOld
     const uint64_t perStep = 52 * N + 4 * C + 8 + (srd ? (8 * NT + 20 * Cs) / srdGap : 0);
     A.held = -1;
     bool hold = K <= kHoldBytes / perStep;
-    if (hold && !ensure_batch_segment(A)) {
-        (void)hipGetLastError();  // no room for it: the run goes on without
+    const uint64_t nColl = srd ? collisions_in(steps, srdGap) : 0;
+    const auto room = [&] {
+        return grow(A.ckpt, A.capCkpt, uint64_t(nck) * stride) && grow(A.hash, A.capHash, NT) &&
+               grow(A.sCell, A.capSCell, N) && grow(A.segIds, A.capIds, N) && grow(A.segSPos, A.capSPos, N) &&
+               grow(A.segOff, A.capOff, C + 2) &&
+               (!srd || (grow(A.shifts, A.capShifts, nColl * b.R * 3) && grow(A.collHash, A.capCollHash, NT) &&
+                         grow(A.collIds, A.capCollIds, NT) && grow(A.collOff, A.capCollOff, Cs + 2) &&
+                         grow(A.collCom, A.capCollCom, Cs)));
+    };
+    if (hold && !(ensure_batch_segment(A) && room())) {
+        drop_batch_segment(A);  // no room for it: the run goes on without
         hold = false;
     }
-    NW_REQUIRE(grow(A.ckpt, A.capCkpt, uint64_t(nck) * stride) && grow(A.hash, A.capHash, NT) &&
-                   grow(A.sCell, A.capSCell, N) && grow(A.segIds, A.capIds, N) && grow(A.segSPos, A.capSPos, N) &&
-                   grow(A.segOff, A.capOff, C + 2),
-               "nwBatchAdjointForward: out of device memory");
+    NW_REQUIRE(room(), "nwBatchAdjointForward: out of device memory");
     if (srd) {
-        const uint64_t nColl = collisions_in(steps, srdGap);
-        NW_REQUIRE(grow(A.shifts, A.capShifts, nColl * b.R * 3) && grow(A.collHash, A.capCollHash, NT) &&
-                       grow(A.collIds, A.capCollIds, NT) && grow(A.collOff, A.capCollOff, Cs + 2) &&
-                       grow(A.collCom, A.capCollCom, Cs),
-                   "nwBatchAdjointForward: out of device memory");
         NW_HIP(hipMemcpy(A.shifts, srdShifts, nColl * b.R * 3 * sizeof(float), hipMemcpyHostToDevice));
     }
     BatchArrays a{};
