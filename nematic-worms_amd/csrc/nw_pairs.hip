@@ -114,15 +114,20 @@ __global__ __launch_bounds__(kBlock) void k_pair_list(float4 *__restrict__ force
     // a wavefront's groups list and take their candidates together; the
     // lists belong to the wavefront, whose lanes run in step
     for (uint32_t base = 0; __any(base < K); base += kListCap) {
-        uint32_t e = first - base;  // mod 2^32: entries before this round wrap past the cap
+        // of each cell the entries of this round alone: a cell crowded beyond
+        // the list is listed once over all rounds, not once in each
+        uint32_t f = first;
 #pragma unroll
-        for (uint32_t j = 0; j < PER; ++j)
+        for (uint32_t j = 0; j < PER; ++j) {
+            const uint32_t k0 = f < base ? min(base - f, len[j]) : 0u;
+            const uint32_t k1 = f < base + kListCap ? min(base + kListCap - f, len[j]) : 0u;
 #pragma unroll 1
-            for (uint32_t k = 0; k < len[j]; ++k, ++e)
-                if (e < kListCap) {
-                    list[g][e] = a[j] + k;
-                    if (!UNIT) listW[g][e] = wt[j];
-                }
+            for (uint32_t k = k0; k < k1; ++k) {
+                list[g][f + k - base] = a[j] + k;
+                if (!UNIT) listW[g][f + k - base] = wt[j];
+            }
+            f += len[j];
+        }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
