@@ -68,10 +68,9 @@ __device__ __forceinline__ void row_pieces(uint32_t x, uint32_t Gx, uint32_t &a0
     b1 = left ? 2u : (right ? 1u : 0u);
 }
 
-// A stage too small for the rows' beads (a collapsed or exploded system; the
-// host gives it two and a half times the average): every lane takes a cell,
-// then a bead, and passes over all cells of the system in bead order.  Slow
-// and exact.  (LDS holds the counts of the rows' cells only.)
+// A stage too small for the rows' beads (a collapsed or exploded system; see
+// rows_cap): every lane takes a cell, then a bead, and passes over all cells of
+// the system in bead order.  Slow and exact.  (LDS holds the counts of the rows' cells only.)
 __device__ __forceinline__ void rows_unstaged(const KP &kp, const RowsArgs &a, uint32_t N, uint32_t idBase,
                                            uint32_t cellBase, uint32_t slotBase, uint32_t y0, uint32_t own,
                                            const uint32_t *cnt) {
@@ -388,15 +387,25 @@ static bool rows_term(const KP &kp) {
            p.gridSize.y < 65536u;  // a row in 16 bits
 }
 
-// beads staged by a workgroup of `rows` rows: two and a half times the
-// average, since rows fill to at most about the close packing of their cells
-static uint32_t rows_cap(uint64_t N, uint32_t Gy, uint32_t rows) {
-    return std::max(1024u, (uint32_t(2.5 * double(N) / Gy * (rows + 2u)) + 255u) & ~255u);
+// Beads staged by a workgroup of `rows` rows: two and a half times the
+// average, and as far as `lds` bytes hold them the close packing of the rows'
+// cells (1.45 beads a cell of the WCA range): worms that gather in bands, or
+// start on a lattice in a part of the box, stay within the stage.
+static uint32_t rows_cap(uint64_t N, uint32_t Gx, uint32_t Gy, uint32_t rows, uint32_t lds) {
+    const uint32_t cells = (rows + 2u) * Gx, fixed = rows_layout(0, cells).total;
+    const uint32_t mean = (uint32_t(2.5 * double(N) / Gy * (rows + 2u)) + 255u) & ~255u;
+    const uint32_t packed = (uint32_t(1.45 * cells) + 255u) & ~255u;
+    const uint32_t room = lds > fixed ? std::min((lds - fixed) / 22u & ~255u, 8192u) : 0u;
+    return std::max({1024u, mean, std::min(packed, room)});
 }
+
+// LDS of a workgroup alone on its CU, and where two share one (batches, whose
+// workgroups may be more than a round)
+constexpr uint32_t kRowsLds = 150u * 1024u, kRowsLdsHalf = 80u * 1024u;
 
 static bool rows_fits(RowsPlan &pl) {
     pl.lds = rows_layout(pl.cap, pl.cells).total;
-    return pl.cells <= 8192u && pl.cap <= 8192u && pl.lds <= 150u * 1024u;
+    return pl.cells <= 8192u && pl.cap <= 8192u && pl.lds <= kRowsLds;
 }
 
 bool rows_plan(uint64_t N, const KP &kp, RowsPlan &out) {
@@ -411,7 +420,7 @@ bool rows_plan(uint64_t N, const KP &kp, RowsPlan &out) {
     out.blocks = (Gy + out.rows - 1u) / out.rows;
     if (double(N) / Gy * out.rows > double(kRowsMaxOwn)) return false;
     out.cells = (out.rows + 2u) * Gx;
-    out.cap = rows_cap(N, Gy, out.rows);
+    out.cap = rows_cap(N, Gx, Gy, out.rows, kRowsLds);
     return rows_fits(out);
 }
 
@@ -447,7 +456,7 @@ bool rows_plan_batch(BatchRep *reps, uint32_t R, RowsPlan &out) {
         const uint32_t blocks = (Gy + q.rows - 1u) / q.rows;
         pl.blocks += blocks;
         pl.cells = std::max(pl.cells, (q.rows + 2u) * Gx);
-        pl.cap = std::max(pl.cap, rows_cap(q.numBeads, Gy, q.rows));
+        pl.cap = std::max(pl.cap, rows_cap(q.numBeads, Gx, Gy, q.rows, kRowsLdsHalf));
     }
     if (!pl.blocks || beads > kRowsMaxBatchBeads || !rows_fits(pl)) return false;
     out = pl;
