@@ -68,8 +68,8 @@ __device__ __forceinline__ void row_pieces(uint32_t x, uint32_t Gx, uint32_t &a0
     b1 = left ? 2u : (right ? 1u : 0u);
 }
 
-// A stage too small for the rows' beads (a collapsed or exploded system; see
-// rows_cap): every lane takes a cell, then a bead, and passes over all cells of
+// A stage too small for the rows' beads by the two rows beside the own
+// ones alone (a collapsed or exploded system; see rows_cap): every lane takes a cell, then a bead, and passes over all cells of
 // the system in bead order.  Slow and exact.  (LDS holds the counts of the rows' cells only.)
 __device__ __forceinline__ void rows_unstaged(const KP &kp, const RowsArgs &a, uint32_t N, uint32_t idBase,
                                            uint32_t cellBase, uint32_t slotBase, uint32_t y0, uint32_t own,
@@ -186,6 +186,46 @@ __device__ __forceinline__ void rows_pairs(const KP &kp, const RowsArgs &a, cons
     }
 }
 
+// More beads than the stage holds, but not in the two rows beside the own
+// ones: the own beads in their slots of `ids`, already there in ascending id
+// per cell, the others' ids in lid (staged slots without the own ones').
+__device__ __forceinline__ void rows_own_in_memory(const KP &kp, const RowsArgs &a, uint32_t idBase,
+                                                   uint32_t cellBase, uint32_t slot0, uint32_t y0, uint32_t s0,
+                                                   uint32_t s1, const uint32_t *cnt, const uint32_t *lid) {
+    const uint32_t Gx = kp.p.gridSize.x;
+    const float rc2 = kp.e.wcaCutoff * kp.e.wcaCutoff;
+    const uint32_t *own = a.ids + slot0;
+    for (uint32_t s = s0 + threadIdx.x; s < s1; s += blockDim.x) {
+        const uint32_t me = own[s - s0] - idBase, cell = a.hash[me];
+        const float4 R = load4(a.pos, me);
+        a.sCell[slot0 + (s - s0)] = cell;
+        a.sPos[slot0 + (s - s0)] = R;
+        int gx, gy, gz;
+        cell_xyz(kp, cell - cellBase, gx, gy, gz);
+        const f3 r = mk(R);
+        uint32_t fil, ch, lo, hi, b0, b1;
+        worm_of(kp, me, fil, ch);
+        row_pieces(uint32_t(gx), Gx, lo, hi, b0, b1);
+        f3 acc = mk(0.f, 0.f, 0.f);
+        for (uint32_t yi = 0; yi < 3u; ++yi) {
+            const uint32_t row = (uint32_t(gy) - y0 + yi) * Gx;  // staged: the one below the own rows first
+            for (uint32_t k = 0; k < 3u; ++k) {
+                const uint32_t d = row + (lo + k < hi ? lo + k : b0 + k - (hi - lo));
+                for (uint32_t u = cnt[d], z = cnt[d + 1u]; u < z; ++u) {
+                    const uint32_t j = u < s0 ? lid[u] : (u < s1 ? own[u - s0] - idBase : lid[u - (s1 - s0)]);
+                    uint32_t fil2, ch2;
+                    worm_of(kp, j, fil2, ch2);
+                    float4 P = load4(a.pos, j);
+                    P.w = __uint_as_float(fil2);
+                    acc += wca_term_masked(kp, r, fil, rc2, P);
+                }
+            }
+        }
+        const float4 F = load4(a.force, me);
+        a.force[me] = make_float4(F.x + acc.x, F.y + acc.y, F.z + acc.z, F.w + 0.0f);
+    }
+}
+
 // Rows [y0, y0 + rows) of one system: N beads whose arrays hash, pos, force
 // start at its first bead; ids, sCell and sPos (indexed by sorted slot) and
 // off (by cell) at its own first entries; bead ids, cells and slots of the
@@ -288,7 +328,31 @@ __device__ __forceinline__ void rows_body(const KP &kp, const RowsArgs &a, uint3
     for (uint32_t c = t; c < own * Gx; c += T) a.off[hOwn + c] = slotBase + cnt[Gx + c] - s0;
     if (y0 + own == Gy && t == 0) a.off[C] = slotAdd + N;
     if (m > cap) {
-        rows_unstaged(kp, a, N, idBase, cellBase, slotBase - slotAdd, y0, own, cnt);
+        const uint32_t slot0 = slotBase - slotAdd, owned = s1 - s0;
+        if (m - owned > cap) {
+            rows_unstaged(kp, a, N, idBase, cellBase, slot0, y0, own, cnt);
+            return;
+        }
+        for (uint32_t k = t; k < words; k += T) {
+            const uint32_t id = bead_of(k), d = local(a.hash[id] - cellBase);
+            if (d >= nc) continue;
+            const uint32_t s = atomicAdd(&cur[d], 1u);
+            if (s >= s0 && s < s1) a.ids[slot0 + (s - s0)] = idBase + id;
+            else lid[s < s0 ? s : s - owned] = id;
+        }
+        __syncthreads();
+        for (uint32_t c = t; c < nc; c += T) {
+            const uint32_t u0 = cnt[c], z = cnt[c + 1u] - u0;
+            uint32_t *cell = c >= Gx && c < (own + 1u) * Gx ? a.ids + slot0 + (u0 - s0) : lid + (u0 < s1 ? u0 : u0 - owned);
+            for (uint32_t u = 1; u < z; ++u) {
+                const uint32_t x = cell[u];
+                uint32_t w = u;
+                for (; w > 0u && cell[w - 1u] > x; --w) cell[w] = cell[w - 1u];
+                cell[w] = x;
+            }
+        }
+        __syncthreads();
+        rows_own_in_memory(kp, a, idBase, cellBase, slot0, y0, s0, s1, cnt, lid);
         return;
     }
     auto place = [&](uint32_t id, uint32_t d) {
