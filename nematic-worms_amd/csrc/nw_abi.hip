@@ -995,6 +995,8 @@ void nwBatchSetReplicas(const NWReplicaParams *reps, uint numReplicas) {
     b.reps.assign(numReplicas, BatchRep{});
     b.beadOff.assign(numReplicas + 1, 0u);
     b.cellOff.assign(numReplicas + 1, 0u);
+    b.tan = false;
+    b.unit = true;
     uint64_t N = 0, C = 0, waves = 0, blocks = 0;
     for (uint r = 0; r < numReplicas; ++r) {
         const NWReplicaParams &q = reps[r];
@@ -1041,8 +1043,6 @@ void nwBatchSetReplicas(const NWReplicaParams *reps, uint numReplicas) {
     b.waves = uint32_t(waves);
     b.blocks = uint32_t(blocks);
     b.mode = numReplicas && reps[0].ext.pairPotential == NW_PAIR_WCA ? 1 : 0;
-    if (b.mode == 0) b.tan = true;
-    if (numReplicas == 0) b.tan = false, b.unit = true;
     b.steps = 0;
     (void)rows_plan_batch(b.reps.data(), numReplicas, b.rows);
     b.sort.assign(numReplicas, SortRep{});
