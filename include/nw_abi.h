@@ -327,8 +327,8 @@ void nwGetTuning(NWTuning *tuning);
    copy of the given state (pos / vel hold the numFilaments worms' beads,
    followed by numSolvent solvent particles) -- the front's workgroup size,
    the MD sort's tile and bucket sizes jointly, the pair kernel's workgroup
-   size, each over `reps` steps with HIP events on the kernels' dispatch
-   packets -- and, when numSolvent > 0, those of nwFusedSrdStep (the SRD
+   size, each judged by all kernels of `reps` steps, with HIP events on their
+   dispatch packets -- and, when numSolvent > 0, those of nwFusedSrdStep (the SRD
    sort's tile and bucket sizes) with the SolventParams of the last
    setSolventParameters.  The fastest choice of each is set (nwSetTuning)
    and written to out.  The state itself is not touched; the generator is

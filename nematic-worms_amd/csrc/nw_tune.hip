@@ -4,11 +4,12 @@
 // nwFusedSrdStep) under each candidate NWTuning, reads the per-kernel timers
 // (HIP events on the kernels' dispatch packets) and keeps the fastest choice
 // of every knob.  The knobs act on different kernels, so they are searched
-// one kernel at a time: the front's workgroup size and the MD sort's tile and
-// bucket sizes on the front and the sort's two levels together (mid-sized
-// systems run the first two as one launch), the pair kernel's workgroup size
-// on the pair kernel, the SRD sort's tile and bucket sizes on the collision's
-// two sort levels.  Choices are cached in a text file, one
+// one at a time: the front's workgroup size, the MD sort's tile and bucket
+// sizes and the pair kernel's workgroup size, each judged by the whole MD
+// step (a knob asked for takes a small system out of the launches that do
+// front and first sort level, or cell order and pairs, at once, so the work
+// moves between the timed families), the SRD sort's tile and bucket sizes on
+// the collision's two sort levels.  Choices are cached in a text file, one
 // line per device and system size.
 #include <hip/hip_runtime.h>
 #include <sys/stat.h>
@@ -99,11 +100,13 @@ void cache_store(const std::string &file, const std::string &dev, const std::str
         << t.srdMembers << ' ' << t.pairBlock << ' ' << t.frontBlock << ' ' << t.pairStage << '\n';
 }
 
+// per launch, which is per step; 0 for a family that the step does not launch
+// (its work is then part of another's launch)
 double avg_ms(const char *fam) {
     double ms = 0.0;
     uint64_t n = 0;
     nwTimerRead(fam, &ms, &n);
-    return n ? ms / double(n) : 1e30;
+    return n ? ms / double(n) : 0.0;
 }
 
 }  // namespace
@@ -156,10 +159,14 @@ extern "C" int nwAutotuneFused(float *pos, float *vel, float *force, float *forc
         nwFusedSrdStep(fP, fV, static_cast<float *>(COM.p), static_cast<uint *>(H.p), static_cast<uint *>(I.p),
                        srdDeltaTime, uint(N), numSolvent, isokinetic);
     };
-    // the summed average duration of `fams` over reps steps under tuning t
+    // the summed average duration of the step's families (an SRD collision's
+    // sort levels) over reps steps under tuning t
     // (one untimed step first: first launches, LDS grants); negative when
-    // the library refused the setting or a step failed
-    auto measure = [&](const NWTuning &t, std::initializer_list<const char *> fams, bool srd) {
+    // the library refused the setting, a step failed or nothing was timed
+    auto measure = [&](const NWTuning &t, bool srd) {
+        static const std::vector<const char *> kMd = {"md_front", "md_tiles", "md_sort", "md_collide"},
+                                               kSrd = {"srdf_tiles", "srdf_cells"};
+        const std::vector<const char *> &fams = srd ? kSrd : kMd;
         nwSetTuning(&t);
         if (nwGetLastError() != 0) return -1.0;
         if (srd) srd_step();
@@ -174,7 +181,7 @@ extern "C" int nwAutotuneFused(float *pos, float *vel, float *force, float *forc
             tot += avg_ms(f);
             nwTimerEnable(f, 0);
         }
-        return nwGetLastError() == 0 ? tot : -1.0;
+        return nwGetLastError() == 0 && tot > 0.0 ? tot : -1.0;
     };
     // the plan a candidate asks for is the plan the step runs (else skipped:
     // it fell back to the built-in plan)
@@ -184,12 +191,12 @@ extern "C" int nwAutotuneFused(float *pos, float *vel, float *force, float *forc
         return out4[2] == items;
     };
     // one knob (or a pair) of `best` over its candidates
-    auto search = [&](std::vector<NWTuning> cands, std::initializer_list<const char *> fams, bool srd) {
-        const double base = measure(best, fams, srd);
+    auto search = [&](std::vector<NWTuning> cands, bool srd) {
+        const double base = measure(best, srd);
         double bestT = base;
         NWTuning pick = best;
         for (const NWTuning &c : cands) {
-            const double t = measure(c, fams, srd);
+            const double t = measure(c, srd);
             if (t >= 0.0 && t < bestT) {
                 bestT = t;
                 pick = c;
@@ -208,8 +215,7 @@ extern "C" int nwAutotuneFused(float *pos, float *vel, float *force, float *forc
             t.frontBlock = fb;
             c.push_back(t);
         }
-        // with the sort's first level, which a small system's built-in front does itself
-        search(c, {"md_front", "md_tiles", "md_sort"}, false);
+        search(c, false);
     }
     {
         std::vector<NWTuning> c;
@@ -222,7 +228,7 @@ extern "C" int nwAutotuneFused(float *pos, float *vel, float *force, float *forc
                 if (nwGetLastError() == 0 && plan_is(N, C, n, items)) c.push_back(t);
             }
         nwSetTuning(&best);
-        search(c, {"md_front", "md_tiles", "md_sort"}, false);
+        search(c, false);
     }
     {
         // the pair workgroup and its stage (0: pairBlock + 128 per row)
@@ -234,8 +240,7 @@ extern "C" int nwAutotuneFused(float *pos, float *vel, float *force, float *forc
                 t.pairStage = stage;
                 c.push_back(t);
             }
-        // with the sort: a small system's built-in choice does both in one launch
-        search(c, {"md_tiles", "md_sort", "md_collide"}, false);
+        search(c, false);
     }
     if (numSolvent) {
         std::vector<NWTuning> c;
@@ -248,7 +253,7 @@ extern "C" int nwAutotuneFused(float *pos, float *vel, float *force, float *forc
                 if (nwGetLastError() == 0 && plan_is(NT, Cs, 0, items)) c.push_back(t);
             }
         nwSetTuning(&best);
-        search(c, {"srdf_tiles", "srdf_cells"}, true);
+        search(c, true);
     }
     (void)hipStreamSynchronize(st);
     nwRngSetSeed(seed, offset);
