@@ -333,7 +333,8 @@ void nwGetTuning(NWTuning *tuning);
    setSolventParameters.  The fastest choice of each is set (nwSetTuning)
    and written to out.  The state itself is not touched; the generator is
    left where it was.  cachePath (NULL: $NW_TUNE_CACHE, else
-   $HOME/.cache/nwamd/tuning.txt; "": no cache) holds one line per device
+   $HOME/.cache/nwamd/tuning.txt; "": no cache) holds one line per device,
+   with the kernels' number and the form of the physics (pair term, stencil),
    and system size (beads, MD cells, beads per worm, solvent, SRD cells):
    with useCache a recorded line is applied without timing.  Returns 2 when
    the choice came from the cache, 1 when it was timed, 0 on an error. */

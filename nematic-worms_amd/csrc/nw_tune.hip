@@ -10,7 +10,7 @@
 // front and first sort level, or cell order and pairs, at once, so the work
 // moves between the timed families), the SRD sort's tile and bucket sizes on
 // the collision's two sort levels.  Choices are cached in a text file, one
-// line per device and system size.
+// line per device with the form of the physics, and system size.
 #include <hip/hip_runtime.h>
 #include <sys/stat.h>
 
@@ -52,6 +52,21 @@ std::string device_key() {
     std::string k = std::string(prop.gcnArchName) + "/" + prop.name + "/" + std::to_string(prop.multiProcessorCount);
     for (char &c : k)
         if (c == ' ' || c == '\t') c = '_';
+    return k;
+}
+
+// The launches that the built-in choice takes, and so what is worth asking
+// for, depend on the pair term and the stencil beside the sizes, and on the
+// kernels: raise the number when a kernel or a built-in rule changes, and
+// lines stored before it are not read any more.
+constexpr int kKernels = 2;
+
+std::string physics_key(const nw::KP &kp) {
+    std::string k = "/k" + std::to_string(kKernels);
+    k += kp.e.pairPotential == NW_PAIR_WCA ? "/wca" : "/dem";
+    if (kp.p.activity != 0.0f) k += "/extensile";
+    k += kp.e.stencil == NW_STENCIL_2D || kp.p.gridSize.z == 1 ? "/layer" : "/layers";
+    if (kp.e.collideKernel != NW_COLLIDE_AUTO) k += "/collide" + std::to_string(int(kp.e.collideKernel));
     return k;
 }
 
@@ -125,7 +140,8 @@ extern "C" int nwAutotuneFused(float *pos, float *vel, float *force, float *forc
         NT >= (1ull << 31) || (numSolvent && Cs == 0))
         return 0;
     if (reps == 0) reps = 5;
-    const std::string file = cache_file(cachePath), dev = device_key(), size = size_key(N, C, n, numSolvent, Cs);
+    const std::string file = cache_file(cachePath), dev = device_key() + physics_key(kp),
+                      size = size_key(N, C, n, numSolvent, Cs);
     NWTuning best{};
     if (useCache && !file.empty() && cache_lookup(file, dev, size, best)) {
         nwSetTuning(&best);

@@ -1,7 +1,8 @@
 """The autotuner against the launches of small systems: the built-in choice
 does cell order and pairs, or the front and the sort's first level, in one
 launch, which a knob asked for takes apart.  The tuner must see all that a
-candidate costs: its pick keeps the launches that are some 40 % faster."""
+candidate costs (its pick keeps the launches that are some 40 % faster), and a
+stored choice holds for its own physics and kernels alone."""
 import ctypes
 
 import numpy as np
@@ -67,3 +68,18 @@ def test_pick_keeps_the_faster_launches(lib, dem, families, expected):
     assert rc == 1
     assert launches(lib, p, d, families) == expected, pick
 
+
+def test_stored_choice_is_of_its_physics_and_kernels(lib, tmp_path):
+    cache = tmp_path / "t.txt"
+    p, d = system(lib)
+    assert tune(lib, p, d, str(cache).encode())[0] == 1
+    device, size, values = cache.read_text().splitlines()[0].split("\t")
+    assert tune(lib, p, d, str(cache).encode())[0] == 2
+    # the same sizes with the extensile term
+    p, d = system(lib, activity=2.0)
+    assert tune(lib, p, d, str(cache).encode())[0] == 1
+    # a line as stored before the kernels were numbered
+    old = tmp_path / "old.txt"
+    old.write_text("\t".join((device.split("/k")[0], size, "4096 512 0 0 256 256 0")) + "\n")
+    p, d = system(lib)
+    assert tune(lib, p, d, str(old).encode())[0] == 1
