@@ -650,7 +650,10 @@ static bool fused_md(const KP &kp, float *pos, float *vel, float *force, float *
     uint32_t frontBlock = 0;
     // (the fixed scratch is carved for the sort's own tiles)
     const bool frontTiles = !oneLaunch && !fixed && front_tiles_plan(numFilaments, n, bp, frontBlock);
-    if (!fixed) NW_HIP_R(ensure_bucket_scratch(s.bucket, bp), false);
+    if (!fixed) {
+        NW_HIP_R(ensure_bucket_scratch(s.bucket, bp), false);
+        if (oneLaunch) NW_HIP_R(ensure_rows_scratch(s.bucket, N), false);
+    }
     BucketScratch base = fixed ? *fixed : s.bucket;
     BucketScratch sc = base;
     if (offOut) sc.off = offOut;
@@ -690,7 +693,7 @@ static bool fused_md(const KP &kp, float *pos, float *vel, float *force, float *
         // a small system: the cell order and the pair forces in one launch
         TimedScope ts(fixed ? noTimer : "md_collide", s.stream, true);
         NW_HIP_R(launch_rows(rows, a.hash, a.wormRows, a.pos, swapForces ? a.forceOld : a.force, gridParticleIndex, sc.off,
-                             sc.sortedCell, reinterpret_cast<float4 *>(sortedPos), uint32_t(N), kp, s.stream), false);
+                             sc.sortedCell, reinterpret_cast<float4 *>(sortedPos), base.spill, uint32_t(N), kp, s.stream), false);
         s.lastHashPtr = nullptr;
         return true;
     }
@@ -766,12 +769,16 @@ void nwFusedMdStepNoAlloc(float *pos, float *vel, float *force, float *forceOld,
                "nwFusedMdStepNoAlloc: %llu beads over %llu cells", (unsigned long long)N, (unsigned long long)cells);
     // the sort's arrays carved from the scratch, 256-byte aligned: the cell
     // of every bead (unless the caller takes it), the packed pairs, the tile
-    // x bucket prefix matrix, the cell of every sorted slot, the CSR offsets
+    // x bucket prefix matrix, the cell of every sorted slot, the CSR offsets,
+    // and for the one-launch order and pairs (some 14 MiB in all at its largest)
+    // its crowded rows
+    RowsPlan rows;
+    const uint64_t spill = rows_plan(N, kp, rows) ? 4 * N : 0;
     const BucketPlan bp = fused_plan(N, cells, false);
     NW_REQUIRE(!*bucket_plan_problem(bp), "nwFusedMdStepNoAlloc: %s", bucket_plan_problem(bp));
     auto words = [](uint64_t n) { return (n * 4 + 255) & ~uint64_t(255); };
     const uint64_t need = (gridParticleHash ? 0 : words(N)) + words(uint64_t(bp.tiles) * bp.tileItems) +
-                          words(uint64_t(bp.tiles) * (bp.buckets + 1)) + words(N) + words(cells + 2);
+                          words(uint64_t(bp.tiles) * (bp.buckets + 1)) + words(N) + words(cells + 2) + words(spill);
     NW_REQUIRE(need <= kNoAllocScratchBytes,
                "nwFusedMdStepNoAlloc: %llu beads over %llu cells need %llu bytes of scratch; the fixed scratch "
                "array holds %llu (use nwFusedMdStep)",
@@ -789,6 +796,7 @@ void nwFusedMdStepNoAlloc(float *pos, float *vel, float *force, float *forceOld,
     sc.P = take(uint64_t(bp.tiles) * (bp.buckets + 1));
     sc.sortedCell = take(N);
     sc.off = take(cells + 2);
+    if (spill) sc.spill = take(spill);
     (void)fused_md(kp, pos, vel, force, forceOld, tangent, gridParticleHash, gridParticleIndex, sortedPos, sortedVel,
                    sortedTangent, deltaTime, langevinGamma, langevinKbT, langevin, numFilaments, nullptr, nullptr,
                    nullptr, nullptr, false, &sc);
@@ -1074,6 +1082,7 @@ void nwBatchSetReplicas(const NWReplicaParams *reps, uint numReplicas) {
         NW_REQUIRE(!*why, "nwBatchSetReplicas: %s", why);
         b.sortDev = reinterpret_cast<SortRep *>(b.table + sortAt);
         NW_HIP(ensure_batch_sort_scratch(b.scratch, b.sortPlan));
+        if (b.rows.blocks) NW_HIP(ensure_rows_scratch(b.scratch, N));
     }
 }
 
@@ -1138,6 +1147,7 @@ void nwBatchMdStep(float *pos, float *vel, float *force, float *forceOld, float 
     a.swapForces = b.swap ? 1 : 0;
     a.hash = b.scratch.hash;
     a.wormRows = b.rows.blocks ? b.scratch.pairs : nullptr;  // the sort's, which is not launched
+    a.spill = b.scratch.spill;
     a.ids = gridParticleIndex;
     a.off = b.scratch.off;
     a.sCell = b.scratch.sortedCell;
@@ -1726,6 +1736,7 @@ void nwBatchAdjointForward(float *pos, float *vel, float *force, float *forceOld
     a.forceOld = reinterpret_cast<float4 *>(forceOld);
     a.hash = A.hash;
     a.wormRows = b.rows.blocks ? b.scratch.pairs : nullptr;
+    a.spill = b.scratch.spill;
     a.sCell = A.sCell;
     // the step velocities are read only for the Langevin partials
     const bool lgv = batch_langevin(b);
@@ -1821,6 +1832,7 @@ void nwBatchAdjointBackward(const float *dLdPos, const float *dLdVel, double *gr
             a.forceOld = G;
             a.hash = A.hash;
             a.wormRows = b.rows.blocks ? b.scratch.pairs : nullptr;
+            a.spill = b.scratch.spill;
             a.ids = A.segIds + uint64_t(j) * N;
             a.off = A.segOff + uint64_t(j) * (C + 2);
             a.sCell = A.sCell;

@@ -36,6 +36,7 @@ struct RowsArgs {
     float4 *force;
     uint32_t *ids, *off, *sCell;
     float4 *sPos;
+    uint32_t *spill;        // scratch, four words a bead
 };
 
 // LDS of a workgroup (bytes): staged beads `cap`, cells of its rows and the two beside them
@@ -66,58 +67,6 @@ __device__ __forceinline__ void row_pieces(uint32_t x, uint32_t Gx, uint32_t &a0
     a1 = left || right ? Gx : x + 2u;
     b0 = 0u;
     b1 = left ? 2u : (right ? 1u : 0u);
-}
-
-// A stage too small for the rows' beads by the two rows beside the own
-// ones alone (a collapsed or exploded system; see rows_cap): every lane takes a cell, then a bead, and passes over all cells of
-// the system in bead order.  Slow and exact.  (LDS holds the counts of the rows' cells only.)
-__device__ __forceinline__ void rows_unstaged(const KP &kp, const RowsArgs &a, uint32_t N, uint32_t idBase,
-                                           uint32_t cellBase, uint32_t slotBase, uint32_t y0, uint32_t own,
-                                           const uint32_t *cnt) {
-    const uint32_t Gx = kp.p.gridSize.x, Gy = kp.p.gridSize.y;
-    const uint32_t first = cnt[Gx];
-    for (uint32_t c = threadIdx.x; c < own * Gx; c += blockDim.x) {
-        const uint32_t cell = cellBase + y0 * Gx + c;
-        uint32_t w = slotBase + cnt[Gx + c] - first;
-        const uint32_t e = slotBase + cnt[Gx + c + 1u] - first;
-        for (uint32_t j = 0; j < N && w < e; ++j) {
-            if (a.hash[j] != cell) continue;
-            a.ids[w] = idBase + j;
-            a.sCell[w] = cell;
-            a.sPos[w] = load4(a.pos, j);
-            ++w;
-        }
-    }
-    __syncthreads();
-    const float rc2 = kp.e.wcaCutoff * kp.e.wcaCutoff;
-    const uint32_t beads = cnt[(own + 1u) * Gx] - first;
-    for (uint32_t s = threadIdx.x; s < beads; s += blockDim.x) {
-        const uint32_t me = a.ids[slotBase + s] - idBase;
-        int gx, gy, gz;
-        cell_xyz(kp, a.sCell[slotBase + s] - cellBase, gx, gy, gz);
-        const f3 r = mk(load4(a.pos, me));
-        uint32_t fil, ch;
-        worm_of(kp, me, fil, ch);
-        f3 acc = mk(0.f, 0.f, 0.f);
-        for (int yi = -1; yi <= 1; ++yi) {
-            const uint32_t y = uint32_t(gy + yi < 0 ? int(Gy) - 1 : (gy + yi == int(Gy) ? 0 : gy + yi));
-            uint32_t lo, hi, b0, b1;
-            row_pieces(uint32_t(gx), Gx, lo, hi, b0, b1);
-            for (uint32_t k = 0; k < 3u; ++k) {
-                const uint32_t cell = cellBase + y * Gx + (lo + k < hi ? lo + k : b0 + k - (hi - lo));
-                for (uint32_t j = 0; j < N; ++j) {
-                    if (a.hash[j] != cell) continue;
-                    uint32_t fil2, ch2;
-                    worm_of(kp, j, fil2, ch2);
-                    float4 P = load4(a.pos, j);
-                    P.w = __uint_as_float(fil2);
-                    acc += wca_term_masked(kp, r, fil, rc2, P);
-                }
-            }
-        }
-        const float4 F = load4(a.force, me);
-        a.force[me] = make_float4(F.x + acc.x, F.y + acc.y, F.z + acc.z, F.w + 0.0f);
-    }
 }
 
 // own beads above which a bead takes one lane instead of four: 229,000 beads
@@ -186,33 +135,68 @@ __device__ __forceinline__ void rows_pairs(const KP &kp, const RowsArgs &a, cons
     }
 }
 
-// More beads than the stage holds, but not in the two rows beside the own
-// ones: the own beads in their slots of `ids`, already there in ascending id
-// per cell, the others' ids in lid (staged slots without the own ones').
-__device__ __forceinline__ void rows_own_in_memory(const KP &kp, const RowsArgs &a, uint32_t idBase,
-                                                   uint32_t cellBase, uint32_t slot0, uint32_t y0, uint32_t s0,
-                                                   uint32_t s1, const uint32_t *cnt, const uint32_t *lid) {
-    const uint32_t Gx = kp.p.gridSize.x;
+// More beads than the stage holds (worms crowded into a few rows): the staged
+// beads' lists in memory.  The own ones stand at their slots, as they arrive in
+// sCell and in ascending id per cell in ids; those of the rows below and above
+// in a.spill, N words each for arrival and order, at the slots that their rows
+// have in the system: a row is below the rows of one workgroup alone, and above
+// those of one, so no two workgroups meet there.
+// A bead counts its own rank among the ids of its cell, so a cell takes the
+// square of its beads over the threads, not one thread's insertion sort (a
+// system collapsed into few cells).  Twelve rows of 5,000 beads: a step 0.65 ms,
+// by the sort and the pair kernel 0.26, by passes over all beads 320; 4,000
+// beads in a cell or two 4.4 ms, by insertion 158.  What bounds it is that the
+// crowded rows' few workgroups do all the work.
+template <typename BeadOf, typename Local>
+__device__ __forceinline__ void rows_in_memory(const KP &kp, const RowsArgs &a, uint32_t N, uint32_t idBase,
+                                               uint32_t cellBase, uint32_t slot0, uint32_t y0, uint32_t own,
+                                               const uint32_t *cnt, uint32_t *cur, uint32_t words,
+                                               const BeadOf &bead_of, const Local &local) {
+    const uint32_t Gx = kp.p.gridSize.x, Gy = kp.p.gridSize.y, nc = (own + 2u) * Gx;
+    const uint32_t s0 = cnt[Gx], s1 = cnt[(own + 1u) * Gx], m = cnt[nc];
+    // of a staged slot u: below u < s0, own, above u >= s1
+    uint32_t *const lo = a.spill + (y0 == 0u ? N - s0 : slot0 - s0);
+    uint32_t *const hi = a.spill + 2u * uint64_t(N) + (y0 + own == Gy ? 0u : slot0 + (s1 - s0));
+    auto raw = [&](uint32_t u) { return u < s0 ? lo + u : (u < s1 ? a.sCell + slot0 + (u - s0) : hi + (u - s1)); };
+    auto fin = [&](uint32_t u) { return u < s0 ? lo + N + u : (u < s1 ? a.ids + slot0 + (u - s0) : hi + N + (u - s1)); };
+    for (uint32_t k = threadIdx.x; k < words; k += blockDim.x) {
+        const uint32_t id = bead_of(k), d = local(a.hash[id] - cellBase);
+        if (d < nc) *raw(atomicAdd(&cur[d], 1u)) = id;
+    }
+    __syncthreads();
+    for (uint32_t s = threadIdx.x; s < m; s += blockDim.x) {
+        const uint32_t id = *raw(s), d = local(a.hash[id] - cellBase);
+        const uint32_t c0 = cnt[d], z = cnt[d + 1u] - c0;
+        const uint32_t *cell = raw(c0);
+        uint32_t r = c0;
+#pragma unroll 4
+        for (uint32_t u = 0; u < z; ++u) r += cell[u] < id ? 1u : 0u;
+        *fin(r) = s >= s0 && s < s1 ? idBase + id : id;
+    }
+    __syncthreads();
     const float rc2 = kp.e.wcaCutoff * kp.e.wcaCutoff;
-    const uint32_t *own = a.ids + slot0;
     for (uint32_t s = s0 + threadIdx.x; s < s1; s += blockDim.x) {
-        const uint32_t me = own[s - s0] - idBase, cell = a.hash[me];
+        const uint32_t me = a.ids[slot0 + (s - s0)] - idBase, cell = a.hash[me];
         const float4 R = load4(a.pos, me);
         a.sCell[slot0 + (s - s0)] = cell;
         a.sPos[slot0 + (s - s0)] = R;
         int gx, gy, gz;
         cell_xyz(kp, cell - cellBase, gx, gy, gz);
         const f3 r = mk(R);
-        uint32_t fil, ch, lo, hi, b0, b1;
+        uint32_t fil, ch, x0, x1, b0, b1;
         worm_of(kp, me, fil, ch);
-        row_pieces(uint32_t(gx), Gx, lo, hi, b0, b1);
+        row_pieces(uint32_t(gx), Gx, x0, x1, b0, b1);
         f3 acc = mk(0.f, 0.f, 0.f);
         for (uint32_t yi = 0; yi < 3u; ++yi) {
-            const uint32_t row = (uint32_t(gy) - y0 + yi) * Gx;  // staged: the one below the own rows first
+            const uint32_t y = uint32_t(gy) - y0 + yi, row = y * Gx;  // staged: the one below the own rows first
+            const bool mine = y >= 1u && y <= own;
+            const uint32_t *ids = y == 0u ? lo + N : (mine ? a.ids + slot0 - s0 : hi + N - s1);
+            const uint32_t base = mine ? idBase : 0u;
             for (uint32_t k = 0; k < 3u; ++k) {
-                const uint32_t d = row + (lo + k < hi ? lo + k : b0 + k - (hi - lo));
+                const uint32_t d = row + (x0 + k < x1 ? x0 + k : b0 + k - (x1 - x0));
+#pragma unroll 2
                 for (uint32_t u = cnt[d], z = cnt[d + 1u]; u < z; ++u) {
-                    const uint32_t j = u < s0 ? lid[u] : (u < s1 ? own[u - s0] - idBase : lid[u - (s1 - s0)]);
+                    const uint32_t j = ids[u] - base;
                     uint32_t fil2, ch2;
                     worm_of(kp, j, fil2, ch2);
                     float4 P = load4(a.pos, j);
@@ -328,31 +312,7 @@ __device__ __forceinline__ void rows_body(const KP &kp, const RowsArgs &a, uint3
     for (uint32_t c = t; c < own * Gx; c += T) a.off[hOwn + c] = slotBase + cnt[Gx + c] - s0;
     if (y0 + own == Gy && t == 0) a.off[C] = slotAdd + N;
     if (m > cap) {
-        const uint32_t slot0 = slotBase - slotAdd, owned = s1 - s0;
-        if (m - owned > cap) {
-            rows_unstaged(kp, a, N, idBase, cellBase, slot0, y0, own, cnt);
-            return;
-        }
-        for (uint32_t k = t; k < words; k += T) {
-            const uint32_t id = bead_of(k), d = local(a.hash[id] - cellBase);
-            if (d >= nc) continue;
-            const uint32_t s = atomicAdd(&cur[d], 1u);
-            if (s >= s0 && s < s1) a.ids[slot0 + (s - s0)] = idBase + id;
-            else lid[s < s0 ? s : s - owned] = id;
-        }
-        __syncthreads();
-        for (uint32_t c = t; c < nc; c += T) {
-            const uint32_t u0 = cnt[c], z = cnt[c + 1u] - u0;
-            uint32_t *cell = c >= Gx && c < (own + 1u) * Gx ? a.ids + slot0 + (u0 - s0) : lid + (u0 < s1 ? u0 : u0 - owned);
-            for (uint32_t u = 1; u < z; ++u) {
-                const uint32_t x = cell[u];
-                uint32_t w = u;
-                for (; w > 0u && cell[w - 1u] > x; --w) cell[w] = cell[w - 1u];
-                cell[w] = x;
-            }
-        }
-        __syncthreads();
-        rows_own_in_memory(kp, a, idBase, cellBase, slot0, y0, s0, s1, cnt, lid);
+        rows_in_memory(kp, a, N, idBase, cellBase, slotBase - slotAdd, y0, own, cnt, cur, words, bead_of, local);
         return;
     }
     auto place = [&](uint32_t id, uint32_t d) {
@@ -421,7 +381,7 @@ __global__ __launch_bounds__(kRowsBlock) void k_rows_batch(BatchArrays a, const 
     const BatchRep &rep = reps[__builtin_amdgcn_readfirstlane(replica_of_row_block(reps, R, b))];
     const uint32_t b0 = rep.beadOffset, c0 = rep.cellOffset;
     const RowsArgs x{a.hash + b0, a.wormRows + b0, a.pos + b0, (a.swapForces ? a.forceOld : a.force) + b0, a.ids + b0,
-                     a.off + c0,     a.sCell + b0, a.sPos + b0};
+                     a.off + c0,     a.sCell + b0, a.sPos + b0, a.spill + 4u * uint64_t(b0)};
     rows_body<kRowsBlock>(rep.kp, x, rep.numBeads, b0, c0, b0, (b - rep.rowBlock) * rep.rows, rep.rows, cap, maxCells,
                           smem);
 }
@@ -536,8 +496,8 @@ hipError_t launch_rows_batch(const RowsPlan &pl, const BatchArrays &a, const Bat
 }
 
 hipError_t launch_rows(const RowsPlan &pl, const uint32_t *hash, const uint32_t *wormRows, const float4 *pos, float4 *force, uint32_t *ids,
-                       uint32_t *off, uint32_t *sCell, float4 *sPos, uint32_t N, const KP &kp, hipStream_t st) {
-    const RowsArgs a{hash, wormRows, pos, force, ids, off, sCell, sPos};
+                       uint32_t *off, uint32_t *sCell, float4 *sPos, uint32_t *spill, uint32_t N, const KP &kp, hipStream_t st) {
+    const RowsArgs a{hash, wormRows, pos, force, ids, off, sCell, sPos, spill};
     const hipError_t e = grant_lds(reinterpret_cast<const void *>(&k_rows), pl.lds);
     if (e != hipSuccess) return e;
     NW_LAUNCH(k_rows, dim3(pl.blocks), dim3(kRowsBlock), pl.lds, st, a, N, pl.rows, pl.cap, pl.cells, kp);
