@@ -22,6 +22,7 @@
 
 #include "nw_bucket.hpp"
 #include "nw_pair.hpp"
+#include "nw_rules.hpp"
 
 namespace nw {
 
@@ -412,13 +413,17 @@ static bool rows_term(const KP &kp) {
 }
 
 // Beads staged by a workgroup of `rows` rows: two and a half times the
-// average, and as far as `lds` bytes hold them the close packing of the rows'
-// cells (1.45 beads a cell of the WCA range): worms that gather in bands, or
-// start on a lattice in a part of the box, stay within the stage.
-static uint32_t rows_cap(uint64_t N, uint32_t Gx, uint32_t Gy, uint32_t rows, uint32_t lds) {
+// average, and as far as `lds` bytes hold them the packing of the rows' cells:
+// worms that gather in bands, or start on a lattice in a part of the box, stay
+// within the stage (200,000 beads in four tenths of their box, 1.75 a cell: a
+// step 75 us, with the packing of single beads, 1.45 a cell, 133).
+static uint32_t rows_cap(uint64_t N, const KP &kp, uint32_t rows, uint32_t lds) {
+    const uint32_t Gx = kp.p.gridSize.x, Gy = kp.p.gridSize.y;
     const uint32_t cells = (rows + 2u) * Gx, fixed = rows_layout(0, cells).total;
     const uint32_t mean = (uint32_t(2.5 * double(N) / Gy * (rows + 2u)) + 255u) & ~255u;
-    const uint32_t packed = (uint32_t(1.45 * cells) + 255u) & ~255u;
+    const double perCell = worms_packed(double(kp.p.cellSize.x) * kp.p.cellSize.y, kp.e.wcaSigma,
+                                        kp.p.filamentSize > 1 ? kp.p.bondSpringL : kp.e.wcaSigma);
+    const uint32_t packed = (uint32_t(perCell * cells) + 255u) & ~255u;
     const uint32_t room = lds > fixed ? std::min((lds - fixed) / 22u & ~255u, 8192u) : 0u;
     return std::max({1024u, mean, std::min(packed, room)});
 }
@@ -444,7 +449,7 @@ bool rows_plan(uint64_t N, const KP &kp, RowsPlan &out) {
     out.blocks = (Gy + out.rows - 1u) / out.rows;
     if (double(N) / Gy * out.rows > double(kRowsMaxOwn)) return false;
     out.cells = (out.rows + 2u) * Gx;
-    out.cap = rows_cap(N, Gx, Gy, out.rows, kRowsLds);
+    out.cap = rows_cap(N, kp, out.rows, kRowsLds);
     return rows_fits(out);
 }
 
@@ -480,7 +485,7 @@ bool rows_plan_batch(BatchRep *reps, uint32_t R, RowsPlan &out) {
         const uint32_t blocks = (Gy + q.rows - 1u) / q.rows;
         pl.blocks += blocks;
         pl.cells = std::max(pl.cells, (q.rows + 2u) * Gx);
-        pl.cap = std::max(pl.cap, rows_cap(q.numBeads, Gx, Gy, q.rows, kRowsLdsHalf));
+        pl.cap = std::max(pl.cap, rows_cap(q.numBeads, q.kp, q.rows, kRowsLdsHalf));
     }
     if (!pl.blocks || beads > kRowsMaxBatchBeads || !rows_fits(pl)) return false;
     out = pl;
