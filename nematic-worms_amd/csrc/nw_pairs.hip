@@ -15,6 +15,7 @@
 // square roots and quotients.
 #include "nw_internal.hpp"
 #include "nw_pair.hpp"
+#include "nw_rules.hpp"
 
 namespace nw {
 
@@ -25,7 +26,11 @@ struct PairCells {
     const uint32_t *start, *end;
 };
 
-constexpr uint32_t kListCap = 64;  // a bead's candidates listed at a time (more: further rounds)
+// A bead's candidates listed at a time (more: further rounds).  With two lanes
+// a bead a workgroup holds 128 lists, and their length sets how many
+// workgroups fit a CU's LDS (1 million soft spheres in one layer, in rows: 54
+// us with 32 entries, 43 with 24).
+constexpr uint32_t list_cap(int lanes) { return lanes <= 2 ? 24u : 64u; }
 
 // exclusive prefix sum of v over the S lanes of a group, and its total
 template <int S>
@@ -48,6 +53,7 @@ __global__ __launch_bounds__(kBlock) void k_pair_list(float4 *__restrict__ force
                                                       const uint32_t *__restrict__ sIdx, PairCells cells,
                                                       const uint32_t *__restrict__ sCell, uint32_t n, KP kp) {
     constexpr uint32_t G = kBlock / S;           // beads of a workgroup
+    constexpr uint32_t kListCap = list_cap(S);
     constexpr uint32_t PER = (CELLS + S - 1) / S;  // cells of a lane
     __shared__ uint32_t list[G][kListCap];
     __shared__ float listW[UNIT ? 1 : G][UNIT ? 1 : kListCap];
@@ -158,13 +164,6 @@ __global__ __launch_bounds__(kBlock) void k_pair_list(float4 *__restrict__ force
     }
 }
 
-// Lanes a bead: 8 while that fills the chip, 4 beyond, where the lanes' lookups
-// and sums are work (through the tables, us with 8 / 4 / 2 lanes): 27 cells, 96,000
-// beads of the soft spheres 27 / 29 / 41, 800,000 160 / 152 / 200, WCA in three
-// dimensions 110 / 93 / 135; 9 cells, 10,000 WCA beads 6.7 with 8, 800,000 70 / 52 /
-// 74; soft spheres in one layer, 800,000, 100 / 115 / 170: 8 throughout.
-constexpr uint32_t kPairFewBeads = 200000;
-
 template <bool CSR, int S, int CELLS>
 static void launch_list_of(float4 *force, const float4 *sPos, const float4 *sVel, const float4 *sTan,
                            const uint32_t *sIdx, const PairCells &c, const uint32_t *sCell, uint32_t n, const KP &kp,
@@ -194,13 +193,14 @@ static hipError_t launch_list(float4 *force, const float4 *sPos, const float4 *s
                               const uint32_t *sIdx, const PairCells &c, const uint32_t *sCell, uint32_t n,
                               const KP &kp, hipStream_t st) {
     if (n == 0) return hipSuccess;
-    const bool few = n <= kPairFewBeads, oneLayer = kp.e.stencil == NW_STENCIL_2D || kp.p.gridSize.z == 1;
+    const bool oneLayer = kp.e.stencil == NW_STENCIL_2D || kp.p.gridSize.z == 1;
+    const int lanes = pair_lanes(n, oneLayer);
 #define NW_LIST_OF(S, CELLS) launch_list_of<CSR, S, CELLS>(force, sPos, sVel, sTan, sIdx, c, sCell, n, kp, st)
     if (oneLayer) {
-        if (few || kp.e.pairPotential != NW_PAIR_WCA) NW_LIST_OF(8, 9);
-        else NW_LIST_OF(4, 9);
+        if (lanes == 8) NW_LIST_OF(8, 9);
+        else NW_LIST_OF(2, 9);
     } else {
-        if (few) NW_LIST_OF(8, 27);
+        if (lanes == 8) NW_LIST_OF(8, 27);
         else NW_LIST_OF(4, 27);
     }
 #undef NW_LIST_OF

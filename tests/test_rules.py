@@ -11,6 +11,7 @@ D, U32, U64 = ctypes.c_double, ctypes.c_uint32, ctypes.c_uint64
 C = """#include "nw_rules.hpp"
 extern "C" {
 double packed(double area, double sigma, double bond) { return nw::worms_packed(area, sigma, bond); }
+int lanes(uint64_t beads, int oneLayer) { return nw::pair_lanes(beads, oneLayer != 0); }
 }
 """
 
@@ -23,6 +24,7 @@ def rules(tmp_path_factory):
                     str(d / "r.cpp"), "-o", str(d / "r.so")], check=True)
     lib = ctypes.CDLL(str(d / "r.so"))
     lib.packed.restype, lib.packed.argtypes = D, [D, D, D]
+    lib.lanes.argtypes = [U64, ctypes.c_int]
     return lib
 
 
@@ -48,3 +50,8 @@ def test_packing_limits(rules):
     assert rules.packed(1.2599, 1.0, 1.0) == pytest.approx(1.455, rel=1e-3)  # hexagonal, a cell of the WCA range
     assert rules.packed(1.44, 1.0, 0.8) > 1.75  # bonds of 0.8 sigma: a band of 1.75 a cell stays in the stage
     assert rules.packed(1.44, 0.0, 0.8) == 16.0 and rules.packed(1.44, 1.0, 0.0) <= 16.0
+
+
+@pytest.mark.parametrize("beads,layer,layers", [(1, 8, 8), (200_000, 8, 8), (200_001, 2, 4), (1 << 31, 2, 4)])
+def test_lanes_of_the_pair_list(rules, beads, layer, layers):
+    assert (rules.lanes(beads, 1), rules.lanes(beads, 0)) == (layer, layers)
