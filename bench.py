@@ -104,8 +104,10 @@ def dispatched_kernel(family, w):
         # the smaller stage where twice the average bucket fits it
         return "k_md_cells<1, 256, 1024>" if 2 * w["N"] <= 1024 * w["md_plan"][1] else "k_md_cells<1, 512, 2048>"
     if family == "srdf_cells":
-        # the larger sorting network above seven particles a cell
-        return f"k_srd_cells<256, {32 if w['NT'] > 7 * w['Cs'] else 16}>"
+        # the larger sorting network for cells of middling density, places behind the scan in dense ones
+        lo, hi = (7, 26) if w["srd_plan"][1] <= 1024 else (9, 21 if w["srd_plan"][1] > 2048 else 0)
+        per = w["NT"] / w["Cs"]
+        return f"k_srd_cells<256, {32 if lo < per <= hi else 16}, {'true' if per > 12 else 'false'}>"
     if family == "md_tiles":
         items = w["md_plan"][2]
         shapes = {1024: "4, 256", 2048: "8, 256", 4096: "4, 1024", 8192: "8, 1024", 16384: "16, 1024"}

@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "nw_bucket.hpp"
+#include "nw_rules.hpp"
 #include "nw_physics.hpp"
 
 namespace nw {
@@ -790,8 +791,9 @@ __device__ __forceinline__ void md_cells_body(const CellsArgs &o, const BucketPl
     }
 }
 
-// SRD, bucket b; staged as the MD sort's
-template <int BLOCK, int NET, int CAP = int(kBucketCap)>
+// SRD, bucket b; staged as the MD sort's.  LATE: a member takes its place in a
+// pass of its own behind the scan, not from the count (srd_late).
+template <int BLOCK, int NET, bool LATE, int CAP = int(kBucketCap)>
 __device__ __forceinline__ void srd_cells_body(const CellsArgs &o, const BucketPlan &bp, uint32_t b,
                                                   unsigned char *smem) {
     constexpr int PER = CAP / BLOCK;
@@ -835,8 +837,12 @@ __device__ __forceinline__ void srd_cells_body(const CellsArgs &o, const BucketP
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
             const uint32_t k = tid + uint32_t(j) * BLOCK;
-            // its place in the cell's run of arrivals beside the cell (both below 2^11)
-            if (k < m) q[j].x |= atomicAdd(&cnt[q[j].x], 1u) << 16;
+            if (LATE) {
+                if (k < m) atomicAdd(&cnt[q[j].x], 1u);
+            } else {
+                // its place in the cell's run of arrivals beside the cell (both below 2^11)
+                if (k < m) q[j].x |= atomicAdd(&cnt[q[j].x], 1u) << 16;
+            }
         }
     } else if (!staged) {
         for (uint32_t k = tid; k < m; k += bd) {
@@ -845,7 +851,7 @@ __device__ __forceinline__ void srd_cells_body(const CellsArgs &o, const BucketP
         }
     }
     __syncthreads();
-    if (staged) scan_cells<BLOCK>(cnt, nc, m, wsum);
+    if (staged && !LATE) scan_cells<BLOCK>(cnt, nc, m, wsum);
     else block_excl_scan<true>(cnt, nc, wsum, cur);
 
     uint32_t *out = o.ids + sb;
@@ -853,9 +859,7 @@ __device__ __forceinline__ void srd_cells_body(const CellsArgs &o, const BucketP
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
             const uint32_t k = tid + uint32_t(j) * BLOCK;
-            if (k < m) {
-                lid[cnt[q[j].x & 0xffffu] + (q[j].x >> 16)] = q[j].y;
-            }
+            if (k < m) lid[LATE ? atomicAdd(&cur[q[j].x], 1u) : cnt[q[j].x & 0xffffu] + (q[j].x >> 16)] = q[j].y;
         }
     } else {
         for (uint32_t k = tid; k < m; k += bd) {
@@ -882,8 +886,8 @@ __device__ __forceinline__ void srd_cells_body(const CellsArgs &o, const BucketP
         }
     }
     // every cell in ascending id order; CSR offsets.  SRD cells hold ~6
-    // particles (a network of 16 takes all but the rare crowded ones).  The
-    // two storages take separate calls so that the staged ids are read as
+    // particles (a network of 16 takes all but the rare crowded ones; denser
+    // solvents: srd_network).  The two storages take separate calls so that the staged ids are read as
     // LDS, not through a generic pointer.
     for (uint32_t c = tid; c < nc; c += bd) {
         const uint32_t a = cnt[c], z = cnt[c + 1];
@@ -928,10 +932,10 @@ __device__ __forceinline__ void srd_cells_body(const CellsArgs &o, const BucketP
     }
 }
 
-template <int BLOCK, int NET>
+template <int BLOCK, int NET, bool LATE>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(NET > 16 ? 4 : 8, 8))) void k_srd_cells(CellsArgs o, BucketPlan bp) {
     extern __shared__ __align__(16) unsigned char smem[];
-    srd_cells_body<BLOCK, NET>(o, bp, xcd_contiguous(blockIdx.x, gridDim.x), smem);
+    srd_cells_body<BLOCK, NET, LATE>(o, bp, xcd_contiguous(blockIdx.x, gridDim.x), smem);
 }
 
 template <int GATHER, int BLOCK, int CAP>
@@ -1430,16 +1434,20 @@ hipError_t launch_md_cells(const BucketPlan &bp, BucketScratch &s, uint32_t *ids
 }
 
 // The network takes a cell whose ids fit it, the sums load half as many
-// velocities together: 32 and 16 where cells hold more than seven particles on
-// average (a million particles of ten a cell in random order: 28.3 us, with 16
-// and 8 30.4: above sixteen the sort is by insertion, and every four velocities
-// past the first batch are another round trip).
+// velocities together (the rules: nw_rules.hpp)
 static hipError_t launch_srd_buckets(const CellsArgs &o, const BucketPlan &bp, hipStream_t st) {
     const CellsLayout L = cells_layout(bp, true);
-    if (uint64_t(bp.n) > 7u * uint64_t(bp.cells))
-        NW_LAUNCH((k_srd_cells<kSrdCellsBlock, 32>), dim3(bp.buckets), dim3(kSrdCellsBlock), L.total, st, o, bp);
-    else
-        NW_LAUNCH((k_srd_cells<kSrdCellsBlock, 16>), dim3(bp.buckets), dim3(kSrdCellsBlock), L.total, st, o, bp);
+#define NW_SRD_CELLS(NET, LATE) \
+    NW_LAUNCH((k_srd_cells<kSrdCellsBlock, NET, LATE>), dim3(bp.buckets), dim3(kSrdCellsBlock), L.total, st, o, bp)
+    const bool late = srd_late(bp.n, bp.cells);
+    if (srd_network(bp.n, bp.cells, bp.buckets) == 32) {
+        if (late) NW_SRD_CELLS(32, true);
+        else NW_SRD_CELLS(32, false);
+    } else {
+        if (late) NW_SRD_CELLS(16, true);
+        else NW_SRD_CELLS(16, false);
+    }
+#undef NW_SRD_CELLS
     return hipGetLastError();
 }
 

@@ -11,6 +11,8 @@ D, U32, U64 = ctypes.c_double, ctypes.c_uint32, ctypes.c_uint64
 C = """#include "nw_rules.hpp"
 extern "C" {
 double packed(double area, double sigma, double bond) { return nw::worms_packed(area, sigma, bond); }
+int network(uint64_t n, uint64_t cells, uint64_t buckets) { return nw::srd_network(n, cells, buckets); }
+int late(uint64_t n, uint64_t cells) { return nw::srd_late(n, cells); }
 int lanes(uint64_t beads, int oneLayer) { return nw::pair_lanes(beads, oneLayer != 0); }
 }
 """
@@ -24,6 +26,7 @@ def rules(tmp_path_factory):
                     str(d / "r.cpp"), "-o", str(d / "r.so")], check=True)
     lib = ctypes.CDLL(str(d / "r.so"))
     lib.packed.restype, lib.packed.argtypes = D, [D, D, D]
+    lib.network.argtypes, lib.late.argtypes = [U64, U64, U64], [U64, U64]
     lib.lanes.argtypes = [U64, ctypes.c_int]
     return lib
 
@@ -55,3 +58,13 @@ def test_packing_limits(rules):
 @pytest.mark.parametrize("beads,layer,layers", [(1, 8, 8), (200_000, 8, 8), (200_001, 2, 4), (1 << 31, 2, 4)])
 def test_lanes_of_the_pair_list(rules, beads, layer, layers):
     assert (rules.lanes(beads, 1), rules.lanes(beads, 0)) == (layer, layers)
+
+
+@pytest.mark.parametrize("per,buckets,network,late", [
+    (5, 700, 16, 0), (7, 700, 16, 0), (8, 700, 32, 0), (12, 1024, 32, 0), (13, 1024, 32, 1), (26, 700, 32, 1),
+    (27, 700, 16, 1), (80, 700, 16, 1),      # dense cells: by insertion, many workgroups
+    (8, 1025, 16, 0), (20, 2048, 16, 1),     # two rounds of the larger network, one of the smaller
+    (9, 2049, 16, 0), (10, 2049, 32, 0), (21, 9000, 32, 1), (22, 9000, 16, 1)])
+def test_network_of_the_srd_cells(rules, per, buckets, network, late):
+    cells = 100_000
+    assert (rules.network(per * cells, cells, buckets), rules.late(per * cells, cells)) == (network, late)
