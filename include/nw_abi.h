@@ -405,9 +405,10 @@ void nwBatchSolventLayout(uint *solventOffset, uint *srdCellOffset);
 /* `steps` nwFusedMdStep steps from (pos, vel, force, forceOld), in place,
    with the SimParams / NWExtParams of the last setParameters /
    nwSetExtParameters; the state and generator offset are checkpointed every
-   checkpointEvery steps for nwAdjointBackward, whose segment store (up to 4
-   GiB) takes the states of the last segment right away.  langevinGamma must equal
-   SimParams.gamma when langevin is on. */
+   checkpointEvery steps for nwAdjointBackward, whose segment store takes the
+   states of the last segment right away, if the store is no more than 4 GiB
+   and a quarter of the free memory; like the checkpoints it is kept for later
+   runs.  langevinGamma must equal SimParams.gamma when langevin is on. */
 void nwAdjointForward(float *pos, float *vel, float *force, float *forceOld, float *tangent, uint numFilaments,
                       float deltaTime, float langevinGamma, float langevinKbT, int langevin, uint steps,
                       uint checkpointEvery);

@@ -1232,37 +1232,87 @@ static KP collision_kp(const State::Adjoint &A, uint32_t c) {
     return kp;
 }
 
-static bool ensure_segment(State::Adjoint &A) {
-    const uint64_t N = A.N, K = A.K, NT = A.NT;
-    if (!(grow(A.segPos, A.capPos, (K + 1) * N) && grow(A.segVel, A.capVel, (K + 1) * N) &&
-          grow(A.segSPos, A.capSPos, K * N) && grow(A.segIds, A.capIds, std::max(K * N, NT)) &&
-          grow(A.segOff, A.capOff, K * (uint64_t(A.C) + 2)) && grow(A.segCell, A.capCell, K * N) &&
-          grow(A.work, A.capWork, 2 * N) && grow(A.lam, A.capLam, 4 * N + NT)))
-        return false;
-    if (!A.srd) return true;
-    // at most this many collisions in a segment of K steps
-    const uint64_t cpS = (K + A.gap - 1) / A.gap + 1;
-    return grow(A.collHash, A.capCollHash, cpS * NT) && grow(A.collIds, A.capCollIds, cpS * NT) &&
-           grow(A.collOff, A.capCollOff, cpS * (uint64_t(A.Cs) + 2)) &&
-           grow(A.collCom, A.capCollCom, cpS * A.Cs) && grow(A.cellSum, A.capCellSum, A.Cs) &&
-           grow(A.wPos, A.capWPos, NT) && grow(A.wVel, A.capWVel, NT);
+extern "C++" {
+// f(buffer, its capacity, the elements needed) for the buffers of one segment
+// and its collisions, until one of them fails
+template <typename F>
+static bool segment_buffers(State::Adjoint &A, F &&f) {
+    const uint64_t N = A.N, K = A.K, NT = A.NT, Cs = A.srd ? A.Cs : 0;
+    const uint64_t colls = A.srd ? (K + A.gap - 1) / A.gap + 1 : 0;  // at most this many in K steps
+    return f(A.segPos, A.capPos, (K + 1) * N) && f(A.segVel, A.capVel, (K + 1) * N) &&
+           f(A.segSPos, A.capSPos, K * N) && f(A.segIds, A.capIds, std::max(K * N, NT)) &&
+           f(A.segOff, A.capOff, K * (uint64_t(A.C) + 2)) && f(A.segCell, A.capCell, K * N) &&
+           f(A.work, A.capWork, 2 * N) && f(A.lam, A.capLam, 4 * N + NT) &&
+           f(A.collHash, A.capCollHash, colls * NT) && f(A.collIds, A.capCollIds, colls * NT) &&
+           f(A.collOff, A.capCollOff, colls * (Cs + 2)) && f(A.collCom, A.capCollCom, colls * Cs) &&
+           f(A.cellSum, A.capCellSum, Cs) && f(A.wPos, A.capWPos, A.srd ? NT : 0) &&
+           f(A.wVel, A.capWVel, A.srd ? NT : 0);
 }
 
-// gives the segment store back, where a forward run that would have kept its
-// last segment does not fit with it
-static void drop_segment(State::Adjoint &A) {
-    drop(A.segPos, A.capPos), drop(A.segVel, A.capVel), drop(A.segSPos, A.capSPos), drop(A.segIds, A.capIds);
-    drop(A.segOff, A.capOff), drop(A.segCell, A.capCell), drop(A.work, A.capWork), drop(A.lam, A.capLam);
-    drop(A.collHash, A.capCollHash), drop(A.collIds, A.capCollIds), drop(A.collOff, A.capCollOff);
-    drop(A.collCom, A.capCollCom), drop(A.cellSum, A.capCellSum), drop(A.wPos, A.capWPos), drop(A.wVel, A.capWVel);
+template <typename F>
+static bool segment_buffers(State::BatchAdjoint &A, F &&f) {
+    const uint64_t N = A.N, K = A.K, NT = A.NT, Cs = A.srd ? A.Cs : 0;
+    const uint64_t colls = A.srd ? (K + A.gap - 1) / A.gap + 1 : 0;
+    return f(A.segPos, A.capPos, (K + 1) * N) && f(A.segVel, A.capVel, (K + 1) * N) &&
+           f(A.segSPos, A.capSPos, K * N) && f(A.segIds, A.capIds, K * N) &&
+           f(A.segOff, A.capOff, K * (uint64_t(A.C) + 2)) && f(A.work, A.capWork, 2 * N) &&
+           f(A.lam, A.capLam, 4 * N + NT) && f(A.wPos, A.capWPos, NT) && f(A.wVel, A.capWVel, NT) &&
+           f(A.partial, A.capPartial, uint64_t(A.waves) * kAdjParams) &&
+           f(A.grad, A.capGrad, uint64_t(A.R) * kAdjParams) && f(A.collHash, A.capCollHash, colls * NT) &&
+           f(A.collIds, A.capCollIds, colls * NT) && f(A.collOff, A.capCollOff, colls * (Cs + 2)) &&
+           f(A.collCom, A.capCollCom, colls * Cs) && f(A.cellSum, A.capCellSum, Cs);
+}
+
+template <typename A>
+static bool ensure_segment(A &adj) {
+    return segment_buffers(adj, [](auto *&p, uint64_t &cap, uint64_t need) { return grow(p, cap, need); });
+}
+
+// gives the segment store back
+template <typename A>
+static void drop_segment(A &adj) {
+    (void)segment_buffers(adj, [](auto *&p, uint64_t &cap, uint64_t) { return drop(p, cap), true; });
     (void)hipGetLastError();
 }
 
 // The forward run leaves its last segment in the segment store, which the
-// backward pass then need not recompute, when the store (allocated by the
-// backward pass in any case) takes at most this much: a forward run alone does
-// not claim more.
+// backward pass then need not recompute, when the whole store (allocated by the
+// backward pass in any case, and kept until a run needs a larger one) takes at
+// most this much and no more than a quarter of the memory that is free: a
+// forward run that is never differentiated leaves the caller the rest.
 constexpr uint64_t kHoldBytes = 4ull << 30;
+
+template <typename A>
+static bool may_hold(A &adj) {
+    double bytes = 0, grown = 0;
+    (void)segment_buffers(adj, [&](auto *&p, uint64_t &cap, uint64_t need) {
+        bytes += double(need) * sizeof(*p);
+        if (need > cap) grown += double(need) * sizeof(*p);
+        return true;
+    });
+    // (so many steps that a product in the sizes could wrap are far above it)
+    if (uint64_t(adj.K) > kHoldBytes / (4u * std::max<uint64_t>(adj.N, 1u)) || bytes > double(kHoldBytes)) return false;
+    if (grown == 0) return true;
+    size_t free = 0, total = 0;
+    return hipMemGetInfo(&free, &total) == hipSuccess && grown <= double(free) / 4;
+}
+
+// Room for a forward run (room(): its own buffers, some of them in the store)
+// and, where it fits, for the segment that it leaves (hold).
+template <typename A, typename F>
+static bool forward_room(A &adj, const F &room, bool &hold) {
+    hold = false;
+    if (!room()) {
+        drop_segment(adj);  // an earlier run's store gives way
+        return room();
+    }
+    if (!may_hold(adj)) return true;
+    hold = ensure_segment(adj);
+    if (hold) return true;
+    drop_segment(adj);
+    return room();
+}
+}
 
 // The forward run of nwAdjointForward / nwAdjointForwardSrd (srd: numSolvent,
 // gap and shifts set in A by the caller, A.srd true).
@@ -1315,19 +1365,14 @@ static void adjoint_forward(float *pos, float *vel, float *force, float *forceOl
     const uint32_t nck = (steps + checkpointEvery - 1) / checkpointEvery;
     const uint64_t NT = A.NT, stride = 2 * NT + 2 * N;
     const uint64_t K = checkpointEvery;
-    const uint64_t perStep = 56 * N + 4 * C + 8 + (A.srd ? (8 * NT + 20 * uint64_t(A.Cs)) / A.gap : 0);
     A.held = -1;
-    bool hold = K <= kHoldBytes / perStep;
+    bool hold = false;
     const auto room = [&] {
         return grow(A.ckpt, A.capCkpt, uint64_t(nck) * stride) && grow(A.segSPos, A.capSPos, N) &&
                grow(A.segIds, A.capIds, NT) &&
                (!A.srd || (grow(A.collCom, A.capCollCom, A.Cs) && grow(A.collHash, A.capCollHash, NT)));
     };
-    if (hold && !(ensure_segment(A) && room())) {
-        drop_segment(A);  // no room for it: the run goes on without
-        hold = false;
-    }
-    NW_REQUIRE(room(), "nwAdjointForward: out of device memory");
+    NW_REQUIRE(forward_room(A, room, hold), "nwAdjointForward: out of device memory");
     A.ckptOffset.assign(nck, 0);
     A.lgvOff.assign(hold ? std::min<uint64_t>(K, steps) : 0, 0);
     uint64_t slots = 0;  // collisions kept
@@ -1632,31 +1677,6 @@ void nwBatchSrdStep(float *pos, float *vel, float *solventCellCOM, uint *gridPar
                               q.shift, deltaTime);
 }
 
-static bool ensure_batch_segment(State::BatchAdjoint &A) {
-    const uint64_t N = A.N, K = A.K, NT = A.NT;
-    if (!(grow(A.segPos, A.capPos, (K + 1) * N) && grow(A.segVel, A.capVel, (K + 1) * N) &&
-          grow(A.segSPos, A.capSPos, K * N) && grow(A.segIds, A.capIds, K * N) &&
-          grow(A.segOff, A.capOff, K * (uint64_t(A.C) + 2)) && grow(A.work, A.capWork, 2 * N) &&
-          grow(A.lam, A.capLam, 4 * N + NT) && grow(A.wPos, A.capWPos, NT) && grow(A.wVel, A.capWVel, NT) &&
-          grow(A.partial, A.capPartial, uint64_t(A.waves) * kAdjParams) &&
-          grow(A.grad, A.capGrad, uint64_t(A.R) * kAdjParams)))
-        return false;
-    if (!A.srd) return true;
-    const uint64_t cpS = (K + A.gap - 1) / A.gap + 1;  // collisions in a segment, at most
-    return grow(A.collHash, A.capCollHash, cpS * NT) && grow(A.collIds, A.capCollIds, cpS * NT) &&
-           grow(A.collOff, A.capCollOff, cpS * (uint64_t(A.Cs) + 2)) &&
-           grow(A.collCom, A.capCollCom, cpS * A.Cs) && grow(A.cellSum, A.capCellSum, A.Cs);
-}
-
-static void drop_batch_segment(State::BatchAdjoint &A) {
-    drop(A.segPos, A.capPos), drop(A.segVel, A.capVel), drop(A.segSPos, A.capSPos), drop(A.segIds, A.capIds);
-    drop(A.segOff, A.capOff), drop(A.work, A.capWork), drop(A.lam, A.capLam);
-    drop(A.wPos, A.capWPos), drop(A.wVel, A.capWVel), drop(A.collHash, A.capCollHash);
-    drop(A.collIds, A.capCollIds), drop(A.collOff, A.capCollOff), drop(A.collCom, A.capCollCom);
-    drop(A.cellSum, A.capCellSum);
-    (void)hipGetLastError();
-}
-
 static bool batch_langevin(const State::Batch &b) {
     bool lgv = false;
     for (const BatchRep &q : b.reps) lgv = lgv || q.langevin != 0;
@@ -1707,11 +1727,10 @@ void nwBatchAdjointForward(float *pos, float *vel, float *force, float *forceOld
     A.ctr0 = b.steps;
     const uint32_t nck = (steps + checkpointEvery - 1) / checkpointEvery;
     const uint64_t stride = 2 * NT + 2 * N;
-    // the last segment stays in the store (see kHoldBytes)
+    // the last segment stays in the store (see may_hold)
     const uint64_t K = checkpointEvery;
-    const uint64_t perStep = 52 * N + 4 * C + 8 + (srd ? (8 * NT + 20 * Cs) / srdGap : 0);
     A.held = -1;
-    bool hold = K <= kHoldBytes / perStep;
+    bool hold = false;
     const uint64_t nColl = srd ? collisions_in(steps, srdGap) : 0;
     const auto room = [&] {
         return grow(A.ckpt, A.capCkpt, uint64_t(nck) * stride) && grow(A.hash, A.capHash, NT) &&
@@ -1721,11 +1740,7 @@ void nwBatchAdjointForward(float *pos, float *vel, float *force, float *forceOld
                          grow(A.collIds, A.capCollIds, NT) && grow(A.collOff, A.capCollOff, Cs + 2) &&
                          grow(A.collCom, A.capCollCom, Cs)));
     };
-    if (hold && !(ensure_batch_segment(A) && room())) {
-        drop_batch_segment(A);  // no room for it: the run goes on without
-        hold = false;
-    }
-    NW_REQUIRE(room(), "nwBatchAdjointForward: out of device memory");
+    NW_REQUIRE(forward_room(A, room, hold), "nwBatchAdjointForward: out of device memory");
     if (srd) {
         NW_HIP(hipMemcpy(A.shifts, srdShifts, nColl * b.R * 3 * sizeof(float), hipMemcpyHostToDevice));
     }
@@ -1789,7 +1804,7 @@ void nwBatchAdjointBackward(const float *dLdPos, const float *dLdVel, double *gr
     NW_REQUIRE(A.ready, "nwBatchAdjointBackward: no nwBatchAdjointForward run to differentiate");
     NW_REQUIRE(dLdPos != nullptr && grad != nullptr, "nwBatchAdjointBackward: NULL argument");
     NW_REQUIRE(b.R == A.R && b.N == A.N, "nwBatchAdjointBackward: the batch changed since the forward run");
-    NW_REQUIRE(ensure_batch_segment(A), "nwBatchAdjointBackward: out of device memory");
+    NW_REQUIRE(ensure_segment(A), "nwBatchAdjointBackward: out of device memory");
     const uint64_t N = A.N, NT = A.NT, K = A.K, C = A.C, stride = 2 * NT + 2 * N;
     const size_t bytes = N * sizeof(float4);
     float4 *lr = A.lam, *lF[2] = {A.lam + N, A.lam + 2 * N}, *lG = A.lam + 3 * N, *lv = A.lam + 4 * N;
