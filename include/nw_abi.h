@@ -363,7 +363,8 @@ typedef struct NWReplicaParams {
     uint32_t reserved[5];
 } NWReplicaParams;
 
-/* Replaces the batch (one per process) and resets its step count. */
+/* Replaces the batch (one per process) and resets its step count.  A refused
+   call leaves the batch as it was. */
 void nwBatchSetReplicas(const NWReplicaParams *reps, uint numReplicas);
 /* numReplicas + 1 bead and cell offsets of the current batch. */
 void nwBatchLayout(uint *beadOffset, uint *cellOffset);

@@ -996,15 +996,11 @@ static hipError_t upload_table(unsigned char *&dev, size_t &cap, const void *src
 void nwBatchSetReplicas(const NWReplicaParams *reps, uint numReplicas) {
     NW_INIT();
     State &s = S();
-    State::Batch &b = s.batch;
+    State::Batch b;  // the new batch; a refused one leaves the old as it is
     NW_REQUIRE(numReplicas == 0 || reps != nullptr, "nwBatchSetReplicas: NULL replicas");
-    s.bsol.R = 0;  // a new batch has no solvent until nwBatchSetSolvent
-    s.badj.ready = false;
     b.reps.assign(numReplicas, BatchRep{});
     b.beadOff.assign(numReplicas + 1, 0u);
     b.cellOff.assign(numReplicas + 1, 0u);
-    b.tan = false;
-    b.unit = true;
     uint64_t N = 0, C = 0, waves = 0, blocks = 0;
     for (uint r = 0; r < numReplicas; ++r) {
         const NWReplicaParams &q = reps[r];
@@ -1051,12 +1047,11 @@ void nwBatchSetReplicas(const NWReplicaParams *reps, uint numReplicas) {
     b.waves = uint32_t(waves);
     b.blocks = uint32_t(blocks);
     b.mode = numReplicas && reps[0].ext.pairPotential == NW_PAIR_WCA ? 1 : 0;
-    b.steps = 0;
     (void)rows_plan_batch(b.reps.data(), numReplicas, b.rows);
     b.sort.assign(numReplicas, SortRep{});
-    b.sortPlan = BatchSortPlan{};
     const char *why = "";
     if (N) why = make_sort_reps(b.beadOff.data(), b.cellOff.data(), numReplicas, b.sort.data(), b.sortPlan);
+    NW_REQUIRE(!*why, "nwBatchSetReplicas: %s", why);
     // one buffer, one copy: the step counter, the records, then their
     // wavefront and workgroup offsets packed (the kernels' replica lookups
     // bisect those), then the sort's records
@@ -1072,18 +1067,27 @@ void nwBatchSetReplicas(const NWReplicaParams *reps, uint numReplicas) {
         off[numReplicas + r] = b.reps[r].blockOffset;
         off[2 * numReplicas + r] = b.reps[r].rowBlock;
     }
-    b.dev = nullptr;
-    b.sortDev = nullptr;
-    b.stepCtr = nullptr;
-    NW_HIP(upload_table(b.table, b.capTable, table.data(), table.size()));
+    s.bsol.R = 0;  // a new batch has no solvent until nwBatchSetSolvent
+    s.badj.ready = false;
+    b.scratch = s.batch.scratch;
+    b.table = s.batch.table;
+    b.capTable = s.batch.capTable;
+    hipError_t he = upload_table(b.table, b.capTable, table.data(), table.size());
+    if (he == hipSuccess && N) he = ensure_batch_sort_scratch(b.scratch, b.sortPlan);
+    if (he == hipSuccess && b.rows.blocks) he = ensure_rows_scratch(b.scratch, N);
+    if (he != hipSuccess) {
+        // no batch rather than one without its tables or scratch
+        s.batch = State::Batch{};
+        s.batch.scratch = b.scratch;
+        s.batch.table = b.table;
+        s.batch.capTable = b.capTable;
+        fail(__FILE__, __LINE__, int(he), "nwBatchSetReplicas: HIP error %d (%s)", int(he), hipGetErrorString(he));
+        return;
+    }
     b.stepCtr = reinterpret_cast<uint64_t *>(b.table);
     if (numReplicas) b.dev = reinterpret_cast<BatchRep *>(b.table + recAt);
-    if (N) {
-        NW_REQUIRE(!*why, "nwBatchSetReplicas: %s", why);
-        b.sortDev = reinterpret_cast<SortRep *>(b.table + sortAt);
-        NW_HIP(ensure_batch_sort_scratch(b.scratch, b.sortPlan));
-        if (b.rows.blocks) NW_HIP(ensure_rows_scratch(b.scratch, N));
-    }
+    if (N) b.sortDev = reinterpret_cast<SortRep *>(b.table + sortAt);
+    s.batch = std::move(b);
 }
 
 void nwBatchLayout(uint *beadOffset, uint *cellOffset) {
