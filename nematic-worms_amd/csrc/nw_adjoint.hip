@@ -398,15 +398,7 @@ __device__ __forceinline__ void adj_group(const AdjStepArgs &a, const KP &kp, ui
         lv = mk(load4(a.lv, m.bead));
         lG = mk(load4(a.lG, m.bead));
     }
-    if (m.active) {
-        const f3 Rt = lr + R + Rp;
-        // the drag -gamma v' is part of F' only with the Langevin thermostat on
-        const f3 V = lv - (a.langevin ? a.gamma : 0.0f) * lam + a.dt * Rt;
-        a.lr[m.bead] = f4(Rt, 0.0f);
-        a.lv[m.bead] = f4(V, 0.0f);
-        a.lFout[m.bead] = f4(lG + (0.5f * a.dt * a.dt) * Rt + (0.5f * a.dt) * V, 0.0f);
-        a.lG[m.bead] = f4((0.5f * a.dt) * V, 0.0f);
-    }
+    if (m.active) adj_update(a, m, lam, R, Rp, lr, lv, lG);
     acc[kAdjEpsilon] = -eps / double(kp.e.wcaEpsilon);  // F is linear in epsilon
     double total = 0.0;
 #pragma unroll

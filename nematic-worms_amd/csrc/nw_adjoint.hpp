@@ -16,14 +16,14 @@ struct AdjStepArgs {
     const float4 *lF;               // adjoint of the step's force
     float4 *lFout;                  // adjoint of the previous force (the other buffer)
     float4 *lr, *lv, *lG;           // updated in place
-    double *partial;                // one row of kAdjParams per workgroup, added to
+    double *partial;                // one row of kAdjParams per front wavefront, added to
     uint32_t W;
     int langevin;
     float lgvStd, gamma, dt;
     uint64_t seed, offLgv;          // the step's Langevin draws
 };
 
-// workgroups of a step (one per front wavefront): rows of partial
+// front wavefronts of a system: rows of partial
 uint32_t adj_step_rows(uint32_t W, uint32_t n);
 hipError_t launch_adj_step(const AdjStepArgs &a, const KP &kp, hipStream_t st);
 // d S / d r of the bond-tangent nematic order: e the unit eigenvector of the
