@@ -537,8 +537,8 @@ uint nwGetDeviceFlags(int clear);
    system's front and first level are one launch), "md_sort", "md_collide" (a small
    system's order and pair forces are one launch, under "md_collide"),
    "srdf_tiles", "srdf_cells", "srdf_rotate"; of the batched step's kernels:
-   "batch_front", "batch_tiles", "batch_sort", "batch_collide"; of the adjoint
-   sweeps: "adj_step", "badj_step"; the solvent
+   "batch_front", "batch_tiles", "batch_sort", "batch_collide", and "batch_step"
+   around all of a step; of the adjoint sweeps: "adj_step", "badj_step"; the solvent
    re-sort nwSortSolvent: "srd_resort". */
 void nwTimerEnable(const char *kernel, int enable);
 /* Synchronises; returns total milliseconds and launch count since enable. */

@@ -1178,7 +1178,11 @@ void nwBatchMdStep(float *pos, float *vel, float *force, float *forceOld, float 
             x.tangent = a.tangent;
             if (ph == 0) x.swapForces = 0;
         }
-        const hipError_t e = batch_step(b, x, gv, gt, a.sVel, a.sTan, deltaTime, s.stream);
+        hipError_t e;
+        {
+            TimedScope ts("batch_step", s.stream);
+            e = batch_step(b, x, gv, gt, a.sVel, a.sTan, deltaTime, s.stream);
+        }
         if (e != hipSuccess) {
             // what the steps before it reached is the caller's: the force
             // arrays' contents in their roles and the tangents; then report
