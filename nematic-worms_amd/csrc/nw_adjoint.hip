@@ -707,7 +707,7 @@ __global__ __launch_bounds__(kTotalBlock) void k_adj_total(const double *__restr
 // launchers
 // ---------------------------------------------------------------------------
 // workgroups of the kernels with a bead a lane
-static uint32_t adj_step_blocks(uint32_t W, uint32_t n) {
+static uint32_t bead_lane_blocks(uint32_t W, uint32_t n) {
     const uint32_t wpw = 64u / n;
     return grid_for(((uint64_t(W) + wpw - 1) / wpw) * 64u);
 }
@@ -729,7 +729,7 @@ hipError_t launch_adj_step(const AdjStepArgs &a, const KP &kp, hipStream_t st) {
 
 hipError_t launch_bond_order_grad(const float4 *pos, uint32_t W, const double e[3], double scale, float4 *out,
                                   const KP &kp, hipStream_t st) {
-    const uint32_t blocks = adj_step_blocks(W, kp.p.filamentSize);
+    const uint32_t blocks = bead_lane_blocks(W, kp.p.filamentSize);
     if (!blocks) return hipSuccess;
     hipLaunchKernelGGL(k_bond_order_grad, dim3(blocks), dim3(kBlock), 0, st, pos, W, float(e[0]), float(e[1]),
                        float(e[2]), float(scale), out, kp);
@@ -749,7 +749,7 @@ hipError_t launch_srd_adj(const uint32_t *ids, const uint32_t *off, const uint32
 
 hipError_t launch_polar_speed_grad(const float4 *pos, const float4 *vel, uint32_t W, double scale, float4 *dPos,
                                    float4 *dVel, const KP &kp, hipStream_t st) {
-    const uint32_t blocks = adj_step_blocks(W, kp.p.filamentSize);
+    const uint32_t blocks = bead_lane_blocks(W, kp.p.filamentSize);
     if (!blocks) return hipSuccess;
     hipLaunchKernelGGL(k_polar_speed_grad, dim3(blocks), dim3(kBlock), 0, st, pos, vel, W, float(scale), dPos, dVel,
                        kp);

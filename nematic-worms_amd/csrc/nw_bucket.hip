@@ -1130,8 +1130,7 @@ hipError_t ensure_bucket_scratch(BucketScratch &s, const BucketPlan &bp) {
 
 hipError_t ensure_rows_scratch(BucketScratch &s, uint64_t n) { return regrow(s.spill, s.cap_spill, 4u * n, 4); }
 
-// LDS beyond 64 KiB is granted per kernel, once (outside any graph capture:
-// the first launch of a size runs directly)
+// LDS beyond 64 KiB is granted per kernel and size, once
 hipError_t grant_lds(const void *fn, size_t lds) {
     static std::vector<std::pair<const void *, size_t>> granted;
     if (lds <= 65536) return hipSuccess;

@@ -233,8 +233,7 @@ __device__ __forceinline__ void row_runs(const uint32_t *__restrict__ off, uint3
 // The candidates of a one-layer stencil (Gx >= 3) from global memory: the
 // row pieces (three rows, one or two x runs each, in stencil order) first,
 // then the flattened candidate list four at a time with the loads of the
-// four issued together.  The same candidates, order and arithmetic as the
-// row-by-row walk below.
+// four issued together: the candidates, order and arithmetic of the LDS walk.
 constexpr int kGlobalBatch = 4;
 
 template <int MODE, bool TAN>

@@ -1,6 +1,6 @@
 // nw_physics.hpp -- device physics shared by the per-call kernels
 // (nw_kernels.hip) and the fused step kernels (nw_fused.hip): boundaries,
-// pair terms, stencil folding, cross-lane shuffles, per-element uniforms.
+// the WCA magnitude, stencil folding, cross-lane shuffles, per-element uniforms.
 #pragma once
 
 #include "nw_device.hpp"

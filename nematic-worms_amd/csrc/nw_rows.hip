@@ -15,9 +15,11 @@
 // (11.7 reading every bead's cell): 1.3 the worms, 2 the order, 1.5 the pairs,
 // the rest the dispatch and barriers.
 //
-// The pairs: four lanes a bead, lane q evaluating candidates q, q + 4, ... of
-// the flattened list, their terms added in list order by quad broadcasts: the
-// sums of k_collide_rows bit for bit, in a quarter of its dependent steps.
+// The pairs: up to some 400 own beads four lanes a bead, lane q evaluating
+// candidates q, q + 4, ... of the flattened list, their terms added in list
+// order by quad broadcasts: a quarter of the dependent steps.  With more beads
+// a workgroup has chains enough and a bead takes one lane (kRowsLaneBeads).
+// Either way the sums of k_collide_rows bit for bit.
 #include <algorithm>
 
 #include "nw_bucket.hpp"
@@ -146,7 +148,7 @@ __device__ __forceinline__ void rows_pairs(const KP &kp, const RowsArgs &a, cons
 // square of its beads over the threads, not one thread's insertion sort (a
 // system collapsed into few cells).  Twelve rows of 5,000 beads: a step 0.65 ms,
 // by the sort and the pair kernel 0.26, by passes over all beads 320; 4,000
-// beads in a cell or two 4.4 ms, by insertion 158.  What bounds it is that the
+// beads in a cell or two 6.1 ms, by insertion 395.  What bounds it is that the
 // crowded rows' few workgroups do all the work.
 template <typename BeadOf, typename Local>
 __device__ __forceinline__ void rows_in_memory(const KP &kp, const RowsArgs &a, uint32_t N, uint32_t idBase,
@@ -392,11 +394,11 @@ __global__ __launch_bounds__(kRowsBlock) void k_rows_batch(BatchArrays a, const 
 // ---------------------------------------------------------------------------
 // A step with the sort and the pair kernel / with this launch, worms of 16: 21.5
 // / 13.0 us at 32,000 beads, 22.1 / 16.0 at 64,000, 25.0 / 19.9 at 128,000, 27.7
-// / 22.6 at 192,000, 28.9 / 27.5 at 256,000, 33.1 / 33.6 at 288,000; where the
-// front and the sort's first level are two launches (front_tiles_plan: more than
-// 4,096 wavefronts), worms of 23: 32.9 / 27.9 at 229,000, 35.8 / 31.4 at 298,000,
-// 39.0 / 38.8 at 344,000.
-constexpr uint64_t kRowsMaxBeads = 262144, kRowsMaxBeadsTwo = 300000;
+// / 22.6 at 192,000, 28.9 / 27.5 at 256,000, 33.1 / 33.6 at 288,000; worms of
+// 23, whose front and first sort level are two launches (front_tiles_plan: more
+// than 4,096 wavefronts, as any system beyond 262,144 beads has): 32.9 / 27.9 at
+// 229,000, 35.8 / 31.4 at 298,000, 39.0 / 38.8 at 344,000.
+constexpr uint64_t kRowsMaxBeads = 300000;
 // every workgroup reads every worm's rows: 22.8 / 20.4 us with 20,000 worms of
 // three, 23.1 / 24.8 with 30,000; of five 22.7 / 19.6 with 15,000, 26.9 / 28.1
 // with 30,000
@@ -443,8 +445,7 @@ bool rows_plan(uint64_t N, const KP &kp, RowsPlan &out) {
     if (!rows_term(kp)) return false;
     // a launch shape asked of the sort or the pair kernel is theirs
     if (t.mdTileItems || t.mdMembers || t.pairBlock || t.pairStage) return false;
-    const uint32_t n = kp.p.filamentSize, waves = uint32_t((N / n + 64u / n - 1u) / (64u / n));
-    if (N == 0 || N / n > kRowsMaxWorms || N > (waves > kFrontTilesWaves ? kRowsMaxBeadsTwo : kRowsMaxBeads)) return false;
+    if (N == 0 || N / kp.p.filamentSize > kRowsMaxWorms || N > kRowsMaxBeads) return false;
     out.rows = std::min((Gy + kRowsMaxBlocks - 1u) / kRowsMaxBlocks, Gy - 2u);
     out.blocks = (Gy + out.rows - 1u) / out.rows;
     if (double(N) / Gy * out.rows > double(kRowsMaxOwn)) return false;

@@ -4,6 +4,8 @@ of each other in one cell, rows at the periodic face.  Against the two-level
 sort and the pair kernel: bit for bit, and in a time of the same order (the
 candidates are the same; passes over the whole system are hundreds of times
 more).  A small wcaEpsilon keeps overlapping beads' forces finite."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -89,3 +91,20 @@ def test_crowded_batch(lib):  # noqa: F811
     for name, x, y in zip(("pos", "vel", "force", "forceOld", "tangent", "ids", "sortedPos"), *got):
         assert np.array_equal(x, y), name
 
+
+
+def test_crowded_without_allocation(lib):  # noqa: F811
+    """The same through nwFusedMdStepNoAlloc, whose crowded rows have their place in its fixed scratch."""
+    p, state = crowd(np.random.default_rng(5), (200, 200), 3200, 10, (0.0, 0.98), (1.0, 0.04))
+    N = p.numParticles
+    want = step(lib, p, ext(), state, NWTuning(mdMembers=512), 0)
+    lib.nwSetTuning(ctypes.byref(NWTuning()))
+    d = [DeviceArray.from_numpy(lib, a) for a in state]
+    i, sp = DeviceArray(lib, 4 * N), DeviceArray(lib, 16 * N)
+    lib.nwRngSetSeed(11, 5)
+    for _ in range(2):
+        lib.nwFusedMdStepNoAlloc(*[x.p for x in d], None, i.p, sp.p, None, None, 1e-4, 2.0, 0.1, 1, p.numFilaments)
+    assert lib.nwGetLastError() == 0, lib.nwGetLastErrorString()
+    got = [x.download(np.uint32, (N, 4)) for x in d] + [i.download(np.uint32, (N,)), sp.download(np.uint32, (N, 4))]
+    for x, y in zip(got, want[:5] + want[6:]):
+        assert np.array_equal(x, y)
