@@ -693,7 +693,7 @@ static bool fused_md(const KP &kp, float *pos, float *vel, float *force, float *
         // a small system: the cell order and the pair forces in one launch
         TimedScope ts(fixed ? noTimer : "md_collide", s.stream, true);
         NW_HIP_R(launch_rows(rows, a.hash, a.wormRows, a.pos, swapForces ? a.forceOld : a.force, gridParticleIndex, sc.off,
-                             sc.sortedCell, reinterpret_cast<float4 *>(sortedPos), base.spill, uint32_t(N), kp, s.stream), false);
+                             sc.sortedCell, reinterpret_cast<float4 *>(sortedPos), uint32_t(N), kp, s.stream), false);
         s.lastHashPtr = nullptr;
         return true;
     }
@@ -769,16 +769,15 @@ void nwFusedMdStepNoAlloc(float *pos, float *vel, float *force, float *forceOld,
                "nwFusedMdStepNoAlloc: %llu beads over %llu cells", (unsigned long long)N, (unsigned long long)cells);
     // the sort's arrays carved from the scratch, 256-byte aligned: the cell
     // of every bead (unless the caller takes it), the packed pairs, the tile
-    // x bucket prefix matrix, the cell of every sorted slot, the CSR offsets,
-    // and for the one-launch order and pairs (some 14 MiB in all at its largest)
-    // its crowded rows
-    RowsPlan rows;
-    const uint64_t spill = rows_plan(N, kp, rows) ? 4 * N : 0;
+    // x bucket prefix matrix, the cell of every sorted slot, the CSR offsets
     const BucketPlan bp = fused_plan(N, cells, false);
     NW_REQUIRE(!*bucket_plan_problem(bp), "nwFusedMdStepNoAlloc: %s", bucket_plan_problem(bp));
     auto words = [](uint64_t n) { return (n * 4 + 255) & ~uint64_t(255); };
-    const uint64_t need = (gridParticleHash ? 0 : words(N)) + words(uint64_t(bp.tiles) * bp.tileItems) +
-                          words(uint64_t(bp.tiles) * (bp.buckets + 1)) + words(N) + words(cells + 2) + words(spill);
+    // (with the one-launch order and pairs some 14 MiB in all at its largest)
+    RowsPlan rows;
+    const uint64_t pairs = std::max(uint64_t(bp.tiles) * bp.tileItems, rows_plan(N, kp, rows) ? kRowsWords * N : 0);
+    const uint64_t need = (gridParticleHash ? 0 : words(N)) + words(pairs) +
+                          words(uint64_t(bp.tiles) * (bp.buckets + 1)) + words(N) + words(cells + 2);
     NW_REQUIRE(need <= kNoAllocScratchBytes,
                "nwFusedMdStepNoAlloc: %llu beads over %llu cells need %llu bytes of scratch; the fixed scratch "
                "array holds %llu (use nwFusedMdStep)",
@@ -792,11 +791,10 @@ void nwFusedMdStepNoAlloc(float *pos, float *vel, float *force, float *forceOld,
     };
     BucketScratch sc{};
     sc.hash = gridParticleHash ? nullptr : take(N);
-    sc.pairs = take(uint64_t(bp.tiles) * bp.tileItems);
+    sc.pairs = take(pairs);
     sc.P = take(uint64_t(bp.tiles) * (bp.buckets + 1));
     sc.sortedCell = take(N);
     sc.off = take(cells + 2);
-    if (spill) sc.spill = take(spill);
     (void)fused_md(kp, pos, vel, force, forceOld, tangent, gridParticleHash, gridParticleIndex, sortedPos, sortedVel,
                    sortedTangent, deltaTime, langevinGamma, langevinKbT, langevin, numFilaments, nullptr, nullptr,
                    nullptr, nullptr, false, &sc);
@@ -1151,7 +1149,6 @@ void nwBatchMdStep(float *pos, float *vel, float *force, float *forceOld, float 
     a.swapForces = b.swap ? 1 : 0;
     a.hash = b.scratch.hash;
     a.wormRows = b.rows.blocks ? b.scratch.pairs : nullptr;  // the sort's, which is not launched
-    a.spill = b.scratch.spill;
     a.ids = gridParticleIndex;
     a.off = b.scratch.off;
     a.sCell = b.scratch.sortedCell;
@@ -1759,7 +1756,6 @@ void nwBatchAdjointForward(float *pos, float *vel, float *force, float *forceOld
     a.forceOld = reinterpret_cast<float4 *>(forceOld);
     a.hash = A.hash;
     a.wormRows = b.rows.blocks ? b.scratch.pairs : nullptr;
-    a.spill = b.scratch.spill;
     a.sCell = A.sCell;
     // the step velocities are read only for the Langevin partials
     const bool lgv = batch_langevin(b);
@@ -1855,7 +1851,6 @@ void nwBatchAdjointBackward(const float *dLdPos, const float *dLdVel, double *gr
             a.forceOld = G;
             a.hash = A.hash;
             a.wormRows = b.rows.blocks ? b.scratch.pairs : nullptr;
-            a.spill = b.scratch.spill;
             a.ids = A.segIds + uint64_t(j) * N;
             a.off = A.segOff + uint64_t(j) * (C + 2);
             a.sCell = A.sCell;

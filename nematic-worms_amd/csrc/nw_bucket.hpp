@@ -81,11 +81,13 @@ struct BucketScratch {
     uint32_t *off = nullptr;         // CSR cell offsets (cells + 1)
     float *lam = nullptr;            // isokinetic factor per SRD cell
     uint32_t *aux = nullptr;         // per particle: the values of a key-value sort
-    uint32_t *spill = nullptr;       // 4 per bead: crowded rows of the one-launch order and pairs
-    uint64_t cap_n = 0, cap_pairs = 0, cap_mat = 0, cap_cells = 0, cap_range = 0, cap_spill = 0;
+    uint64_t cap_n = 0, cap_pairs = 0, cap_mat = 0, cap_cells = 0, cap_range = 0;
 };
 
 hipError_t ensure_bucket_scratch(BucketScratch &s, const BucketPlan &bp);
+// the one-launch order and pairs uses pairs, five words a bead: the worms'
+// words and its crowded rows
+constexpr uint64_t kRowsWords = 5;
 hipError_t ensure_rows_scratch(BucketScratch &s, uint64_t n);
 
 struct MdFrontArgs {
@@ -171,8 +173,9 @@ struct RowsPlan {
 };
 // whether the launch takes this system, and its shape
 bool rows_plan(uint64_t N, const KP &kp, RowsPlan &out);
-hipError_t launch_rows(const RowsPlan &pl, const uint32_t *hash, const uint32_t *wormRows, const float4 *pos, float4 *force, uint32_t *ids,
-                       uint32_t *off, uint32_t *sCell, float4 *sPos, uint32_t *spill, uint32_t N, const KP &kp, hipStream_t st);
+hipError_t launch_rows(const RowsPlan &pl, const uint32_t *hash, uint32_t *wormRows, const float4 *pos, float4 *force,
+                       uint32_t *ids, uint32_t *off, uint32_t *sCell, float4 *sPos, uint32_t N, const KP &kp,
+                       hipStream_t st);
 // LDS beyond 64 KiB, granted per kernel once
 hipError_t grant_lds(const void *fn, size_t lds);
 
@@ -282,8 +285,9 @@ hipError_t launch_srd_rotate_batch(const uint32_t *hash, const float4 *com, floa
 struct BatchArrays {
     float4 *pos, *vel, *force, *forceOld, *tangent;
     float4 *keepPos, *keepVel;  // the new state once more (NULL: not)
-    uint32_t *wormRows;         // every worm's rows of cells, from its replica's first bead on (NULL: not)
-    uint32_t *spill;            // with wormRows: scratch, four words a bead
+    // every worm's rows of cells, from its replica's first bead on (NULL: not);
+    // behind the batch's beads four words of scratch a bead
+    uint32_t *wormRows;
     // nonzero: the new force goes to forceOld's buffer (pairs add there too)
     // and force's buffer is left as the old force (no replica reverses)
     int swapForces;

@@ -34,12 +34,11 @@ constexpr int kRowsBlock = 1024;
 
 struct RowsArgs {
     const uint32_t *hash;   // cell of every bead, bead order
-    const uint32_t *worms;  // rows of every worm (worm_rows_word)
+    uint32_t *worms;        // rows of every worm (worm_rows_word); behind a system's words is its scratch
     const float4 *pos;
     float4 *force;
     uint32_t *ids, *off, *sCell;
     float4 *sPos;
-    uint32_t *spill;        // scratch, four words a bead
 };
 
 // LDS of a workgroup (bytes): staged beads `cap`, cells of its rows and the two beside them
@@ -141,7 +140,7 @@ __device__ __forceinline__ void rows_pairs(const KP &kp, const RowsArgs &a, cons
 // More beads than the stage holds (worms crowded into a few rows): the staged
 // beads' lists in memory.  The own ones stand at their slots, as they arrive in
 // sCell and in ascending id per cell in ids; those of the rows below and above
-// in a.spill, N words each for arrival and order, at the slots that their rows
+// in spill, N words each for arrival and order, at the slots that their rows
 // have in the system: a row is below the rows of one workgroup alone, and above
 // those of one, so no two workgroups meet there.
 // A bead counts its own rank among the ids of its cell, so a cell takes the
@@ -151,15 +150,15 @@ __device__ __forceinline__ void rows_pairs(const KP &kp, const RowsArgs &a, cons
 // beads in a cell or two 6.1 ms, by insertion 395.  What bounds it is that the
 // crowded rows' few workgroups do all the work.
 template <typename BeadOf, typename Local>
-__device__ __forceinline__ void rows_in_memory(const KP &kp, const RowsArgs &a, uint32_t N, uint32_t idBase,
+__device__ __forceinline__ void rows_in_memory(const KP &kp, const RowsArgs &a, uint32_t *spill, uint32_t N, uint32_t idBase,
                                                uint32_t cellBase, uint32_t slot0, uint32_t y0, uint32_t own,
                                                const uint32_t *cnt, uint32_t *cur, uint32_t words,
                                                const BeadOf &bead_of, const Local &local) {
     const uint32_t Gx = kp.p.gridSize.x, Gy = kp.p.gridSize.y, nc = (own + 2u) * Gx;
     const uint32_t s0 = cnt[Gx], s1 = cnt[(own + 1u) * Gx], m = cnt[nc];
     // of a staged slot u: below u < s0, own, above u >= s1
-    uint32_t *const lo = a.spill + (y0 == 0u ? N - s0 : slot0 - s0);
-    uint32_t *const hi = a.spill + 2u * uint64_t(N) + (y0 + own == Gy ? 0u : slot0 + (s1 - s0));
+    uint32_t *const lo = spill + (y0 == 0u ? N - s0 : slot0 - s0);
+    uint32_t *const hi = spill + 2u * uint64_t(N) + (y0 + own == Gy ? 0u : slot0 + (s1 - s0));
     auto raw = [&](uint32_t u) { return u < s0 ? lo + u : (u < s1 ? a.sCell + slot0 + (u - s0) : hi + (u - s1)); };
     auto fin = [&](uint32_t u) { return u < s0 ? lo + N + u : (u < s1 ? a.ids + slot0 + (u - s0) : hi + N + (u - s1)); };
     for (uint32_t k = threadIdx.x; k < words; k += blockDim.x) {
@@ -216,11 +215,13 @@ __device__ __forceinline__ void rows_in_memory(const KP &kp, const RowsArgs &a, 
 // Rows [y0, y0 + rows) of one system: N beads whose arrays hash, pos, force
 // start at its first bead; ids, sCell and sPos (indexed by sorted slot) and
 // off (by cell) at its own first entries; bead ids, cells and slots of the
-// system are written with idBase, cellBase and slotBase added.
-template <int T>
+// system are written with idBase, cellBase and slotBase added.  spill(): scratch
+// of four words a bead (an argument of the launch more took 0.1 us: it has
+// its place behind the worms' words).
+template <int T, typename Spill>
 __device__ __forceinline__ void rows_body(const KP &kp, const RowsArgs &a, uint32_t N, uint32_t idBase,
                                           uint32_t cellBase, uint32_t slotAdd, uint32_t y0, uint32_t rows,
-                                          uint32_t cap, uint32_t maxCells, unsigned char *smem) {
+                                          uint32_t cap, uint32_t maxCells, unsigned char *smem, const Spill &spill) {
     const RowsLayout L = rows_layout(cap, maxCells);
     float4 *lpos = reinterpret_cast<float4 *>(smem + L.pos);
     uint32_t *list = reinterpret_cast<uint32_t *>(smem + L.pos);  // until the positions come: 4 cap words
@@ -315,7 +316,7 @@ __device__ __forceinline__ void rows_body(const KP &kp, const RowsArgs &a, uint3
     for (uint32_t c = t; c < own * Gx; c += T) a.off[hOwn + c] = slotBase + cnt[Gx + c] - s0;
     if (y0 + own == Gy && t == 0) a.off[C] = slotAdd + N;
     if (m > cap) {
-        rows_in_memory(kp, a, N, idBase, cellBase, slotBase - slotAdd, y0, own, cnt, cur, words, bead_of, local);
+        rows_in_memory(kp, a, spill(), N, idBase, cellBase, slotBase - slotAdd, y0, own, cnt, cur, words, bead_of, local);
         return;
     }
     auto place = [&](uint32_t id, uint32_t d) {
@@ -370,7 +371,7 @@ __global__ __launch_bounds__(kRowsBlock) void k_rows(RowsArgs a, uint32_t N, uin
                                                      uint32_t maxCells, KP kp) {
     extern __shared__ __align__(16) unsigned char smem[];
     const uint32_t b = xcd_contiguous(blockIdx.x, gridDim.x);
-    rows_body<kRowsBlock>(kp, a, N, 0u, 0u, 0u, b * rows, rows, cap, maxCells, smem);
+    rows_body<kRowsBlock>(kp, a, N, 0u, 0u, 0u, b * rows, rows, cap, maxCells, smem, [&] { return a.worms + N; });
 }
 
 // the same of every replica of a batch: a workgroup belongs to one replica
@@ -384,9 +385,12 @@ __global__ __launch_bounds__(kRowsBlock) void k_rows_batch(BatchArrays a, const 
     const BatchRep &rep = reps[__builtin_amdgcn_readfirstlane(replica_of_row_block(reps, R, b))];
     const uint32_t b0 = rep.beadOffset, c0 = rep.cellOffset;
     const RowsArgs x{a.hash + b0, a.wormRows + b0, a.pos + b0, (a.swapForces ? a.forceOld : a.force) + b0, a.ids + b0,
-                     a.off + c0,     a.sCell + b0, a.sPos + b0, a.spill + 4u * uint64_t(b0)};
+                     a.off + c0,     a.sCell + b0, a.sPos + b0};
     rows_body<kRowsBlock>(rep.kp, x, rep.numBeads, b0, c0, b0, (b - rep.rowBlock) * rep.rows, rep.rows, cap, maxCells,
-                          smem);
+                          smem, [&] {
+                              const BatchRep &last = reps[R - 1u];
+                              return a.wormRows + last.beadOffset + last.numBeads + 4u * uint64_t(b0);
+                          });
 }
 
 // ---------------------------------------------------------------------------
@@ -501,9 +505,10 @@ hipError_t launch_rows_batch(const RowsPlan &pl, const BatchArrays &a, const Bat
     return hipGetLastError();
 }
 
-hipError_t launch_rows(const RowsPlan &pl, const uint32_t *hash, const uint32_t *wormRows, const float4 *pos, float4 *force, uint32_t *ids,
-                       uint32_t *off, uint32_t *sCell, float4 *sPos, uint32_t *spill, uint32_t N, const KP &kp, hipStream_t st) {
-    const RowsArgs a{hash, wormRows, pos, force, ids, off, sCell, sPos, spill};
+hipError_t launch_rows(const RowsPlan &pl, const uint32_t *hash, uint32_t *wormRows, const float4 *pos, float4 *force,
+                       uint32_t *ids, uint32_t *off, uint32_t *sCell, float4 *sPos, uint32_t N, const KP &kp,
+                       hipStream_t st) {
+    const RowsArgs a{hash, wormRows, pos, force, ids, off, sCell, sPos};
     const hipError_t e = grant_lds(reinterpret_cast<const void *>(&k_rows), pl.lds);
     if (e != hipSuccess) return e;
     NW_LAUNCH(k_rows, dim3(pl.blocks), dim3(kRowsBlock), pl.lds, st, a, N, pl.rows, pl.cap, pl.cells, kp);
