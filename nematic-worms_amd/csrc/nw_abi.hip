@@ -773,9 +773,9 @@ void nwFusedMdStepNoAlloc(float *pos, float *vel, float *force, float *forceOld,
     const BucketPlan bp = fused_plan(N, cells, false);
     NW_REQUIRE(!*bucket_plan_problem(bp), "nwFusedMdStepNoAlloc: %s", bucket_plan_problem(bp));
     auto words = [](uint64_t n) { return (n * 4 + 255) & ~uint64_t(255); };
-    // (with the one-launch order and pairs some 14 MiB in all at its largest)
+    // (with the one-launch order and pairs some 24 MiB in all at its largest)
     RowsPlan rows;
-    const uint64_t pairs = std::max(uint64_t(bp.tiles) * bp.tileItems, rows_plan(N, kp, rows) ? kRowsWords * N : 0);
+    const uint64_t pairs = std::max(uint64_t(bp.tiles) * bp.tileItems, rows_plan(N, kp, rows) ? kRowsWords * N + 4 : 0);
     const uint64_t need = (gridParticleHash ? 0 : words(N)) + words(pairs) +
                           words(uint64_t(bp.tiles) * (bp.buckets + 1)) + words(N) + words(cells + 2);
     NW_REQUIRE(need <= kNoAllocScratchBytes,

@@ -1128,7 +1128,7 @@ hipError_t ensure_bucket_scratch(BucketScratch &s, const BucketPlan &bp) {
     return hipSuccess;
 }
 
-hipError_t ensure_rows_scratch(BucketScratch &s, uint64_t n) { return regrow(s.pairs, s.cap_pairs, kRowsWords * n, 4); }
+hipError_t ensure_rows_scratch(BucketScratch &s, uint64_t n) { return regrow(s.pairs, s.cap_pairs, kRowsWords * n + 4u, 4); }
 
 // LDS beyond 64 KiB is granted per kernel and size, once
 hipError_t grant_lds(const void *fn, size_t lds) {

@@ -85,9 +85,9 @@ struct BucketScratch {
 };
 
 hipError_t ensure_bucket_scratch(BucketScratch &s, const BucketPlan &bp);
-// the one-launch order and pairs uses pairs, five words a bead: the worms'
-// words and its crowded rows
-constexpr uint64_t kRowsWords = 5;
+// the one-launch order and pairs uses pairs, eleven words a bead (and three to
+// align): the worms' words and its crowded rows
+constexpr uint64_t kRowsWords = 11;
 hipError_t ensure_rows_scratch(BucketScratch &s, uint64_t n);
 
 struct MdFrontArgs {
@@ -286,7 +286,7 @@ struct BatchArrays {
     float4 *pos, *vel, *force, *forceOld, *tangent;
     float4 *keepPos, *keepVel;  // the new state once more (NULL: not)
     // every worm's rows of cells, from its replica's first bead on (NULL: not);
-    // behind the batch's beads four words of scratch a bead
+    // behind the batch's beads the scratch of crowded rows
     uint32_t *wormRows;
     // nonzero: the new force goes to forceOld's buffer (pairs add there too)
     // and force's buffer is left as the old force (no replica reverses)

@@ -137,30 +137,45 @@ __device__ __forceinline__ void rows_pairs(const KP &kp, const RowsArgs &a, cons
     }
 }
 
+// The scratch behind the words of a launch's worms (n beads in all): the beads
+// of crowded rows beside a workgroup's own, two roles a row, as they arrive
+// and in order.
+struct RowsSpill {
+    uint32_t *raw;  // 2 n ids
+    float4 *pos;    // 2 n records: position, worm
+    uint64_t n;
+};
+__device__ __forceinline__ RowsSpill rows_spill(uint32_t *worms, uint64_t n) {
+    return {worms + n, reinterpret_cast<float4 *>(worms + ((3u * n + 3u) & ~uint64_t(3))), n};
+}
+
 // More beads than the stage holds (worms crowded into a few rows): the staged
 // beads' lists in memory.  The own ones stand at their slots, as they arrive in
-// sCell and in ascending id per cell in ids; those of the rows below and above
-// in spill, N words each for arrival and order, at the slots that their rows
-// have in the system: a row is below the rows of one workgroup alone, and above
-// those of one, so no two workgroups meet there.
+// sCell and in ascending id per cell in ids and sPos; those of the rows below
+// and above in the spill, at the slots that their rows have in the system
+// (at: its first bead): a row is below the rows of one workgroup alone, and above those of
+// one, so no two workgroups meet there.
 // A bead counts its own rank among the ids of its cell, so a cell takes the
 // square of its beads over the threads, not one thread's insertion sort (a
-// system collapsed into few cells).  Twelve rows of 5,000 beads: a step 0.65 ms,
-// by the sort and the pair kernel 0.26, by passes over all beads 320; 4,000
-// beads in a cell or two 6.1 ms, by insertion 395.  What bounds it is that the
-// crowded rows' few workgroups do all the work.
+// system collapsed into few cells); and it goes to its place as the record
+// that the walk reads, one load a candidate.  Twelve rows of 5,000 beads: a step
+// 0.57 ms, by the sort and the pair kernel 0.27, by passes over all beads 320;
+// 4,000 beads in a cell or two 4.4 ms, by insertion 395; 250,000 beads in four
+// tenths of their box 118 us, before the launch 101.  What bounds it is that
+// the crowded rows' few workgroups do all the work.
 template <typename BeadOf, typename Local>
-__device__ __forceinline__ void rows_in_memory(const KP &kp, const RowsArgs &a, uint32_t *spill, uint32_t N, uint32_t idBase,
-                                               uint32_t cellBase, uint32_t slot0, uint32_t y0, uint32_t own,
-                                               const uint32_t *cnt, uint32_t *cur, uint32_t words,
-                                               const BeadOf &bead_of, const Local &local) {
+__device__ __forceinline__ void rows_in_memory(const KP &kp, const RowsArgs &a, const RowsSpill &sp, uint32_t at,
+                                               uint32_t N, uint32_t idBase, uint32_t cellBase, uint32_t slot0,
+                                               uint32_t y0, uint32_t own, const uint32_t *cnt, uint32_t *cur,
+                                               uint32_t words, const BeadOf &bead_of, const Local &local) {
     const uint32_t Gx = kp.p.gridSize.x, Gy = kp.p.gridSize.y, nc = (own + 2u) * Gx;
     const uint32_t s0 = cnt[Gx], s1 = cnt[(own + 1u) * Gx], m = cnt[nc];
-    // of a staged slot u: below u < s0, own, above u >= s1
-    uint32_t *const lo = spill + (y0 == 0u ? N - s0 : slot0 - s0);
-    uint32_t *const hi = spill + 2u * uint64_t(N) + (y0 + own == Gy ? 0u : slot0 + (s1 - s0));
-    auto raw = [&](uint32_t u) { return u < s0 ? lo + u : (u < s1 ? a.sCell + slot0 + (u - s0) : hi + (u - s1)); };
-    auto fin = [&](uint32_t u) { return u < s0 ? lo + N + u : (u < s1 ? a.ids + slot0 + (u - s0) : hi + N + (u - s1)); };
+    // of a staged slot u: below u < s0, own, above u >= s1; its place in the spill
+    const uint64_t lo = at + (y0 == 0u ? N - s0 : slot0 - s0);
+    const uint64_t hi = sp.n + at + (y0 + own == Gy ? 0u : slot0 + (s1 - s0));
+    auto raw = [&](uint32_t u) {
+        return u < s0 ? sp.raw + lo + u : (u < s1 ? a.sCell + slot0 + (u - s0) : sp.raw + hi + (u - s1));
+    };
     for (uint32_t k = threadIdx.x; k < words; k += blockDim.x) {
         const uint32_t id = bead_of(k), d = local(a.hash[id] - cellBase);
         if (d < nc) *raw(atomicAdd(&cur[d], 1u)) = id;
@@ -168,23 +183,29 @@ __device__ __forceinline__ void rows_in_memory(const KP &kp, const RowsArgs &a, 
     __syncthreads();
     for (uint32_t s = threadIdx.x; s < m; s += blockDim.x) {
         const uint32_t id = *raw(s), d = local(a.hash[id] - cellBase);
+        const float4 P = load4(a.pos, id);
         const uint32_t c0 = cnt[d], z = cnt[d + 1u] - c0;
         const uint32_t *cell = raw(c0);
         uint32_t r = c0;
 #pragma unroll 4
         for (uint32_t u = 0; u < z; ++u) r += cell[u] < id ? 1u : 0u;
-        *fin(r) = s >= s0 && s < s1 ? idBase + id : id;
+        if (s >= s0 && s < s1) {
+            a.ids[slot0 + (r - s0)] = idBase + id;
+            a.sPos[slot0 + (r - s0)] = P;
+        } else {
+            uint32_t fil, ch;
+            worm_of(kp, id, fil, ch);
+            sp.pos[s < s0 ? lo + r : hi + (r - s1)] = make_float4(P.x, P.y, P.z, __uint_as_float(fil));
+        }
     }
     __syncthreads();
     const float rc2 = kp.e.wcaCutoff * kp.e.wcaCutoff;
     for (uint32_t s = s0 + threadIdx.x; s < s1; s += blockDim.x) {
         const uint32_t me = a.ids[slot0 + (s - s0)] - idBase, cell = a.hash[me];
-        const float4 R = load4(a.pos, me);
         a.sCell[slot0 + (s - s0)] = cell;
-        a.sPos[slot0 + (s - s0)] = R;
         int gx, gy, gz;
         cell_xyz(kp, cell - cellBase, gx, gy, gz);
-        const f3 r = mk(R);
+        const f3 r = mk(load4(a.sPos, slot0 + (s - s0)));
         uint32_t fil, ch, x0, x1, b0, b1;
         worm_of(kp, me, fil, ch);
         row_pieces(uint32_t(gx), Gx, x0, x1, b0, b1);
@@ -192,17 +213,18 @@ __device__ __forceinline__ void rows_in_memory(const KP &kp, const RowsArgs &a, 
         for (uint32_t yi = 0; yi < 3u; ++yi) {
             const uint32_t y = uint32_t(gy) - y0 + yi, row = y * Gx;  // staged: the one below the own rows first
             const bool mine = y >= 1u && y <= own;
-            const uint32_t *ids = y == 0u ? lo + N : (mine ? a.ids + slot0 - s0 : hi + N - s1);
-            const uint32_t base = mine ? idBase : 0u;
-            for (uint32_t k = 0; k < 3u; ++k) {
-                const uint32_t d = row + (x0 + k < x1 ? x0 + k : b0 + k - (x1 - x0));
+            const float4 *rec = mine ? a.sPos + slot0 - s0 : sp.pos + (y == 0u ? lo : hi - s1);
+            // the row's three cells in one run, or in two across the wrap
+            for (uint32_t k = 0; k < 2u; ++k) {
+                const uint32_t z = cnt[row + (k ? b1 : x1)];
 #pragma unroll 2
-                for (uint32_t u = cnt[d], z = cnt[d + 1u]; u < z; ++u) {
-                    const uint32_t j = ids[u] - base;
-                    uint32_t fil2, ch2;
-                    worm_of(kp, j, fil2, ch2);
-                    float4 P = load4(a.pos, j);
-                    P.w = __uint_as_float(fil2);
+                for (uint32_t u = cnt[row + (k ? b0 : x0)]; u < z; ++u) {
+                    float4 P = load4(rec, u);
+                    if (mine) {
+                        uint32_t fil2, ch2;
+                        worm_of(kp, a.ids[slot0 + (u - s0)] - idBase, fil2, ch2);
+                        P.w = __uint_as_float(fil2);
+                    }
                     acc += wca_term_masked(kp, r, fil, rc2, P);
                 }
             }
@@ -215,9 +237,9 @@ __device__ __forceinline__ void rows_in_memory(const KP &kp, const RowsArgs &a, 
 // Rows [y0, y0 + rows) of one system: N beads whose arrays hash, pos, force
 // start at its first bead; ids, sCell and sPos (indexed by sorted slot) and
 // off (by cell) at its own first entries; bead ids, cells and slots of the
-// system are written with idBase, cellBase and slotBase added.  spill(): scratch
-// of four words a bead (an argument of the launch more took 0.1 us: it has
-// its place behind the worms' words).
+// system are written with idBase, cellBase and slotBase added.  spill(): the
+// launch's scratch (an argument of the launch more took 0.1 us: it has its
+// place behind the worms' words).
 template <int T, typename Spill>
 __device__ __forceinline__ void rows_body(const KP &kp, const RowsArgs &a, uint32_t N, uint32_t idBase,
                                           uint32_t cellBase, uint32_t slotAdd, uint32_t y0, uint32_t rows,
@@ -316,7 +338,7 @@ __device__ __forceinline__ void rows_body(const KP &kp, const RowsArgs &a, uint3
     for (uint32_t c = t; c < own * Gx; c += T) a.off[hOwn + c] = slotBase + cnt[Gx + c] - s0;
     if (y0 + own == Gy && t == 0) a.off[C] = slotAdd + N;
     if (m > cap) {
-        rows_in_memory(kp, a, spill(), N, idBase, cellBase, slotBase - slotAdd, y0, own, cnt, cur, words, bead_of, local);
+        rows_in_memory(kp, a, spill(), slotAdd, N, idBase, cellBase, slotBase - slotAdd, y0, own, cnt, cur, words, bead_of, local);
         return;
     }
     auto place = [&](uint32_t id, uint32_t d) {
@@ -371,7 +393,7 @@ __global__ __launch_bounds__(kRowsBlock) void k_rows(RowsArgs a, uint32_t N, uin
                                                      uint32_t maxCells, KP kp) {
     extern __shared__ __align__(16) unsigned char smem[];
     const uint32_t b = xcd_contiguous(blockIdx.x, gridDim.x);
-    rows_body<kRowsBlock>(kp, a, N, 0u, 0u, 0u, b * rows, rows, cap, maxCells, smem, [&] { return a.worms + N; });
+    rows_body<kRowsBlock>(kp, a, N, 0u, 0u, 0u, b * rows, rows, cap, maxCells, smem, [&] { return rows_spill(a.worms, N); });
 }
 
 // the same of every replica of a batch: a workgroup belongs to one replica
@@ -389,7 +411,7 @@ __global__ __launch_bounds__(kRowsBlock) void k_rows_batch(BatchArrays a, const 
     rows_body<kRowsBlock>(rep.kp, x, rep.numBeads, b0, c0, b0, (b - rep.rowBlock) * rep.rows, rep.rows, cap, maxCells,
                           smem, [&] {
                               const BatchRep &last = reps[R - 1u];
-                              return a.wormRows + last.beadOffset + last.numBeads + 4u * uint64_t(b0);
+                              return rows_spill(a.wormRows, last.beadOffset + last.numBeads);
                           });
 }
 
