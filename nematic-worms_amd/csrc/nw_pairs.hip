@@ -11,8 +11,8 @@
 // Measured at 96,000 beads, 64 x 64 x 32 cells: 86 -> 23.7 us against one lane a
 // bead (22,600 instructions of unrolled walk, nine divisions a candidate); at
 // 30,000 beads through the reference's tables 80 -> 12.5 us.  What bounds it now
-// is the issue of some 1,000 VALU a wavefront (8 beads), a fifth of them exact
-// square roots and quotients.
+// is the issue of some 950 VALU a wavefront (8 beads), exact square roots and
+// quotients among them.
 #include "nw_internal.hpp"
 #include "nw_pair.hpp"
 #include "nw_rules.hpp"
